@@ -15,6 +15,7 @@ namespace alpha_moe {
 namespace {
 
 constexpr int kAlignSeg = 1024;        // routing slots per workgroup of the histogram and placement kernels
+constexpr int kAlignSmall = 4096;      // most routing slots one workgroup aligns by itself (9 us near there; two launches: 13)
 constexpr int kAlignMaxExperts = 4096;
 
 // ---- quantisation ------------------------------------------------------------------------------------------
@@ -68,158 +69,243 @@ __global__ __launch_bounds__(256) void quant_group128_kernel(const T *__restrict
 }
 
 // ---- alignment ---------------------------------------------------------------------------------------------
-// Exclusive prefix sum over `n` values held in LDS (n <= kAlignMaxExperts), in place; returns the total.
-// Every thread of the workgroup calls it.
-__device__ int block_exclusive_scan(int *vals, int n, int *partial /* [blockDim.x + 1] */)
+// A stable counting sort of the routing slots by expert.  What bounds it is latency: a few hundred KiB of integers, so
+// everything serial counts.  A wavefront ranks 64 consecutive slots among the equal experts of its chunk with one ballot
+// per bit of the expert id (same_expert) - a loop over the chunk's distinct experts, ~60 LDS round trips for 64 slots
+// of 257 experts, is what took most of 398 us for 2997 slots and of 193 us for 73 728 - and every wavefront counts and
+// places a run of slots of its own behind cursors of its own.  MI355X, kernel trace, 257 experts: 9 us for 2997 slots,
+// 17 us (two launches) for 73 728; nine slots take 5.3 us (8.1 with a serial scan over the experts).
+typedef unsigned long long lanes_t;
+
+// The lanes of this wavefront whose slot has the same expert as this lane's (e < 0: no slot, no lanes); all 64 lanes
+// call it.
+__device__ __forceinline__ lanes_t same_expert(int e, int id_bits)
 {
+    lanes_t same = __ballot(e >= 0);
+    for (int b = 0; b < id_bits; b++) {
+        const bool set = (e >> b) & 1;
+        const lanes_t with = __ballot(set);
+        same &= set ? with : ~with;
+    }
+    return e >= 0 ? same : 0;
+}
+
+__device__ __forceinline__ int expert_of_slot(const int32_t *ids, int i, int end, int E)
+{
+    const int e = i < end ? ids[i] : -1;
+    return e < E ? e : -1;
+}
+
+__device__ __forceinline__ lanes_t lanes_below() { return (1ull << (threadIdx.x & 63)) - 1ull; }
+
+// LDS accesses of one wavefront complete in order; this keeps the compiler to the written order
+__device__ __forceinline__ void lds_order()
+{
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// counts[e] += slots of expert e in ids[lo, hi).  One wavefront, its own counters.
+__device__ __forceinline__ void count_run(const int32_t *ids, int lo, int hi, int E, int id_bits, uint16_t *counts)
+{
+    for (int base = lo; base < hi; base += 64) {
+        const int e = expert_of_slot(ids, base + (threadIdx.x & 63), hi, E);
+        const lanes_t same = same_expert(e, id_bits);
+        if (e >= 0 && (same & lanes_below()) == 0) counts[e] += (uint16_t)__builtin_popcountll(same);
+        lds_order();
+    }
+}
+
+// sorted_ids[start[e] + cursor[e] ...] = the slots of expert e in ids[lo, hi), in order.  One wavefront, its own cursors.
+__device__ __forceinline__ void place_run(const int32_t *ids, int lo, int hi, int E, int id_bits, const int *start,
+                                          uint16_t *cursor, int32_t *sorted_ids)
+{
+    for (int base = lo; base < hi; base += 64) {
+        const int i = base + (threadIdx.x & 63);
+        const int e = expert_of_slot(ids, i, hi, E);
+        const lanes_t same = same_expert(e, id_bits);
+        const int rank = __builtin_popcountll(same & lanes_below());
+        const int at = e >= 0 ? cursor[e] : 0;
+        lds_order();
+        if (e >= 0) {
+            sorted_ids[start[e] + at + rank] = i;
+            if (rank == 0) cursor[e] = (uint16_t)(at + __builtin_popcountll(same));
+        }
+        lds_order();
+    }
+}
+
+// cursors[w][e] of the n_waves wavefronts: counts -> exclusive prefix over the wavefronts; returns the sum
+__device__ __forceinline__ int prefix_over_waves(uint16_t *cursors, int E, int e, int n_waves)
+{
+    int run = 0;
+    for (int w = 0; w < n_waves; w++) {
+        const int t = cursors[w * E + e];
+        cursors[w * E + e] = (uint16_t)run;
+        run += t;
+    }
+    return run;
+}
+
+// Exclusive prefix sum over the n values of LDS array `vals`, in place; returns their sum.  All threads call it.
+__device__ int block_exclusive_scan(int *vals, int n, int *wave_sums /* [blockDim.x / 64] */)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
     const int per = (n + blockDim.x - 1) / blockDim.x;
-    const int lo = threadIdx.x * per, hi = lo + per < n ? lo + per : n;
+    const int lo = min((int)threadIdx.x * per, n), hi = min(lo + per, n);
     int sum = 0;
     for (int i = lo; i < hi; i++) sum += vals[i];
-    partial[threadIdx.x] = sum;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int run = 0;
-        for (unsigned i = 0; i < blockDim.x; i++) {
-            const int t = partial[i];
-            partial[i] = run;
-            run += t;
-        }
-        partial[blockDim.x] = run;
+    int incl = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int t = __shfl_up(incl, d);
+        if (lane >= d) incl += t;
     }
+    if (lane == 63) wave_sums[wave] = incl;
     __syncthreads();
-    int run = partial[threadIdx.x];
+    int run = incl - sum, total = 0;
+    for (int w = 0; w < n_waves; w++) {
+        const int t = wave_sums[w];
+        if (w < wave) run += t;
+        total += t;
+    }
     for (int i = lo; i < hi; i++) {
         const int t = vals[i];
         vals[i] = run;
         run += t;
     }
     __syncthreads();
-    return partial[blockDim.x];
+    return total;
 }
 
-// Stable placement of one wavefront's 64 consecutive slots: lanes with the same expert take consecutive positions
-// in lane order behind cursor[expert]; the cursor advances by their number.  All 64 lanes call it (e < 0: no slot).
-__device__ __forceinline__ void place_chunk(int e, int flat_id, int *cursor, int32_t *sorted_ids)
+__device__ __forceinline__ int pad_to(int v, int block_size) { return (v + block_size - 1) / block_size * block_size; }
+
+// expert_ids and the padded total from the starts of the experts' padded segments (total behind the last one): workgroup
+// `part` of `parts` writes its share.
+__device__ void write_blocks(const int *start, int E, int block_size, int total, int32_t *expert_ids, int n_blocks,
+                             int32_t *ntpp, int part, int parts)
 {
-    const int lane = threadIdx.x & 63;
-    unsigned long long todo = __ballot(e >= 0);
-    while (todo) {
-        const int leader_lane = __builtin_ctzll(todo);
-        const int leader = __shfl(e, leader_lane);
-        const unsigned long long same = __ballot(e == leader) & todo;
-        if (e == leader) {
-            const int rank = __builtin_popcountll(same & ((1ull << lane) - 1));
-            sorted_ids[cursor[leader] + rank] = flat_id;
+    const int tid = part * blockDim.x + threadIdx.x, stride = parts * blockDim.x;
+    const int used = total / block_size;
+    for (int b = tid; b < n_blocks; b += stride) {
+        int e = -1;
+        if (b < used) {   // the last expert whose segment starts at or before the block (empty segments start there too)
+            int lo = 0, hi = E;
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (start[mid] <= b * block_size) lo = mid;
+                else hi = mid;
+            }
+            e = lo;
         }
-        __builtin_amdgcn_wave_barrier();
-        if (lane == leader_lane) cursor[leader] += __builtin_popcountll(same);
-        __builtin_amdgcn_wave_barrier();
-        todo &= ~same;
+        expert_ids[b] = e;
     }
+    if (tid == 0) ntpp[0] = total;
 }
 
-// Fills expert_ids and the padded total from the experts' padded segment starts (`start`, exclusive scan of `padded`).
-__device__ void write_blocks(const int *start, const int *padded, int E, int block_size, int total, int32_t *expert_ids,
-                             int n_blocks, int32_t *ntpp)
+__device__ __forceinline__ void fill_sentinel(int32_t *sorted_ids, int sorted_num, int numel, int tid, int stride)
 {
-    for (int e = threadIdx.x; e < E; e += blockDim.x)
-        for (int b = start[e] / block_size, end = (start[e] + padded[e]) / block_size; b < end && b < n_blocks; b++)
-            expert_ids[b] = e;
-    for (int b = total / block_size + threadIdx.x; b < n_blocks; b += blockDim.x) expert_ids[b] = -1;
-    if (threadIdx.x == 0) ntpp[0] = total;
+    // 16 bytes per store from the first aligned element on
+    const int head = min((int)((0u - (unsigned)(reinterpret_cast<uintptr_t>(sorted_ids) >> 2)) & 3u), sorted_num);
+    const int quads = (sorted_num - head) >> 2;
+    v4i *body = reinterpret_cast<v4i *>(sorted_ids + head);
+    for (int i = tid; i < quads; i += stride) body[i] = (v4i){numel, numel, numel, numel};
+    for (int i = tid; i < head; i += stride) sorted_ids[i] = numel;
+    for (int i = head + 4 * quads + tid; i < sorted_num; i += stride) sorted_ids[i] = numel;
 }
 
-// One workgroup does everything: up to a few thousand slots (decode).
-__global__ __launch_bounds__(256) void align_small_kernel(const int32_t *__restrict__ ids, int numel, int E, int block_size,
-                                                          int32_t *sorted_ids, int sorted_num, int32_t *expert_ids,
-                                                          int n_blocks, int32_t *ntpp)
+// One workgroup does everything (up to kAlignSmall slots).  n_waves of its wavefronts count and place `run` slots each.
+__global__ __launch_bounds__(1024) void align_small_kernel(const int32_t *__restrict__ ids, int numel, int E, int id_bits,
+                                                           int block_size, int32_t *sorted_ids, int sorted_num,
+                                                           int32_t *expert_ids, int n_blocks, int32_t *ntpp, int n_waves,
+                                                           int run)
 {
-    extern __shared__ int lds[];   // [E] counts -> cursors | [E] padded | [257] scan partials
-    int *cnt = lds, *padded = lds + E, *partial = lds + 2 * E;
-    for (int i = threadIdx.x; i < E; i += blockDim.x) cnt[i] = 0;
-    for (int i = threadIdx.x; i < sorted_num; i += blockDim.x) sorted_ids[i] = numel;
+    extern __shared__ __attribute__((aligned(16))) int lds[];   // [E] starts | [16] | [n_waves][E] cursors (16 bit)
+    int *start = lds, *wave_sums = lds + E;
+    uint16_t *cursors = reinterpret_cast<uint16_t *>(lds + E + 16);
+    const int wave = threadIdx.x >> 6;
+    for (int i = threadIdx.x; i < (n_waves * E + 1) / 2; i += blockDim.x) reinterpret_cast<int *>(cursors)[i] = 0;
+    fill_sentinel(sorted_ids, sorted_num, numel, threadIdx.x, blockDim.x);
     __syncthreads();
-    for (int i = threadIdx.x; i < numel; i += blockDim.x) {
-        const int e = ids[i];
-        if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
-    }
+    const int lo = wave * run, hi = min(lo + run, numel);
+    if (wave < n_waves) count_run(ids, lo, hi, E, id_bits, cursors + wave * E);
     __syncthreads();
-    for (int i = threadIdx.x; i < E; i += blockDim.x) {
-        padded[i] = (cnt[i] + block_size - 1) / block_size * block_size;
-        cnt[i] = padded[i];
-    }
+    for (int e = threadIdx.x; e < E; e += blockDim.x) start[e] = pad_to(prefix_over_waves(cursors, E, e, n_waves), block_size);
     __syncthreads();
-    const int total = block_exclusive_scan(cnt, E, partial);   // cnt: start of each expert's padded segment
-    write_blocks(cnt, padded, E, block_size, total, expert_ids, n_blocks, ntpp);
-    __syncthreads();   // the sentinel fill is done and write_blocks has read the starts before the cursors move
-    if (threadIdx.x < 64) {
-        for (int base = 0; base < numel; base += 64) {
-            const int i = base + threadIdx.x;
-            int e = i < numel ? ids[i] : -1;
-            if (e >= E) e = -1;
-            place_chunk(e, i, cnt, sorted_ids);
-        }
-    }
+    const int total = block_exclusive_scan(start, E, wave_sums);
+    // (the barriers above have also completed the sentinel fill before any slot is placed)
+    if (wave < n_waves) place_run(ids, lo, hi, E, id_bits, start, cursors + wave * E, sorted_ids);
+    write_blocks(start, E, block_size, total, expert_ids, n_blocks, ntpp, 0, 1);
 }
 
-// Large inputs, pass 1: per-segment expert histograms; also the sentinel fill.
+// Larger inputs, pass 1: one workgroup per segment of kAlignSeg slots writes the segment's expert histogram (16-bit
+// counts, two per word); also the sentinel fill.
 __global__ __launch_bounds__(256) void align_hist_kernel(const int32_t *__restrict__ ids, int numel, int E, int *hist,
-                                                         int32_t *sorted_ids, int sorted_num)
+                                                         int words, int32_t *sorted_ids, int sorted_num)
 {
-    extern __shared__ int lds[];
-    for (int i = threadIdx.x; i < E; i += blockDim.x) lds[i] = 0;
+    extern __shared__ int lds[];   // [words]
+    for (int i = threadIdx.x; i < words; i += blockDim.x) lds[i] = 0;
     __syncthreads();
-    const int lo = blockIdx.x * kAlignSeg, hi = lo + kAlignSeg < numel ? lo + kAlignSeg : numel;
+    const int lo = blockIdx.x * kAlignSeg, hi = min(lo + kAlignSeg, numel);
     for (int i = lo + threadIdx.x; i < hi; i += blockDim.x) {
         const int e = ids[i];
-        if (e >= 0 && e < E) atomicAdd(&lds[e], 1);
+        if (e >= 0 && e < E) atomicAdd(&lds[e >> 1], 1 << (16 * (e & 1)));
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < E; i += blockDim.x) hist[(size_t)blockIdx.x * E + i] = lds[i];
-    const int per = (sorted_num + gridDim.x - 1) / gridDim.x;
-    const int flo = blockIdx.x * per, fhi = flo + per < sorted_num ? flo + per : sorted_num;
-    for (int i = flo + threadIdx.x; i < fhi; i += blockDim.x) sorted_ids[i] = numel;
+    for (int i = threadIdx.x; i < words; i += blockDim.x) hist[(size_t)blockIdx.x * words + i] = lds[i];
+    fill_sentinel(sorted_ids, sorted_num, numel, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 
-// Pass 2 (one workgroup): hist[s][e] becomes the position where segment s starts writing expert e.
-__global__ __launch_bounds__(1024) void align_scan_kernel(int *hist, int n_seg, int E, int block_size, int32_t *expert_ids,
-                                                          int n_blocks, int32_t *ntpp)
+// Pass 2, one workgroup per segment: every workgroup adds the histograms up itself (columns of two experts, sixteen
+// segments in flight; a third launch of one workgroup for the sums took 17 - 42 us), scans the padded totals and places
+// its segment, each of its four wavefronts a quarter of it.
+__global__ __launch_bounds__(256) void align_place_kernel(const int32_t *__restrict__ ids, int numel, int E, int id_bits,
+                                                          int block_size, const int *__restrict__ hist, int words,
+                                                          int32_t *sorted_ids, int32_t *expert_ids, int n_blocks,
+                                                          int32_t *ntpp)
 {
-    extern __shared__ int lds[];   // [E] starts | [E] padded | [1025] scan partials
-    int *start = lds, *padded = lds + E, *partial = lds + 2 * E;
-    for (int e = threadIdx.x; e < E; e += blockDim.x) {
-        int run = 0;
-        for (int s = 0; s < n_seg; s++) {
-            const int t = hist[(size_t)s * E + e];
-            hist[(size_t)s * E + e] = run;
-            run += t;
+    // [2 words] starts | [2 words] slots of earlier segments | [4][E] cursors (16 bit; first the scan's partial sums)
+    extern __shared__ __attribute__((aligned(16))) int lds[];
+    int *start = lds, *before = lds + 2 * words;
+    uint16_t *cursors = reinterpret_cast<uint16_t *>(lds + 4 * words);
+    const int wave = threadIdx.x >> 6, n_seg = gridDim.x, seg = blockIdx.x;
+    for (int c = threadIdx.x; c < words; c += blockDim.x) {
+        int b0 = 0, b1 = 0, t0 = 0, t1 = 0;
+        for (int s0 = 0; s0 < n_seg; s0 += 16) {
+            unsigned v[16];
+#pragma unroll
+            for (int k = 0; k < 16; k++) v[k] = s0 + k < n_seg ? (unsigned)hist[(size_t)(s0 + k) * words + c] : 0u;
+#pragma unroll
+            for (int k = 0; k < 16; k++) {
+                const int c0 = v[k] & 0xffffu, c1 = v[k] >> 16;
+                t0 += c0;
+                t1 += c1;
+                if (s0 + k < seg) {
+                    b0 += c0;
+                    b1 += c1;
+                }
+            }
         }
-        padded[e] = (run + block_size - 1) / block_size * block_size;
-        start[e] = padded[e];
+        start[2 * c] = pad_to(t0, block_size);
+        start[2 * c + 1] = pad_to(t1, block_size);
+        before[2 * c] = b0;
+        before[2 * c + 1] = b1;
     }
     __syncthreads();
-    const int total = block_exclusive_scan(start, E, partial);
-    write_blocks(start, padded, E, block_size, total, expert_ids, n_blocks, ntpp);
-    for (int e = threadIdx.x; e < E; e += blockDim.x)
-        for (int s = 0; s < n_seg; s++) hist[(size_t)s * E + e] += start[e];
-}
-
-// Pass 3: one wavefront per segment places its slots in order.
-__global__ __launch_bounds__(64) void align_place_kernel(const int32_t *__restrict__ ids, int numel, int E, const int *hist,
-                                                         int32_t *sorted_ids)
-{
-    extern __shared__ int lds[];   // [E] cursors
-    for (int i = threadIdx.x; i < E; i += 64) lds[i] = hist[(size_t)blockIdx.x * E + i];
-    __builtin_amdgcn_wave_barrier();
+    const int total = block_exclusive_scan(start, E, lds + 4 * words);
+    for (int i = threadIdx.x; i < 2 * E; i += blockDim.x) reinterpret_cast<int *>(cursors)[i] = 0;
+    write_blocks(start, E, block_size, total, expert_ids, n_blocks, ntpp, seg, n_seg);
     __syncthreads();
-    const int lo = blockIdx.x * kAlignSeg, hi = lo + kAlignSeg < numel ? lo + kAlignSeg : numel;
-    for (int base = lo; base < hi; base += 64) {
-        const int i = base + threadIdx.x;
-        int e = i < hi ? ids[i] : -1;
-        if (e >= E) e = -1;
-        place_chunk(e, i, lds, sorted_ids);
+    constexpr int kRun = kAlignSeg / 4;
+    const int lo = seg * kAlignSeg + wave * kRun, hi = min(lo + kRun, numel);
+    count_run(ids, lo, hi, E, id_bits, cursors + wave * E);
+    __syncthreads();
+    for (int e = threadIdx.x; e < E; e += blockDim.x) {
+        prefix_over_waves(cursors, E, e, 4);
+        start[e] += before[e];
     }
+    __syncthreads();
+    place_run(ids, lo, hi, E, id_bits, start, cursors + wave * E, sorted_ids);
 }
 
 }  // namespace
@@ -264,19 +350,27 @@ extern "C" int alpha_moe_moe_align_block_size(const int32_t *topk_ids, int numel
         return ALPHA_MOE_ERR_SHAPE;
     hipStream_t hs = static_cast<hipStream_t>(stream);
     const int E = num_experts;
-    if (numel <= 4 * kAlignSeg) {
-        hipLaunchKernelGGL(align_small_kernel, dim3(1), dim3(256), (2 * E + 257) * sizeof(int), hs, topk_ids, numel, E,
-                           block_size, sorted_token_ids, sorted_num, expert_ids, n_blocks, num_tokens_post_padded);
+    int id_bits = 0;
+    while ((1 << id_bits) < E) id_bits++;
+    if (numel <= kAlignSmall) {
+        // as many wavefronts as there are chunks of 64 slots, and no more than have room for their cursors
+        int n_waves = (numel + 63) / 64;
+        if (n_waves > 16) n_waves = 16;
+        const int room = (40 << 10) / (E * (int)sizeof(uint16_t));
+        if (n_waves > room) n_waves = room;
+        const int run = ((numel + n_waves - 1) / n_waves + 63) / 64 * 64;
+        const size_t lds = (E + 16) * sizeof(int) + ((size_t)n_waves * E + 1) / 2 * sizeof(int);
+        hipLaunchKernelGGL(align_small_kernel, dim3(1), dim3(1024), lds, hs, topk_ids, numel, E, id_bits, block_size,
+                           sorted_token_ids, sorted_num, expert_ids, n_blocks, num_tokens_post_padded, n_waves, run);
         return hipGetLastError() == hipSuccess ? ALPHA_MOE_OK : ALPHA_MOE_ERR_LAUNCH;
     }
     if (!workspace || workspace_bytes < alpha_moe_align_workspace_bytes(numel, E)) return ALPHA_MOE_ERR_WORKSPACE;
-    const int n_seg = (numel + kAlignSeg - 1) / kAlignSeg;
+    const int n_seg = (numel + kAlignSeg - 1) / kAlignSeg, words = (E + 1) / 2;
     int *hist = static_cast<int *>(workspace);
-    hipLaunchKernelGGL(align_hist_kernel, dim3(n_seg), dim3(256), E * sizeof(int), hs, topk_ids, numel, E, hist,
+    hipLaunchKernelGGL(align_hist_kernel, dim3(n_seg), dim3(256), words * sizeof(int), hs, topk_ids, numel, E, hist, words,
                        sorted_token_ids, sorted_num);
-    hipLaunchKernelGGL(align_scan_kernel, dim3(1), dim3(1024), (2 * E + 1025) * sizeof(int), hs, hist, n_seg, E,
-                       block_size, expert_ids, n_blocks, num_tokens_post_padded);
-    hipLaunchKernelGGL(align_place_kernel, dim3(n_seg), dim3(64), E * sizeof(int), hs, topk_ids, numel, E, hist,
-                       sorted_token_ids);
+    const size_t lds = (4 * words + (2 * E > 16 ? 2 * E : 16)) * sizeof(int);   // 64 KiB at kAlignMaxExperts
+    hipLaunchKernelGGL(align_place_kernel, dim3(n_seg), dim3(256), lds, hs, topk_ids, numel, E, id_bits, block_size, hist,
+                       words, sorted_token_ids, expert_ids, n_blocks, num_tokens_post_padded);
     return hipGetLastError() == hipSuccess ? ALPHA_MOE_OK : ALPHA_MOE_ERR_LAUNCH;
 }

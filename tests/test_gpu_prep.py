@@ -47,6 +47,34 @@ def test_align_matches_oracle_bit_for_bit(M, top_k, E, block):
     assert torch.equal(s_ids.cpu(), r_ids)
 
 
+@pytest.mark.parametrize("numel,E,block", [(1, 1, 8), (63, 2, 8), (65, 3, 128), (1025, 1, 16), (4096, 512, 56),
+                                            (4096, 4096, 8), (4097, 4096, 8), (4097, 1, 128), (5120, 257, 64),
+                                            (40000, 3, 8), (81920, 512, 96)])
+def test_align_at_the_edges_of_its_runs_and_segments(numel, E, block):
+    """one chunk, one segment and their remainders; one workgroup (up to 4096 slots) and several; an even and an odd number
+    of experts, one, and the most there can be; slots without an expert among them"""
+    from alpha_moe_python import prep_hip
+    g = torch.Generator().manual_seed(numel + E)
+    ids = torch.randint(-1, E + 1, (numel, 1), generator=g).to(torch.int32)
+    ids[: numel // 3] = E // 2          # a hot expert over several chunks
+    print(f"case align numel={numel} E={E} block={block}", flush=True)
+    s_ids, e_ids, total = prep_hip.moe_align_block_size(ids.to(DEV), block, E)
+    torch.cuda.synchronize()
+    flat = ids.flatten().long()
+    keep = torch.nonzero((flat >= 0) & (flat < E)).flatten()
+    r_ids, r_e = torch.full_like(s_ids.cpu(), numel), torch.full_like(e_ids.cpu(), -1)
+    at = 0
+    for e in torch.unique(flat[keep]).tolist():
+        slots = keep[flat[keep] == e]
+        r_ids[at:at + len(slots)] = slots.to(torch.int32)
+        padded = (len(slots) + block - 1) // block * block
+        r_e[at // block:(at + padded) // block] = e
+        at += padded
+    assert total.item() == at
+    assert torch.equal(e_ids.cpu(), r_e)
+    assert torch.equal(s_ids.cpu(), r_ids)
+
+
 def test_align_drops_slots_with_an_expert_out_of_range():
     from alpha_moe_python import prep_hip
     ids = torch.tensor([[0, 3], [7, -1], [9, 3]], dtype=torch.int32)
