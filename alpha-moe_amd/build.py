@@ -31,6 +31,7 @@ HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
 HIP_SOURCES = {
     "moe_api.hip": [],
     "moe_direct.hip": [],
+    "moe_small.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "moe_stream.hip": [],
     "moe_tile.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "moe_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],

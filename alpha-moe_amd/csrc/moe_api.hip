@@ -31,7 +31,7 @@ void load_tunables_once()
             const char *e = getenv(t.name);
             if (!e) continue;
             if (!strcmp(t.name, "ALPHA_MOE_PATH"))
-                t.value = !strcmp(e, "direct") ? 1 : !strcmp(e, "stream") ? 2 : !strcmp(e, "tile") ? 3 : !strcmp(e, "wide") ? 4 : kTunableUnset;
+                t.value = !strcmp(e, "direct") ? 1 : !strcmp(e, "stream") ? 2 : !strcmp(e, "tile") ? 3 : !strcmp(e, "wide") ? 4 : !strcmp(e, "small") ? 5 : kTunableUnset;
             else
                 t.value = atoi(e);
         }
@@ -40,9 +40,9 @@ void load_tunables_once()
     (void)done;
 }
 
-enum Path { kDirect, kStream, kTile, kWide };
+enum Path { kDirect, kStream, kTile, kWide, kSmall };
 
-// Streaming kernel for row blocks of at most 32 rows (decode); above that (prefill) warp_n picks the token tiles a
+// At most 16 tokens: small kernels.  Streaming kernel for row blocks of at most 32 rows (decode); above that (prefill) warp_n picks the token tiles a
 // wavefront multiplies per step: 8 -> wide kernel (macro blocks of 256 rows), 4 -> tile kernel (one row block).  The
 // direct kernel is the fallback for shapes none of them takes.
 Path choose_path(int top_k, int M, int K, int N, int E, int sorted_num, int block_m, int warp_n)
@@ -55,6 +55,7 @@ Path choose_path(int top_k, int M, int K, int N, int E, int sorted_num, int bloc
     if (f == 2 && s_ok) return kStream;
     if (f == 3 && t_ok) return kTile;
     if (f == 4 && w_ok) return kWide;
+    if ((f == 0 || f == 5) && small_supported(top_k, M, K, N, block_m)) return kSmall;
     if (s_ok) return kStream;
     if (w_ok && (warp_n == 8 || !t_ok)) return kWide;
     if (t_ok) return kTile;
@@ -112,7 +113,9 @@ extern "C" size_t alpha_moe_workspace_bytes(int top_k, int M, int K, int N, int 
     const size_t wide = wide_supported(top_k, M, K, N, num_experts, sorted_num, block_m)
                             ? wide_workspace_bytes(top_k, M, K, N, num_experts, sorted_num, block_m)
                             : 0;
+    const size_t small = small_supported(top_k, M, K, N, block_m) ? small_workspace_bytes(top_k, M, N) : 0;
     size_t m = direct > stream ? direct : stream;
+    m = m > small ? m : small;
     m = m > tile ? m : tile;
     return m > wide ? m : wide;
 }
@@ -153,7 +156,9 @@ int run_fused_moe(const uint8_t *x, const float *x_scale, const uint8_t *w, cons
     hipStream_t hs = static_cast<hipStream_t>(stream);
     hipError_t err;
     const Path path = choose_path(top_k, M, K, N, num_experts, sorted_num, block_m, warp_n);
-    if (path == kStream) {
+    if (path == kSmall) {
+        err = launch_small(p, workspace, hs);
+    } else if (path == kStream) {
         err = launch_stream(p, warp_n, stages, workspace, hs);
     } else if (path == kWide) {
         err = launch_wide(p, stages, workspace, hs);

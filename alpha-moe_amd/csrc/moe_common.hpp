@@ -254,7 +254,7 @@ __device__ __noinline__ inline void spin_all_ge(const int *addr, int count, int 
 // alpha_moe_set_tunable(): no launch ever calls getenv.  A value of kTunableUnset means "the library decides".
 constexpr int kTunableUnset = INT32_MIN;
 enum Tunable {
-    kTunPath,          // ALPHA_MOE_PATH: 1 direct, 2 stream, 3 tile (where the family applies)
+    kTunPath,          // ALPHA_MOE_PATH: 1 direct, 2 stream, 3 tile, 4 wide, 5 small (where the family applies)
     kTunStrictQueue,   // ALPHA_MOE_STRICT_QUEUE: 0 hands the first gridDim.x items of the streaming kernel out by index
     kTunKbpi,          // ALPHA_MOE_KBPI: K blocks per UP item of the streaming kernel
     kTunTpi,           // ALPHA_MOE_TPI: 16-column tiles per DOWN item of the streaming kernel
@@ -277,6 +277,11 @@ int tunable(Tunable which, int dflt);   // the override if one is set, else dflt
 hipError_t launch_zero_acc(const MoeParams &p, hipStream_t stream);
 hipError_t launch_direct(const MoeParams &p, int warp_n, int stages, hipStream_t stream);
 hipError_t launch_finalize(const MoeParams &p, hipStream_t stream);   // out = bf16(out + acc), or bf16(acc)
+
+// Two launches for at most 16 tokens: UP work split over w1 rows, DOWN work over output columns; block_m <= 32.
+bool small_supported(int top_k, int M, int K, int N, int block_m);
+size_t small_workspace_bytes(int top_k, int M, int N);
+hipError_t launch_small(const MoeParams &p, void *workspace, hipStream_t stream);
 
 // Persistent work-queue kernel for decode-sized batches (block_m <= 32 and bounded sizes): split-K up items ->
 // SwiGLU/requant -> column-slab down items -> per-token reduction, chained through counters in the workspace.

@@ -640,6 +640,27 @@ def test_tiny_batches(name, ds_weights, qn_weights):
                            f"{name} M={M} out pre-filled")
 
 
+@pytest.mark.parametrize("M,E,top_k,K,I", [(1, 3, 2, 128, 128),       # one K block: seven wavefronts multiply zeros
+                                            (16, 160, 10, 1152, 256),   # nine K blocks over eight wavefronts; the most rows
+                                            (5, 7, 3, 3712, 384),       # 29 K blocks; parts that end inside a tile
+                                            (16, 40, 10, 2048, 1024),   # eight slices: rows quantised in groups
+                                            (13, 64, 8, 7168, 768),     # the deepest K; two w2 blocks in an output range
+                                            (2, 2, 2, 7168, 128)])
+def test_small_kernel_at_the_edges_of_its_parts(M, E, top_k, K, I):
+    """At most 16 tokens: ranges of intermediate columns of unequal tiles, output ranges across scale blocks, several row
+    blocks of one expert (block_m 8), adding and storing, two launches bit for bit, against the oracle."""
+    shape = Shape("small", E=E, top_k=top_k, K=K, I=I, shared_expert=False, routing="softmax_renorm", scaling_factor=1.3)
+    P = make_problem(make_weights(shape, device=DEV, seed=M + K), M, seed=9)
+    refs = oracle_variants(P)
+    for knobs in ((16, 32, 8, 4), (8, 64, 4, 2), (32, 32, 8, 1)):
+        print(f"case small M={M} E={E} K={K} I={I} knobs {knobs}", flush=True)
+        got = run_op(P, *knobs, via="c_abi")
+        assert_parity_rows(got, refs, f"small {knobs}")
+        assert torch.equal(got, run_op(P, *knobs, via="c_abi"))
+        junk = torch.full((M, K), float("nan"), dtype=torch.bfloat16, device=DEV)
+        assert torch.equal(run_op(P, *knobs, out=junk, via="c_abi", store=True), got)
+
+
 def test_an_up_sum_on_a_bf16_boundary(ds_weights):
     """The one problem on which the device and the oracle disagree by more than the bar (DeepSeek-V3 shard, M=2): the
     disagreement is the oracle's own discontinuity.  Seventeen of the eighteen (token, slot) rows agree; in the shared
