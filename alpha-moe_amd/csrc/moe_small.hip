@@ -349,12 +349,18 @@ __device__ __forceinline__ uint2 quantise_row(const v4i raw, float *scale)
     float m = kAmaxFloor;
 #pragma unroll
     for (int i = 0; i < 8; i++) m = fmaxf(m, fabsf(v[i]));
-    const float sa = divide(max_of_16_lanes(m), kFp8Max, 1.0f / kFp8Max);
+    m = max_of_16_lanes(m);
+    // a row with an infinity: its scale is infinite, a finite value over it is 0 and an infinity over it NaN; NaN is clamped
+    // to -448 (as in the other kernels)
+    const bool inf = m == __builtin_inff();
+    const float sa = inf ? m : divide(m, kFp8Max, 1.0f / kFp8Max);
     float r = __builtin_amdgcn_rcpf(sa);
-    r = __builtin_fmaf(__builtin_fmaf(-sa, r, 1.0f), r, r);
-    uint2 o;   // (no value exceeds the row's maximum: nothing to clamp)
-    o.x = pack_fp8x4(divide(v[0], sa, r), divide(v[1], sa, r), divide(v[2], sa, r), divide(v[3], sa, r));
-    o.y = pack_fp8x4(divide(v[4], sa, r), divide(v[5], sa, r), divide(v[6], sa, r), divide(v[7], sa, r));
+    r = inf ? 0.f : __builtin_fmaf(__builtin_fmaf(-sa, r, 1.0f), r, r);
+    const float s = inf ? 0.f : sa;
+    auto code = [&](float a) { return clamp_fp8(divide(a, s, r)); };
+    uint2 o;
+    o.x = pack_fp8x4(code(v[0]), code(v[1]), code(v[2]), code(v[3]));
+    o.y = pack_fp8x4(code(v[4]), code(v[5]), code(v[6]), code(v[7]));
     *scale = sa;
     return o;
 }

@@ -661,6 +661,28 @@ def test_small_kernel_at_the_edges_of_its_parts(M, E, top_k, K, I):
         assert torch.equal(run_op(P, *knobs, out=junk, via="c_abi", store=True), got)
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("nan"), 3e38])
+def test_small_kernel_requantises_what_is_not_finite_like_the_streaming_kernel(bad):
+    """A token whose up/gate sums are infinite, not a number or overflow on the way: NaN and infinite elements in the same
+    places as from the streaming kernel, the other tokens' rows untouched."""
+    shape = Shape("small", E=6, top_k=2, K=512, I=256, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
+    P = make_problem(make_weights(shape, device=DEV, seed=3), 5, seed=4)
+    clean = run_op(P, 16, 32, 8, 4, via="c_abi")
+    P.x_scale = P.x_scale.clone()
+    P.x_scale[2, 1] = bad
+    print(f"case not finite {bad}", flush=True)
+    got = run_op(P, 16, 32, 8, 4, via="c_abi")
+    with tunables(ALPHA_MOE_PATH=2):
+        want = run_op(P, 16, 32, 8, 4, via="c_abi")
+    rest = [0, 1, 3, 4]
+    assert torch.equal(got[rest], clean[rest])
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    finite = torch.isfinite(want)
+    assert torch.equal(torch.sign(got[~finite].nan_to_num(0.)), torch.sign(want[~finite].nan_to_num(0.)))
+    # (two bf16 roundings of sums in another order)
+    assert torch.allclose(got[finite].float(), want[finite].float(), rtol=2 ** -7, atol=float(clean.float().abs().max()) * 1e-2)
+
+
 def test_an_up_sum_on_a_bf16_boundary(ds_weights):
     """The one problem on which the device and the oracle disagree by more than the bar (DeepSeek-V3 shard, M=2): the
     disagreement is the oracle's own discontinuity.  Seventeen of the eighteen (token, slot) rows agree; in the shared
