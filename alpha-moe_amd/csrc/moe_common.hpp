@@ -196,9 +196,8 @@ struct StreamCtl {
     int head;        // streaming kernel: next work item
     int done;        // streaming kernel: workgroups that have left
     int epoch;       // completed launches on this workspace (any kernel family)
-    int pad_e;
-    int fin_done;    // tile kernels: reduce-kernel workgroups that have left
-    int tile_done;   // tile kernel: workgroups that have left
+    int pad_e[2];
+    int tile_done;   // tile kernels: workgroups that have left
     int pad0[2];
     int tile_head[8];   // tile kernel: next work item of each of the eight queues
     int pad1a[16];
@@ -304,12 +303,12 @@ bool wide_supported(int top_k, int M, int K, int N, int E, int sorted_num, int b
 size_t wide_workspace_bytes(int top_k, int M, int K, int N, int E, int sorted_num, int block_m);
 hipError_t launch_wide(const MoeParams &p, int stages, void *workspace, hipStream_t stream);
 
-// out[t] = bf16(out[t] + sum over the token's live slots of y[slot]) (or bf16(sum) when p.overwrite); closes the
-// workspace's launch epoch.  Shared by the tile and wide kernels, which write each (token, slot) row once into y.
+// out[t] = bf16(out[t] + sum over the token's live slots of y[slot]) (or bf16(sum) when p.overwrite).  Runs behind the
+// kernel that wrote the rows and closed the launch epoch.  Shared by the tile and wide kernels, which write each (token, slot) row once into y.
 struct RowsReduce {
     MoeParams p;
     StreamCtl *ctl;
-    const int *live;      // [slots] == epoch + 1 of the control block for rows written in this launch
+    const int *live;      // [slots] == epoch of the control block for rows written in this call
     const uint16_t *y;    // [slots][K] bf16
 };
 hipError_t launch_rows_reduce(const RowsReduce &r, hipStream_t stream);

@@ -534,65 +534,62 @@ __global__ __launch_bounds__(512) void moe_tile_kernel(const TileParams s)
         if (left == (int)gridDim.x - 1) {
             for (int i = 0; i < 8; i++) store_agent(&s.ctl->tile_head[i], 0);
             store_agent(&s.ctl->tile_done, 0);
+            store_agent(&s.ctl->epoch, epoch);   // everybody has read the old one; the reduce kernel compares with this
         }
     }
 }
 
-// out[t] = bf16(out[t] + sum over the token's live slots of y[slot]); the last workgroup to leave closes the epoch.
-// A unit is (token, 2048 columns): a thread owns 8 columns and keeps up to 8 row loads in flight.  Workgroups stride
-// over the units so that the closing counter sees a few thousand arrivals, not one per unit.
-__global__ __launch_bounds__(256) void moe_tile_reduce_kernel(const RowsReduce s, int chunks_per_token, int n_units)
+// out[t] = bf16(out[t] + sum over the token's live slots of y[slot]).
+// A workgroup is (token, 2048 columns): a thread owns 8 columns, and all rows of a token with up to 12 slots are in flight at
+// once.  Bound by HBM: the rows are read once.  Nothing else is waited for: the launch epoch was closed by the
+// kernel that wrote the rows.  (The last of this kernel's workgroups used to close it: arrivals at one counter are served
+// one by one, ~10 ns each, so 4096 workgroups took 41 us whatever they had to read.)
+// MI355X, kernel trace, before and after: Qwen3-Next M=4096 60 -> 38 us, Qwen3-30B M=1024 18 -> 9.7 and M=8192 78 -> 46,
+// DeepSeek shard M=2048 76 -> 61 and M=8192 204 -> 198 (1.18 GB, 6.0 TB/s).  Workgroups that stride over units are slower
+// (M=8192 with 1024 of them: 220 us).
+constexpr int kReduceInFlight = 12;
+__global__ __launch_bounds__(256) void moe_tile_reduce_kernel(const RowsReduce s, int chunks_per_token)
 {
     const MoeParams &p = s.p;
-    const int epoch = (int)((unsigned)s.ctl->epoch + 1u);
+    const int epoch = s.ctl->epoch;   // of the kernel before this one
     // a bounded wait that ran out (in this call's tile kernel or in any earlier launch on this workspace: the word is
     // sticky) means result rows may be missing: the output then says so itself, NaN in every element
     // (an ordinary load: this kernel starts after the tile kernel has ended, and every wavefront asking the memory side
     // for the same word with an agent-scope load cost ~100 us per call)
     const bool poisoned = s.ctl->error != 0;
-    for (int unit = blockIdx.x; unit < n_units; unit += gridDim.x) {
-        const int t = unit / chunks_per_token;
-        const int c = (unit - t * chunks_per_token) * 2048 + threadIdx.x * 8;
-        if (c >= p.K) continue;
-        float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        auto add = [&](const v4i v) {
+    const int t = blockIdx.x / chunks_per_token;
+    const int c = ((int)blockIdx.x - t * chunks_per_token) * 2048 + threadIdx.x * 8;
+    if (c >= p.K) return;
+    float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    auto add = [&](const v4i v) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                sum[2 * i] += __builtin_bit_cast(float, (uint32_t)v[i] << 16);
-                sum[2 * i + 1] += __builtin_bit_cast(float, (uint32_t)v[i] & 0xffff0000u);
-            }
-        };
-        v4i *op = reinterpret_cast<v4i *>(p.out + (size_t)t * p.K + c);
-        v4i prior = {0, 0, 0, 0};
-        if (!p.overwrite) prior = *op;
-        const int *live = s.live + t * p.top_k;
-        const uint16_t *yrow = s.y + (size_t)t * p.top_k * p.K + c;
-        for (int s0 = 0; s0 < p.top_k; s0 += 8) {   // slot order: the sum depends on nothing but the inputs
-            bool on[8];
-            v4i v[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) on[j] = s0 + j < p.top_k && live[s0 + j] == epoch;
-#pragma unroll
-            for (int j = 0; j < 8; j++)
-                if (on[j]) v[j] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(yrow + (size_t)(s0 + j) * p.K));
-#pragma unroll
-            for (int j = 0; j < 8; j++)
-                if (on[j]) add(v[j]);
+        for (int i = 0; i < 4; i++) {
+            sum[2 * i] += __builtin_bit_cast(float, (uint32_t)v[i] << 16);
+            sum[2 * i + 1] += __builtin_bit_cast(float, (uint32_t)v[i] & 0xffff0000u);
         }
-        add(prior);
-        v4i o;
+    };
+    v4i *op = reinterpret_cast<v4i *>(p.out + (size_t)t * p.K + c);
+    v4i prior = {0, 0, 0, 0};
+    if (!p.overwrite) prior = *op;
+    const int *live = s.live + t * p.top_k;
+    const uint16_t *yrow = s.y + (size_t)t * p.top_k * p.K + c;
+    for (int s0 = 0; s0 < p.top_k; s0 += kReduceInFlight) {   // slot order: the sum depends on nothing but the inputs
+        bool on[kReduceInFlight];
+        v4i v[kReduceInFlight];
 #pragma unroll
-        for (int i = 0; i < 4; i++) o[i] = poisoned ? 0x7fc07fc0 : (int)pack_bf16x2(sum[2 * i], sum[2 * i + 1]);
-        *op = o;
+        for (int j = 0; j < kReduceInFlight; j++) on[j] = s0 + j < p.top_k && live[s0 + j] == epoch;
+#pragma unroll
+        for (int j = 0; j < kReduceInFlight; j++)
+            if (on[j]) v[j] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(yrow + (size_t)(s0 + j) * p.K));
+#pragma unroll
+        for (int j = 0; j < kReduceInFlight; j++)
+            if (on[j]) add(v[j]);
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const int left = __hip_atomic_fetch_add(&s.ctl->fin_done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (left == (int)gridDim.x - 1) {
-            __hip_atomic_store(&s.ctl->fin_done, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(&s.ctl->epoch, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-    }
+    add(prior);
+    v4i o;
+#pragma unroll
+    for (int i = 0; i < 4; i++) o[i] = poisoned ? 0x7fc07fc0 : (int)pack_bf16x2(sum[2 * i], sum[2 * i + 1]);
+    *op = o;
 }
 
 size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -732,9 +729,7 @@ hipError_t launch_tile(const MoeParams &p, int stages, void *workspace, hipStrea
 hipError_t launch_rows_reduce(const RowsReduce &r, hipStream_t stream)
 {
     const int chunks = (r.p.K + 2047) / 2048;
-    const int n_units = r.p.M * chunks;
-    hipLaunchKernelGGL(moe_tile_reduce_kernel, dim3((unsigned)(n_units < 4096 ? n_units : 4096)), dim3(256), 0, stream, r,
-                       chunks, n_units);
+    hipLaunchKernelGGL(moe_tile_reduce_kernel, dim3((unsigned)(r.p.M * chunks)), dim3(256), 0, stream, r, chunks);
     return hipGetLastError();
 }
 

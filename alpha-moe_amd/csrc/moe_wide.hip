@@ -1061,6 +1061,7 @@ __global__ __launch_bounds__(512) void moe_wide_kernel(const WideParams s)
         if (left == (int)gridDim.x - 1) {
             for (int i = 0; i < 8; i++) store_agent(&s.ctl->tile_head[i], 0);
             store_agent(&s.ctl->tile_done, 0);
+            store_agent(&s.ctl->epoch, epoch);   // everybody has read the old one; the reduce kernel compares with this
         }
     }
 }

@@ -189,6 +189,21 @@ def test_ragged_small_shapes(M, E, top_k, K, I):
         assert_parity(run_op(P, bm, bn, wn, st), ref, f"{(M, E, top_k, K, I)} knobs {(bm, bn, wn, st)}")
 
 
+@pytest.mark.parametrize("top_k", [1, 12, 13, 25])
+def test_prefill_rows_are_summed_for_any_top_k(top_k):
+    """The sum over a token's rows takes 12 of them at a time, 2048 columns a workgroup: below, at and beyond both."""
+    shape = Shape("t", E=27, top_k=top_k, K=2176, I=128, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
+    W = make_weights(shape, device=DEV, seed=top_k)
+    P = make_problem(W, 70, seed=top_k)
+    ref = oracle_out(P)
+    junk = torch.full((P.M, shape.K), float("nan"), dtype=torch.bfloat16, device=DEV)
+    for knobs in ((48, 64, 4, 3), (64, 32, 8, 2)):   # tile kernel, wide kernel
+        print(f"case rows top_k={top_k} knobs {knobs}", flush=True)
+        for store in (False, True, False):           # one workspace: every call has to see its own rows as live
+            out = junk.clone() if store else None
+            assert_parity(run_op(P, *knobs, out=out, store=store), ref, f"top_k {top_k} {knobs} store {store}")
+
+
 def test_duplicate_experts_and_negative_scales():
     """Duplicate expert ids inside one token's top-k and negative block scales are legal inputs
     (test_moe_correctness.py:42,59-60 of the reference generates both)."""
