@@ -196,20 +196,19 @@ struct StreamCtl {
     int head;        // streaming kernel: next work item
     int done;        // streaming kernel: workgroups that have left
     int epoch;       // completed launches on this workspace (any kernel family)
-    int pad_e[2];
+    int poisoned;    // the epoch of a launch that found `mark` set (for the kernel that sums the rows)
+    int pad_e;
     int tile_done;   // tile kernels: workgroups that have left
     int pad0[2];
     int tile_head[8];   // tile kernel: next work item of each of the eight queues
     int pad1a[16];
-    // a 128-byte line of its own: idle workgroups poll it while the others still fetch items through `head`
-    int down_done;   // streaming kernel: finished DOWN items of this launch (+ kExpiredBit after an expired wait)
-    int error;       // sticky: a bounded wait ran out (word kErrorWord of the workspace); read with the same poll
+    int mark;        // kExpiredBit: one call through the small or the streaming kernel answers NaN and clears it
+    int error;       // sticky: a bounded wait ran out (word kErrorWord of the workspace)
     int pad1[30];
 };
 constexpr int kErrorWord = 33;
 static_assert(sizeof(StreamCtl) == 256, "control block is one 256-byte line group");
-static_assert(offsetof(StreamCtl, error) == kErrorWord * sizeof(int) && offsetof(StreamCtl, down_done) % 128 == 0,
-              "the error word sits right behind the DOWN counter, on that counter's line");
+static_assert(offsetof(StreamCtl, error) == kErrorWord * sizeof(int), "where the tests and the check look for it");
 
 constexpr size_t kOffArrive = 256;
 constexpr size_t kOffFlag = kOffArrive + sizeof(int) * kMaxUnits;
@@ -223,14 +222,11 @@ constexpr size_t kPrefixBytes = kOffLive + sizeof(int) * kMaxSlots;
 // "a >= b" for counters and epochs that wrap around: true while a is at most 2^31 - 1 steps ahead of b
 __device__ __forceinline__ bool reached(int a, int b) { return (int)((unsigned)a - (unsigned)b) >= 0; }
 
+constexpr int kExpiredBit = 1 << 30;
+
 // A whole wavefront, `count` <= 64 consecutive flags, one per lane: every poll is ONE load, so the wait costs one round
 // trip however many flags there are.
-// `also`: a counter that other workgroups are (or will be) waiting on; an expiry sets kExpiredBit in it (an OR: several
-// wavefronts of a workgroup may expire together and must not cancel each other), so that they stop waiting and learn
-// about the expiry from the very word they poll.
-constexpr int kExpiredBit = 1 << 30;
-__device__ __noinline__ inline void spin_all_ge(const int *addr, int count, int target, StreamCtl *ctl,
-                                                int *also = nullptr)
+__device__ __noinline__ inline void spin_all_ge(const int *addr, int count, int target, StreamCtl *ctl)
 {
     const int lane = threadIdx.x & 63;
     for (int it = 0; it < (1 << 22); it++) {
@@ -242,10 +238,7 @@ __device__ __noinline__ inline void spin_all_ge(const int *addr, int count, int 
         if (it < 16) __builtin_amdgcn_s_sleep(4);
         else __builtin_amdgcn_s_sleep(32);
     }
-    if (lane == 0) {
-        store_agent(&ctl->error, 1);
-        if (also) __hip_atomic_fetch_or(also, kExpiredBit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (lane == 0) store_agent(&ctl->error, 1);
 }
 
 // ---- tuning overrides (experiments and tests) ---------------------------------------------------------------
@@ -283,7 +276,7 @@ size_t small_workspace_bytes(int top_k, int M, int N);
 hipError_t launch_small(const MoeParams &p, void *workspace, hipStream_t stream);
 
 // Persistent work-queue kernel for decode-sized batches (block_m <= 32 and bounded sizes): split-K up items ->
-// SwiGLU/requant -> column-slab down items -> per-token reduction, chained through counters in the workspace.
+// SwiGLU/requant -> column-slab down items, chained through flags in the workspace; then the per-token reduction.
 // Weights HBM -> LDS with direct-to-LDS loads.  The first stream_prefix_bytes() of the workspace belong to it.
 size_t stream_prefix_bytes();
 bool stream_supported(int top_k, int M, int K, int N, int E, int sorted_num, int block_m);
@@ -304,12 +297,14 @@ size_t wide_workspace_bytes(int top_k, int M, int K, int N, int E, int sorted_nu
 hipError_t launch_wide(const MoeParams &p, int stages, void *workspace, hipStream_t stream);
 
 // out[t] = bf16(out[t] + sum over the token's live slots of y[slot]) (or bf16(sum) when p.overwrite).  Runs behind the
-// kernel that wrote the rows and closed the launch epoch.  Shared by the tile and wide kernels, which write each (token, slot) row once into y.
+// kernel that wrote the rows and closed the launch epoch.  Shared by the streaming, tile and wide kernels, which write each (token,
+// slot) row once into y.
 struct RowsReduce {
     MoeParams p;
     StreamCtl *ctl;
     const int *live;      // [slots] == epoch of the control block for rows written in this call
-    const uint16_t *y;    // [slots][K] bf16
+    const void *y;        // [slots][K] bf16 or fp32
+    int y_is_f32;
 };
 hipError_t launch_rows_reduce(const RowsReduce &r, hipStream_t stream);
 

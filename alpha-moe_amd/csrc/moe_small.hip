@@ -232,10 +232,9 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
             if (row != id) s_act.same[id] = row;
         });
         if (tid == 0) {
-            // A wait that ran out in an earlier launch on this workspace (sticky), or a counter that such a launch left
-            // marked (once): the output says so itself, NaN in every element.
-            const bool marked = (s.ctl->down_done & kExpiredBit) != 0;
-            if (marked) s.ctl->down_done = 0;
+            // A wait that ran out in an earlier launch on this workspace (sticky), or a marked control block (once): the output says so itself, NaN in every element.
+            const bool marked = (s.ctl->mark & kExpiredBit) != 0;
+            if (marked) s.ctl->mark = 0;
             s_act.n = n_act;
             s_act.poison = marked || s.ctl->error != 0;
         }

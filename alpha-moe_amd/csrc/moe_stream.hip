@@ -14,9 +14,11 @@
 //             flag[u] = epoch.
 //   DOWN item (row block mb, column slab cs): waits for the flags of all I/128 slices of mb, then contracts the
 //             full intermediate against tpi 16-column tiles of w2[e] and stores each valid (token, slot) row's
-//             fp32 result to y[slot] - every element of y has exactly one writer.  Bumps down_done.
-//   FIN item  (token t, 1024 output columns): waits for down_done == number of DOWN items, then
-//             out[t] = bf16(out[t] + sum over the token's live slots of y[slot]) - one rounding, fixed order.
+//             fp32 result to y[slot] - every element of y has exactly one writer.
+// A second launch (launch_rows_reduce) then sums each token's live rows: out[t] = bf16(out[t] + sum of y[slot]), one
+// rounding, fixed order.  As items of the queue that waited for a count of finished DOWN items these sums cost more than a
+// launch: every DOWN item had to wait for its rows to be acknowledged before it could be counted.  Operator calls, before
+// and after: DeepSeek shard M=64 227.6 -> 214 us, M=333 (layer call) 304 -> 287, Qwen3-Next M=256 167 -> 149.
 //
 // There is no floating-point atomic anywhere: the result is bit-reproducible from run to run.
 //
@@ -26,7 +28,7 @@
 // being able to starve each other.  (ALPHA_MOE_STRICT_QUEUE=0 hands the first gridDim.x items out by workgroup index
 // instead, which saves the first round trip to the counter but is only correct when the whole grid is resident at
 // once; it is an experiment switch, not a mode to serve with.)  Each spin is bounded and sets ctl->error instead of
-// hanging; the items that write `out` then fill it with NaN, in that launch and in every later one on the workspace.
+// hanging; the second launch then fills `out` with NaN, in that call and in every later one on the workspace.
 // The workspace starts zero-filled; its first kPrefixBytes hold the control block, the arrival counters (reset by the
 // last arrival) and epoch-stamped flags, so nothing has to be cleared between launches; the rest (aq, sa, hpart, y)
 // is only ever read after it was written in the same launch.
@@ -50,7 +52,6 @@ namespace {
 
 constexpr int kItemKBlocks = 64;     // most K blocks one UP item covers
 constexpr int kMaxIb = 16;           // most 128-column slices of the intermediate (I <= 2048)
-constexpr int kFinCols = 1024;       // output columns per FIN item
 constexpr int kMaxDynamicLds = 140 << 10;   // of the 160 KiB of a compute unit; the kernel's static tables take ~16 KiB
 
 struct StreamPlan {
@@ -66,8 +67,6 @@ struct StreamPlan {
     int n_ib, nkb, n_ct, n_mb_max;
     int kbpi, ks;    // K blocks per UP item, UP items per unit
     int tpi, n_cs;   // 16-column tiles per DOWN item, DOWN items per row block
-    int n_fc;        // 1024-column chunks per token
-    int fin_w;       // chunks per FIN item (1 or 2)
     int lag;         // row blocks between a block's UP items and its DOWN items in the queue
     int bm_pad;
     int strict_queue;   // every item, the first one too, comes from the counter: correct with any number of resident workgroups
@@ -149,8 +148,7 @@ __global__ __launch_bounds__(WN * 64) void moe_stream_kernel(const StreamPlan s)
     const int n_units = n_mb * s.n_ib;
     const int n_up = n_units * s.ks;
     const int n_down = n_mb * s.n_cs;
-    const int n_fin = (p.M * s.n_fc + s.fin_w - 1) / s.fin_w;
-    const int total = n_up + n_down + n_fin;
+    const int total = n_up + n_down;
     const int epoch = (int)((unsigned)__builtin_amdgcn_readfirstlane(s.ctl->epoch) + 1u);
     const uint8_t *dummy = p.x;   // where loads past the end of an item are pointed: always mapped, always cached
 
@@ -449,7 +447,7 @@ __global__ __launch_bounds__(WN * 64) void moe_stream_kernel(const StreamPlan s)
             }
             prime();
             // rare (a DOWN item is queued long after the UP items it needs): a poll returns behind the ring's loads
-            if (!__all(reached(flag0, epoch))) spin_all_ge(&s.flag[mb * n_ib], n_ib, epoch, s.ctl, &s.ctl->down_done);
+            if (!__all(reached(flag0, epoch))) spin_all_ge(&s.flag[mb * n_ib], n_ib, epoch, s.ctl);
 
             // requantised activations of all slices -> LDS as operand tiles, their scales -> s_xs[row][ib]
             for (int i = wave; i < n_ib * TM; i += WN) {
@@ -524,6 +522,14 @@ __global__ __launch_bounds__(WN * 64) void moe_stream_kernel(const StreamPlan s)
                         for (int t = 0; t < TM; t++) res[gg][t] = d[t] * tw[t];
                     }
                 }
+                if (g0 + NG >= wng) {
+                    // Behind the last tile: the next item's ticket and the ring's loads past the end come back before the
+                    // rows go out, so that nothing of this item waits for memory to acknowledge them (a ticket asked
+                    // for behind them would).
+                    fetch_next();
+                    drain_vmem();
+                    asm volatile("" : "+v"(next_item));
+                }
 #pragma unroll
                 for (int gg = 0; gg < NG; gg++)
                     if (g0 + gg < wng) {
@@ -533,115 +539,21 @@ __global__ __launch_bounds__(WN * 64) void moe_stream_kernel(const StreamPlan s)
                     }
             }
         }
-        // (Asking for the next item when the last tile is issued, and counting the item only behind the next item's
-        // prologue instead of waiting for its rows here, were both tried: 1 - 3 % slower at M = 16 and 64.)
-        fetch_next();
-        drain_vmem();
-        __syncthreads();
-        if (tid == 0) __hip_atomic_fetch_add(&s.ctl->down_done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    };
-
-    // FIN item: two dependent round trips.  (1) Wavefront 0 polls the DOWN counter; an expired wait anywhere in this
-    // launch has set kExpiredBit in that very counter, and lane 1 reads the sticky error word of earlier launches
-    // with the same instruction.  (2) The stamps of the token's slots, the rows of ALL its slots and the prior output
-    // go out together; rows of slots that are not live this launch are dropped after the fact (they are stale bytes of
-    // this workspace, nothing else).
-    auto fin_item = [&](int f) {
-        if (wave == 0) {
-            int v = 0;
-            bool up = false;
-            for (int it = 0; it < (1 << 22) && !up; it++) {
-                v = load_agent(lane == 1 ? &s.ctl->error : &s.ctl->down_done);
-                up = reached(__builtin_amdgcn_readlane(v, 0), n_down);
-                if (!up) {
-                    if (it < 16) __builtin_amdgcn_s_sleep(4);
-                    else __builtin_amdgcn_s_sleep(32);
-                }
-            }
-            if (lane == 0) {
-                if (!up) store_agent(&s.ctl->error, 1);
-                // a result row may be missing: the output says so itself, NaN in every element
-                s_bcast[1] = !up || __builtin_amdgcn_readlane(v, 1) != 0 || (__builtin_amdgcn_readlane(v, 0) & kExpiredBit) != 0;
-            }
-        }
-        __syncthreads();
-        acquire_fence();   // the result rows are read from here on, not before the DOWN counter was seen up
-        // an item sums fin_w (1 or 2) chunks of 1024 columns: with more chunks than workgroups, two per item halve the
-        // rounds of dependent memory round trips that close the call
-        const bool poisoned = s_bcast[1] != 0;
-        const int n_chunks = p.M * s.n_fc;
-        int tk[2], col[2], stamp[2];
-        bool mine[2];
-        uint2 *op[2];
-        uint2 o[2];
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int ch = f * s.fin_w + j;
-            const bool on = j < s.fin_w && ch < n_chunks;
-            tk[j] = on ? ch / s.n_fc : 0;
-            col[j] = (on ? ch - tk[j] * s.n_fc : 0) * kFinCols + tid * 4;
-            mine[j] = on && tid < kFinCols / 4 && col[j] < K;
-            // lane k fetches the stamp of the token's slot k (top_k <= 64)
-            stamp[j] = load_agent(&s.live[tk[j] * p.top_k + (lane < p.top_k ? lane : 0)]);
-            op[j] = reinterpret_cast<uint2 *>(p.out + (size_t)tk[j] * K + (mine[j] ? col[j] : 0));
-            o[j] = make_uint2(0u, 0u);
-            if (mine[j] && !p.overwrite && !poisoned) o[j] = *op[j];
-        }
-        v4f sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-        // slot order: the sum depends on nothing but the inputs.  Sixteen rows per chunk are in flight at a time.
-        for (int s0 = 0; s0 < p.top_k; s0 += 16) {
-            v4i lo[2][8], hi[2][8];
-#pragma unroll
-            for (int j = 0; j < 2; j++)
-#pragma unroll
-                for (int k = 0; k < 8; k++) {
-                    lo[j][k] = (v4i){0, 0, 0, 0};
-                    hi[j][k] = (v4i){0, 0, 0, 0};
-                    const uint32_t row = ((uint32_t)(tk[j] * p.top_k + s0 + k) * (uint32_t)K + (uint32_t)col[j]) * 4u;
-                    if (mine[j] && s0 + k < p.top_k) lo[j][k] = ldg128_agent(s.y, row);
-                    if (mine[j] && s0 + 8 + k < p.top_k) hi[j][k] = ldg128_agent(s.y, row + 32u * (uint32_t)K);
-                }
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const unsigned long long live_mask = __ballot(lane < p.top_k && stamp[j] == epoch) >> s0;
-#pragma unroll
-                for (int k = 0; k < 8; k++)
-                    if ((live_mask >> k) & 1) sum[j] += __builtin_bit_cast(v4f, lo[j][k]);
-#pragma unroll
-                for (int k = 0; k < 8; k++)
-                    if ((live_mask >> (8 + k)) & 1) sum[j] += __builtin_bit_cast(v4f, hi[j][k]);
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 2; j++)
-            if (mine[j]) {
-                uint2 r = o[j];
-                if (poisoned) {
-                    r = make_uint2(0x7fc07fc0u, 0x7fc07fc0u);
-                } else {
-                    const float o0 = __builtin_bit_cast(float, r.x << 16), o1 = __builtin_bit_cast(float, r.x & 0xffff0000u);
-                    const float o2 = __builtin_bit_cast(float, r.y << 16), o3 = __builtin_bit_cast(float, r.y & 0xffff0000u);
-                    r.x = pack_bf16x2(o0 + sum[j][0], o1 + sum[j][1]);
-                    r.y = pack_bf16x2(o2 + sum[j][2], o3 + sum[j][3]);
-                }
-                *op[j] = r;
-            }
+        // (Asking for the next item when the last tile is issued was tried: 1 - 3 % slower at M = 16 and 64.)
     };
 
     // ---- work queue ---------------------------------------------------------------------------------------
     // Order: round r holds the UP items of row block r followed by the DOWN items of row block r - lag, so the two
     // kinds overlap, a DOWN item is taken long after the UP items it waits for, and only `lag` blocks' worth of
-    // DOWN items remain when the UP items run out.  FIN items come last.
+    // DOWN items remain when the UP items run out.
     const int per_up = s.n_ib * s.ks, per_down = s.n_cs;
     const int lag = s.lag < n_mb ? s.lag : n_mb;
     const int head_items = lag * per_up;                          // rounds 0 .. lag-1: UP only
     const int mid_items = (n_mb - lag) * (per_up + per_down);     // rounds lag .. n_mb-1: UP then DOWN
     // every item kind has exactly one call site: the compiler inlines the item bodies into the loop
     auto run_item = [&](int item) {
-        int up = -1, down = -1, fin = -1;
-        if (item >= n_up + n_down) {
-            fin = item - n_up - n_down;
-        } else if (item < head_items) {
+        int up = -1, down = -1;
+        if (item < head_items) {
             up = item;
         } else if (item < head_items + mid_items) {
             const int i = item - head_items;
@@ -655,9 +567,7 @@ __global__ __launch_bounds__(WN * 64) void moe_stream_kernel(const StreamPlan s)
             down = (n_mb - lag) * per_down + (item - head_items - mid_items);
         }
         if (up >= 0) up_item(up);
-        else if (down >= 0) down_item(down);
-        else fin_item(fin);
-        return up >= 0 ? 1 : down >= 0 ? 2 : 3;
+        else down_item(down);
     };
     int item = blockIdx.x;   // no round trip to the queue before the first item
     if (s.strict_queue) {    // unless the caller cannot promise that the whole grid is resident at once
@@ -669,12 +579,11 @@ __global__ __launch_bounds__(WN * 64) void moe_stream_kernel(const StreamPlan s)
     }
     while (item < total) {
         next_item = -1;
-        const int kind = run_item(item);
-        (void)kind;
-        fetch_next();   // paths that did not get there themselves (skipped blocks, FIN items)
-        __syncthreads();
+        run_item(item);
+        fetch_next();    // items that did not get there themselves
+        lds_barrier();   // (not __syncthreads, which would wait for a DOWN item's result rows)
         if (tid == 0) s_bcast[0] = next_item;
-        __syncthreads();
+        lds_barrier();
         item = __builtin_amdgcn_readfirstlane(s_bcast[0]);
     }
     if (tid == 0) {
@@ -682,8 +591,11 @@ __global__ __launch_bounds__(WN * 64) void moe_stream_kernel(const StreamPlan s)
         if (left == (int)gridDim.x - 1) {
             store_agent(&s.ctl->head, 0);
             store_agent(&s.ctl->done, 0);
-            store_agent(&s.ctl->down_done, 0);
-            store_agent(&s.ctl->epoch, epoch);
+            if (load_agent(&s.ctl->mark) & kExpiredBit) {
+                store_agent(&s.ctl->mark, 0);
+                store_agent(&s.ctl->poisoned, epoch);
+            }
+            store_agent(&s.ctl->epoch, epoch);   // everybody has read the old one; the reduce kernel compares with this
         }
     }
 }
@@ -695,7 +607,7 @@ size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 struct HostPlan {
     bool ok;
     int bm_pad, n_ib, nkb, n_ct, n_mb_max, units;
-    int kbpi, ks, tpi, n_cs, n_fc, fin_w, lag;
+    int kbpi, ks, tpi, n_cs, lag;
     size_t off_sa, off_aq, off_hpart, off_y, total;
 };
 
@@ -763,8 +675,6 @@ HostPlan make_plan(int top_k, int M, int K, int N, int E, int sorted_num, int bl
     h.n_cs = (h.n_ct + tpi - 1) / tpi;
     h.tpi = ((h.n_ct + h.n_cs - 1) / h.n_cs + 15) / 16 * 16;   // even split, whole multiples of 16 tiles
     h.n_cs = (h.n_ct + h.tpi - 1) / h.tpi;
-    h.n_fc = (K + kFinCols - 1) / kFinCols;
-    h.fin_w = (int64_t)M * h.n_fc > cus ? 2 : 1;
     // how many row blocks later a block's DOWN items enter the queue than its UP items
     // (measured: overlapping the two kinds lowers the total rate - DOWN items stream less efficiently than UP items -
     // so by default the lag is "all blocks", i.e. UP items first, then DOWN items)
@@ -906,8 +816,6 @@ hipError_t launch_stream(const MoeParams &p, int warp_n, int stages, void *works
     s.ks = h.ks;
     s.tpi = h.tpi;
     s.n_cs = h.n_cs;
-    s.n_fc = h.n_fc;
-    s.fin_w = h.fin_w;
     s.lag = h.lag;
     s.strict_queue = tunable(kTunStrictQueue, 1) != 0;
 
@@ -923,15 +831,23 @@ hipError_t launch_stream(const MoeParams &p, int warp_n, int stages, void *works
     }
     if (lds_bytes > kMaxDynamicLds) return hipErrorInvalidValue;
     int slots = 0;
-    const hipError_t err = resident_slots(v, lds_bytes, &slots);
+    hipError_t err = resident_slots(v, lds_bytes, &slots);
     if (err != hipSuccess) return err;
 
-    const int64_t max_items = (int64_t)h.units * h.ks + (int64_t)h.n_mb_max * h.n_cs + (int64_t)p.M * h.n_fc;
+    const int64_t max_items = (int64_t)h.units * h.ks + (int64_t)h.n_mb_max * h.n_cs;
     int grid = tunable(kTunGrid, slots);
     if (grid > max_items) grid = (int)max_items;
     if (grid < 1) grid = 1;
     hipLaunchKernelGGL(v.fn, dim3((unsigned)grid), dim3((unsigned)v.threads), lds_bytes, stream, s);
-    return hipGetLastError();
+    err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    RowsReduce r;
+    r.p = p;
+    r.ctl = s.ctl;
+    r.live = s.live;
+    r.y = s.y;
+    r.y_is_f32 = 1;
+    return launch_rows_reduce(r, stream);
 }
 
 }  // namespace alpha_moe

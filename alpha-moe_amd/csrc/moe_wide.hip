@@ -1175,6 +1175,7 @@ hipError_t launch_wide(const MoeParams &p, int stages, void *workspace, hipStrea
     r.ctl = s.ctl;
     r.live = s.live;
     r.y = s.y;
+    r.y_is_f32 = 0;
     return launch_rows_reduce(r, stream);
 }
 
