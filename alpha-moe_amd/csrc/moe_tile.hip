@@ -180,6 +180,19 @@ __global__ __launch_bounds__(512) void moe_tile_kernel(const TileParams s)
 
     v4f acc[4][TH];
 
+    auto blocks_of = [&](int queue) {
+        const int left = n_live - queue * per_q;
+        return left < 0 ? 0 : (left < per_q ? left : per_q);
+    };
+    // The next item's ticket is asked for where an item has nothing left to wait for but its own results (earlier it could
+    // hold an item that a waiting workgroup waits for); thread 0 keeps it.  With the result rows of a down item no longer
+    // waited for, layer calls: DeepSeek shard M=2048 432 -> 428 us, Qwen3-Next M=4096 297 -> 293.
+    int qq = blockIdx.x & 7, visited = 0, ticket = -1;   // state of thread 0
+    auto ask_ticket = [&]() {
+        if (tid == 0 && ticket < 0 && visited < 8)
+            ticket = __hip_atomic_fetch_add(&s.ctl->tile_head[qq], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+
     // ---- UP item: slice ib of row block mb -> requantised operand tiles + scales in scratch, then the unit's flag ----
     // An expert with a single row block streams its weights with non-temporal loads (measured on the DeepSeek-V3 shard:
     // -13 % at M = 512 where nearly every expert has one block, +8 % at M = 8192 if applied to experts whose blocks run
@@ -277,6 +290,7 @@ __global__ __launch_bounds__(512) void moe_tile_kernel(const TileParams s)
             }
         }
         wait_vmcnt<0>();
+        ask_ticket();
 
         // SwiGLU, per-token amax over the slice's 128 columns, FP8 requant into operand tiles
 #pragma unroll
@@ -430,6 +444,13 @@ __global__ __launch_bounds__(512) void moe_tile_kernel(const TileParams s)
                     __builtin_amdgcn_sched_barrier(0);
                     cib++;
                     if (cib == n_ib) {
+                        if (s0 + h + 1 == n_steps) {
+                            // behind the last step: the ring's loads past the end land and the ticket comes back before
+                            // the last rows go out, and nothing waits for memory to acknowledge those
+                            ask_ticket();
+                            wait_vmcnt<0>();
+                            asm volatile("" : "+v"(ticket));
+                        }
 #pragma unroll
                         for (int t = 0; t < THD; t++) {
                             if (valid[t] && cg < my_groups) {
@@ -454,7 +475,6 @@ __global__ __launch_bounds__(512) void moe_tile_kernel(const TileParams s)
                 }
             }
         }
-        wait_vmcnt<0>();
     };
     // token parts of a DOWN item: the host picks the smallest divisor of TH whose tiles fit next to the weight ring
     auto run_down = [&](int mb, int sub) {
@@ -476,32 +496,27 @@ __global__ __launch_bounds__(512) void moe_tile_kernel(const TileParams s)
     // blocks.  A down item waits for the flags of its block's up/gate items, which are EARLIER in the same queue:
     // whoever took them is running and waits for nothing later, so the queues drain with any number of resident
     // workgroups.  A workgroup that finds its queue empty moves on to the next one.
-    auto blocks_of = [&](int qq) {
-        const int left = n_live - qq * per_q;
-        return left < 0 ? 0 : (left < per_q ? left : per_q);
-    };
-    // (Asking for the next item's ticket while the current item runs was tried: the round trip it hides, ~2 us per item,
-    // does not show in a call's time - the kernel is bound by what all compute units pull together, not by one of them.)
-    int qq = blockIdx.x & 7, visited = 0;   // state of thread 0
     while (true) {
         if (tid == 0) {
             int it = -1;
             while (visited < 8) {
-                const int nb = blocks_of(qq);
-                const int idx = nb > 0 ? __hip_atomic_fetch_add(&s.ctl->tile_head[qq], 1, __ATOMIC_RELAXED,
-                                                                __HIP_MEMORY_SCOPE_AGENT)
-                                       : 0;
-                if (idx < nb * (per_up + per_down)) {
-                    it = idx;
-                    break;
+                const int n_items = blocks_of(qq) * (per_up + per_down);
+                if (n_items > 0) {
+                    ask_ticket();
+                    if (ticket < n_items) {
+                        it = ticket;
+                        break;
+                    }
                 }
+                ticket = -1;
                 qq = (qq + 1) & 7;
                 visited++;
             }
+            ticket = -1;
             s_item[0] = it;
             s_item[1] = qq;
         }
-        __syncthreads();
+        lds_barrier();
         const int item = __builtin_amdgcn_readfirstlane(s_item[0]);
         const int qi = __builtin_amdgcn_readfirstlane(s_item[1]);
         if (item < 0) break;
@@ -527,7 +542,7 @@ __global__ __launch_bounds__(512) void moe_tile_kernel(const TileParams s)
         } else {
             run_down(qi * per_q + down / per_down, down % per_down);
         }
-        __syncthreads();   // everybody is done with the item's LDS tables and rings before the next item refills them
+        lds_barrier();   // everybody is done with the item's LDS tables and rings before the next item refills them
     }
     if (tid == 0) {
         const int left = __hip_atomic_fetch_add(&s.ctl->tile_done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
