@@ -60,6 +60,9 @@ c_abi.alpha_moe_moe_align_block_size.restype = ctypes.c_int
 c_abi.alpha_moe_moe_align_block_size.argtypes = (
     [ctypes.c_void_p] + [ctypes.c_int] * 3 + [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_int,
                                               ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p])
+c_abi.alpha_moe_prepare_inputs.restype = ctypes.c_int
+c_abi.alpha_moe_prepare_inputs.argtypes = (
+    c_abi.alpha_moe_per_token_group_quant_fp8.argtypes[:-1] + c_abi.alpha_moe_moe_align_block_size.argtypes)
 
 __version__ = c_abi.alpha_moe_version().decode()
 

@@ -42,6 +42,11 @@ def _moe_align_block_size_fake(topk_ids, block_size, num_experts):
             topk_ids.new_empty((1,)))
 
 
+@torch.library.register_fake("alpha_moe::prepare_inputs")
+def _prepare_inputs_fake(x, topk_ids, group_size, block_size, num_experts):
+    return (*_per_token_group_quant_fp8_fake(x, group_size), *_moe_align_block_size_fake(topk_ids, block_size, num_experts))
+
+
 def fused_moe_w8a8_up_down(
     x: torch.Tensor,
     x_scale: torch.Tensor,

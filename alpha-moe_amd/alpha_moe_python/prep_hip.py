@@ -2,7 +2,7 @@
 ``torch.ops.alpha_moe.per_token_group_quant_fp8`` and ``torch.ops.alpha_moe.moe_align_block_size``.
 
 Same names, arguments and results as the torch restatements in ``alpha_moe_python.prep`` (and as the SGLang functions
-the reference's callers use, jit_moe.py:142,158), bit for bit; these run as one to three small kernels on the current
+the reference's callers use, jit_moe.py:142,158), bit for bit; these run as one or two small kernels on the current
 stream and need the built extension.
 """
 from typing import Tuple
@@ -22,3 +22,11 @@ def moe_align_block_size(topk_ids: torch.Tensor, block_size: int, num_experts: i
     if topk_ids.dtype != torch.int32:
         topk_ids = topk_ids.to(torch.int32)
     return torch.ops.alpha_moe.moe_align_block_size(topk_ids.contiguous(), block_size, num_experts)
+
+
+def prepare_inputs(x: torch.Tensor, topk_ids: torch.Tensor, group_size: int, block_size: int, num_experts: int):
+    """Both of the above for one layer call, in one launch less: ``(q, scale, sorted_token_ids, expert_ids,
+    num_tokens_post_padded)``."""
+    if topk_ids.dtype != torch.int32:
+        topk_ids = topk_ids.to(torch.int32)
+    return torch.ops.alpha_moe.prepare_inputs(x, topk_ids.contiguous(), group_size, block_size, num_experts)

@@ -45,15 +45,14 @@ __device__ __forceinline__ void load8<float>(const float *p, float (&v)[8])
     }
 }
 
+// The groups of workgroup `part` of `parts`; a thread has the loads of two groups in flight.
 template <typename T>
-__global__ __launch_bounds__(256) void quant_group128_kernel(const T *__restrict__ x, uint8_t *__restrict__ q,
-                                                             float *__restrict__ scale, long long n_groups)
+__device__ __forceinline__ void quant_groups(const T *__restrict__ x, uint8_t *__restrict__ q, float *__restrict__ scale,
+                                             long long n_groups, int part, int parts)
 {
-    const int sub = threadIdx.x & 15;
-    const long long stride = (long long)gridDim.x * 16;
-    for (long long g = (long long)blockIdx.x * 16 + (threadIdx.x >> 4); g < n_groups; g += stride) {
-        float v[8];
-        load8<T>(x + g * 128 + sub * 8, v);
+    const int sub = threadIdx.x & 15, per = blockDim.x >> 4;
+    const long long stride = (long long)parts * per;
+    auto quantise = [&](long long g, const float (&v)[8]) {
         float m = 0.f;
 #pragma unroll
         for (int i = 0; i < 8; i++) m = fmaxf(m, fabsf(v[i]));
@@ -65,7 +64,22 @@ __global__ __launch_bounds__(256) void quant_group128_kernel(const T *__restrict
         o.y = pack_fp8x4(clamp_fp8(v[4] / s), clamp_fp8(v[5] / s), clamp_fp8(v[6] / s), clamp_fp8(v[7] / s));
         *reinterpret_cast<uint2 *>(q + g * 128 + sub * 8) = o;
         if (sub == 0) scale[g] = s;
+    };
+    for (long long g = (long long)part * per + (threadIdx.x >> 4); g < n_groups; g += 2 * stride) {
+        const bool second = g + stride < n_groups;   // the same for the 16 lanes of a group
+        float v[8], u[8];
+        load8<T>(x + g * 128 + sub * 8, v);
+        if (second) load8<T>(x + (g + stride) * 128 + sub * 8, u);
+        quantise(g, v);
+        if (second) quantise(g + stride, u);
     }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void quant_group128_kernel(const T *__restrict__ x, uint8_t *__restrict__ q,
+                                                             float *__restrict__ scale, long long n_groups)
+{
+    quant_groups<T>(x, q, scale, n_groups, blockIdx.x, gridDim.x);
 }
 
 // ---- alignment ---------------------------------------------------------------------------------------------
@@ -215,11 +229,22 @@ __device__ __forceinline__ void fill_sentinel(int32_t *sorted_ids, int sorted_nu
 }
 
 // One workgroup does everything (up to kAlignSmall slots).  n_waves of its wavefronts count and place `run` slots each.
-__global__ __launch_bounds__(1024) void align_small_kernel(const int32_t *__restrict__ ids, int numel, int E, int id_bits,
-                                                           int block_size, int32_t *sorted_ids, int sorted_num,
-                                                           int32_t *expert_ids, int n_blocks, int32_t *ntpp, int n_waves,
-                                                           int run)
+struct AlignSmall {
+    const int32_t *ids;
+    int numel, E, id_bits, block_size;
+    int32_t *sorted_ids;
+    int sorted_num;
+    int32_t *expert_ids;
+    int n_blocks;
+    int32_t *ntpp;
+    int n_waves, run;
+};
+__device__ __forceinline__ void align_small(const AlignSmall &a)
 {
+    const int32_t *__restrict__ ids = a.ids;
+    const int numel = a.numel, E = a.E, id_bits = a.id_bits, block_size = a.block_size, sorted_num = a.sorted_num;
+    const int n_waves = a.n_waves, run = a.run;
+    int32_t *sorted_ids = a.sorted_ids;
     extern __shared__ __attribute__((aligned(16))) int lds[];   // [E] starts | [16] | [n_waves][E] cursors (16 bit)
     int *start = lds, *wave_sums = lds + E;
     uint16_t *cursors = reinterpret_cast<uint16_t *>(lds + E + 16);
@@ -235,13 +260,27 @@ __global__ __launch_bounds__(1024) void align_small_kernel(const int32_t *__rest
     const int total = block_exclusive_scan(start, E, wave_sums);
     // (the barriers above have also completed the sentinel fill before any slot is placed)
     if (wave < n_waves) place_run(ids, lo, hi, E, id_bits, start, cursors + wave * E, sorted_ids);
-    write_blocks(start, E, block_size, total, expert_ids, n_blocks, ntpp, 0, 1);
+    write_blocks(start, E, block_size, total, a.expert_ids, a.n_blocks, a.ntpp, 0, 1);
+}
+
+__global__ __launch_bounds__(1024) void align_small_kernel(const AlignSmall a) { align_small(a); }
+
+// Both preparations of a layer call in one launch: workgroup 0 aligns, the others quantise.  Neither needs the other's
+// result, and at decode sizes each is ~5 us of latency: layer calls,
+// DeepSeek shard M=1 30.3 -> 26.3 us, M=7 63.8 -> 61.5, M=333 287 -> 283, Qwen3-30B M=61 104 -> 100.
+template <typename T>
+__global__ __launch_bounds__(1024) void prepare_small_kernel(const AlignSmall a, const T *__restrict__ x,
+                                                             uint8_t *__restrict__ q, float *__restrict__ scale,
+                                                             long long n_groups)
+{
+    if (blockIdx.x == 0) align_small(a);
+    else quant_groups<T>(x, q, scale, n_groups, (int)blockIdx.x - 1, (int)gridDim.x - 1);
 }
 
 // Larger inputs, pass 1: one workgroup per segment of kAlignSeg slots writes the segment's expert histogram (16-bit
 // counts, two per word); also the sentinel fill.
-__global__ __launch_bounds__(256) void align_hist_kernel(const int32_t *__restrict__ ids, int numel, int E, int *hist,
-                                                         int words, int32_t *sorted_ids, int sorted_num)
+__device__ __forceinline__ void align_hist(const int32_t *__restrict__ ids, int numel, int E, int *hist, int words,
+                                           int32_t *sorted_ids, int sorted_num, int n_seg)
 {
     extern __shared__ int lds[];   // [words]
     for (int i = threadIdx.x; i < words; i += blockDim.x) lds[i] = 0;
@@ -253,7 +292,24 @@ __global__ __launch_bounds__(256) void align_hist_kernel(const int32_t *__restri
     }
     __syncthreads();
     for (int i = threadIdx.x; i < words; i += blockDim.x) hist[(size_t)blockIdx.x * words + i] = lds[i];
-    fill_sentinel(sorted_ids, sorted_num, numel, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
+    fill_sentinel(sorted_ids, sorted_num, numel, blockIdx.x * blockDim.x + threadIdx.x, n_seg * blockDim.x);
+}
+
+__global__ __launch_bounds__(256) void align_hist_kernel(const int32_t *__restrict__ ids, int numel, int E, int *hist,
+                                                         int words, int32_t *sorted_ids, int sorted_num)
+{
+    align_hist(ids, numel, E, hist, words, sorted_ids, sorted_num, gridDim.x);
+}
+
+// Pass 1 and the quantiser in one launch: the first n_seg workgroups count, the others quantise.
+template <typename T>
+__global__ __launch_bounds__(256) void prepare_hist_kernel(const int32_t *__restrict__ ids, int numel, int E, int *hist,
+                                                           int words, int32_t *sorted_ids, int sorted_num, int n_seg,
+                                                           const T *__restrict__ x, uint8_t *__restrict__ q,
+                                                           float *__restrict__ scale, long long n_groups)
+{
+    if ((int)blockIdx.x < n_seg) align_hist(ids, numel, E, hist, words, sorted_ids, sorted_num, n_seg);
+    else quant_groups<T>(x, q, scale, n_groups, (int)blockIdx.x - n_seg, (int)gridDim.x - n_seg);
 }
 
 // Pass 2, one workgroup per segment: every workgroup adds the histograms up itself (columns of two experts, sixteen
@@ -308,6 +364,82 @@ __global__ __launch_bounds__(256) void align_place_kernel(const int32_t *__restr
     place_run(ids, lo, hi, E, id_bits, start, cursors + wave * E, sorted_ids);
 }
 
+// What is quantised beside an alignment (x == nullptr: nothing).
+struct Quant {
+    const void *x;
+    int is_f32;
+    uint8_t *q;
+    float *scale;
+    int M, K;
+};
+
+int check_quant(const Quant &z)
+{
+    if (!z.x || !z.q || !z.scale) return ALPHA_MOE_ERR_NULL_POINTER;
+    if (z.M <= 0 || z.K <= 0 || z.K % 128 != 0) return ALPHA_MOE_ERR_SHAPE;
+    return ALPHA_MOE_OK;
+}
+
+// workgroups of `threads` threads for the groups of z
+unsigned quant_grid(const Quant &z, int threads)
+{
+    const long long per = threads / 16, want = ((long long)z.M * (z.K / 128) + per - 1) / per, most = 8192 * 256 / threads;
+    return (unsigned)(want < most ? want : most);
+}
+
+int align(const int32_t *topk_ids, int numel, int num_experts, int block_size, int32_t *sorted_token_ids, int sorted_num,
+          int32_t *expert_ids, int n_blocks, int32_t *num_tokens_post_padded, void *workspace, size_t workspace_bytes,
+          const Quant &z, hipStream_t hs)
+{
+    if (!topk_ids || !sorted_token_ids || !expert_ids || !num_tokens_post_padded) return ALPHA_MOE_ERR_NULL_POINTER;
+    if (numel <= 0 || num_experts <= 0 || num_experts > kAlignMaxExperts || block_size <= 0) return ALPHA_MOE_ERR_SHAPE;
+    if ((long long)sorted_num != (long long)numel + (long long)num_experts * (block_size - 1) ||
+        (long long)n_blocks != ((long long)sorted_num + block_size - 1) / block_size)
+        return ALPHA_MOE_ERR_SHAPE;
+    const int E = num_experts;
+    const long long n_groups = z.x ? (long long)z.M * (z.K / 128) : 0;
+    int id_bits = 0;
+    while ((1 << id_bits) < E) id_bits++;
+    if (numel <= kAlignSmall) {
+        // as many wavefronts as there are chunks of 64 slots, and no more than have room for their cursors
+        int n_waves = (numel + 63) / 64;
+        if (n_waves > 16) n_waves = 16;
+        const int room = (40 << 10) / (E * (int)sizeof(uint16_t));
+        if (n_waves > room) n_waves = room;
+        const int run = ((numel + n_waves - 1) / n_waves + 63) / 64 * 64;
+        const size_t lds = (E + 16) * sizeof(int) + ((size_t)n_waves * E + 1) / 2 * sizeof(int);
+        const AlignSmall a = {topk_ids, numel, E, id_bits, block_size, sorted_token_ids, sorted_num, expert_ids, n_blocks,
+                              num_tokens_post_padded, n_waves, run};
+        if (!z.x)
+            hipLaunchKernelGGL(align_small_kernel, dim3(1), dim3(1024), lds, hs, a);
+        else if (z.is_f32)
+            hipLaunchKernelGGL(prepare_small_kernel<float>, dim3(1 + quant_grid(z, 1024)), dim3(1024), lds, hs, a,
+                               static_cast<const float *>(z.x), z.q, z.scale, n_groups);
+        else
+            hipLaunchKernelGGL(prepare_small_kernel<uint16_t>, dim3(1 + quant_grid(z, 1024)), dim3(1024), lds, hs, a,
+                               static_cast<const uint16_t *>(z.x), z.q, z.scale, n_groups);
+        return hipGetLastError() == hipSuccess ? ALPHA_MOE_OK : ALPHA_MOE_ERR_LAUNCH;
+    }
+    if (!workspace || workspace_bytes < alpha_moe_align_workspace_bytes(numel, E)) return ALPHA_MOE_ERR_WORKSPACE;
+    const int n_seg = (numel + kAlignSeg - 1) / kAlignSeg, words = (E + 1) / 2;
+    int *hist = static_cast<int *>(workspace);
+    if (!z.x)
+        hipLaunchKernelGGL(align_hist_kernel, dim3(n_seg), dim3(256), words * sizeof(int), hs, topk_ids, numel, E, hist,
+                           words, sorted_token_ids, sorted_num);
+    else if (z.is_f32)
+        hipLaunchKernelGGL(prepare_hist_kernel<float>, dim3(n_seg + quant_grid(z, 256)), dim3(256), words * sizeof(int), hs,
+                           topk_ids, numel, E, hist, words, sorted_token_ids, sorted_num, n_seg,
+                           static_cast<const float *>(z.x), z.q, z.scale, n_groups);
+    else
+        hipLaunchKernelGGL(prepare_hist_kernel<uint16_t>, dim3(n_seg + quant_grid(z, 256)), dim3(256), words * sizeof(int),
+                           hs, topk_ids, numel, E, hist, words, sorted_token_ids, sorted_num, n_seg,
+                           static_cast<const uint16_t *>(z.x), z.q, z.scale, n_groups);
+    const size_t lds = (4 * words + (2 * E > 16 ? 2 * E : 16)) * sizeof(int);   // 64 KiB at kAlignMaxExperts
+    hipLaunchKernelGGL(align_place_kernel, dim3(n_seg), dim3(256), lds, hs, topk_ids, numel, E, id_bits, block_size, hist,
+                       words, sorted_token_ids, expert_ids, n_blocks, num_tokens_post_padded);
+    return hipGetLastError() == hipSuccess ? ALPHA_MOE_OK : ALPHA_MOE_ERR_LAUNCH;
+}
+
 }  // namespace
 }  // namespace alpha_moe
 
@@ -316,18 +448,18 @@ using namespace alpha_moe;
 extern "C" int alpha_moe_per_token_group_quant_fp8(const void *x, int x_is_f32, uint8_t *q, float *scale, int M, int K,
                                                    void *stream)
 {
-    if (!x || !q || !scale) return ALPHA_MOE_ERR_NULL_POINTER;
-    if (M <= 0 || K <= 0 || K % 128 != 0) return ALPHA_MOE_ERR_SHAPE;
+    const Quant z = {x, x_is_f32, q, scale, M, K};
+    const int rc = check_quant(z);
+    if (rc != ALPHA_MOE_OK) return rc;
+    const dim3 grid(quant_grid(z, 256));
     const long long n_groups = (long long)M * (K / 128);
-    const long long want = (n_groups + 15) / 16;
-    const unsigned grid = (unsigned)(want < 8192 ? want : 8192);
     hipStream_t hs = static_cast<hipStream_t>(stream);
     if (x_is_f32)
-        hipLaunchKernelGGL(quant_group128_kernel<float>, dim3(grid), dim3(256), 0, hs, static_cast<const float *>(x), q,
-                           scale, n_groups);
+        hipLaunchKernelGGL(quant_group128_kernel<float>, grid, dim3(256), 0, hs, static_cast<const float *>(x), q, scale,
+                           n_groups);
     else
-        hipLaunchKernelGGL(quant_group128_kernel<uint16_t>, dim3(grid), dim3(256), 0, hs,
-                           static_cast<const uint16_t *>(x), q, scale, n_groups);
+        hipLaunchKernelGGL(quant_group128_kernel<uint16_t>, grid, dim3(256), 0, hs, static_cast<const uint16_t *>(x), q,
+                           scale, n_groups);
     return hipGetLastError() == hipSuccess ? ALPHA_MOE_OK : ALPHA_MOE_ERR_LAUNCH;
 }
 
@@ -343,34 +475,19 @@ extern "C" int alpha_moe_moe_align_block_size(const int32_t *topk_ids, int numel
                                               int n_blocks, int32_t *num_tokens_post_padded, void *workspace,
                                               size_t workspace_bytes, void *stream)
 {
-    if (!topk_ids || !sorted_token_ids || !expert_ids || !num_tokens_post_padded) return ALPHA_MOE_ERR_NULL_POINTER;
-    if (numel <= 0 || num_experts <= 0 || num_experts > kAlignMaxExperts || block_size <= 0) return ALPHA_MOE_ERR_SHAPE;
-    if ((long long)sorted_num != (long long)numel + (long long)num_experts * (block_size - 1) ||
-        (long long)n_blocks != ((long long)sorted_num + block_size - 1) / block_size)
-        return ALPHA_MOE_ERR_SHAPE;
-    hipStream_t hs = static_cast<hipStream_t>(stream);
-    const int E = num_experts;
-    int id_bits = 0;
-    while ((1 << id_bits) < E) id_bits++;
-    if (numel <= kAlignSmall) {
-        // as many wavefronts as there are chunks of 64 slots, and no more than have room for their cursors
-        int n_waves = (numel + 63) / 64;
-        if (n_waves > 16) n_waves = 16;
-        const int room = (40 << 10) / (E * (int)sizeof(uint16_t));
-        if (n_waves > room) n_waves = room;
-        const int run = ((numel + n_waves - 1) / n_waves + 63) / 64 * 64;
-        const size_t lds = (E + 16) * sizeof(int) + ((size_t)n_waves * E + 1) / 2 * sizeof(int);
-        hipLaunchKernelGGL(align_small_kernel, dim3(1), dim3(1024), lds, hs, topk_ids, numel, E, id_bits, block_size,
-                           sorted_token_ids, sorted_num, expert_ids, n_blocks, num_tokens_post_padded, n_waves, run);
-        return hipGetLastError() == hipSuccess ? ALPHA_MOE_OK : ALPHA_MOE_ERR_LAUNCH;
-    }
-    if (!workspace || workspace_bytes < alpha_moe_align_workspace_bytes(numel, E)) return ALPHA_MOE_ERR_WORKSPACE;
-    const int n_seg = (numel + kAlignSeg - 1) / kAlignSeg, words = (E + 1) / 2;
-    int *hist = static_cast<int *>(workspace);
-    hipLaunchKernelGGL(align_hist_kernel, dim3(n_seg), dim3(256), words * sizeof(int), hs, topk_ids, numel, E, hist, words,
-                       sorted_token_ids, sorted_num);
-    const size_t lds = (4 * words + (2 * E > 16 ? 2 * E : 16)) * sizeof(int);   // 64 KiB at kAlignMaxExperts
-    hipLaunchKernelGGL(align_place_kernel, dim3(n_seg), dim3(256), lds, hs, topk_ids, numel, E, id_bits, block_size, hist,
-                       words, sorted_token_ids, expert_ids, n_blocks, num_tokens_post_padded);
-    return hipGetLastError() == hipSuccess ? ALPHA_MOE_OK : ALPHA_MOE_ERR_LAUNCH;
+    return align(topk_ids, numel, num_experts, block_size, sorted_token_ids, sorted_num, expert_ids, n_blocks,
+                 num_tokens_post_padded, workspace, workspace_bytes, Quant{}, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int alpha_moe_prepare_inputs(const void *x, int x_is_f32, uint8_t *q, float *scale, int M, int K,
+                                        const int32_t *topk_ids, int numel, int num_experts, int block_size,
+                                        int32_t *sorted_token_ids, int sorted_num, int32_t *expert_ids, int n_blocks,
+                                        int32_t *num_tokens_post_padded, void *workspace, size_t workspace_bytes,
+                                        void *stream)
+{
+    const Quant z = {x, x_is_f32, q, scale, M, K};
+    const int rc = check_quant(z);
+    if (rc != ALPHA_MOE_OK) return rc;
+    return align(topk_ids, numel, num_experts, block_size, sorted_token_ids, sorted_num, expert_ids, n_blocks,
+                 num_tokens_post_padded, workspace, workspace_bytes, z, static_cast<hipStream_t>(stream));
 }

@@ -288,6 +288,41 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> moe_align_block_size(const at::Te
     return {sorted_ids, expert_ids, total};
 }
 
+// (q, scale, sorted_token_ids, expert_ids, num_tokens_post_padded): the two functions above for one layer call.
+std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor, at::Tensor>
+prepare_inputs(const at::Tensor &x, const at::Tensor &topk_ids, int64_t group_size, int64_t block_size, int64_t num_experts)
+{
+    TORCH_CHECK(x.is_cuda() && topk_ids.is_cuda() && x.device() == topk_ids.device(), "x and topk_ids must be on one GPU");
+    TORCH_CHECK(group_size == 128, "group_size must be 128");
+    TORCH_CHECK(x.dim() == 2 && x.size(1) % 128 == 0 && x.size(0) > 0, "x must be [M, K] with K % 128 == 0");
+    TORCH_CHECK(x.scalar_type() == at::kBFloat16 || x.scalar_type() == at::kFloat, "x must be bfloat16 or float32");
+    TORCH_CHECK(x.is_contiguous(), "x must be contiguous");
+    TORCH_CHECK(topk_ids.scalar_type() == at::kInt, "topk_ids must be int32");
+    TORCH_CHECK(topk_ids.is_contiguous() && topk_ids.numel() > 0, "topk_ids must be contiguous and not empty");
+    TORCH_CHECK(block_size > 0 && num_experts > 0, "block_size and num_experts must be positive");
+    const int64_t numel = topk_ids.numel();
+    const int64_t sorted_num = numel + num_experts * (block_size - 1);
+    const int64_t n_blocks = (sorted_num + block_size - 1) / block_size;
+    TORCH_CHECK(sorted_num <= INT32_MAX, "too many routing slots");
+    const c10::hip::OptionalHIPGuardMasqueradingAsCUDA guard(x.device());
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
+    at::Tensor q = at::empty(x.sizes(), x.options().dtype(at::kFloat8_e4m3fn));
+    at::Tensor scale = at::empty({x.size(0), x.size(1) / 128}, x.options().dtype(at::kFloat));
+    const auto opts = topk_ids.options();
+    at::Tensor sorted_ids = at::empty({sorted_num}, opts), expert_ids = at::empty({n_blocks}, opts),
+               total = at::empty({1}, opts);
+    const size_t ws_bytes = alpha_moe_align_workspace_bytes(static_cast<int>(numel), static_cast<int>(num_experts));
+    at::Tensor ws = at::empty({static_cast<int64_t>(ws_bytes)}, opts.dtype(at::kByte));
+    const int rc = alpha_moe_prepare_inputs(
+        x.const_data_ptr(), x.scalar_type() == at::kFloat, static_cast<uint8_t *>(q.data_ptr()), scale.data_ptr<float>(),
+        static_cast<int>(x.size(0)), static_cast<int>(x.size(1)), topk_ids.const_data_ptr<int32_t>(),
+        static_cast<int>(numel), static_cast<int>(num_experts), static_cast<int>(block_size), sorted_ids.data_ptr<int32_t>(),
+        static_cast<int>(sorted_num), expert_ids.data_ptr<int32_t>(), static_cast<int>(n_blocks), total.data_ptr<int32_t>(),
+        ws.data_ptr(), ws_bytes, static_cast<void *>(stream));
+    TORCH_CHECK(rc == ALPHA_MOE_OK, "alpha_moe_prepare_inputs failed: ", alpha_moe_status_string(rc));
+    return {q, scale, sorted_ids, expert_ids, total};
+}
+
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(alpha_moe, m)
@@ -296,6 +331,9 @@ TORCH_LIBRARY_FRAGMENT(alpha_moe, m)
     m.impl("per_token_group_quant_fp8", c10::DispatchKey::CUDA, &per_token_group_quant_fp8);
     m.def("moe_align_block_size(Tensor topk_ids, int block_size, int num_experts) -> (Tensor, Tensor, Tensor)");
     m.impl("moe_align_block_size", c10::DispatchKey::CUDA, &moe_align_block_size);
+    m.def("prepare_inputs(Tensor x, Tensor topk_ids, int group_size, int block_size, int num_experts) -> "
+          "(Tensor, Tensor, Tensor, Tensor, Tensor)");
+    m.impl("prepare_inputs", c10::DispatchKey::CUDA, &prepare_inputs);
     m.def("reserve_workspace(Tensor like, int bytes) -> ()");
     m.impl("reserve_workspace", c10::DispatchKey::CUDA, &reserve_workspace);
     m.def("scratch_buffers(Tensor like) -> int[]");

@@ -205,6 +205,15 @@ int alpha_moe_moe_align_block_size(const int32_t *topk_ids, int numel, int num_e
                                    int32_t *num_tokens_post_padded, void *workspace, size_t workspace_bytes,
                                    void *stream /* hipStream_t */);
 
+/*
+ * Both of the above for one layer call, with their arguments and results, in one launch less: neither needs the
+ * other's result.
+ */
+int alpha_moe_prepare_inputs(const void *x, int x_is_f32, uint8_t *q, float *scale, int M, int K, const int32_t *topk_ids,
+                             int numel, int num_experts, int block_size, int32_t *sorted_token_ids, int sorted_num,
+                             int32_t *expert_ids, int n_blocks, int32_t *num_tokens_post_padded, void *workspace,
+                             size_t workspace_bytes, void *stream /* hipStream_t */);
+
 /* Human-readable text for a status code (static storage). */
 const char *alpha_moe_status_string(int status);
 

@@ -75,6 +75,27 @@ def test_align_at_the_edges_of_its_runs_and_segments(numel, E, block):
     assert torch.equal(s_ids.cpu(), r_ids)
 
 
+@pytest.mark.parametrize("M,K,top_k,E,block,dtype", [
+    (1, 128, 1, 3, 16, torch.bfloat16),        # one group, one slot
+    (7, 7168, 9, 257, 8, torch.bfloat16),
+    (65, 2048, 10, 512, 16, torch.float32),    # an odd number of groups per thread
+    (512, 256, 8, 128, 64, torch.bfloat16),    # 4096 slots: the last size with one workgroup for the alignment
+    (513, 384, 8, 128, 64, torch.float32),     # two launches
+    (3000, 7168, 9, 257, 96, torch.bfloat16)])
+def test_prepare_inputs_equals_the_two_separate_calls(M, K, top_k, E, block, dtype):
+    from alpha_moe_python import prep_hip
+    g = torch.Generator().manual_seed(M + K)
+    x = torch.randn((M, K), generator=g).to(dtype).to(DEV)
+    ids = torch.randint(0, E, (M, top_k), generator=g, dtype=torch.int32).to(DEV)
+    print(f"case prepare M={M} K={K} top_k={top_k} E={E} {dtype}", flush=True)
+    got = prep_hip.prepare_inputs(x, ids, 128, block, E)
+    torch.cuda.synchronize()
+    q_ref, s_ref = O.quant_group_reference(x.cpu())
+    assert torch.equal(got[0].cpu().view(torch.uint8), q_ref.view(torch.uint8)) and torch.equal(got[1].cpu(), s_ref)
+    for a, b in zip(got[2:], O.align_reference(ids.cpu(), block, E)):
+        assert torch.equal(a.cpu(), b)
+
+
 def test_align_drops_slots_with_an_expert_out_of_range():
     from alpha_moe_python import prep_hip
     ids = torch.tensor([[0, 3], [7, -1], [9, 3]], dtype=torch.int32)
