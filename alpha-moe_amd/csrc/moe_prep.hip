@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256) void quant_group128_kernel(const T *__restrict
 // per bit of the expert id (same_expert) - a loop over the chunk's distinct experts, ~60 LDS round trips for 64 slots
 // of 257 experts, is what took most of 398 us for 2997 slots and of 193 us for 73 728 - and every wavefront counts and
 // places a run of slots of its own behind cursors of its own.  MI355X, kernel trace, 257 experts: 9 us for 2997 slots,
-// 17 us (two launches) for 73 728; nine slots take 5.3 us (8.1 with a serial scan over the experts).
+// 16 us (two launches) for 73 728; nine slots take 5.3 us (8.1 with a serial scan over the experts).
 typedef unsigned long long lanes_t;
 
 // The lanes of this wavefront whose slot has the same expert as this lane's (e < 0: no slot, no lanes); all 64 lanes
@@ -312,56 +312,64 @@ __global__ __launch_bounds__(256) void prepare_hist_kernel(const int32_t *__rest
     else quant_groups<T>(x, q, scale, n_groups, (int)blockIdx.x - n_seg, (int)gridDim.x - n_seg);
 }
 
-// Pass 2, one workgroup per segment: every workgroup adds the histograms up itself (columns of two experts, sixteen
-// segments in flight; a third launch of one workgroup for the sums took 17 - 42 us), scans the padded totals and places
-// its segment, each of its four wavefronts a quarter of it.
-__global__ __launch_bounds__(256) void align_place_kernel(const int32_t *__restrict__ ids, int numel, int E, int id_bits,
-                                                          int block_size, const int *__restrict__ hist, int words,
-                                                          int32_t *sorted_ids, int32_t *expert_ids, int n_blocks,
-                                                          int32_t *ntpp)
+// Pass 2, one workgroup per segment: every workgroup adds the histograms up itself (columns of two experts, the segments
+// split over the threads that share a column, sixteen in flight each; a third launch of one workgroup for the sums took
+// 17 - 42 us), scans the padded totals and places its segment, each of its n_waves wavefronts a part of it.
+// 1024 threads: every step is a dependent round trip of memory or LDS, and four times the threads take a quarter of the
+// rounds: 257 experts, 18 432 slots 13 -> 10 us, 73 728 slots 15 -> 11, 512 experts, 40 960 slots 12 -> 10 (before: 256).
+__global__ __launch_bounds__(1024) void align_place_kernel(const int32_t *__restrict__ ids, int numel, int E, int id_bits,
+                                                           int block_size, const int *__restrict__ hist, int words,
+                                                           int32_t *sorted_ids, int32_t *expert_ids, int n_blocks,
+                                                           int32_t *ntpp, int n_waves)
 {
-    // [2 words] starts | [2 words] slots of earlier segments | [4][E] cursors (16 bit; first the scan's partial sums)
+    // [2 words] starts | [2 words] slots of earlier segments | [n_waves][E] cursors (16 bit; first the scan's partial sums)
     extern __shared__ __attribute__((aligned(16))) int lds[];
     int *start = lds, *before = lds + 2 * words;
     uint16_t *cursors = reinterpret_cast<uint16_t *>(lds + 4 * words);
     const int wave = threadIdx.x >> 6, n_seg = gridDim.x, seg = blockIdx.x;
-    for (int c = threadIdx.x; c < words; c += blockDim.x) {
+    for (int i = threadIdx.x; i < 4 * words; i += blockDim.x) lds[i] = 0;
+    __syncthreads();
+    const int share = words < (int)blockDim.x ? blockDim.x / words : 1;   // threads of a column
+    const int part = words < (int)blockDim.x ? threadIdx.x / words : 0;
+    for (int c = (int)threadIdx.x - part * words; c < words && part < share; c += blockDim.x) {
         int b0 = 0, b1 = 0, t0 = 0, t1 = 0;
-        for (int s0 = 0; s0 < n_seg; s0 += 16) {
+        for (int s0 = part; s0 < n_seg; s0 += 16 * share) {
             unsigned v[16];
 #pragma unroll
-            for (int k = 0; k < 16; k++) v[k] = s0 + k < n_seg ? (unsigned)hist[(size_t)(s0 + k) * words + c] : 0u;
+            for (int k = 0; k < 16; k++) v[k] = s0 + k * share < n_seg ? (unsigned)hist[(size_t)(s0 + k * share) * words + c] : 0u;
 #pragma unroll
             for (int k = 0; k < 16; k++) {
                 const int c0 = v[k] & 0xffffu, c1 = v[k] >> 16;
                 t0 += c0;
                 t1 += c1;
-                if (s0 + k < seg) {
+                if (s0 + k * share < seg) {
                     b0 += c0;
                     b1 += c1;
                 }
             }
         }
-        start[2 * c] = pad_to(t0, block_size);
-        start[2 * c + 1] = pad_to(t1, block_size);
-        before[2 * c] = b0;
-        before[2 * c + 1] = b1;
+        atomicAdd(&start[2 * c], t0);
+        atomicAdd(&start[2 * c + 1], t1);
+        atomicAdd(&before[2 * c], b0);
+        atomicAdd(&before[2 * c + 1], b1);
     }
     __syncthreads();
+    for (int i = threadIdx.x; i < 2 * words; i += blockDim.x) start[i] = pad_to(start[i], block_size);
+    __syncthreads();
     const int total = block_exclusive_scan(start, E, lds + 4 * words);
-    for (int i = threadIdx.x; i < 2 * E; i += blockDim.x) reinterpret_cast<int *>(cursors)[i] = 0;
+    for (int i = threadIdx.x; i < (n_waves * E + 1) / 2; i += blockDim.x) reinterpret_cast<int *>(cursors)[i] = 0;
     write_blocks(start, E, block_size, total, expert_ids, n_blocks, ntpp, seg, n_seg);
     __syncthreads();
-    constexpr int kRun = kAlignSeg / 4;
-    const int lo = seg * kAlignSeg + wave * kRun, hi = min(lo + kRun, numel);
-    count_run(ids, lo, hi, E, id_bits, cursors + wave * E);
+    const int run = kAlignSeg / n_waves;
+    const int lo = seg * kAlignSeg + wave * run, hi = min(lo + run, numel);
+    if (wave < n_waves) count_run(ids, lo, hi, E, id_bits, cursors + wave * E);
     __syncthreads();
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
-        prefix_over_waves(cursors, E, e, 4);
+        prefix_over_waves(cursors, E, e, n_waves);
         start[e] += before[e];
     }
     __syncthreads();
-    place_run(ids, lo, hi, E, id_bits, start, cursors + wave * E, sorted_ids);
+    if (wave < n_waves) place_run(ids, lo, hi, E, id_bits, start, cursors + wave * E, sorted_ids);
 }
 
 // What is quantised beside an alignment (x == nullptr: nothing).
@@ -434,9 +442,12 @@ int align(const int32_t *topk_ids, int numel, int num_experts, int block_size, i
         hipLaunchKernelGGL(prepare_hist_kernel<uint16_t>, dim3(n_seg + quant_grid(z, 256)), dim3(256), words * sizeof(int),
                            hs, topk_ids, numel, E, hist, words, sorted_token_ids, sorted_num, n_seg,
                            static_cast<const uint16_t *>(z.x), z.q, z.scale, n_groups);
-    const size_t lds = (4 * words + (2 * E > 16 ? 2 * E : 16)) * sizeof(int);   // 64 KiB at kAlignMaxExperts
-    hipLaunchKernelGGL(align_place_kernel, dim3(n_seg), dim3(256), lds, hs, topk_ids, numel, E, id_bits, block_size, hist,
-                       words, sorted_token_ids, expert_ids, n_blocks, num_tokens_post_padded);
+    // sixteen wavefronts where their cursors fit 32 KiB, at least four (64 KiB of LDS in all at kAlignMaxExperts)
+    const int n_waves = E <= 1024 ? 16 : E <= 2048 ? 8 : 4;
+    const int cursor_words = (n_waves * E + 1) / 2;
+    const size_t lds = (4 * words + (cursor_words > 16 ? cursor_words : 16)) * sizeof(int);
+    hipLaunchKernelGGL(align_place_kernel, dim3(n_seg), dim3(1024), lds, hs, topk_ids, numel, E, id_bits, block_size, hist,
+                       words, sorted_token_ids, expert_ids, n_blocks, num_tokens_post_padded, n_waves);
     return hipGetLastError() == hipSuccess ? ALPHA_MOE_OK : ALPHA_MOE_ERR_LAUNCH;
 }
 

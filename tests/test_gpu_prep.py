@@ -75,6 +75,18 @@ def test_align_at_the_edges_of_its_runs_and_segments(numel, E, block):
     assert torch.equal(s_ids.cpu(), r_ids)
 
 
+@pytest.mark.parametrize("E", [1024, 1025, 2045, 2046, 2048, 2049])
+def test_align_where_the_wavefronts_of_a_segment_change(E):
+    """16, 8 and 4 wavefronts place a segment; columns of the histogram are shared by threads up to 1023 of them"""
+    from alpha_moe_python import prep_hip
+    g = torch.Generator().manual_seed(E)
+    ids = torch.randint(0, E, (4500, 1), generator=g, dtype=torch.int32)
+    print(f"case align E={E}", flush=True)
+    got = prep_hip.moe_align_block_size(ids.to(DEV), 8, E)
+    for a, b in zip(got, O.align_reference(ids, 8, E)):
+        assert torch.equal(a.cpu(), b)
+
+
 @pytest.mark.parametrize("M,K,top_k,E,block,dtype", [
     (1, 128, 1, 3, 16, torch.bfloat16),        # one group, one slot
     (7, 7168, 9, 257, 8, torch.bfloat16),
