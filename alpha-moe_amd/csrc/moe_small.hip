@@ -85,6 +85,7 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
     __shared__ __attribute__((aligned(1024))) uint8_t s_ring[kWaves * kRingBytes];
     __shared__ v4f s_red[2][TB][kWaves][64];   // partial sums
     __shared__ Active s_act;
+    __shared__ __attribute__((aligned(16))) int s_row[kMaxRows][kMaxTokens];   // s_act.row, a word each
     __shared__ short s_of_mb[kMaxRows];        // row block -> its expert's place in the list
     __shared__ __attribute__((aligned(16))) float s_ws[kWaves][2][16];   // [128-column block & 1][gate | up][K block]
     __shared__ int s_cnt[3];
@@ -128,7 +129,7 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
         x_sc[i] = 0.f;
         if (n < p.M && kb0 + i < nkb) x_sc[i] = p.x_scale[(size_t)n * nkb + kb0 + i];
     }
-    for (int i = tid; i < kMaxRows * kMaxTokens / 4; i += kThreads) reinterpret_cast<int *>(s_act.row)[i] = -1;
+    for (int i = tid; i < kMaxRows * kMaxTokens / 4; i += kThreads) reinterpret_cast<v4i *>(s_row)[i] = (v4i){255, 255, 255, 255};
     for (int i = tid; i < kMaxRows; i += kThreads) s_act.same[i] = 255;
 
     // the active experts: row blocks whose expert is not the one of the block before
@@ -217,20 +218,25 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
     }
 
     // ---- while the first tiles are on their way: which row holds a token's share of an expert ----------------------
-    // (a token that names an expert twice: one of its rows stands for both)
+    // A token that names an expert more than once: its lowest row stands for all.  (The choice must not depend on the order
+    // of the wavefronts: every workgroup makes it for itself, and the second launch reads what workgroup 0 chose.)
     auto for_rows = [&](auto f) {
         for (int idx = tid; idx < n_ids && idx < n_mb * p.block_m; idx += kThreads) {
             const int id = idx == tid ? id0 : p.sorted_ids[idx];
             const int a = s_of_mb[idx / p.block_m];
-            if (id >= 0 && id < s.rows && a >= 0) f(id, s_act.row[a][id / p.top_k]);
+            if (id >= 0 && id < s.rows && a >= 0) f(id, s_row[a][id / p.top_k]);
         }
     };
-    for_rows([&](int id, uint8_t &row) { row = (uint8_t)id; });
+    for_rows([&](int id, int &row) { atomicMin(&row, id); });
     lds_barrier();
     if (blockIdx.x == 0) {   // for the second launch
-        for_rows([&](int id, uint8_t &row) {
-            if (row != id) s_act.same[id] = row;
+        for_rows([&](int id, int &row) {
+            if (row != id) s_act.same[id] = (uint8_t)row;
         });
+        for (int i = tid; i < kMaxRows * kMaxTokens / 4; i += kThreads) {
+            const v4i r = reinterpret_cast<const v4i *>(s_row)[i];
+            reinterpret_cast<int *>(s_act.row)[i] = r.x | r.y << 8 | r.z << 16 | r.w << 24;
+        }
         if (tid == 0) {
             // A wait that ran out in an earlier launch on this workspace (sticky), or a marked control block (once): the output says so itself, NaN in every element.
             const bool marked = (s.ctl->mark & kExpiredBit) != 0;
@@ -298,7 +304,7 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
                 for (int w = 1; w < kWaves; w++) v += s_red[buf][tb][w][lane];
                 // lanes q < 2 hold the gate sums of columns 4 q .. 4 q + 3, lanes q + 2 the up sums
                 const int a = expert_of(tile_c[tb]);
-                const int row = s_act.row[a][n];
+                const int row = s_row[a][n];
                 const int col = tile_c[tb] + 4 * (q & 1);
 #pragma unroll
                 for (int j = 0; j < 4; j++) {

@@ -676,6 +676,44 @@ def test_small_kernel_at_the_edges_of_its_parts(M, E, top_k, K, I):
         assert torch.equal(run_op(P, *knobs, out=junk, via="c_abi", store=True), got)
 
 
+def _named_more_than_once(what):
+    """16 tokens' expert ids, each token naming one expert many times; where the expert's rows stand in the sorted ids."""
+    if what == 64:       # nine slots a token on one expert: token 7 holds positions 63 .. 71
+        return torch.zeros((16, 9), dtype=torch.int32)
+    ids = torch.full((16, 10), 15, dtype=torch.int32)   # fifteen blocks of one row each, then an expert with 145 rows:
+    ids[:15, 0] = torch.arange(15, dtype=torch.int32)   # with blocks of 32, token 3 holds positions 507 .. 515
+    return ids
+
+
+@pytest.mark.parametrize("edge,block_m", [(64, 8), (64, 16), (64, 32), (512, 32), (512, 16)])
+def test_small_kernel_expert_named_more_than_once_by_a_token(edge, block_m):
+    """A token's rows of one expert on both sides of a wavefront's 64 sorted ids (and of a workgroup's 512): every workgroup
+    has to take the same row for the token, so the result is the oracle's and the same in every launch.  Scratch rows start
+    as NaN: a row that nobody wrote would show."""
+    import alpha_moe
+    ids = _named_more_than_once(edge)
+    shape = Shape("dup", E=16, top_k=ids.shape[1], K=1024, I=256, shared_expert=False, routing="softmax_renorm", scaling_factor=1.5)
+    P = make_problem(make_weights(shape, device=DEV, seed=edge), 16, seed=block_m)
+    P.topk_ids = ids.to(DEV)
+    P.aligned.clear()
+    s_ids, e_ids, _ = [t.cpu() for t in P.align(block_m)]
+    if block_m == 32 or edge == 64:
+        pair = s_ids[edge - 1:edge + 1]
+        assert pair.max() < ids.numel() and pair[0] // shape.top_k == pair[1] // shape.top_k
+        assert ids.flatten()[pair[0]] == ids.flatten()[pair[1]]
+    ref = oracle_out(P)
+    need = alpha_moe.c_abi.alpha_moe_workspace_bytes(shape.top_k, P.M, shape.K, shape.N, shape.E, s_ids.numel(), block_m)
+    first = None
+    for rep in range(6):
+        print(f"case named more than once edge {edge} block_m {block_m} launch {rep}", flush=True)
+        ws = torch.full((need,), 255, dtype=torch.uint8, device=DEV)
+        ws[: alpha_moe.c_abi.alpha_moe_workspace_zero_bytes()] = 0
+        got = run_op(P, block_m, 32, 8, 4, via="c_abi", workspace=ws)
+        assert_parity(got, ref, f"named more than once {edge} {block_m}")
+        first = got if first is None else first
+        assert torch.equal(got, first), rep
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan"), 3e38])
 def test_small_kernel_requantises_what_is_not_finite_like_the_streaming_kernel(bad):
     """A token whose up/gate sums are infinite, not a number or overflow on the way: NaN and infinite elements in the same
