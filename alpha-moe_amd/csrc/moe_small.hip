@@ -53,7 +53,8 @@ constexpr int kMaxLds = 158 << 10;
 struct Active {
     int n;                                  // active experts
     int poison;                             // results on this workspace are not to be trusted: answer NaN
-    int pad[2];
+    int repeats;                            // a token names an expert more than once: `same` has entries
+    int pad;
     int expert[kMaxRows];
     uint8_t row[kMaxRows][kMaxTokens];      // [expert][token] -> (token, slot) row, 255: not routed
     uint8_t same[kMaxRows];                 // row -> the row that stands for the same (expert, token), 255: itself
@@ -131,6 +132,7 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
     }
     for (int i = tid; i < kMaxRows * kMaxTokens / 4; i += kThreads) reinterpret_cast<v4i *>(s_row)[i] = (v4i){255, 255, 255, 255};
     for (int i = tid; i < kMaxRows; i += kThreads) s_act.same[i] = 255;
+    if (tid == 0) s_act.repeats = 0;
 
     // the active experts: row blocks whose expert is not the one of the block before
     int n_mb = (__builtin_amdgcn_readfirstlane(ntpp) + p.block_m - 1) / p.block_m;
@@ -231,7 +233,10 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
     lds_barrier();
     if (blockIdx.x == 0) {   // for the second launch
         for_rows([&](int id, int &row) {
-            if (row != id) s_act.same[id] = (uint8_t)row;
+            if (row != id) {
+                s_act.same[id] = (uint8_t)row;
+                s_act.repeats = 1;
+            }
         });
         for (int i = tid; i < kMaxRows * kMaxTokens / 4; i += kThreads) {
             const v4i r = reinterpret_cast<const v4i *>(s_row)[i];
@@ -523,7 +528,14 @@ __global__ __launch_bounds__(kThreads) void moe_small_down_kernel(const SmallPar
 #pragma unroll
             for (int u = 0; u < kW2sLoads; u++)
                 if (tid + u * kThreads < n_act * n_ib * 2) s_w2s[tid + u * kThreads] = w2s_reg[u];
-            if (tid < s.rows && s_act.same[tid] != 255) atomicAdd(&s_tw[s_act.same[tid]], tw_reg);
+            // a row that stands for others of its token takes their weights over, in ascending order (a fixed one: the result
+            // does not depend on which wavefront comes first)
+            if (s_act.repeats && tid < s.rows && s_act.same[tid] == 255) {
+                float tw = tw_reg;
+                for (int r = tid + 1, end = (tid / p.top_k + 1) * p.top_k; r < end; r++)
+                    if (s_act.same[r] == tid) tw += s_tw[r];
+                s_tw[tid] = tw;
+            }
         }
         lds_barrier();
         for (int a = wave; a < n_act; a += kWaves) {

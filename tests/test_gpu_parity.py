@@ -714,6 +714,29 @@ def test_small_kernel_expert_named_more_than_once_by_a_token(edge, block_m):
         assert torch.equal(got, first), rep
 
 
+def test_small_kernel_sums_the_weights_of_a_repeated_expert_in_row_order():
+    """Token 6 names one expert ten times, rows 60 .. 69: two wavefronts' worth of weights.  In ascending order the three ones
+    vanish in 2^24 and the weights sum to 0.75; with rows 64 .. 69 first they sum to 3.75.  The same call with that sum as the
+    first row's weight and zeros behind it gives the same bits."""
+    shape = Shape("dup", E=10, top_k=10, K=512, I=128, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
+    P = make_problem(make_weights(shape, device=DEV, seed=1), 9, seed=1)
+    P.topk_ids = (torch.arange(90, dtype=torch.int32).view(9, 10) % 4).to(DEV)
+    P.topk_ids[6] = 2
+    P.aligned.clear()
+    w = P.topk_weights.clone()
+    big = 2.0 ** 24
+    w[6] = torch.tensor([big, 1, 1, 1, -big, 0.5, 0.25, 0, 0, 0], device=DEV)
+    once = w.clone()
+    once[6] = torch.tensor([0.75] + [0.0] * 9, device=DEV)
+    P.topk_weights = once
+    want = run_op(P, 16, 32, 8, 4, via="c_abi")
+    assert_parity(want, oracle_out(P), "one weight")
+    P.topk_weights = w
+    for rep in range(3):
+        print(f"case repeated expert, order of the weights, launch {rep}", flush=True)
+        assert torch.equal(run_op(P, 16, 32, 8, 4, via="c_abi"), want), rep
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan"), 3e38])
 def test_small_kernel_requantises_what_is_not_finite_like_the_streaming_kernel(bad):
     """A token whose up/gate sums are infinite, not a number or overflow on the way: NaN and infinite elements in the same
