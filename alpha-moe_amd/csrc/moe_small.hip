@@ -287,6 +287,11 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
                             f[k] = w_lo[k];
                             f[4 + k] = w_hi[k];
                         }
+                        if (kb0 + NKW > nkb) {   // past the end: nothing, also where the last block's scale is infinite
+#pragma unroll
+                            for (int k = 0; k < NKW; k++)
+                                if (kb0 + k >= nkb) f[k] = 0.f;
+                        }
                     }
                     const uint8_t *tile = ring + slot_r * 2048;
                     slot_r = slot_r + 1 == R ? 0 : slot_r + 1;

@@ -737,6 +737,26 @@ def test_small_kernel_sums_the_weights_of_a_repeated_expert_in_row_order():
         assert torch.equal(run_op(P, 16, 32, 8, 4, via="c_abi"), want), rep
 
 
+@pytest.mark.parametrize("K,block", [(1152, 8), (512, 3), (1152, 0)])
+def test_small_kernel_infinite_weight_scale_with_wavefronts_past_the_end_of_k(K, block):
+    """Nine and four K blocks over eight wavefronts: what a wavefront multiplies past the end of K is nothing, whatever scale
+    stands at the last block.  Infinite and NaN elements in the same places as from the streaming kernel."""
+    shape = Shape("small", E=6, top_k=2, K=K, I=256, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
+    W = make_weights(shape, device=DEV, seed=3)
+    W.w1_scale[1, 0, block] = float("inf")   # expert 1, the gate columns of the first slice
+    P = make_problem(W, 7, seed=4)
+    print(f"case infinite weight scale K={K} block {block}", flush=True)
+    got = run_op(P, 16, 32, 8, 4, via="c_abi")
+    with tunables(ALPHA_MOE_PATH=2):
+        want = run_op(P, 16, 32, 8, 4, via="c_abi")
+    assert not torch.isfinite(want.float()).all() and torch.isfinite(want.float()).any()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    finite = torch.isfinite(want)
+    assert torch.equal(torch.sign(got[torch.isinf(want)]), torch.sign(want[torch.isinf(want)]))
+    # (two bf16 roundings of sums in another order)
+    assert torch.allclose(got[finite].float(), want[finite].float(), rtol=2 ** -7, atol=float(want[finite].float().abs().max()) * 1e-2)
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan"), 3e38])
 def test_small_kernel_requantises_what_is_not_finite_like_the_streaming_kernel(bad):
     """A token whose up/gate sums are infinite, not a number or overflow on the way: NaN and infinite elements in the same
