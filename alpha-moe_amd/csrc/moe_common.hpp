@@ -196,15 +196,14 @@ struct StreamCtl {
     int head;        // streaming kernel: next work item
     int done;        // streaming kernel: workgroups that have left
     int epoch;       // completed launches on this workspace (any kernel family)
-    int poisoned;    // the epoch of a launch that found `mark` set (for the kernel that sums the rows)
-    int pad_e;
+    int pad_e[2];
     int tile_done;   // tile kernels: workgroups that have left
     int pad0[2];
     int tile_head[8];   // tile kernel: next work item of each of the eight queues
     int pad1a[16];
-    int mark;        // kExpiredBit: one call through the small or the streaming kernel answers NaN and clears it
+    int pad1;
     int error;       // sticky: a bounded wait ran out (word kErrorWord of the workspace)
-    int pad1[30];
+    int pad2[30];
 };
 constexpr int kErrorWord = 33;
 static_assert(sizeof(StreamCtl) == 256, "control block is one 256-byte line group");
@@ -221,8 +220,6 @@ constexpr size_t kPrefixBytes = kOffLive + sizeof(int) * kMaxSlots;
 // (measured).
 // "a >= b" for counters and epochs that wrap around: true while a is at most 2^31 - 1 steps ahead of b
 __device__ __forceinline__ bool reached(int a, int b) { return (int)((unsigned)a - (unsigned)b) >= 0; }
-
-constexpr int kExpiredBit = 1 << 30;
 
 // A whole wavefront, `count` <= 64 consecutive flags, one per lane: every poll is ONE load, so the wait costs one round
 // trip however many flags there are.

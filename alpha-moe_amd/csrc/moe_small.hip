@@ -243,11 +243,9 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
             reinterpret_cast<int *>(s_act.row)[i] = r.x | r.y << 8 | r.z << 16 | r.w << 24;
         }
         if (tid == 0) {
-            // A wait that ran out in an earlier launch on this workspace (sticky), or a marked control block (once): the output says so itself, NaN in every element.
-            const bool marked = (s.ctl->mark & kExpiredBit) != 0;
-            if (marked) s.ctl->mark = 0;
+            // a wait that ran out in an earlier launch on this workspace (sticky): the output says so itself, NaN in every element
             s_act.n = n_act;
-            s_act.poison = marked || s.ctl->error != 0;
+            s_act.poison = s.ctl->error != 0;
         }
         lds_barrier();
         for (int i = tid; i < (int)sizeof(Active) / 4; i += kThreads)

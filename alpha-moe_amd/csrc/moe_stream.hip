@@ -591,10 +591,6 @@ __global__ __launch_bounds__(WN * 64) void moe_stream_kernel(const StreamPlan s)
         if (left == (int)gridDim.x - 1) {
             store_agent(&s.ctl->head, 0);
             store_agent(&s.ctl->done, 0);
-            if (load_agent(&s.ctl->mark) & kExpiredBit) {
-                store_agent(&s.ctl->mark, 0);
-                store_agent(&s.ctl->poisoned, epoch);
-            }
             store_agent(&s.ctl->epoch, epoch);   // everybody has read the old one; the reduce kernel compares with this
         }
     }

@@ -575,7 +575,7 @@ __global__ __launch_bounds__(256) void moe_rows_reduce_kernel(const RowsReduce s
     // sticky) means result rows may be missing: the output then says so itself, NaN in every element
     // (an ordinary load: this kernel starts after the other has ended, and every wavefront asking the memory side
     // for the same word with an agent-scope load cost ~100 us per call)
-    const bool poisoned = s.ctl->error != 0 || (F32 && s.ctl->poisoned == epoch);
+    const bool poisoned = s.ctl->error != 0;
     const int t = blockIdx.x / chunks_per_token;
     const int c = (((int)blockIdx.x - t * chunks_per_token) * 256 + (int)threadIdx.x) * COLS;
     if (c >= p.K) return;

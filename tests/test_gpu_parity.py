@@ -530,7 +530,7 @@ def test_nothing_routed(c1, knobs):
 
 
 def test_workspace_check_reports_an_expired_wait(c1):
-    """alpha_moe_workspace_check: 0 after ordinary launches of both kernels; 8 once the sticky word that a workgroup
+    """alpha_moe_workspace_check: 0 after ordinary launches of every kernel family; 8 once the sticky word that a workgroup
     writes when its bounded wait runs out is set (set here from the host: no kernel is made to wait)."""
     import alpha_moe
     P, ref = c1
@@ -538,30 +538,46 @@ def test_workspace_check_reports_an_expired_wait(c1):
                                                          P.align(bm)[0].numel(), bm) for bm in (16, 64))
     ws = torch.zeros(need, dtype=torch.uint8, device=DEV)
     stream = torch.cuda.current_stream().cuda_stream
-    for knobs in ((16, 32, 8, 5), (64, 64, 4, 3)):
-        assert_parity(run_op(P, *knobs, via="c_abi", workspace=ws), ref, f"knobs {knobs}")
+    families = ((2, (16, 32, 8, 5)), (5, (16, 32, 8, 5)), (3, (64, 64, 4, 3)), (4, (64, 32, 8, 2)))   # streaming, small, tile, wide
+    for path, knobs in families:
+        with tunables(ALPHA_MOE_PATH=path):
+            assert_parity(run_op(P, *knobs, via="c_abi", workspace=ws), ref, f"path {path} knobs {knobs}")
         assert alpha_moe.c_abi.alpha_moe_workspace_check(ws.data_ptr(), stream) == 0
     error_word = 33   # the control block's sticky error word (kErrorWord in csrc/moe_common.hpp)
     ws.view(torch.int32)[error_word] = 1
     rc = alpha_moe.c_abi.alpha_moe_workspace_check(ws.data_ptr(), stream)
     assert rc == 8 and b"wait" in alpha_moe.c_abi.alpha_moe_status_string(rc)
     # while the word is set, every call on the workspace says so in its output: NaN everywhere, adding or storing,
-    # from the streaming kernel and from the tile kernel
-    for knobs in ((16, 32, 8, 5), (64, 64, 4, 3)):
+    # from every kernel family that works on it
+    for path, knobs in families:
         for store in (False, True):
-            got = run_op(P, *knobs, via="c_abi", workspace=ws, store=store)
-            assert torch.isnan(got.float()).all(), (knobs, store)
+            with tunables(ALPHA_MOE_PATH=path):
+                got = run_op(P, *knobs, via="c_abi", workspace=ws, store=store)
+            assert torch.isnan(got.float()).all(), (path, knobs, store)
     ws.view(torch.int32)[error_word] = 0
-    assert_parity(run_op(P, 16, 32, 8, 5, via="c_abi", workspace=ws), ref, "after clearing the error word")
-    # An expiry DURING a launch of the streaming kernel reaches the closing items through the counter they poll: the
-    # waiter sets a high bit in it (an OR, so the value below is what the kernel produces).  Set from the host here, the bit makes that one launch answer NaN (its closing items
-    # do not wait and do not trust what they read); the launch resets the counter, and the next one is clean again.
-    down_counter, expired_bit = 32, 1 << 30   # StreamCtl::down_done and kExpiredBit in csrc/moe_common.hpp
-    ws.view(torch.int32)[down_counter] = expired_bit
-    got = run_op(P, 16, 32, 8, 5, via="c_abi", workspace=ws)
-    assert torch.isnan(got.float()).all()
-    assert_parity(run_op(P, 16, 32, 8, 5, via="c_abi", workspace=ws), ref, "the launch after a marked counter")
+    for path, knobs in families:
+        with tunables(ALPHA_MOE_PATH=path):
+            assert_parity(run_op(P, *knobs, via="c_abi", workspace=ws), ref, f"path {path} after clearing the error word")
     assert alpha_moe.c_abi.alpha_moe_workspace_check(ws.data_ptr(), stream) == 0
+
+
+@pytest.mark.parametrize("path,knobs", [(2, (16, 32, 8, 5)), (5, (16, 32, 8, 5)), (3, (64, 64, 4, 3)), (4, (64, 32, 8, 2))])
+def test_epoch_of_a_workspace_may_wrap(c1, path, knobs):
+    """Four calls over the wrap of the launch epoch: stamps of 2^32 - 1 earlier launches, nothing wrong on the workspace."""
+    import alpha_moe
+    P, ref = c1
+    need = alpha_moe.c_abi.alpha_moe_workspace_bytes(P.shape.top_k, P.M, P.shape.K, P.shape.N, P.shape.E,
+                                                     P.align(knobs[0])[0].numel(), knobs[0])
+    ws = torch.zeros(need, dtype=torch.uint8, device=DEV)
+    words = ws[: alpha_moe.c_abi.alpha_moe_workspace_zero_bytes()].view(torch.int32)
+    epoch_word, flags = 2, 64 + 65536   # StreamCtl::epoch; the flags and stamps behind the arrival counters
+    words[flags:] = -2
+    words[epoch_word] = -2
+    for call in range(4):
+        print(f"case epoch wrap path {path} call {call}", flush=True)
+        with tunables(ALPHA_MOE_PATH=path):
+            assert_parity(run_op(P, *knobs, via="c_abi", workspace=ws), ref, f"path {path} call {call}")
+    assert alpha_moe.c_abi.alpha_moe_workspace_check(ws.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
 
 
 def test_queue_survives_a_grid_the_device_cannot_hold(ds_weights):
