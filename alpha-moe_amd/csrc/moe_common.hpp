@@ -186,8 +186,8 @@ __device__ __forceinline__ void store_agent(int *p, int v)
 
 // ---- workspace prefix shared by the kernel families --------------------------------------------------------
 // The first kPrefixBytes of the workspace are zero-initialised by the caller once and maintained by the kernels:
-// counters return to zero by themselves, flags are stamped with a launch epoch that grows by one per launch and is
-// compared modulo 2^32 (reached()), so it may wrap.  Its size does not depend on the problem, so calls of different
+// counters return to zero by themselves, flags are stamped with a launch epoch that grows by one per launch
+// and may wrap (next_epoch()).  Its size does not depend on the problem, so calls of different
 // sizes can share one buffer.
 constexpr int kMaxUnits = 1 << 16;   // most (row block, slice) units of one streaming launch
 constexpr int kMaxSlots = 1 << 18;   // most (token, slot) rows whose results go through per-slot rows
@@ -218,17 +218,19 @@ constexpr size_t kPrefixBytes = kOffLive + sizeof(int) * kMaxSlots;
 // the control block instead of a hang.  The sleep grows from 0.1 us to 0.9 us: a hundred workgroups polling one address
 // every 0.2 us keep that L2 channel busy enough to slow the loads of the workgroups still streaming weights threefold
 // (measured).
-// "a >= b" for counters and epochs that wrap around: true while a is at most 2^31 - 1 steps ahead of b
-__device__ __forceinline__ bool reached(int a, int b) { return (int)((unsigned)a - (unsigned)b) >= 0; }
+// The stamp of a launch: the launches before it on this workspace, and one more.  Never 0, which is what a flag or a slot
+// holds that no launch has stamped yet; flags and slots are compared for equality, so nothing else is up either, however
+// many launches ago it was stamped.
+__device__ __forceinline__ int next_epoch(int epoch) { return epoch == -1 ? 1 : epoch + 1; }
 
 // A whole wavefront, `count` <= 64 consecutive flags, one per lane: every poll is ONE load, so the wait costs one round
 // trip however many flags there are.
-__device__ __noinline__ inline void spin_all_ge(const int *addr, int count, int target, StreamCtl *ctl)
+__device__ __noinline__ inline void spin_all_eq(const int *addr, int count, int target, StreamCtl *ctl)
 {
     const int lane = threadIdx.x & 63;
     for (int it = 0; it < (1 << 22); it++) {
         const int v = lane < count ? load_agent(addr + lane) : target;
-        if (__all(reached(v, target))) {
+        if (__all(v == target)) {
             acquire_fence();
             return;
         }

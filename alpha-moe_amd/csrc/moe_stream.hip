@@ -149,7 +149,7 @@ __global__ __launch_bounds__(WN * 64) void moe_stream_kernel(const StreamPlan s)
     const int n_up = n_units * s.ks;
     const int n_down = n_mb * s.n_cs;
     const int total = n_up + n_down;
-    const int epoch = (int)((unsigned)__builtin_amdgcn_readfirstlane(s.ctl->epoch) + 1u);
+    const int epoch = next_epoch(__builtin_amdgcn_readfirstlane(s.ctl->epoch));
     const uint8_t *dummy = p.x;   // where loads past the end of an item are pointed: always mapped, always cached
 
     auto read_tile = [&](const uint8_t *tile) -> v8i {
@@ -447,7 +447,7 @@ __global__ __launch_bounds__(WN * 64) void moe_stream_kernel(const StreamPlan s)
             }
             prime();
             // rare (a DOWN item is queued long after the UP items it needs): a poll returns behind the ring's loads
-            if (!__all(reached(flag0, epoch))) spin_all_ge(&s.flag[mb * n_ib], n_ib, epoch, s.ctl);
+            if (!__all(flag0 == epoch)) spin_all_eq(&s.flag[mb * n_ib], n_ib, epoch, s.ctl);
 
             // requantised activations of all slices -> LDS as operand tiles, their scales -> s_xs[row][ib]
             for (int i = wave; i < n_ib * TM; i += WN) {

@@ -156,7 +156,7 @@ __global__ __launch_bounds__(512) void moe_tile_kernel(const TileParams s)
     const int q = lane >> 4;
     const int K = p.K, I = p.N >> 1;
     const int n_ib = s.n_ib, nkb = s.nkb;
-    const int epoch = (int)((unsigned)__builtin_amdgcn_readfirstlane(s.ctl->epoch) + 1u);
+    const int epoch = next_epoch(__builtin_amdgcn_readfirstlane(s.ctl->epoch));
     uint8_t *a_ring = lds_dyn + w * (kStages * 8192);
     uint8_t *xbuf = lds_dyn + kARingBytes;
 
@@ -401,7 +401,7 @@ __global__ __launch_bounds__(512) void moe_tile_kernel(const TileParams s)
         // the weights do not depend on the up/gate phase: first two steps go out before the wait
         issue2(0);
         issue2(1);
-        if (wave == 0) spin_all_ge(&s.flag[mb * n_ib], n_ib, epoch, s.ctl);
+        if (wave == 0) spin_all_eq(&s.flag[mb * n_ib], n_ib, epoch, s.ctl);
         __syncthreads();
         // the requantised tiles of this part and their scales come from scratch into LDS: [slice][tile of the part]
         uint8_t *aq = xbuf;

@@ -436,7 +436,7 @@ __global__ __launch_bounds__(512) void moe_wide_kernel(const WideParams s)
     const int q = lane >> 4;
     const int K = p.K, I = p.N >> 1;
     const int n_ib = s.n_ib, nkb = s.nkb;
-    const int epoch = (int)((unsigned)rfl(s.ctl->epoch) + 1u);
+    const int epoch = next_epoch(rfl(s.ctl->epoch));
     uint8_t *a_ring = lds_dyn;
     uint8_t *xbuf = lds_dyn + 2 * kWStageA;
 
@@ -903,7 +903,7 @@ __global__ __launch_bounds__(512) void moe_wide_kernel(const WideParams s)
         // the weights do not depend on the up/gate phase: the first step's go out before the wait
 #pragma unroll
         for (int i = 0; i < 4; i++) issue_op(0, i);
-        if (wave == 0) spin_all_ge(&s.flag[mc.mb0 * n_ib], n_ib, epoch, s.ctl);
+        if (wave == 0) spin_all_eq(&s.flag[mc.mb0 * n_ib], n_ib, epoch, s.ctl);
         __syncthreads();
         n_tiles = tiles_of();
         const int nt_w = n_tiles > g ? (n_tiles - g + 1) >> 1 : 0;

@@ -562,8 +562,10 @@ def test_workspace_check_reports_an_expired_wait(c1):
 
 
 @pytest.mark.parametrize("path,knobs", [(2, (16, 32, 8, 5)), (5, (16, 32, 8, 5)), (3, (64, 64, 4, 3)), (4, (64, 32, 8, 2))])
-def test_epoch_of_a_workspace_may_wrap(c1, path, knobs):
-    """Four calls over the wrap of the launch epoch: stamps of 2^32 - 1 earlier launches, nothing wrong on the workspace."""
+@pytest.mark.parametrize("epoch,stamps", [(-2, -2), (-2, 0), (2 ** 31 - 2, 0), (2 ** 31 - 2, -(2 ** 31) + 5)])
+def test_epoch_of_a_workspace_may_wrap(c1, path, knobs, epoch, stamps):
+    """Four calls over the wrap of the launch epoch and over its change of sign.  Flags and slots hold the stamp of an earlier
+    launch or none (0): no item may take them for this launch's, and a slot that was never written adds nothing."""
     import alpha_moe
     P, ref = c1
     need = alpha_moe.c_abi.alpha_moe_workspace_bytes(P.shape.top_k, P.M, P.shape.K, P.shape.N, P.shape.E,
@@ -571,12 +573,22 @@ def test_epoch_of_a_workspace_may_wrap(c1, path, knobs):
     ws = torch.zeros(need, dtype=torch.uint8, device=DEV)
     words = ws[: alpha_moe.c_abi.alpha_moe_workspace_zero_bytes()].view(torch.int32)
     epoch_word, flags = 2, 64 + 65536   # StreamCtl::epoch; the flags and stamps behind the arrival counters
-    words[flags:] = -2
-    words[epoch_word] = -2
-    for call in range(4):
-        print(f"case epoch wrap path {path} call {call}", flush=True)
+    words[flags:] = stamps
+    words[epoch_word] = epoch
+    # the first half of the slots stay without an expert: their rows are whatever scratch holds
+    s_ids, e_ids, total = P.align(knobs[0])
+    half = s_ids.numel() // knobs[0] // 2
+    P.aligned[knobs[0]] = (s_ids, torch.where(torch.arange(e_ids.numel(), device=DEV) < half, -1, e_ids).to(torch.int32), total)
+    try:
         with tunables(ALPHA_MOE_PATH=path):
-            assert_parity(run_op(P, *knobs, via="c_abi", workspace=ws), ref, f"path {path} call {call}")
+            want = run_op(P, *knobs, via="c_abi")
+            ws[alpha_moe.c_abi.alpha_moe_workspace_zero_bytes():] = 255
+            for call in range(4):
+                print(f"case epoch {epoch} stamps {stamps} path {path} call {call}", flush=True)
+                assert torch.equal(run_op(P, *knobs, via="c_abi", workspace=ws), want), call
+    finally:
+        P.aligned.clear()
+    assert torch.isfinite(want.float()).all()
     assert alpha_moe.c_abi.alpha_moe_workspace_check(ws.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
 
 
