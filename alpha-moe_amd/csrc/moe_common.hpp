@@ -186,7 +186,7 @@ __device__ __forceinline__ void store_agent(int *p, int v)
 
 // ---- workspace prefix shared by the kernel families --------------------------------------------------------
 // The first kPrefixBytes of the workspace are zero-initialised by the caller once and maintained by the kernels:
-// counters return to zero by themselves, flags are stamped with a launch epoch that grows by one per launch
+// counters return to zero by themselves, flags are stamped with a launch epoch that grows with every launch
 // and may wrap (next_epoch()).  Its size does not depend on the problem, so calls of different
 // sizes can share one buffer.
 constexpr int kMaxUnits = 1 << 16;   // most (row block, slice) units of one streaming launch
@@ -195,7 +195,7 @@ constexpr int kMaxSlots = 1 << 18;   // most (token, slot) rows whose results go
 struct StreamCtl {
     int head;        // streaming kernel: next work item
     int done;        // streaming kernel: workgroups that have left
-    int epoch;       // completed launches on this workspace (any kernel family)
+    int epoch;       // stamp of the last completed launch on this workspace (any kernel family)
     int pad_e[2];
     int tile_done;   // tile kernels: workgroups that have left
     int pad0[2];
@@ -218,19 +218,22 @@ constexpr size_t kPrefixBytes = kOffLive + sizeof(int) * kMaxSlots;
 // the control block instead of a hang.  The sleep grows from 0.1 us to 0.9 us: a hundred workgroups polling one address
 // every 0.2 us keep that L2 channel busy enough to slow the loads of the workgroups still streaming weights threefold
 // (measured).
-// The stamp of a launch: the launches before it on this workspace, and one more.  Never 0, which is what a flag or a slot
-// holds that no launch has stamped yet; flags and slots are compared for equality, so nothing else is up either, however
-// many launches ago it was stamped.
-__device__ __forceinline__ int next_epoch(int epoch) { return epoch == -1 ? 1 : epoch + 1; }
+// The stamp of a launch from that of the launch before it on this workspace: the odd numbers in turn, so never 0, which is
+// what a flag or a slot holds that no launch has stamped yet.  Flags and slots are compared for equality: nothing else is
+// up either, however many launches ago it was stamped.  (Without a branch: a comparison and a select here cost the wide
+// kernel's calls 7 - 10 %, again through its registers.)
+__device__ __forceinline__ int next_epoch(int epoch) { return (int)((unsigned)epoch + 2u) | 1; }
 
-// A whole wavefront, `count` <= 64 consecutive flags, one per lane: every poll is ONE load, so the wait costs one round
-// trip however many flags there are.
+// A whole wavefront, consecutive flags, one per lane: every poll is ONE load for up to 64 flags, so the wait costs one round
+// trip however many of them there are.  (The wide kernel's registers depend on those this function uses: handing the flags
+// out 64 at a time around the loop instead cost its calls 3 %.)
 __device__ __noinline__ inline void spin_all_eq(const int *addr, int count, int target, StreamCtl *ctl)
 {
     const int lane = threadIdx.x & 63;
     for (int it = 0; it < (1 << 22); it++) {
-        const int v = lane < count ? load_agent(addr + lane) : target;
-        if (__all(v == target)) {
+        bool up = true;
+        for (int i = lane; i < count; i += 64) up &= load_agent(addr + i) == target;
+        if (__all(up)) {
             acquire_fence();
             return;
         }
