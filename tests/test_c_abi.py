@@ -135,3 +135,16 @@ def test_prep_entry_points_refuse_bad_arguments_without_touching_a_device(lib):
     assert lib.alpha_moe_moe_align_block_size(8, 32, 5000, 16, 8, 32 + 5000 * 15, 8, 4690, 8, None, 0, None) == 2
     # more than 4096 slots need the scratch buffer
     assert lib.alpha_moe_moe_align_block_size(8, 5000, 8, 16, 8, 5120, 8, 320, 8, None, 0, None) == 7
+
+
+def test_static_scratch_holds_every_batch_up_to_the_documented_sizes(lib):
+    """With the shipped tables the entry point without a workspace takes every batch up to these sizes, also where a table
+    keeps the streaming kernel and its fp32 rows (Qwen3-Next shard, 752 .. 768 tokens: 65.4 MiB)."""
+    from alpha_moe_python.utils import get_best_config
+    limit = int(re.search(r"ALPHA_MOE_STATIC_SCRATCH_BYTES \(\(size_t\)(\d+) << 20\)", open(HEADER).read()).group(1)) << 20
+    for E, N, K, top_k, upto in ((257, 512, 7168, 9, 250), (512, 512, 2048, 10, 1355), (128, 1536, 2048, 8, 1565)):
+        table = os.path.join(ROOT, "alpha-moe_amd", "configs", f"moe_jit_{E}_{N}_{K}.json")
+        for M in range(1, upto + 2):
+            bm = get_best_config(table, M)["block_m"]
+            need = lib.alpha_moe_workspace_bytes(top_k, M, K, N, E, M * top_k + E * (bm - 1), bm)
+            assert (need <= limit) == (M <= upto), (E, M, need)

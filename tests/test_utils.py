@@ -130,3 +130,14 @@ def test_sglang_weight_loader_bookkeeping():
         done.append(il.shard_loaded(param[e], e, shard))
     assert done == [False, False, False, True, True, True]
     assert torch.equal(param, interleave_tensor(ckpt, 8))
+
+
+def test_shipped_tables_keep_fp32_rows_where_they_had_them():
+    """Up to 32-row blocks a token's per-slot rows are summed in fp32, above they are rounded to bf16 once more.  No caller of
+    the layer call chose the entry, so an entry may not move a batch size to the less exact kernels: the largest batch that
+    each table serves in fp32, and none above it."""
+    configs = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "alpha-moe_amd", "configs")
+    for name, largest in (("moe_jit_257_512_7168.json", 384), ("moe_jit_512_512_2048.json", 768), ("moe_jit_128_1536_2048.json", 384)):
+        for M in range(1, 8193):
+            small_blocks = get_best_config(os.path.join(configs, name), M)["block_m"] <= 32
+            assert small_blocks == (M <= largest), (name, M)
