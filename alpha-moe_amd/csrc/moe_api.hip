@@ -42,9 +42,9 @@ void load_tunables_once()
 
 enum Path { kDirect, kStream, kTile, kWide, kSmall };
 
-// At most 16 tokens: small kernels.  Streaming kernel for row blocks of at most 32 rows (decode); above that (prefill) warp_n picks the token tiles a
-// wavefront multiplies per step: 8 -> wide kernel (macro blocks of 256 rows), 4 -> tile kernel (one row block).  The
-// direct kernel is the fallback for shapes none of them takes.
+// At most 16 tokens: small kernels where they are ahead (small_pays).  Streaming kernel for row blocks of at most 32 rows
+// (decode); above that (prefill) warp_n picks the token tiles a wavefront multiplies per step: 8 -> wide kernel (macro blocks
+// of 256 rows), 4 -> tile kernel (one row block).  The direct kernel is the fallback for shapes none of them takes.
 Path choose_path(int top_k, int M, int K, int N, int E, int sorted_num, int block_m, int warp_n)
 {
     const bool s_ok = stream_supported(top_k, M, K, N, E, sorted_num, block_m);
@@ -55,7 +55,8 @@ Path choose_path(int top_k, int M, int K, int N, int E, int sorted_num, int bloc
     if (f == 2 && s_ok) return kStream;
     if (f == 3 && t_ok) return kTile;
     if (f == 4 && w_ok) return kWide;
-    if ((f == 0 || f == 5) && small_supported(top_k, M, K, N, block_m)) return kSmall;
+    const bool small_ok = small_supported(top_k, M, K, N, block_m);
+    if (small_ok && (f == 5 || (f == 0 && (!s_ok || small_pays(top_k, M, K, N, E))))) return kSmall;
     if (s_ok) return kStream;
     if (w_ok && (warp_n == 8 || !t_ok)) return kWide;
     if (t_ok) return kTile;

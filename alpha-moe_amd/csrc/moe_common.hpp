@@ -274,6 +274,7 @@ hipError_t launch_finalize(const MoeParams &p, hipStream_t stream);   // out = b
 
 // Two launches for at most 16 tokens: UP work split over w1 rows, DOWN work over output columns; block_m <= 32.
 bool small_supported(int top_k, int M, int K, int N, int block_m);
+bool small_pays(int top_k, int M, int K, int N, int E);   // ahead of the streaming kernel
 size_t small_workspace_bytes(int top_k, int M, int N);
 hipError_t launch_small(const MoeParams &p, void *workspace, hipStream_t stream);
 

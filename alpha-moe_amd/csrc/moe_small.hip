@@ -697,6 +697,21 @@ hipError_t allow_dynamic_lds(int h, int ring, SmallFn fn)
 
 bool small_supported(int top_k, int M, int K, int N, int block_m) { return make_plan(top_k, M, K, N, block_m).ok; }
 
+// Every part of the second launch quantises all rows and walks all experts' slices, whatever K is: on narrow layers with many
+// rows that chain takes longer than the streaming kernel's whole call; on wide ones the weights' bytes hide it.  With
+// u = (4 min(E, rows) + rows) I / 5, a measure of that chain, the small kernels are ahead while u (1 - K / 2496) is at most
+// 19 Ki.  MI355X, cold weights, small / streaming us a call, experts drawn evenly: K = 512, I = 512: 32 rows (u 16 Ki) 21.8 /
+// 23.1, 64 (32 Ki) 28.3 / 24.9, 160 (80 Ki) 57.3 / 36.5; K = 1024, I = 256: 96 rows (24 Ki) 28.2 / 34.7, 128 (32 Ki) 31.8 / 31.5,
+// 160 (40 Ki) 39.9 / 34.4; K = 1536, I = 768: 64 rows (48 Ki) 47.6 / 51.2, 96 (72 Ki) 58.8 / 55.3; K = 2048, I = 768: 64 rows
+// (48 Ki) 54.1 / 58.1, 128 (96 Ki) 77.4 / 76.5 (with Zipf popularity 60.0 / 58.9, 112 rows 53.9 / 54.9); from K = 3072 on the
+// small kernels take at most 1.06 of the streaming kernel's time, mostly 0.65 - 0.95 (K = 5120 and 6144, 128 rows of I = 256:
+// 68 / 73 and 74 / 82).
+bool small_pays(int top_k, int M, int K, int N, int E)
+{
+    const long long rows = (long long)M * top_k, u5 = (4 * (rows < E ? rows : E) + rows) * (N / 2);
+    return K >= 2496 || u5 * (2496 - K) <= 5ll * 19456 * 2496;
+}
+
 size_t small_workspace_bytes(int top_k, int M, int N)
 {
     return align_up(kPrefixBytes) + align_up(sizeof(Active)) + align_up((size_t)M * top_k * (N / 2) * sizeof(uint16_t));

@@ -703,17 +703,38 @@ def test_tiny_batches(name, ds_weights, qn_weights):
                                             (2, 2, 2, 7168, 128)])
 def test_small_kernel_at_the_edges_of_its_parts(M, E, top_k, K, I):
     """At most 16 tokens: ranges of intermediate columns of unequal tiles, output ranges across scale blocks, several row
-    blocks of one expert (block_m 8), adding and storing, two launches bit for bit, against the oracle."""
+    blocks of one expert (block_m 8), adding and storing, two launches bit for bit, against the oracle.  (Where the streaming
+    kernel is ahead the small kernels are asked for.)"""
     shape = Shape("small", E=E, top_k=top_k, K=K, I=I, shared_expert=False, routing="softmax_renorm", scaling_factor=1.3)
     P = make_problem(make_weights(shape, device=DEV, seed=M + K), M, seed=9)
     refs = oracle_variants(P)
     for knobs in ((16, 32, 8, 4), (8, 64, 4, 2), (32, 32, 8, 1)):
         print(f"case small M={M} E={E} K={K} I={I} knobs {knobs}", flush=True)
-        got = run_op(P, *knobs, via="c_abi")
-        assert_parity_rows(got, refs, f"small {knobs}")
-        assert torch.equal(got, run_op(P, *knobs, via="c_abi"))
-        junk = torch.full((M, K), float("nan"), dtype=torch.bfloat16, device=DEV)
-        assert torch.equal(run_op(P, *knobs, out=junk, via="c_abi", store=True), got)
+        with tunables(ALPHA_MOE_PATH=5):
+            got = run_op(P, *knobs, via="c_abi")
+            assert_parity_rows(got, refs, f"small {knobs}")
+            assert torch.equal(got, run_op(P, *knobs, via="c_abi"))
+            junk = torch.full((M, K), float("nan"), dtype=torch.bfloat16, device=DEV)
+            assert torch.equal(run_op(P, *knobs, out=junk, via="c_abi", store=True), got)
+
+
+@pytest.mark.parametrize("M,E,top_k,K,I,small", [(8, 64, 4, 512, 512, True), (16, 64, 4, 512, 512, False),      # u 16 Ki, 32 Ki
+                                                  (11, 128, 8, 1024, 256, True), (16, 256, 10, 1024, 256, False),   # 22, 40
+                                                  (8, 128, 8, 1536, 768, True), (12, 128, 8, 1536, 768, False),    # 48, 72
+                                                  (16, 128, 8, 2048, 768, True), (16, 256, 10, 2048, 768, False),   # 96, 120
+                                                  (16, 256, 10, 2560, 768, True)])
+def test_which_kernel_serves_sixteen_tokens(M, E, top_k, K, I, small):
+    """Both sides of the line between the small kernels and the streaming kernel, against the oracle.  The streaming kernel
+    stamps the workspace (StreamCtl::epoch), the small ones do not."""
+    import alpha_moe
+    shape = Shape("line", E=E, top_k=top_k, K=K, I=I, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
+    P = make_problem(make_weights(shape, device=DEV, seed=M), M, seed=2)
+    need = alpha_moe.c_abi.alpha_moe_workspace_bytes(top_k, M, K, shape.N, E, P.align(16)[0].numel(), 16)
+    ws = torch.zeros(need, dtype=torch.uint8, device=DEV)
+    print(f"case line M={M} E={E} K={K} I={I}", flush=True)
+    got = run_op(P, 16, 32, 8, 4, via="c_abi", workspace=ws)
+    assert (ws.view(torch.int32)[2].item() == 0) == small
+    assert_parity_rows(got, oracle_variants(P), "line")
 
 
 def _named_more_than_once(what):
@@ -748,7 +769,8 @@ def test_small_kernel_expert_named_more_than_once_by_a_token(edge, block_m):
         print(f"case named more than once edge {edge} block_m {block_m} launch {rep}", flush=True)
         ws = torch.full((need,), 255, dtype=torch.uint8, device=DEV)
         ws[: alpha_moe.c_abi.alpha_moe_workspace_zero_bytes()] = 0
-        got = run_op(P, block_m, 32, 8, 4, via="c_abi", workspace=ws)
+        with tunables(ALPHA_MOE_PATH=5):
+            got = run_op(P, block_m, 32, 8, 4, via="c_abi", workspace=ws)
         assert_parity(got, ref, f"named more than once {edge} {block_m}")
         first = got if first is None else first
         assert torch.equal(got, first), rep
@@ -786,7 +808,8 @@ def test_small_kernel_infinite_weight_scale_with_wavefronts_past_the_end_of_k(K,
     W.w1_scale[1, 0, block] = float("inf")   # expert 1, the gate columns of the first slice
     P = make_problem(W, 7, seed=4)
     print(f"case infinite weight scale K={K} block {block}", flush=True)
-    got = run_op(P, 16, 32, 8, 4, via="c_abi")
+    with tunables(ALPHA_MOE_PATH=5):
+        got = run_op(P, 16, 32, 8, 4, via="c_abi")
     with tunables(ALPHA_MOE_PATH=2):
         want = run_op(P, 16, 32, 8, 4, via="c_abi")
     assert not torch.isfinite(want.float()).all() and torch.isfinite(want.float()).any()
@@ -803,11 +826,13 @@ def test_small_kernel_requantises_what_is_not_finite_like_the_streaming_kernel(b
     places as from the streaming kernel, the other tokens' rows untouched."""
     shape = Shape("small", E=6, top_k=2, K=512, I=256, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
     P = make_problem(make_weights(shape, device=DEV, seed=3), 5, seed=4)
-    clean = run_op(P, 16, 32, 8, 4, via="c_abi")
+    with tunables(ALPHA_MOE_PATH=5):
+        clean = run_op(P, 16, 32, 8, 4, via="c_abi")
     P.x_scale = P.x_scale.clone()
     P.x_scale[2, 1] = bad
     print(f"case not finite {bad}", flush=True)
-    got = run_op(P, 16, 32, 8, 4, via="c_abi")
+    with tunables(ALPHA_MOE_PATH=5):
+        got = run_op(P, 16, 32, 8, 4, via="c_abi")
     with tunables(ALPHA_MOE_PATH=2):
         want = run_op(P, 16, 32, 8, 4, via="c_abi")
     rest = [0, 1, 3, 4]
