@@ -14,7 +14,10 @@
 namespace alpha_moe {
 namespace {
 
-constexpr int kAlignSeg = 1024;        // routing slots per workgroup of the histogram and placement kernels
+constexpr int kAlignSeg = 1024;        // routing slots per workgroup (segment) of the histogram and placement kernels, and
+constexpr int kAlignMaxSeg = 512;      // most segments before they get longer: every workgroup reads all segments' histograms
+                                       // (4 Mi slots, 4096 experts: 10.2 ms in 4096 segments, 272 us in 512;
+                                       // 600 000 slots, 257 experts: 42 us in 586, 26 in 293)
 constexpr int kAlignSmall = 4096;      // most routing slots one workgroup aligns by itself (9 us near there; two launches: 13)
 constexpr int kAlignMaxExperts = 4096;
 
@@ -273,15 +276,15 @@ __global__ __launch_bounds__(1024) void prepare_small_kernel(const AlignSmall a,
     else quant_groups<T>(x, q, scale, n_groups, (int)blockIdx.x - 1, (int)gridDim.x - 1);
 }
 
-// Larger inputs, pass 1: one workgroup per segment of kAlignSeg slots writes the segment's expert histogram (16-bit
+// Larger inputs, pass 1: one workgroup per segment of `seg` slots writes the segment's expert histogram (16-bit
 // counts, two per word); also the sentinel fill.
 __device__ __forceinline__ void align_hist(const int32_t *__restrict__ ids, int numel, int E, int *hist, int words,
-                                           int32_t *sorted_ids, int sorted_num, int n_seg)
+                                           int32_t *sorted_ids, int sorted_num, int n_seg, int seg)
 {
     extern __shared__ int lds[];   // [words]
     for (int i = threadIdx.x; i < words; i += blockDim.x) lds[i] = 0;
     __syncthreads();
-    const int lo = blockIdx.x * kAlignSeg, hi = min(lo + kAlignSeg, numel);
+    const int lo = blockIdx.x * seg, hi = min(lo + seg, numel);
     for (int i = lo + threadIdx.x; i < hi; i += blockDim.x) {
         const int e = ids[i];
         if (e >= 0 && e < E) atomicAdd(&lds[e >> 1], 1 << (16 * (e & 1)));
@@ -292,19 +295,19 @@ __device__ __forceinline__ void align_hist(const int32_t *__restrict__ ids, int 
 }
 
 __global__ __launch_bounds__(256) void align_hist_kernel(const int32_t *__restrict__ ids, int numel, int E, int *hist,
-                                                         int words, int32_t *sorted_ids, int sorted_num)
+                                                         int words, int32_t *sorted_ids, int sorted_num, int seg)
 {
-    align_hist(ids, numel, E, hist, words, sorted_ids, sorted_num, gridDim.x);
+    align_hist(ids, numel, E, hist, words, sorted_ids, sorted_num, gridDim.x, seg);
 }
 
 // Pass 1 and the quantiser in one launch: the first n_seg workgroups count, the others quantise.
 template <typename T>
 __global__ __launch_bounds__(256) void prepare_hist_kernel(const int32_t *__restrict__ ids, int numel, int E, int *hist,
-                                                           int words, int32_t *sorted_ids, int sorted_num, int n_seg,
+                                                           int words, int32_t *sorted_ids, int sorted_num, int n_seg, int seg,
                                                            const T *__restrict__ x, uint8_t *__restrict__ q,
                                                            float *__restrict__ scale, long long n_groups)
 {
-    if ((int)blockIdx.x < n_seg) align_hist(ids, numel, E, hist, words, sorted_ids, sorted_num, n_seg);
+    if ((int)blockIdx.x < n_seg) align_hist(ids, numel, E, hist, words, sorted_ids, sorted_num, n_seg, seg);
     else quant_groups<T>(x, q, scale, n_groups, (int)blockIdx.x - n_seg, (int)gridDim.x - n_seg);
 }
 
@@ -316,7 +319,7 @@ __global__ __launch_bounds__(256) void prepare_hist_kernel(const int32_t *__rest
 __global__ __launch_bounds__(1024) void align_place_kernel(const int32_t *__restrict__ ids, int numel, int E, int id_bits,
                                                            int block_size, const int *__restrict__ hist, int words,
                                                            int32_t *sorted_ids, int32_t *expert_ids, int n_blocks,
-                                                           int32_t *ntpp, int n_waves)
+                                                           int32_t *ntpp, int n_waves, int seg_slots)
 {
     // [2 words] starts | [2 words] slots of earlier segments | [n_waves][E] cursors (16 bit; first the scan's partial sums)
     extern __shared__ __attribute__((aligned(16))) int lds[];
@@ -356,8 +359,8 @@ __global__ __launch_bounds__(1024) void align_place_kernel(const int32_t *__rest
     for (int i = threadIdx.x; i < (n_waves * E + 1) / 2; i += blockDim.x) reinterpret_cast<int *>(cursors)[i] = 0;
     write_blocks(start, E, block_size, total, expert_ids, n_blocks, ntpp, seg, n_seg);
     __syncthreads();
-    const int run = kAlignSeg / n_waves;
-    const int lo = seg * kAlignSeg + wave * run, hi = min(lo + run, numel);
+    const int run = seg_slots / n_waves;
+    const int lo = seg * seg_slots + wave * run, hi = min(lo + run, numel);
     if (wave < n_waves) count_run(ids, lo, hi, E, id_bits, cursors + wave * E);
     __syncthreads();
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
@@ -425,25 +428,27 @@ int align(const int32_t *topk_ids, int numel, int num_experts, int block_size, i
         return hipGetLastError() == hipSuccess ? ALPHA_MOE_OK : ALPHA_MOE_ERR_LAUNCH;
     }
     if (!workspace || workspace_bytes < alpha_moe_align_workspace_bytes(numel, E)) return ALPHA_MOE_ERR_WORKSPACE;
-    const int n_seg = (numel + kAlignSeg - 1) / kAlignSeg, words = (E + 1) / 2;
+    int seg = kAlignSeg;   // (counts and cursors of a segment are 16 bits wide)
+    while (seg < (32 << 10) && (numel - 1) / seg >= kAlignMaxSeg) seg *= 2;
+    const int n_seg = (numel - 1) / seg + 1, words = (E + 1) / 2;
     int *hist = static_cast<int *>(workspace);
     if (!z.x)
         hipLaunchKernelGGL(align_hist_kernel, dim3(n_seg), dim3(256), words * sizeof(int), hs, topk_ids, numel, E, hist,
-                           words, sorted_token_ids, sorted_num);
+                           words, sorted_token_ids, sorted_num, seg);
     else if (z.is_f32)
         hipLaunchKernelGGL(prepare_hist_kernel<float>, dim3(n_seg + quant_grid(z, 256)), dim3(256), words * sizeof(int), hs,
-                           topk_ids, numel, E, hist, words, sorted_token_ids, sorted_num, n_seg,
+                           topk_ids, numel, E, hist, words, sorted_token_ids, sorted_num, n_seg, seg,
                            static_cast<const float *>(z.x), z.q, z.scale, n_groups);
     else
         hipLaunchKernelGGL(prepare_hist_kernel<uint16_t>, dim3(n_seg + quant_grid(z, 256)), dim3(256), words * sizeof(int),
-                           hs, topk_ids, numel, E, hist, words, sorted_token_ids, sorted_num, n_seg,
+                           hs, topk_ids, numel, E, hist, words, sorted_token_ids, sorted_num, n_seg, seg,
                            static_cast<const uint16_t *>(z.x), z.q, z.scale, n_groups);
     // sixteen wavefronts where their cursors fit 32 KiB, at least four (64 KiB of LDS in all at kAlignMaxExperts)
     const int n_waves = E <= 1024 ? 16 : E <= 2048 ? 8 : 4;
     const int cursor_words = (n_waves * E + 1) / 2;
     const size_t lds = (4 * words + (cursor_words > 16 ? cursor_words : 16)) * sizeof(int);
     hipLaunchKernelGGL(align_place_kernel, dim3(n_seg), dim3(1024), lds, hs, topk_ids, numel, E, id_bits, block_size, hist,
-                       words, sorted_token_ids, expert_ids, n_blocks, num_tokens_post_padded, n_waves);
+                       words, sorted_token_ids, expert_ids, n_blocks, num_tokens_post_padded, n_waves, seg);
     return hipGetLastError() == hipSuccess ? ALPHA_MOE_OK : ALPHA_MOE_ERR_LAUNCH;
 }
 

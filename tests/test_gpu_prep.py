@@ -49,9 +49,11 @@ def test_align_matches_oracle_bit_for_bit(M, top_k, E, block):
 
 @pytest.mark.parametrize("numel,E,block", [(1, 1, 8), (63, 2, 8), (65, 3, 128), (1025, 1, 16), (4096, 512, 56),
                                             (4096, 4096, 8), (4097, 4096, 8), (4097, 1, 128), (5120, 257, 64),
-                                            (40000, 3, 8), (81920, 512, 96)])
+                                            (40000, 3, 8), (81920, 512, 96),
+                                            (524288, 3, 8), (524289, 40, 16), (1048577, 301, 64)])
 def test_align_at_the_edges_of_its_runs_and_segments(numel, E, block):
-    """one chunk, one segment and their remainders; one workgroup (up to 4096 slots) and several; an even and an odd number
+    """one chunk, one segment and their remainders; one workgroup (up to 4096 slots) and several; segments of 1024,
+    2048 and 4096 slots (beyond 512 segments); an even and an odd number
     of experts, one, and the most there can be; slots without an expert among them"""
     from alpha_moe_python import prep_hip
     g = torch.Generator().manual_seed(numel + E)
