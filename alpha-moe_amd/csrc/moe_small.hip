@@ -329,8 +329,8 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
 }
 
 // a / s from r ~ 1 / s (one rounding off at most) by one residual correction: three instructions where the division takes
-// ten.  For s = 448 it is the quotient; for the FP8 quantisation the codes of all bf16 values and row maxima are those of the
-// exact division (both checked exhaustively).
+// ten.  For s = 448 it is the quotient, for every bf16 row maximum; the FP8 codes are those of the exact division (the CPU tests
+// compare both, the codes for all mantissas of row maximum and value at eleven exponents).
 __device__ __forceinline__ float divide(float a, float s, float r)
 {
     const float t = a * r;

@@ -90,3 +90,51 @@ def test_block_quant():
                 ref = torch.from_numpy(O.fp8_e4m3fn_encode((blk / s[e, i, j]).clamp(-448, 448).numpy()))
                 assert torch.equal(q[e, 128 * i:128 * i + 128, 128 * j:128 * j + 128].view(torch.uint8), ref)
     assert int((O.fp8_to_float(q).abs() == 448.0).sum()) >= 3 * 2 * 3   # each block's amax maps to +-448
+
+
+def _fma32(a, b, c):
+    """a * b + c of float32 arrays, rounded once: the product is exact in float64, the sum is rounded to odd there."""
+    p, c = a.astype(np.float64) * b.astype(np.float64), c.astype(np.float64)
+    s = p + c
+    t = s - p
+    err = (p - (s - t)) + (c - t)
+    even = (s.view(np.int64) & 1) == 0
+    return np.where((err != 0) & even, np.nextafter(s, np.copysign(np.inf, err)), s).astype(np.float32)
+
+
+def _divide32(a, s, r):
+    """What the small kernels take for a / s: one residual correction of a * r (r about 1 / s)."""
+    t = a * r
+    return _fma32(_fma32(-t, s, a), r, t)
+
+
+def _bf16_values(exponents):
+    return np.concatenate([np.float32(2.0) ** np.float32(e) * (1 + np.arange(128, dtype=np.float32) / 128) for e in exponents])
+
+
+def test_requantisation_without_a_division_gives_the_codes_of_the_division():
+    """Scale m / 448 and codes a / scale as moe_small.hip computes them, against the exact float32 division: every bf16 row
+    maximum (scale), and every mantissa of maximum and value with the value up to 2^20 below the maximum (smaller ones are 0
+    either way) at eleven of the maximum's exponents, the ends of its range among them; the reciprocal estimate right to one
+    unit in the last place, either way."""
+    f448 = np.float32(448.0)
+    every = np.concatenate([np.array([1e-10], np.float32), _bf16_values(range(-33, 128))])
+    every = every[every >= np.float32(1e-10)]
+    assert np.array_equal(_divide32(every, f448, np.full_like(every, np.float32(1.0) / f448)), every / f448)
+    checked = 0
+    for e_m in (-33, -32, -31, -20, -1, 0, 1, 40, 125, 126, 127):
+        for m in np.concatenate([_bf16_values([e_m]), np.array([1e-10], np.float32) if e_m == -33 else np.array([], np.float32)]):
+            if m < np.float32(1e-10):
+                continue
+            a = _bf16_values(range(max(e_m - 20, -126), e_m + 1))
+            a = a[a <= m]
+            s = np.full_like(a, m / f448)
+            want = torch.from_numpy(np.minimum(a / s, f448)).to(torch.float8_e4m3fn).view(torch.uint8)
+            for ulps in (-1, 0, 1):
+                r = (np.float32(1.0) / s).view(np.int32) + np.int32(ulps)
+                r = r.view(np.float32)
+                r = _fma32(_fma32(-s, r, np.ones_like(s)), r, r)
+                got = torch.from_numpy(np.minimum(_divide32(a, s, r), f448)).to(torch.float8_e4m3fn).view(torch.uint8)
+                assert torch.equal(got, want), (float(m), ulps)
+                checked += got.numel()
+    assert checked > 10_000_000
