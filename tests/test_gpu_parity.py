@@ -22,14 +22,22 @@ def c1():
     return P, oracle_out(P)
 
 
-def test_c1_default_knobs_torch_op_and_c_abi(c1):
+@pytest.fixture(params=[0, 2], ids=["default", "stream"])
+def decode_path(request):
+    """Batches of at most 16 tokens take the small kernels by default; the second run asks for the streaming kernel, which
+    serves the larger ones (row blocks above 32 take the prefill kernels in both)."""
+    with tunables(ALPHA_MOE_PATH=request.param):
+        yield request.param
+
+
+def test_c1_default_knobs_torch_op_and_c_abi(c1, decode_path):
     P, ref = c1
     print("case c1 M=16 block_m=16 (64,4) stages=3", flush=True)
     assert_parity(run_op(P, 16, 64, 4, 3, via="torch"), ref, "torch op")
     assert_parity(run_op(P, 16, 64, 4, 3, via="c_abi"), ref, "c abi")
 
 
-def test_c_abi_workspace_is_reusable_without_clearing(c1):
+def test_c_abi_workspace_is_reusable_without_clearing(c1, decode_path):
     """One zero-filled workspace, many calls with different knobs (and so different kernels and layouts inside it)."""
     import alpha_moe
     P, ref = c1
@@ -50,9 +58,14 @@ def test_c_abi_workspace_is_reusable_without_clearing(c1):
         for (prob, knobs), want in zip(cases, fresh):
             print(f"case shared workspace round {rep} M={prob.M} knobs {knobs}", flush=True)
             assert torch.equal(run_op(prob, *knobs, via="c_abi", workspace=ws2), want), (rep, prob.M, knobs)
+    # small and streaming kernels taking turns on it
+    for rep in range(3):
+        for path in (5, 2):
+            with tunables(ALPHA_MOE_PATH=path):
+                assert_parity(run_op(P, 16, 32, 8, 5, via="c_abi", workspace=ws2), ref, f"shared ws path {path} round {rep}")
 
 
-def test_c1_result_independent_of_every_knob(c1):
+def test_c1_result_independent_of_every_knob(c1, decode_path):
     """The reference's correctness sweep runs every (block_m, block_n/warp_n, stages) it accepts
     (test_moe_correctness.py:172-190); the result may not depend on them."""
     P, ref = c1
@@ -61,7 +74,7 @@ def test_c1_result_independent_of_every_knob(c1):
         assert_parity(run_op(P, bm, bn, wn, st), ref, f"knobs {(bm, bn, wn, st)}")
 
 
-def test_add_semantics_scaling_and_zero_weights(c1):
+def test_add_semantics_scaling_and_zero_weights(c1, decode_path):
     P, ref = c1
     pre = torch.full((P.M, P.shape.K), 0.25, dtype=torch.bfloat16, device=DEV)
     got = run_op(P, 16, 32, 8, 2, out=pre.clone())
@@ -74,7 +87,7 @@ def test_add_semantics_scaling_and_zero_weights(c1):
 
 
 @pytest.mark.parametrize("knobs", [(16, 32, 8, 2), (16, 64, 4, 5), (64, 64, 4, 3), (128, 64, 4, 3)])
-def test_store_variant_overwrites_whatever_out_held(c1, knobs):
+def test_store_variant_overwrites_whatever_out_held(c1, knobs, decode_path):
     """fused_moe_w8a8_up_down_store: out = bf16(sum) on every element, NaN-filled or not, and bit for bit what the
     adding call leaves in a zero-filled out - streaming and tile kernels, torch op and C ABI."""
     P, ref = c1
@@ -188,7 +201,7 @@ def test_store_variant_fallback_kernel():
 
 
 @pytest.mark.parametrize("M,E,top_k,K,I", [(1, 4, 2, 128, 128), (3, 5, 3, 384, 256), (37, 3, 2, 256, 384), (200, 2, 1, 128, 128)])
-def test_ragged_small_shapes(M, E, top_k, K, I):
+def test_ragged_small_shapes(M, E, top_k, K, I, decode_path):
     """K a single block, K % 256 == 128 (the reference silently drops the last 128 columns there), more I blocks,
     more tokens than one block, experts without tokens."""
     shape = Shape("t", E=E, top_k=top_k, K=K, I=I, shared_expert=False, routing="softmax_renorm", scaling_factor=1.3,
@@ -256,9 +269,12 @@ def ds_weights():
 def test_deepseek_shard_decode_full_size(ds_weights, M, knobs):
     """The headline decode configuration at its real size: E=257, top_k=9, K=7168, I=256."""
     P = make_problem(ds_weights, M, seed=0)
-    print(f"case ds M={M} knobs {knobs}", flush=True)
-    m = assert_parity(run_op(P, *knobs), oracle_out(P), f"ds M={M} knobs {knobs}")
-    print("metrics", m, flush=True)
+    ref = oracle_out(P)
+    for path in (0, 2) if M <= 16 else (0,):   # small kernels, streaming kernel
+        print(f"case ds M={M} knobs {knobs} path {path}", flush=True)
+        with tunables(ALPHA_MOE_PATH=path):
+            m = assert_parity(run_op(P, *knobs), ref, f"ds M={M} knobs {knobs} path {path}")
+        print("metrics", m, flush=True)
 
 
 @pytest.mark.parametrize("knobs", [(48, 64, 4, 3), (64, 32, 8, 2), (128, 64, 4, 3)])
@@ -434,7 +450,7 @@ def test_tile_kernel_result_independent_of_item_schedule():
 
 
 @pytest.mark.parametrize("knobs", [(16, 32, 8, 5), (64, 64, 4, 3)])
-def test_workspace_needs_only_its_prefix_zeroed(c1, knobs):
+def test_workspace_needs_only_its_prefix_zeroed(c1, knobs, decode_path):
     """Everything behind alpha_moe_workspace_zero_bytes() may hold anything: fill it with 0xff."""
     import alpha_moe
     P, ref = c1
@@ -449,7 +465,7 @@ def test_workspace_needs_only_its_prefix_zeroed(c1, knobs):
 
 
 @pytest.mark.parametrize("knobs,store", [((16, 32, 8, 5), False), ((16, 64, 4, 2), True), ((64, 64, 4, 3), False)])
-def test_hip_graph_capture_and_replay(c1, knobs, store):
+def test_hip_graph_capture_and_replay(c1, knobs, store, decode_path):
     """The operator allocates and synchronises nothing once it has run on a stream, so it can be captured into a HIP
     graph there.  Replays with new activations in the captured buffers agree bit for bit with eager calls, with eager
     work and synchronisations between the replays."""
@@ -516,11 +532,15 @@ def test_random_small_shapes_and_knobs():
         got = run_op(P, block_m, bn, wn, stages, via="c_abi")
         # The 1e-2 bar per token row, against the oracle or one of its neighbours within rounding-order noise of the
         # up/gate sums: a sum on a bf16 rounding boundary that decides a group's FP8 scale may fall on either side.
-        assert_parity_rows(got, oracle_variants(P), f"rnd{case}")
+        variants = oracle_variants(P)
+        assert_parity_rows(got, variants, f"rnd{case}")
+        if M <= 16 and block_m <= 32:
+            with tunables(ALPHA_MOE_PATH=2):
+                assert_parity_rows(run_op(P, block_m, bn, wn, stages, via="c_abi"), variants, f"rnd{case} streaming")
 
 
 @pytest.mark.parametrize("knobs", [(16, 32, 8, 5), (64, 64, 4, 3)])
-def test_nothing_routed(c1, knobs):
+def test_nothing_routed(c1, knobs, decode_path):
     """No live row block at all (num_tokens_post_padded = 0), and row blocks whose expert id is out of range: the adding
     call leaves `out` as it was, the storing call writes zeros - both kernels."""
     import alpha_moe
@@ -610,12 +630,13 @@ def test_queue_survives_a_grid_the_device_cannot_hold(ds_weights):
     overlap launches on several streams.  Handing the first items out by workgroup index (ALPHA_MOE_STRICT_QUEUE=0, an
     experiment switch) gives the same result on a grid the device holds."""
     import time
-    P = make_problem(ds_weights, 16, seed=4)
-    base = run_op(P, 16, 32, 8, 5, via="c_abi")
+    P = make_problem(ds_weights, 16, seed=4)   # K-split UP items (the small kernels, which this size takes by default, have no queue)
+    with tunables(ALPHA_MOE_PATH=2):
+        base = run_op(P, 16, 32, 8, 5, via="c_abi")
     assert_parity(base, oracle_out(P), "ds M=16")
-    with tunables(ALPHA_MOE_STRICT_QUEUE=0):
+    with tunables(ALPHA_MOE_PATH=2, ALPHA_MOE_STRICT_QUEUE=0):
         assert torch.equal(run_op(P, 16, 32, 8, 5, via="c_abi"), base)
-    with tunables(ALPHA_MOE_GRID=1024):
+    with tunables(ALPHA_MOE_PATH=2, ALPHA_MOE_GRID=1024):
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         got = run_op(P, 16, 32, 8, 5, via="c_abi")
@@ -667,8 +688,9 @@ def test_two_streams_at_once(ds_weights):
 
 @pytest.mark.parametrize("name", ["ds", "qn"])
 def test_tiny_batches(name, ds_weights, qn_weights):
-    """M in {1, 2, 4, 8, 16}: K-split UP items whose partial sums the last arrival adds up (in batches of eight
-    splits), on both shards, several knobs, adding and storing, two launches bit for bit; against the oracle.  The 1e-2
+    """M in {1, 2, 4, 8, 16}: the small kernels, and the streaming kernel with K-split UP items whose partial sums the last
+    arrival adds up (in batches of eight splits; fourteen at M = 1 of the DeepSeek-V3 shard), on both shards, several knobs,
+    adding and storing, two launches bit for bit; against the oracle.  The 1e-2
     bar holds on every size: on the benchmark sizes against the oracle as it is, on the sizes in between per token row
     against the oracle or its neighbours within rounding-order noise of the up/gate sums (at M=2 of the DeepSeek-V3
     shard one up-projection sum of the shared expert, the largest activation of its group, sits 6e-6 of its size from a
@@ -680,19 +702,23 @@ def test_tiny_batches(name, ds_weights, qn_weights):
         P = make_problem(W, M, seed=20 + M)
         ref = oracle_out(P)
         variants = None if M in benchmark_sizes else oracle_variants(P)
-        for knobs in ((16, 32, 8, 5), (16, 64, 4, 3), (8, 32, 8, 2), (32, 64, 4, 4)):
-            print(f"case {name} M={M} knobs {knobs}", flush=True)
-            got = run_op(P, *knobs, via="c_abi")
-            if M in benchmark_sizes:
-                assert_parity(got, ref, f"{name} M={M} knobs {knobs}")
-            else:
-                assert_parity_rows(got, variants, f"{name} M={M} knobs {knobs}")
-            assert torch.equal(got, run_op(P, *knobs, via="c_abi")), (name, M, knobs)
-            junk = torch.full((P.M, P.shape.K), float("nan"), dtype=torch.bfloat16, device=DEV)
-            assert torch.equal(run_op(P, *knobs, out=junk, via="c_abi", store=True), got), (name, M, knobs, "store")
         pre = torch.full((P.M, P.shape.K), 0.25, dtype=torch.bfloat16, device=DEV)
-        assert_parity_rows(run_op(P, 16, 32, 8, 5, out=pre.clone(), via="c_abi"), oracle_variants(P, out=pre.cpu()),
-                           f"{name} M={M} out pre-filled")
+        pre_variants = oracle_variants(P, out=pre.cpu())
+        for path in (5, 2):
+            with tunables(ALPHA_MOE_PATH=path):
+                for knobs in ((16, 32, 8, 5), (16, 64, 4, 3), (8, 32, 8, 2), (32, 64, 4, 4)):
+                    what = f"{name} M={M} knobs {knobs} path {path}"
+                    print(f"case {what}", flush=True)
+                    got = run_op(P, *knobs, via="c_abi")
+                    if M in benchmark_sizes:
+                        assert_parity(got, ref, what)
+                    else:
+                        assert_parity_rows(got, variants, what)
+                    assert torch.equal(got, run_op(P, *knobs, via="c_abi")), what
+                    junk = torch.full((P.M, P.shape.K), float("nan"), dtype=torch.bfloat16, device=DEV)
+                    assert torch.equal(run_op(P, *knobs, out=junk, via="c_abi", store=True), got), (what, "store")
+                assert_parity_rows(run_op(P, 16, 32, 8, 5, out=pre.clone(), via="c_abi"), pre_variants,
+                                   f"{name} M={M} out pre-filled path {path}")
 
 
 @pytest.mark.parametrize("M,E,top_k,K,I", [(1, 3, 2, 128, 128),       # one K block: seven wavefronts multiply zeros
@@ -852,7 +878,6 @@ def test_an_up_sum_on_a_bf16_boundary(ds_weights):
     of the output range - onto the device's."""
     from oracle import moe_oracle as O
     P = make_problem(ds_weights, 2, seed=22)
-    got = run_op(P, 16, 32, 8, 5, via="c_abi")
     plain, up, down = oracle_variants(P)
     scale = float(plain.float().abs().max())
     row = lambda a, b, t: float((a[t].float().cpu() - b[t].float().cpu()).abs().max()) / scale
@@ -860,12 +885,15 @@ def test_an_up_sum_on_a_bf16_boundary(ds_weights):
     assert max(row(plain, up, 0), row(plain, down, 0)) > 1e-2
     assert max(row(plain, up, 1), row(plain, down, 1)) <= 5e-3
     # the device is within the bar of the neighbour and, on token 1, of the oracle as it is
-    assert min(row(got, up, 0), row(got, down, 0)) <= 5e-3
-    assert row(got, plain, 1) <= 5e-3
-    assert O.error_metrics(got, plain)["cosine"] >= 0.9999
+    for path in (5, 2):
+        with tunables(ALPHA_MOE_PATH=path):
+            got = run_op(P, 16, 32, 8, 5, via="c_abi")
+        assert min(row(got, up, 0), row(got, down, 0)) <= 5e-3, path
+        assert row(got, plain, 1) <= 5e-3, path
+        assert O.error_metrics(got, plain)["cosine"] >= 0.9999, path
 
 
-def test_tiny_batch_duplicates_padding_and_missing_experts():
+def test_tiny_batch_duplicates_padding_and_missing_experts(decode_path):
     """A tiny batch with what makes the bookkeeping interesting: a token that picks one expert twice (two rows of one
     block), row blocks whose expert id is out of range (skipped), K % 256 == 128, three 128-column slices."""
     shape = Shape("t", E=6, top_k=4, K=384, I=384, shared_expert=False, routing="softmax_renorm", scaling_factor=2.5,
@@ -1033,7 +1061,7 @@ def _run_prepacked(P, packed, knobs, store=False, via="c_abi", out=None):
     return out
 
 
-def test_prepacked_weights_give_the_same_bits(c1, ds_weights, q3_weights):
+def test_prepacked_weights_give_the_same_bits(c1, ds_weights, q3_weights, decode_path):
     """fused_moe_w8a8_up_down_prepacked on prepack_weights(w, w2) against the operator on w, w2: bit for bit, streaming
     and tile kernels, adding and storing, torch op and C ABI - on the CPU-sized case, the DeepSeek-V3 shard at M=256 and
     the Zipf shard at M=200 (six slices)."""
@@ -1048,7 +1076,8 @@ def test_prepacked_weights_give_the_same_bits(c1, ds_weights, q3_weights):
         junk = torch.full((P.M, P.shape.K), float("nan"), dtype=torch.bfloat16, device=DEV)
         assert torch.equal(_run_prepacked(P, packed, knobs, store=True, out=junk), want), (knobs, "store")
     assert_parity(_run_prepacked(P, packed, (16, 32, 8, 5)), ref, "prepacked c1")
-    for W, M, knob_list in ((ds_weights, 256, ((16, 64, 4, 3), (64, 64, 4, 3), (128, 64, 4, 3))),
+    for W, M, knob_list in ((ds_weights, 16, ((16, 32, 8, 4),)),
+                            (ds_weights, 256, ((16, 64, 4, 3), (64, 64, 4, 3), (128, 64, 4, 3))),
                             (q3_weights, 200, ((16, 32, 8, 5), (64, 64, 4, 3), (128, 64, 4, 2)))):
         Q = make_problem(W, M, seed=1)
         packed = prepack_weights(W.w1, W.w2)
