@@ -75,6 +75,14 @@ struct SmallParams {
 // UP tiles that are summed between two barriers
 constexpr int batch_of(int nkw) { return nkw <= 2 ? 2 : 1; }
 
+// *at = min(*at, v) in LDS; complete behind the next lds_barrier().  (Not atomicMin: the compiler lets it wait for every
+// direct-to-LDS load in flight, here the weights' first tiles: 0.3 - 0.8 us a call.)
+__device__ __forceinline__ void lds_min(int *at, int v)
+{
+    const unsigned addr = (unsigned)(size_t)(__attribute__((address_space(3))) int *)at;
+    asm volatile("ds_min_i32 %0, %1" ::"v"(addr), "v"(v) : "memory");
+}
+
 // NKW: 128-byte K blocks per wavefront.
 template <int NKW>
 __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParams s)
@@ -86,7 +94,7 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
     __shared__ __attribute__((aligned(1024))) uint8_t s_ring[kWaves * kRingBytes];
     __shared__ v4f s_red[2][TB][kWaves][64];   // partial sums
     __shared__ Active s_act;
-    __shared__ __attribute__((aligned(16))) int s_row[kMaxRows][kMaxTokens];   // s_act.row, a word each
+    __shared__ __attribute__((aligned(16))) int s_row[kMaxRows][kMaxTokens];   // Active::row, a word each
     __shared__ short s_of_mb[kMaxRows];        // row block -> its expert's place in the list
     __shared__ __attribute__((aligned(16))) float s_ws[kWaves][2][16];   // [128-column block & 1][gate | up][K block]
     __shared__ int s_cnt[3];
@@ -229,7 +237,7 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
             if (id >= 0 && id < s.rows && a >= 0) f(id, s_row[a][id / p.top_k]);
         }
     };
-    for_rows([&](int id, int &row) { atomicMin(&row, id); });
+    for_rows([&](int id, int &row) { lds_min(&row, id); });
     lds_barrier();
     if (blockIdx.x == 0) {   // for the second launch
         for_rows([&](int id, int &row) {
@@ -238,18 +246,21 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
                 s_act.repeats = 1;
             }
         });
-        for (int i = tid; i < kMaxRows * kMaxTokens / 4; i += kThreads) {
-            const v4i r = reinterpret_cast<const v4i *>(s_row)[i];
-            reinterpret_cast<int *>(s_act.row)[i] = r.x | r.y << 8 | r.z << 16 | r.w << 24;
-        }
         if (tid == 0) {
             // a wait that ran out in an earlier launch on this workspace (sticky): the output says so itself, NaN in every element
             s_act.n = n_act;
             s_act.poison = s.ctl->error != 0;
         }
         lds_barrier();
-        for (int i = tid; i < (int)sizeof(Active) / 4; i += kThreads)
-            reinterpret_cast<int *>(s.active)[i] = reinterpret_cast<const int *>(&s_act)[i];
+        constexpr int kRow0 = offsetof(Active, row) / 4, kRow1 = kRow0 + kMaxRows * kMaxTokens / 4;
+        for (int i = tid; i < (int)sizeof(Active) / 4; i += kThreads) {
+            int word = reinterpret_cast<const int *>(&s_act)[i];
+            if (i >= kRow0 && i < kRow1) {
+                const v4i r = reinterpret_cast<const v4i *>(s_row)[i - kRow0];
+                word = r.x | r.y << 8 | r.z << 16 | r.w << 24;
+            }
+            reinterpret_cast<int *>(s.active)[i] = word;
+        }
     }
 
     int buf = 0;    // partial-sum buffer of the next batch
@@ -455,6 +466,7 @@ __global__ __launch_bounds__(kThreads) void moe_small_down_kernel(const SmallPar
     lds_barrier();
     const int n_act = __builtin_amdgcn_readfirstlane(s_act.n);
     const bool poisoned = s_act.poison != 0;
+    const int repeats = __builtin_amdgcn_readfirstlane(s_act.repeats);
 
     // ---- the weights; units of a wavefront's ring: slice group, then experts wave, wave + 8,
     // ..., then the group's slices
@@ -533,7 +545,7 @@ __global__ __launch_bounds__(kThreads) void moe_small_down_kernel(const SmallPar
                 if (tid + u * kThreads < n_act * n_ib * 2) s_w2s[tid + u * kThreads] = w2s_reg[u];
             // a row that stands for others of its token takes their weights over, in ascending order (a fixed one: the result
             // does not depend on which wavefront comes first)
-            if (s_act.repeats && tid < s.rows && s_act.same[tid] == 255) {
+            if (repeats && tid < s.rows && s_act.same[tid] == 255) {
                 float tw = tw_reg;
                 for (int r = tid + 1, end = (tid / p.top_k + 1) * p.top_k; r < end; r++)
                     if (s_act.same[r] == tid) tw += s_tw[r];
