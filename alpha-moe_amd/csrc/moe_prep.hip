@@ -18,7 +18,9 @@ constexpr int kAlignSeg = 1024;        // routing slots per workgroup (segment) 
 constexpr int kAlignMaxSeg = 512;      // most segments before they get longer: every workgroup reads all segments' histograms
                                        // (4 Mi slots, 4096 experts: 10.2 ms in 4096 segments, 272 us in 512;
                                        // 600 000 slots, 257 experts: 42 us in 586, 26 in 293)
-constexpr int kAlignSmall = 4096;      // most routing slots one workgroup aligns by itself (9 us near there; two launches: 13)
+// Most routing slots one workgroup aligns by itself.  MI355X, one workgroup / two launches, 128 - 512 experts: 3072 slots
+// 8.5 - 10.2 / 9.4 - 10.9 us, 4096 9.8 - 11.7 / 9.4 - 11.2, 5120 11.0 - 13.2 / 9.7 - 11.1.
+constexpr int kAlignSmall = 4096;
 constexpr int kAlignMaxExperts = 4096;
 
 // ---- quantisation ------------------------------------------------------------------------------------------
@@ -86,8 +88,8 @@ __global__ __launch_bounds__(256) void quant_group128_kernel(const T *__restrict
 // everything serial counts.  A wavefront ranks 64 consecutive slots among the equal experts of its chunk with one ballot
 // per bit of the expert id (same_expert) - a loop over the chunk's distinct experts, ~60 LDS round trips for 64 slots
 // of 257 experts, is what took most of 398 us for 2997 slots and of 193 us for 73 728 - and every wavefront counts and
-// places a run of slots of its own behind cursors of its own.  MI355X, kernel trace, 257 experts: 9 us for 2997 slots,
-// 16 us (two launches) for 73 728; nine slots take 5.3 us (8.1 with a serial scan over the experts).
+// places a run of slots of its own behind cursors of its own.  MI355X, 257 experts: 9 us for 2997 slots, 12 us (two
+// launches) for 73 728; nine slots take 5.3 us (8.1 with a serial scan over the experts).
 typedef unsigned long long lanes_t;
 
 // The lanes of this wavefront whose slot has the same expert as this lane's (e < 0: no slot, no lanes); all 64 lanes
