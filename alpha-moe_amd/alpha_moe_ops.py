@@ -47,6 +47,12 @@ def _prepare_inputs_fake(x, topk_ids, group_size, block_size, num_experts):
     return (*_per_token_group_quant_fp8_fake(x, group_size), *_moe_align_block_size_fake(topk_ids, block_size, num_experts))
 
 
+@torch.library.register_fake("alpha_moe::fused_experts")
+def _fused_experts_fake(hidden_states, topk_ids, w, w_scale, w2, w2_scale, topk_weights, group_size, block_m, block_n, warp_n,
+                        stages, scaling_factor):
+    return None
+
+
 def fused_moe_w8a8_up_down(
     x: torch.Tensor,
     x_scale: torch.Tensor,

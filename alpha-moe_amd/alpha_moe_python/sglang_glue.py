@@ -47,15 +47,12 @@ def fused_experts(hidden_states: torch.Tensor, w13: torch.Tensor, w2: torch.Tens
     routing, the fused operator.  ``hidden_states`` ``[M, K]`` bf16 is overwritten with the result and returned, as in
     the reference (which zero-fills it and adds; the storing variant needs no zero-fill)."""
     import alpha_moe  # noqa: F401  registers the operators
-    from .prep_hip import prepare_inputs
 
     config_path = config_path or os.environ["ALPHA_MOE_CONFIG"]
-    M, top_k, E = hidden_states.shape[0], topk_ids.shape[1], w13.shape[0]
-    cfg = get_best_config(config_path, M)
-    a_q, a_scale, sorted_token_ids, expert_ids, num_tokens_post_padded = prepare_inputs(
-        hidden_states, topk_ids, group_size, cfg["block_m"], E)
-    torch.ops.alpha_moe.fused_moe_w8a8_up_down_store(
-        a_q, a_scale, w13, w13_scale, w2, w2_scale, sorted_token_ids, expert_ids, num_tokens_post_padded,
-        topk_weights.to(torch.float32), hidden_states, top_k, cfg["block_m"], cfg["block_n"], cfg["warp_n"], cfg["stages"],
-        routed_scaling_factor or 1.0)
+    cfg = get_best_config(config_path, hidden_states.shape[0])
+    if topk_ids.dtype != torch.int32:
+        topk_ids = topk_ids.to(torch.int32)
+    torch.ops.alpha_moe.fused_experts(
+        hidden_states, topk_ids.contiguous(), w13, w13_scale, w2, w2_scale, topk_weights.to(torch.float32), group_size,
+        cfg["block_m"], cfg["block_n"], cfg["warp_n"], cfg["stages"], routed_scaling_factor or 1.0)
     return hidden_states

@@ -158,7 +158,7 @@ int run_fused_moe(const uint8_t *x, const float *x_scale, const uint8_t *w, cons
     hipError_t err;
     const Path path = choose_path(top_k, M, K, N, num_experts, sorted_num, block_m, warp_n);
     if (path == kSmall) {
-        err = launch_small(p, workspace, hs);
+        err = launch_small(p, nullptr, nullptr, workspace, hs);
     } else if (path == kStream) {
         err = launch_stream(p, warp_n, stages, workspace, hs);
     } else if (path == kWide) {
@@ -219,6 +219,43 @@ extern "C" int alpha_moe_fused_moe_w8a8_up_down_prepacked(const uint8_t *x, cons
     return run_fused_moe(x, x_scale, w_packed, w_scale, w2_packed, w2_scale, out, sorted_token_ids, expert_ids,
                          num_tokens_post_padded, topk_weights, top_k, M, K, N, num_experts, sorted_num, block_m, block_n,
                          warp_n, stages, scaling_factor, workspace, workspace_bytes, stream, store != 0, 1);
+}
+
+extern "C" int alpha_moe_layer_call_supported(int top_k, int M, int K, int N, int num_experts, int block_m, int block_n,
+                                              int warp_n, int stages)
+{
+    const int64_t sorted_num = (int64_t)M * top_k + (int64_t)num_experts * (block_m - 1);
+    if (M <= 0 || top_k <= 0 || num_experts <= 0 || block_m <= 0 || sorted_num > INT32_MAX) return 0;
+    if (alpha_moe_validate(top_k, M, K, N, num_experts, (int)sorted_num, block_m, block_n, warp_n, stages) != ALPHA_MOE_OK) return 0;
+    return layer_supported(num_experts) && choose_path(top_k, M, K, N, num_experts, (int)sorted_num, block_m, warp_n) == kSmall;
+}
+
+extern "C" int alpha_moe_layer_call(const uint16_t *x, const int32_t *topk_ids, const uint8_t *w, const float *w_scale,
+                                    const uint8_t *w2, const float *w2_scale, const float *topk_weights, uint16_t *out,
+                                    int top_k, int M, int K, int N, int num_experts, int block_m, int block_n, int warp_n,
+                                    int stages, float scaling_factor, void *workspace, size_t workspace_bytes, void *stream)
+{
+    if (!x || !topk_ids || !w || !w_scale || !w2 || !w2_scale || !topk_weights || !out) return ALPHA_MOE_ERR_NULL_POINTER;
+    if ((reinterpret_cast<uintptr_t>(x) & 15) != 0 ||
+        !alpha_moe_layer_call_supported(top_k, M, K, N, num_experts, block_m, block_n, warp_n, stages))
+        return ALPHA_MOE_ERR_SHAPE;
+    const int sorted_num = M * top_k + num_experts * (block_m - 1);
+    if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255) != 0 ||
+        workspace_bytes < alpha_moe_workspace_bytes(top_k, M, K, N, num_experts, sorted_num, block_m))
+        return ALPHA_MOE_ERR_WORKSPACE;
+    MoeParams p = {};
+    p.w = w; p.w_scale = w_scale; p.w2 = w2; p.w2_scale = w2_scale;
+    p.out = out;
+    p.topk_w = topk_weights;
+    p.top_k = top_k; p.M = M; p.K = K; p.N = N; p.E = num_experts; p.sorted_num = sorted_num; p.block_m = block_m;
+    p.scaling = scaling_factor;
+    p.overwrite = 1;
+    p.w_rs = (size_t)K;
+    p.w_ks = 128;
+    p.w2_rs = (size_t)N / 2;
+    p.w2_ks = 128;
+    return launch_small(p, x, topk_ids, workspace, static_cast<hipStream_t>(stream)) == hipSuccess ? ALPHA_MOE_OK
+                                                                                                   : ALPHA_MOE_ERR_LAUNCH;
 }
 
 // ---- the entry point for callers that cannot allocate ------------------------------------------------------

@@ -276,7 +276,10 @@ hipError_t launch_finalize(const MoeParams &p, hipStream_t stream);   // out = b
 bool small_supported(int top_k, int M, int K, int N, int block_m);
 bool small_pays(int top_k, int M, int K, int N, int E);   // ahead of the streaming kernel
 size_t small_workspace_bytes(int top_k, int M, int N);
-hipError_t launch_small(const MoeParams &p, void *workspace, hipStream_t stream);
+// x16, topk_ids: a layer call's bf16 activations and routing, prepared inside the first launch (the operator's inputs of p
+// are not read then; layer_supported()), or null.
+bool layer_supported(int E);
+hipError_t launch_small(const MoeParams &p, const uint16_t *x16, const int32_t *topk_ids, void *workspace, hipStream_t stream);
 
 // Persistent work-queue kernel for decode-sized batches (block_m <= 32 and bounded sizes): split-K up items ->
 // SwiGLU/requant -> column-slab down items, chained through flags in the workspace; then the per-token reduction.

@@ -65,6 +65,8 @@ struct SmallParams {
     StreamCtl *ctl;
     Active *active;
     uint16_t *act;     // [rows][I] bf16 SwiGLU output of each (token, slot) row
+    const uint16_t *x16;       // LAYER: the activations before quantisation [M][K] bf16, and
+    const int32_t *topk_ids;   // the experts of each (token, slot) row
     int n_ib, nkb, n_mb_max, rows;
     unsigned ib_magic; // x / n_ib == x * ib_magic >> 16 for x <= kMaxRows * kMaxSlices
     int dcols;         // output columns per DOWN part
@@ -75,6 +77,8 @@ struct SmallParams {
 // UP tiles that are summed between two barriers
 constexpr int batch_of(int nkw) { return nkw <= 2 ? 2 : 1; }
 
+constexpr int kLayerExperts = 4096;    // LAYER: most experts (as many as the aligner takes)
+
 // *at = min(*at, v) in LDS; complete behind the next lds_barrier().  (Not atomicMin: the compiler lets it wait for every
 // direct-to-LDS load in flight, here the weights' first tiles: 0.3 - 0.8 us a call.)
 __device__ __forceinline__ void lds_min(int *at, int v)
@@ -82,9 +86,83 @@ __device__ __forceinline__ void lds_min(int *at, int v)
     const unsigned addr = (unsigned)(size_t)(__attribute__((address_space(3))) int *)at;
     asm volatile("ds_min_i32 %0, %1" ::"v"(addr), "v"(v) : "memory");
 }
+__device__ __forceinline__ void lds_or(unsigned *at, unsigned v)
+{
+    const unsigned addr = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned *)at;
+    asm volatile("ds_or_b32 %0, %1" ::"v"(addr), "v"(v) : "memory");
+}
 
-// NKW: 128-byte K blocks per wavefront.
-template <int NKW>
+// A store to LDS; complete behind the next lds_barrier(), and for what the same wavefront reads from LDS after it.  (Not a plain
+// store, for the same reason.)
+__device__ __forceinline__ void lds_store(void *at, uint2 v)
+{
+    const unsigned addr = (unsigned)(size_t)(__attribute__((address_space(3))) void *)at;
+    asm volatile("ds_write_b64 %0, %1" ::"v"(addr), "v"(v) : "memory");
+}
+__device__ __forceinline__ void lds_store(float *at, float v)
+{
+    const unsigned addr = (unsigned)(size_t)(__attribute__((address_space(3))) float *)at;
+    asm volatile("ds_write_b32 %0, %1" ::"v"(addr), "v"(v) : "memory");
+}
+
+// a / s from r ~ 1 / s (one rounding off at most) by one residual correction: three instructions where the division takes
+// ten.  For s = 448 it is the quotient, for every bf16 row maximum; the FP8 codes are those of the exact division (the CPU tests
+// compare both, the codes for all mantissas of row maximum and value at eleven exponents).
+__device__ __forceinline__ float divide(float a, float s, float r)
+{
+    const float t = a * r;
+    return __builtin_fmaf(__builtin_fmaf(-t, s, a), r, t);
+}
+
+// the largest of the values of the 16 lanes of a row (lanes 16 k .. 16 k + 15), in all of them: rotations within the row
+__device__ __forceinline__ float max_of_16_lanes(float m)
+{
+    auto turned = [](float v, auto by) {
+        const int b = __builtin_bit_cast(int, v);
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(b, b, 0x120 + decltype(by)::value, 0xf, 0xf, false));
+    };
+    m = fmaxf(m, turned(m, std::integral_constant<int, 8>()));
+    m = fmaxf(m, turned(m, std::integral_constant<int, 4>()));
+    m = fmaxf(m, turned(m, std::integral_constant<int, 2>()));
+    return fmaxf(m, turned(m, std::integral_constant<int, 1>()));
+}
+
+// 128 columns of a row on 16 lanes, 8 each: FP8 codes and the row's scale (in all 16 lanes)
+__device__ __forceinline__ uint2 quantise_row(const v4i raw, float *scale)
+{
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        v[2 * i] = __builtin_bit_cast(float, (uint32_t)raw[i] << 16);
+        v[2 * i + 1] = __builtin_bit_cast(float, (uint32_t)raw[i] & 0xffff0000u);
+    }
+    float m = kAmaxFloor;
+#pragma unroll
+    for (int i = 0; i < 8; i++) m = fmaxf(m, fabsf(v[i]));
+    m = max_of_16_lanes(m);
+    // a row with an infinity: its scale is infinite, a finite value over it is 0 and an infinity over it NaN; NaN is clamped
+    // to -448 (as in the other kernels)
+    const bool inf = m == __builtin_inff();
+    const float sa = inf ? m : divide(m, kFp8Max, 1.0f / kFp8Max);
+    float r = __builtin_amdgcn_rcpf(sa);
+    r = inf ? 0.f : __builtin_fmaf(__builtin_fmaf(-sa, r, 1.0f), r, r);
+    const float s = inf ? 0.f : sa;
+    auto code = [&](float a) { return clamp_fp8(divide(a, s, r)); };
+    uint2 o;
+    o.x = pack_fp8x4(code(v[0]), code(v[1]), code(v[2]), code(v[3]));
+    o.y = pack_fp8x4(code(v[4]), code(v[5]), code(v[6]), code(v[7]));
+    *scale = sa;
+    return o;
+}
+
+// NKW: 128-byte K blocks per wavefront.  LAYER: what a layer call starts from - bf16 activations and the router's output -
+// is prepared here, by every workgroup for itself: the active experts come from a bit map of the rows' experts (ascending, as
+// the aligner sorts them), and a wavefront quantises its K range of all tokens while its first weights are on their way.  That
+// saves the preparation's launch (5.1 us of a chain of a few dependent steps on one workgroup, and the gap behind it).  MI355X,
+// cold weights, us a layer call, three launches / two: DeepSeek shard 1 token 31.9 / 28.0, 8 tokens 71.4 / 67.4, 16 tokens 109.8 /
+// 109.9 (there the activations, read at twice the width by 256 workgroups, take what the launch did); Qwen3-Next shard 24.7 /
+// 19.6, 44.8 / 38.8, 61.4 / 56.2; Qwen3-MoE shard 30.4 / 25.6, 48.4 / 43.6, 68.8 / 63.8.
+template <int NKW, bool LAYER>
 __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParams s)
 {
     constexpr int TB = batch_of(NKW);
@@ -98,6 +176,9 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
     __shared__ short s_of_mb[kMaxRows];        // row block -> its expert's place in the list
     __shared__ __attribute__((aligned(16))) float s_ws[kWaves][2][16];   // [128-column block & 1][gate | up][K block]
     __shared__ int s_cnt[3];
+    // LAYER: the experts that have a row; the scales of a wavefront's quantised K block
+    __shared__ unsigned s_bits[LAYER ? kLayerExperts / 32 : 1];
+    __shared__ float s_xs[LAYER ? kWaves : 1][kMaxTokens];
 
     const MoeParams &p = s.p;
     const int tid = threadIdx.x;
@@ -113,63 +194,115 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
     const int ld_row = lane >> 3;   // loader side: row l / 8 (+ 8), chunk slot l % 8
     const int chunk0 = 16 * ((lane & 7) ^ (ld_row >> 1)), chunk1 = chunk0 ^ 64;
 
-    // ---- one round trip: this wavefront's K range of all tokens, as operand tiles in the ring (and, where it holds one tile
-    // less, where the partial sums go later), and the routing arrays.  (Operand loads straight into registers are 16 rows x
-    // 64 bytes each: 3 us of them for 16 tokens.)
-    auto x_tile = [&](int i) { return i < R ? ring + i * 2048 : reinterpret_cast<uint8_t *>(s_red) + wave * 2048; };
-    static_assert(NKW <= R + 1 && sizeof(s_red) >= kWaves * 2048, "room for the token tiles");
-#pragma unroll
-    for (int i = 0; i < NKW; i++) {
-        const uint8_t *src = p.x + (size_t)(kb0 + i < nkb ? kb0 + i : nkb - 1) * 128;
-        dma16<0>(src + (size_t)(ld_row < p.M ? ld_row : p.M - 1) * K + chunk0, x_tile(i));
-        dma16<0>(src + (size_t)(8 + ld_row < p.M ? 8 + ld_row : p.M - 1) * K + chunk1, x_tile(i) + 1024);
-    }
-    int e_mb = -1, e_before = -1;
-    if (tid < s.n_mb_max) {
-        e_mb = p.expert_ids[tid];
-        if (tid > 0) e_before = p.expert_ids[tid - 1];
-    }
-    const int n_ids = s.n_mb_max * p.block_m < p.sorted_num ? s.n_mb_max * p.block_m : p.sorted_num;
-    const int id0 = tid < n_ids ? p.sorted_ids[tid] : -1;
-    const int ntpp = p.ntpp[0];
-    float x_sc[NKW];
-#pragma unroll
-    for (int i = 0; i < NKW; i++) {
-        x_sc[i] = 0.f;
-        if (n < p.M && kb0 + i < nkb) x_sc[i] = p.x_scale[(size_t)n * nkb + kb0 + i];
-    }
-    for (int i = tid; i < kMaxRows * kMaxTokens / 4; i += kThreads) reinterpret_cast<v4i *>(s_row)[i] = (v4i){255, 255, 255, 255};
-    for (int i = tid; i < kMaxRows; i += kThreads) s_act.same[i] = 255;
-    if (tid == 0) s_act.repeats = 0;
-
-    // the active experts: row blocks whose expert is not the one of the block before
-    int n_mb = (__builtin_amdgcn_readfirstlane(ntpp) + p.block_m - 1) / p.block_m;
-    n_mb = n_mb < s.n_mb_max ? n_mb : s.n_mb_max;
     // operand read offsets inside a 16x128 tile: chunk c of row m sits at c ^ ((m >> 1) & 7)
     const int f_n = (n >> 1) & 7;
     const int frag_lo = n * 128 + 16 * (q ^ f_n);
     const int frag_hi = n * 128 + 16 * ((q ^ f_n) ^ 4);
-    drain_vmem();
     v8i x_frag[NKW];   // (columns of tokens behind the last are dropped, K blocks behind the last are zero)
+    float x_sc[NKW];
+    int n_ids = 0, id0 = -1, n_mb = 0, n_act;
+    // LAYER: a wavefront's 4 tokens x 128 columns of a K block, 16 lanes x 8 columns per token
+    constexpr int TG = kMaxTokens / 4;
+    v4i x_raw[LAYER ? NKW : 1][TG];
+    int place = -1;   // LAYER: the place of row tid's expert in the list
+    for (int i = tid; i < kMaxRows * kMaxTokens / 4; i += kThreads) reinterpret_cast<v4i *>(s_row)[i] = (v4i){255, 255, 255, 255};
+    for (int i = tid; i < kMaxRows; i += kThreads) s_act.same[i] = 255;
+    if (tid == 0) s_act.repeats = 0;
+    if constexpr (LAYER) {
+        // one round trip: the rows' experts, then the activations
+        const int e = tid < s.rows ? s.topk_ids[tid] : -1;
 #pragma unroll
-    for (int i = 0; i < NKW; i++) {
-        x_frag[i] = cat(*reinterpret_cast<const v4i *>(x_tile(i) + frag_lo), *reinterpret_cast<const v4i *>(x_tile(i) + frag_hi));
-        if (kb0 + i >= nkb) x_frag[i] = (v8i){0, 0, 0, 0, 0, 0, 0, 0};
+        for (int i = 0; i < NKW; i++)
+#pragma unroll
+            for (int j = 0; j < TG; j++) {
+                const int t = 4 * j + (lane >> 4);
+                if (4 * j < p.M)
+                    x_raw[i][j] = *reinterpret_cast<const v4i *>(s.x16 + (size_t)(t < p.M ? t : p.M - 1) * K +
+                                                                 (size_t)(kb0 + i < nkb ? kb0 + i : nkb - 1) * 128 + 8 * (lane & 15));
+            }
+        const bool ok = e >= 0 && e < p.E;
+        for (int i = tid; i < kLayerExperts / 32; i += kThreads) s_bits[i] = 0;
+        lds_barrier();
+        if (ok) lds_or(&s_bits[e >> 5], 1u << (e & 31));
+        lds_barrier();
+        if (wave < 3) {   // rows are on the first three wavefronts
+            // experts in the words before this lane's: two words per lane cover the map
+            const unsigned w0 = s_bits[2 * lane], w1 = s_bits[2 * lane + 1];
+            const int own = __builtin_popcount(w0) + __builtin_popcount(w1);
+            int incl = own;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int o = __shfl_up(incl, d);
+                if (lane >= d) incl += o;
+            }
+            const int word = ok ? e >> 5 : 0;
+            int before = __shfl(incl - own, word >> 1);
+            if (word & 1) before += __builtin_popcount(s_bits[word - 1]);
+            before += __builtin_popcount(s_bits[word] & ((1u << (e & 31)) - 1u));
+            if (ok) {
+                place = before;
+                s_act.expert[place] = e;   // (equal rows write the same)
+            }
+            if (tid == 63) s_cnt[0] = incl;
+        }
+        lds_barrier();
+        n_act = __builtin_amdgcn_readfirstlane(s_cnt[0]);
+        // (the activations have arrived: what is loaded from here on is not waited for by their quantisation)
+#pragma unroll
+        for (int i = 0; i < NKW; i++)
+#pragma unroll
+            for (int j = 0; j < TG; j++)
+                if (4 * j < p.M) asm volatile("" ::"v"(x_raw[i][j]));
+    } else {
+        // one round trip: this wavefront's K range of all tokens, as operand tiles in the ring (and, where it holds one tile
+        // less, where the partial sums go later), and the routing arrays.  (Operand loads straight into registers are 16 rows
+        // x 64 bytes each: 3 us of them for 16 tokens.)
+        auto x_tile = [&](int i) { return i < R ? ring + i * 2048 : reinterpret_cast<uint8_t *>(s_red) + wave * 2048; };
+        static_assert(NKW <= R + 1 && sizeof(s_red) >= kWaves * 2048, "room for the token tiles");
+#pragma unroll
+        for (int i = 0; i < NKW; i++) {
+            const uint8_t *src = p.x + (size_t)(kb0 + i < nkb ? kb0 + i : nkb - 1) * 128;
+            dma16<0>(src + (size_t)(ld_row < p.M ? ld_row : p.M - 1) * K + chunk0, x_tile(i));
+            dma16<0>(src + (size_t)(8 + ld_row < p.M ? 8 + ld_row : p.M - 1) * K + chunk1, x_tile(i) + 1024);
+        }
+        int e_mb = -1, e_before = -1;
+        if (tid < s.n_mb_max) {
+            e_mb = p.expert_ids[tid];
+            if (tid > 0) e_before = p.expert_ids[tid - 1];
+        }
+        n_ids = s.n_mb_max * p.block_m < p.sorted_num ? s.n_mb_max * p.block_m : p.sorted_num;
+        id0 = tid < n_ids ? p.sorted_ids[tid] : -1;
+        const int ntpp = p.ntpp[0];
+#pragma unroll
+        for (int i = 0; i < NKW; i++) {
+            x_sc[i] = 0.f;
+            if (n < p.M && kb0 + i < nkb) x_sc[i] = p.x_scale[(size_t)n * nkb + kb0 + i];
+        }
+
+        // the active experts: row blocks whose expert is not the one of the block before
+        n_mb = (__builtin_amdgcn_readfirstlane(ntpp) + p.block_m - 1) / p.block_m;
+        n_mb = n_mb < s.n_mb_max ? n_mb : s.n_mb_max;
+        drain_vmem();
+#pragma unroll
+        for (int i = 0; i < NKW; i++) {
+            x_frag[i] = cat(*reinterpret_cast<const v4i *>(x_tile(i) + frag_lo), *reinterpret_cast<const v4i *>(x_tile(i) + frag_hi));
+            if (kb0 + i >= nkb) x_frag[i] = (v8i){0, 0, 0, 0, 0, 0, 0, 0};
+        }
+        const bool live = tid < n_mb && e_mb >= 0 && e_mb < p.E;
+        const bool first = live && (tid == 0 || e_mb != e_before);
+        const unsigned long long fm = __ballot(first);
+        if (wave < 3 && lane == 0) s_cnt[wave] = __builtin_popcountll(fm);
+        lds_barrier();
+        {
+            int at = __builtin_popcountll(fm & (~0ull >> (63 - lane)));   // with this lane
+            for (int v = 0; v < 3; v++)
+                if (v < wave) at += s_cnt[v];
+            if (first) s_act.expert[at - 1] = e_mb;
+            if (tid < n_mb) s_of_mb[tid] = live ? (short)(at - 1) : (short)-1;
+        }
+        n_act = __builtin_amdgcn_readfirstlane(s_cnt[0] + s_cnt[1] + s_cnt[2]);
+        lds_barrier();
     }
-    const bool live = tid < n_mb && e_mb >= 0 && e_mb < p.E;
-    const bool first = live && (tid == 0 || e_mb != e_before);
-    const unsigned long long fm = __ballot(first);
-    if (wave < 3 && lane == 0) s_cnt[wave] = __builtin_popcountll(fm);
-    lds_barrier();
-    {
-        int at = __builtin_popcountll(fm & (~0ull >> (63 - lane)));   // with this lane
-        for (int v = 0; v < 3; v++)
-            if (v < wave) at += s_cnt[v];
-        if (first) s_act.expert[at - 1] = e_mb;
-        if (tid < n_mb) s_of_mb[tid] = live ? (short)(at - 1) : (short)-1;
-    }
-    const int n_act = __builtin_amdgcn_readfirstlane(s_cnt[0] + s_cnt[1] + s_cnt[2]);
-    lds_barrier();
 
     // ---- this workgroup's part: an equal range of the C = experts x I intermediate columns ------------------------
     const int C = n_act * I, parts = (int)gridDim.x;
@@ -231,6 +364,10 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
     // A token that names an expert more than once: its lowest row stands for all.  (The choice must not depend on the order
     // of the wavefronts: every workgroup makes it for itself, and the second launch reads what workgroup 0 chose.)
     auto for_rows = [&](auto f) {
+        if constexpr (LAYER) {
+            if (place >= 0) f(tid, s_row[place][tid / p.top_k]);
+            return;
+        }
         for (int idx = tid; idx < n_ids && idx < n_mb * p.block_m; idx += kThreads) {
             const int id = idx == tid ? id0 : p.sorted_ids[idx];
             const int a = s_of_mb[idx / p.block_m];
@@ -260,6 +397,32 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
                 word = r.x | r.y << 8 | r.z << 16 | r.w << 24;
             }
             reinterpret_cast<int *>(s.active)[i] = word;
+        }
+    }
+
+    if constexpr (LAYER) {
+        // this wavefront's K range of the activations: quantised row by row (16 lanes a row), through LDS into the operand
+        // layout - where its own partial sums go later, 8 tokens in each buffer.  One wavefront's LDS accesses complete in
+        // order: no barrier.
+        static_assert(kMaxTokens == 16 && sizeof(s_red[0][0][0]) == 8 * 128, "a buffer holds 8 tokens' K block");
+        const int t = lane >> 4, sub = lane & 15;
+        auto at = [&](int row) { return reinterpret_cast<uint8_t *>(s_red[row >> 3][0][wave]) + (row & 7) * 128; };
+#pragma unroll
+        for (int i = 0; i < NKW; i++) {
+#pragma unroll
+            for (int j = 0; j < TG; j++)
+                if (4 * j < p.M) {
+                    float sa;
+                    const uint2 o = quantise_row(x_raw[i][j], &sa);
+                    const int row = 4 * j + t;
+                    lds_store(at(row) + 16 * ((sub >> 1) ^ ((row >> 1) & 7)) + 8 * (sub & 1), o);
+                    if (sub == 0) lds_store(&s_xs[wave][row], sa);
+                }
+            // (columns of tokens behind the last are dropped)
+            x_frag[i] = cat(*reinterpret_cast<const v4i *>(at(n) + 16 * (q ^ f_n)),
+                            *reinterpret_cast<const v4i *>(at(n) + 16 * ((q ^ f_n) ^ 4)));
+            x_sc[i] = n < p.M && kb0 + i < nkb ? s_xs[wave][n] : 0.f;
+            if (kb0 + i >= nkb) x_frag[i] = (v8i){0, 0, 0, 0, 0, 0, 0, 0};
         }
     }
 
@@ -337,56 +500,6 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
         turn += TB;
         buf ^= 1;
     }
-}
-
-// a / s from r ~ 1 / s (one rounding off at most) by one residual correction: three instructions where the division takes
-// ten.  For s = 448 it is the quotient, for every bf16 row maximum; the FP8 codes are those of the exact division (the CPU tests
-// compare both, the codes for all mantissas of row maximum and value at eleven exponents).
-__device__ __forceinline__ float divide(float a, float s, float r)
-{
-    const float t = a * r;
-    return __builtin_fmaf(__builtin_fmaf(-t, s, a), r, t);
-}
-
-// the largest of the values of the 16 lanes of a row (lanes 16 k .. 16 k + 15), in all of them: rotations within the row
-__device__ __forceinline__ float max_of_16_lanes(float m)
-{
-    auto turned = [](float v, auto by) {
-        const int b = __builtin_bit_cast(int, v);
-        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(b, b, 0x120 + decltype(by)::value, 0xf, 0xf, false));
-    };
-    m = fmaxf(m, turned(m, std::integral_constant<int, 8>()));
-    m = fmaxf(m, turned(m, std::integral_constant<int, 4>()));
-    m = fmaxf(m, turned(m, std::integral_constant<int, 2>()));
-    return fmaxf(m, turned(m, std::integral_constant<int, 1>()));
-}
-
-// 128 columns of a row on 16 lanes, 8 each: FP8 codes and the row's scale (in all 16 lanes)
-__device__ __forceinline__ uint2 quantise_row(const v4i raw, float *scale)
-{
-    float v[8];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        v[2 * i] = __builtin_bit_cast(float, (uint32_t)raw[i] << 16);
-        v[2 * i + 1] = __builtin_bit_cast(float, (uint32_t)raw[i] & 0xffff0000u);
-    }
-    float m = kAmaxFloor;
-#pragma unroll
-    for (int i = 0; i < 8; i++) m = fmaxf(m, fabsf(v[i]));
-    m = max_of_16_lanes(m);
-    // a row with an infinity: its scale is infinite, a finite value over it is 0 and an infinity over it NaN; NaN is clamped
-    // to -448 (as in the other kernels)
-    const bool inf = m == __builtin_inff();
-    const float sa = inf ? m : divide(m, kFp8Max, 1.0f / kFp8Max);
-    float r = __builtin_amdgcn_rcpf(sa);
-    r = inf ? 0.f : __builtin_fmaf(__builtin_fmaf(-sa, r, 1.0f), r, r);
-    const float s = inf ? 0.f : sa;
-    auto code = [&](float a) { return clamp_fp8(divide(a, s, r)); };
-    uint2 o;
-    o.x = pack_fp8x4(code(v[0]), code(v[1]), code(v[2]), code(v[3]));
-    o.y = pack_fp8x4(code(v[4]), code(v[5]), code(v[6]), code(v[7]));
-    *scale = sa;
-    return o;
 }
 
 // H: groups of 8 output columns per part.  RING: bytes of a wavefront's ring.
@@ -667,13 +780,14 @@ SmallPlan make_plan(int top_k, int M, int K, int N, int block_m)
 
 typedef void (*SmallFn)(const SmallParams);
 
+template <bool LAYER>
 SmallFn pick_up(int nkw)
 {
     switch (nkw) {
-    case 1: return moe_small_up_kernel<1>;
-    case 2: return moe_small_up_kernel<2>;
-    case 4: return moe_small_up_kernel<4>;
-    default: return moe_small_up_kernel<7>;
+    case 1: return moe_small_up_kernel<1, LAYER>;
+    case 2: return moe_small_up_kernel<2, LAYER>;
+    case 4: return moe_small_up_kernel<4, LAYER>;
+    default: return moe_small_up_kernel<7, LAYER>;
     }
 }
 
@@ -729,7 +843,9 @@ size_t small_workspace_bytes(int top_k, int M, int N)
     return align_up(kPrefixBytes) + align_up(sizeof(Active)) + align_up((size_t)M * top_k * (N / 2) * sizeof(uint16_t));
 }
 
-hipError_t launch_small(const MoeParams &p, void *workspace, hipStream_t stream)
+bool layer_supported(int E) { return E <= kLayerExperts; }
+
+hipError_t launch_small(const MoeParams &p, const uint16_t *x16, const int32_t *topk_ids, void *workspace, hipStream_t stream)
 {
     const SmallPlan h = make_plan(p.top_k, p.M, p.K, p.N, p.block_m);
     if (!h.ok) return hipErrorInvalidValue;
@@ -739,6 +855,8 @@ hipError_t launch_small(const MoeParams &p, void *workspace, hipStream_t stream)
     s.ctl = reinterpret_cast<StreamCtl *>(ws);
     s.active = reinterpret_cast<Active *>(ws + align_up(kPrefixBytes));
     s.act = reinterpret_cast<uint16_t *>(ws + align_up(kPrefixBytes) + align_up(sizeof(Active)));
+    s.x16 = x16;
+    s.topk_ids = topk_ids;
     s.n_ib = p.N / 256;
     s.nkb = p.K / 128;
     s.rows = p.M * p.top_k;
@@ -752,7 +870,7 @@ hipError_t launch_small(const MoeParams &p, void *workspace, hipStream_t stream)
     const SmallFn down = pick_down(h.h, h.ring);
     hipError_t err = allow_dynamic_lds(h.h, h.ring, down);
     if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(pick_up(h.nkw), dim3((unsigned)h.up_parts), dim3(kThreads), 0, stream, s);
+    hipLaunchKernelGGL(x16 ? pick_up<true>(h.nkw) : pick_up<false>(h.nkw), dim3((unsigned)h.up_parts), dim3(kThreads), 0, stream, s);
     err = hipGetLastError();
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(down, dim3((unsigned)h.n_down), dim3(kThreads), h.lds_bytes, stream, s);

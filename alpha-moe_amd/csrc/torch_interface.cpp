@@ -115,29 +115,14 @@ void check_tensor(const at::Tensor &t, const char *name, at::ScalarType dtype, c
     TORCH_CHECK(t.is_contiguous(), name, " must be contiguous");
 }
 
-void run_fused_moe(const at::Tensor &x, const at::Tensor &x_scale, const at::Tensor &w, const at::Tensor &w_scale,
-                   const at::Tensor &w2, const at::Tensor &w2_scale, const at::Tensor &sorted_token_ids,
-                   const at::Tensor &expert_ids, const at::Tensor &num_tokens_post_padded,
-                   const at::Tensor &topk_weights, at::Tensor &out, int64_t top_k, int64_t block_m, int64_t block_n,
-                   int64_t warp_n, int64_t stages, double scaling_factor, bool store, bool prepacked = false)
+// The expert weights of a call with K columns; returns (experts, N).
+std::pair<int64_t, int64_t> check_weights(const at::Tensor &w, const at::Tensor &w_scale, const at::Tensor &w2,
+                                          const at::Tensor &w2_scale, int64_t K, const at::Device &dev, bool prepacked)
 {
-    TORCH_CHECK(x.is_cuda(), "x must be a GPU tensor");
-    const at::Device dev = x.device();
-    check_tensor(x, "x", at::kFloat8_e4m3fn, dev);
-    check_tensor(x_scale, "x_scale", at::kFloat, dev);
     check_tensor(w, "w", at::kFloat8_e4m3fn, dev);
     check_tensor(w_scale, "w_scale", at::kFloat, dev);
     check_tensor(w2, "w2", at::kFloat8_e4m3fn, dev);
     check_tensor(w2_scale, "w2_scale", at::kFloat, dev);
-    check_tensor(sorted_token_ids, "sorted_token_ids", at::kInt, dev);
-    check_tensor(expert_ids, "expert_ids", at::kInt, dev);
-    check_tensor(num_tokens_post_padded, "num_tokens_post_padded", at::kInt, dev);
-    check_tensor(topk_weights, "topk_weights", at::kFloat, dev);
-    check_tensor(out, "out", at::kBFloat16, dev);
-
-    TORCH_CHECK(x.dim() == 2 && x.size(0) > 0, "x must be [M, K] with M > 0");
-    const int64_t M = x.size(0), K = x.size(1);
-    TORCH_CHECK(K % 128 == 0, "K dimension must be a multiple of 128");
     int64_t E, N;
     if (!prepacked) {
         TORCH_CHECK(w.dim() == 3 && w.size(2) == K, "w must be [E, N, K] with the K of x");
@@ -152,9 +137,32 @@ void run_fused_moe(const at::Tensor &x, const at::Tensor &x_scale, const at::Ten
         TORCH_CHECK(w2.dim() == 4 && w2.size(0) == E && w2.size(1) == N / 256 && w2.size(2) == K && w2.size(3) == 128,
                     "w2_packed must be [E, N/256, K, 128]");
     }
-    TORCH_CHECK(x_scale.numel() == M * (K / 128), "x_scale must be [M, K/128]");
     TORCH_CHECK(w_scale.numel() == E * (N / 128) * (K / 128), "w_scale must be [E, N/128, K/128]");
     TORCH_CHECK(w2_scale.numel() == E * (K / 128) * (N / 256), "w2_scale must be [E, K/128, N/256]");
+    return {E, N};
+}
+
+void run_fused_moe(const at::Tensor &x, const at::Tensor &x_scale, const at::Tensor &w, const at::Tensor &w_scale,
+                   const at::Tensor &w2, const at::Tensor &w2_scale, const at::Tensor &sorted_token_ids,
+                   const at::Tensor &expert_ids, const at::Tensor &num_tokens_post_padded,
+                   const at::Tensor &topk_weights, at::Tensor &out, int64_t top_k, int64_t block_m, int64_t block_n,
+                   int64_t warp_n, int64_t stages, double scaling_factor, bool store, bool prepacked = false)
+{
+    TORCH_CHECK(x.is_cuda(), "x must be a GPU tensor");
+    const at::Device dev = x.device();
+    check_tensor(x, "x", at::kFloat8_e4m3fn, dev);
+    check_tensor(x_scale, "x_scale", at::kFloat, dev);
+    check_tensor(sorted_token_ids, "sorted_token_ids", at::kInt, dev);
+    check_tensor(expert_ids, "expert_ids", at::kInt, dev);
+    check_tensor(num_tokens_post_padded, "num_tokens_post_padded", at::kInt, dev);
+    check_tensor(topk_weights, "topk_weights", at::kFloat, dev);
+    check_tensor(out, "out", at::kBFloat16, dev);
+
+    TORCH_CHECK(x.dim() == 2 && x.size(0) > 0, "x must be [M, K] with M > 0");
+    const int64_t M = x.size(0), K = x.size(1);
+    TORCH_CHECK(K % 128 == 0, "K dimension must be a multiple of 128");
+    const auto [E, N] = check_weights(w, w_scale, w2, w2_scale, K, dev, prepacked);
+    TORCH_CHECK(x_scale.numel() == M * (K / 128), "x_scale must be [M, K/128]");
     TORCH_CHECK(out.dim() == 2 && out.size(0) == M && out.size(1) == K, "out must be [M, K]");
     TORCH_CHECK(top_k > 0 && topk_weights.numel() == M * top_k, "topk_weights must hold M * top_k values");
     TORCH_CHECK((block_n == 64 && warp_n == 4) || (block_n == 32 && warp_n == 8),
@@ -323,6 +331,54 @@ prepare_inputs(const at::Tensor &x, const at::Tensor &topk_ids, int64_t group_si
     return {q, scale, sorted_ids, expert_ids, total};
 }
 
+// A whole layer call: hidden_states [M, K] bf16 is quantised, the routing aligned, and the operator's result takes its
+// place.  The smallest batches do without the preparation and its tensors (alpha_moe_layer_call); otherwise this is
+// prepare_inputs and fused_moe_w8a8_up_down_store.
+void fused_experts(at::Tensor &hidden, const at::Tensor &topk_ids, const at::Tensor &w, const at::Tensor &w_scale,
+                   const at::Tensor &w2, const at::Tensor &w2_scale, const at::Tensor &topk_weights, int64_t group_size,
+                   int64_t block_m, int64_t block_n, int64_t warp_n, int64_t stages, double scaling_factor)
+{
+    TORCH_CHECK_INDEX(topk_ids.dim() >= 2 && w.dim() >= 1, "topk_ids must be [M, top_k], w [E, N, K]");
+    const int64_t top_k = topk_ids.size(1), E = w.size(0);
+    // (what prepare_inputs and the operator would refuse is left to them)
+    const bool whole = hidden.is_cuda() && hidden.dim() == 2 && hidden.scalar_type() == at::kBFloat16 && hidden.is_contiguous() &&
+                       group_size == 128 && topk_ids.device() == hidden.device() && topk_ids.scalar_type() == at::kInt &&
+                       topk_ids.is_contiguous() && hidden.size(0) <= 64 && topk_ids.numel() == hidden.size(0) * top_k &&
+                       (reinterpret_cast<uintptr_t>(hidden.const_data_ptr()) & 15) == 0 && w.dim() == 3 &&
+                       w.size(1) <= INT32_MAX && hidden.size(1) <= INT32_MAX && E <= INT32_MAX && top_k <= INT32_MAX &&
+                       block_m > 0 && block_m <= 128 && block_n <= 128 && warp_n <= 128 && stages <= 128 &&
+                       alpha_moe_layer_call_supported(static_cast<int>(top_k), static_cast<int>(hidden.size(0)),
+                                                      static_cast<int>(hidden.size(1)), static_cast<int>(w.size(1)),
+                                                      static_cast<int>(E), static_cast<int>(block_m), static_cast<int>(block_n),
+                                                      static_cast<int>(warp_n), static_cast<int>(stages));
+    if (!whole) {
+        const auto [q, scale, sorted_ids, expert_ids, total] = prepare_inputs(hidden, topk_ids, group_size, block_m, E);
+        run_fused_moe(q, scale, w, w_scale, w2, w2_scale, sorted_ids, expert_ids, total, topk_weights, hidden, top_k, block_m,
+                      block_n, warp_n, stages, scaling_factor, true);
+        return;
+    }
+    const at::Device dev = hidden.device();
+    const int64_t M = hidden.size(0), K = hidden.size(1);
+    const int64_t N = check_weights(w, w_scale, w2, w2_scale, K, dev, false).second;
+    check_tensor(topk_weights, "topk_weights", at::kFloat, dev);
+    TORCH_CHECK(topk_weights.numel() == M * top_k, "topk_weights must hold M * top_k values");
+    const c10::hip::OptionalHIPGuardMasqueradingAsCUDA device_guard(dev);
+    hipStream_t stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
+    const int64_t sorted_num = M * top_k + E * (block_m - 1);
+    const size_t ws_bytes =
+        alpha_moe_workspace_bytes(static_cast<int>(top_k), static_cast<int>(M), static_cast<int>(K), static_cast<int>(N),
+                                  static_cast<int>(E), static_cast<int>(sorted_num), static_cast<int>(block_m));
+    at::Tensor ws = workspace_for(dev, stream, ws_bytes);
+    uint16_t *x = static_cast<uint16_t *>(hidden.data_ptr());
+    const int rc = alpha_moe_layer_call(
+        x, topk_ids.const_data_ptr<int32_t>(), static_cast<const uint8_t *>(w.const_data_ptr()), w_scale.const_data_ptr<float>(),
+        static_cast<const uint8_t *>(w2.const_data_ptr()), w2_scale.const_data_ptr<float>(), topk_weights.const_data_ptr<float>(),
+        x, static_cast<int>(top_k), static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), static_cast<int>(E),
+        static_cast<int>(block_m), static_cast<int>(block_n), static_cast<int>(warp_n), static_cast<int>(stages),
+        static_cast<float>(scaling_factor), ws.data_ptr(), static_cast<size_t>(ws.numel()), static_cast<void *>(stream));
+    TORCH_CHECK(rc == ALPHA_MOE_OK, "alpha_moe_layer_call failed: ", alpha_moe_status_string(rc));
+}
+
 }  // namespace
 
 TORCH_LIBRARY_FRAGMENT(alpha_moe, m)
@@ -334,6 +390,9 @@ TORCH_LIBRARY_FRAGMENT(alpha_moe, m)
     m.def("prepare_inputs(Tensor x, Tensor topk_ids, int group_size, int block_size, int num_experts) -> "
           "(Tensor, Tensor, Tensor, Tensor, Tensor)");
     m.impl("prepare_inputs", c10::DispatchKey::CUDA, &prepare_inputs);
+    m.def("fused_experts(Tensor(a!) hidden_states, Tensor topk_ids, Tensor w, Tensor w_scale, Tensor w2, Tensor w2_scale, "
+          "Tensor topk_weights, int group_size, int block_m, int block_n, int warp_n, int stages, float scaling_factor) -> ()");
+    m.impl("fused_experts", c10::DispatchKey::CUDA, &fused_experts);
     m.def("reserve_workspace(Tensor like, int bytes) -> ()");
     m.impl("reserve_workspace", c10::DispatchKey::CUDA, &reserve_workspace);
     m.def("scratch_buffers(Tensor like) -> int[]");

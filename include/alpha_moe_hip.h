@@ -214,6 +214,20 @@ int alpha_moe_prepare_inputs(const void *x, int x_is_f32, uint8_t *q, float *sca
                              int32_t *expert_ids, int n_blocks, int32_t *num_tokens_post_padded, void *workspace,
                              size_t workspace_bytes, void *stream /* hipStream_t */);
 
+/*
+ * A whole layer call on the smallest batches: quantise, align and the storing operator in two launches.  x [M, K] bf16
+ * (16-byte aligned) and topk_ids [M * top_k] are what alpha_moe_prepare_inputs takes, everything else is as in
+ * alpha_moe_fused_moe_w8a8_up_down_store for the row-block size block_m, and so is the result, bit for bit; out may be x.
+ * alpha_moe_layer_call_supported() says (1 or 0) whether these sizes and knobs are taken: those for which the operator
+ * would run its kernels for at most 16 tokens, with at most 4096 experts.  Others are refused (ALPHA_MOE_ERR_SHAPE).
+ */
+int alpha_moe_layer_call_supported(int top_k, int M, int K, int N, int num_experts, int block_m, int block_n, int warp_n,
+                                   int stages);
+int alpha_moe_layer_call(const uint16_t *x, const int32_t *topk_ids, const uint8_t *w, const float *w_scale,
+                         const uint8_t *w2, const float *w2_scale, const float *topk_weights, uint16_t *out, int top_k, int M,
+                         int K, int N, int num_experts, int block_m, int block_n, int warp_n, int stages,
+                         float scaling_factor, void *workspace, size_t workspace_bytes, void *stream /* hipStream_t */);
+
 /* Human-readable text for a status code (static storage). */
 const char *alpha_moe_status_string(int status);
 

@@ -68,3 +68,67 @@ def test_fused_experts_matches_the_oracle_on_the_checkpoint_tensors(M, tmp_path)
                              top_k, 16, 2.5)
     m = O.error_metrics(got, ref)
     assert m["max_abs_over_max_ref"] <= MAX_ABS_OVER_MAX_REF and m["cosine"] >= MIN_COSINE, m
+
+
+@pytest.mark.parametrize("M,top_k,K,I,E,block_m", [
+    (1, 1, 128, 128, 1, 8), (1, 9, 7168, 256, 257, 16),             # one row of one block; the widest K of a wavefront
+    (2, 20, 1024, 128, 4096, 8), (3, 4, 1152, 256, 33, 16),         # the most experts; K blocks that do not fill the wavefronts
+    (4, 5, 2176, 128, 40, 24), (5, 8, 4096, 384, 64, 32), (7, 9, 4224, 256, 257, 16),
+    (8, 20, 2560, 128, 64, 8), (8, 8, 640, 256, 31, 64),
+    (9, 4, 1152, 256, 33, 16), (16, 10, 3072, 128, 512, 8),         # the second eight tokens; the most tokens and rows
+    (17, 4, 1152, 256, 33, 16)])                                    # one token too many; blocks of 64: the three steps as well
+def test_layer_call_equals_its_three_steps_bit_for_bit(M, top_k, K, I, E, block_m):
+    """The smallest batches are quantised and aligned inside the operator's first launch; quantiser, aligner and storing
+    operator called one by one are the general path.  Rows with an expert twice, slots without an expert, an infinity, a
+    NaN and an all-zero group among them; int64 routing, a base that is not 16-byte aligned, replays of a graph."""
+    import alpha_moe
+    from alpha_moe_python import prep_hip
+    g = torch.Generator().manual_seed(M * 131 + K)
+    gd = torch.Generator(device=DEV).manual_seed(M * 131 + K)
+    w13 = (torch.randn((E, 2 * I, K), generator=gd, device=DEV) * 0.5).to(torch.float8_e4m3fn)
+    w2 = (torch.randn((E, K, I), generator=gd, device=DEV) * 0.5).to(torch.float8_e4m3fn)
+    w13_s = torch.rand((E, 2 * I // 128, K // 128), generator=gd, device=DEV) * 0.1
+    w2_s = torch.rand((E, K // 128, I // 128), generator=gd, device=DEV) * 0.1
+    taken = alpha_moe.c_abi.alpha_moe_layer_call_supported(top_k, M, K, 2 * I, E, block_m, 32, 8, 4)
+    assert taken == (M <= 16 and block_m <= 32)
+    for kind in ("plain", "odd", "wild"):
+        x = (torch.randn((M, K), generator=g) * 2).to(torch.bfloat16)
+        ids = torch.randint(0, E, (M, top_k), generator=g).to(torch.int32)
+        if kind != "plain":
+            ids.view(-1)[::3] = torch.tensor([-1, E, E - 1], dtype=torch.int32)[torch.arange(0, M * top_k, 3) // 3 % 3]
+            x[0, :128] = 0
+        if kind == "wild":
+            x[M - 1, K - 1], x[M // 2, K // 2] = float("inf"), float("nan")
+            x[0, 0] = torch.finfo(torch.bfloat16).max
+        x, ids, weights = x.to(DEV), ids.to(DEV), torch.rand((M, top_k), generator=g).to(DEV)
+        print(f"case layer call M={M} top_k={top_k} K={K} I={I} E={E} block_m={block_m} {kind}", flush=True)
+        q, q_s, *routing = prep_hip.prepare_inputs(x, ids, 128, block_m, E)
+        want = torch.empty_like(x)
+        torch.ops.alpha_moe.fused_moe_w8a8_up_down_store(q, q_s, w13, w13_s, w2, w2_s, *routing, weights, want, top_k,
+                                                         block_m, 32, 8, 4, 2.5)
+
+        def call(h):
+            torch.ops.alpha_moe.fused_experts(h, ids, w13, w13_s, w2, w2_s, weights, 128, block_m, 32, 8, 4, 2.5)
+
+        def same(h, want):
+            torch.cuda.synchronize()
+            assert torch.equal(h.view(torch.int16), want.view(torch.int16)), kind
+
+        h = x.clone()
+        call(h)
+        same(h, want)
+        odd = torch.empty(M * K + 4, dtype=torch.bfloat16, device=DEV)[4:].view(M, K)
+        odd.copy_(x)
+        call(odd)
+        same(odd, want)
+        graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            call(h)   # scratch memory is per stream and is not allocated under capture
+        stream.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            call(h)
+        for _ in range(3):
+            h.copy_(x)
+            graph.replay()
+            same(h, want)
+            assert not torch.zeros(4, device=DEV).any()
