@@ -41,7 +41,6 @@ constexpr int kMaxRows = 160;        // most (token, slot) rows, and so most exp
 constexpr int kMaxSlices = 8;        // most 128-column slices of the intermediate (I <= 1024)
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
-constexpr int kW2sLoads = 2 * kMaxRows * kMaxSlices / kThreads;   // w2 scales per thread of a DOWN part
 constexpr int kPassRows = kThreads / 16, kPasses = kMaxRows / kPassRows;   // quantisation: 16 lanes per row
 constexpr int kRingBytes = 12 << 10;   // per wavefront
 constexpr int kBigRing = 16 << 10;     // DOWN launch, where there is room, and
@@ -208,6 +207,9 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
     for (int i = tid; i < kMaxRows * kMaxTokens / 4; i += kThreads) reinterpret_cast<v4i *>(s_row)[i] = (v4i){255, 255, 255, 255};
     for (int i = tid; i < kMaxRows; i += kThreads) s_act.same[i] = 255;
     if (tid == 0) s_act.repeats = 0;
+    // (loaded here: behind the weights' first tiles it would hold up the first workgroup's)
+    unsigned error = 0;
+    if (blockIdx.x == 0 && tid == 0) error = s.ctl->error;
     if constexpr (LAYER) {
         // one round trip: the rows' experts, then the activations
         const int e = tid < s.rows ? s.topk_ids[tid] : -1;
@@ -247,6 +249,7 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
         }
         lds_barrier();
         n_act = __builtin_amdgcn_readfirstlane(s_cnt[0]);
+        asm volatile("" ::"v"(error));
         // (the activations have arrived: what is loaded from here on is not waited for by their quantisation)
 #pragma unroll
         for (int i = 0; i < NKW; i++)
@@ -283,6 +286,7 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
         n_mb = (__builtin_amdgcn_readfirstlane(ntpp) + p.block_m - 1) / p.block_m;
         n_mb = n_mb < s.n_mb_max ? n_mb : s.n_mb_max;
         drain_vmem();
+        asm volatile("" ::"v"(error));
 #pragma unroll
         for (int i = 0; i < NKW; i++) {
             x_frag[i] = cat(*reinterpret_cast<const v4i *>(x_tile(i) + frag_lo), *reinterpret_cast<const v4i *>(x_tile(i) + frag_hi));
@@ -386,7 +390,7 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
         if (tid == 0) {
             // a wait that ran out in an earlier launch on this workspace (sticky): the output says so itself, NaN in every element
             s_act.n = n_act;
-            s_act.poison = s.ctl->error != 0;
+            s_act.poison = error != 0;
         }
         lds_barrier();
         constexpr int kRow0 = offsetof(Active, row) / 4, kRow1 = kRow0 + kMaxRows * kMaxTokens / 4;
@@ -503,6 +507,10 @@ __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParam
 }
 
 // H: groups of 8 output columns per part.  RING: bytes of a wavefront's ring.
+// Until its first product a part is a chain of round trips: what the first launch has left, then the weights.  Nothing may wait
+// in between - a load that is multiplied where it is loaded, a use of a register that might have been loaded behind the ring, a
+// plain store to LDS cost 1.0 - 1.6 us a call together (MI355X, us an operator call: DeepSeek shard 1 token 22.6 -> 21.3, 7 tokens
+// 57.8 -> 56.3; Qwen3-Next shard 14.7 -> 14.1, 32.2 -> 30.8; Qwen3-MoE shard 21.8 -> 19.4, 38.8 -> 37.7).
 template <int H, int RING>
 __global__ __launch_bounds__(kThreads) void moe_small_down_kernel(const SmallParams s)
 {
@@ -550,7 +558,8 @@ __global__ __launch_bounds__(kThreads) void moe_small_down_kernel(const SmallPar
         const int i = tid + k * kThreads;
         act_reg[k] = i < kActWords ? reinterpret_cast<const int *>(s.active)[i] : 0;
     }
-    const float tw_reg = tid < s.rows ? p.topk_w[tid] * p.scaling : 0.f;
+    float tw_reg = 0.f;
+    if (tid < s.rows) tw_reg = p.topk_w[tid];
     // Rows to quantise: 16 lanes x 8 columns per row, 32 rows a pass; two slices in flight (what is loaded behind the ring's
     // first tiles arrives behind them, too).
     const int sub = tid & 15;
@@ -571,6 +580,7 @@ __global__ __launch_bounds__(kThreads) void moe_small_down_kernel(const SmallPar
         const int i = tid + k * kThreads;
         if (i < kActWords) reinterpret_cast<int *>(&s_act)[i] = act_reg[k];
     }
+    tw_reg *= p.scaling;
     if (tid < s.rows) s_tw[tid] = tw_reg;
     // (all of this has arrived, whatever is loaded from here on)
     asm volatile("" ::"v"(prior.x), "v"(prior.y));
@@ -607,18 +617,15 @@ __global__ __launch_bounds__(kThreads) void moe_small_down_kernel(const SmallPar
             }
         }
     };
-    // the w2 scales of the part's one or two 128-column blocks, all loads in flight and ahead of the ring's
+    // the w2 scales of the part's one or two 128-column blocks, ahead of the ring's loads
     const int blk0 = d0 >> 7;
-    float w2s_reg[kW2sLoads];
-#pragma unroll
-    for (int u = 0; u < kW2sLoads; u++) {
-        const int i = tid + u * kThreads;
-        w2s_reg[u] = 0.f;
+    for (int i0 = wave * 64; i0 < n_act * n_ib * 2; i0 += kThreads) {
+        const int i = i0 + lane;
         if (i < n_act * n_ib * 2) {
             const int ai = i >> 1, a = (int)(((unsigned)ai * s.ib_magic) >> 16);
             int blk = blk0 + (i & 1);
             blk = blk < (K >> 7) ? blk : (K >> 7) - 1;
-            w2s_reg[u] = p.w2_scale[((size_t)s_act.expert[a] * (K >> 7) + blk) * n_ib + (ai - a * n_ib)];
+            dma4(p.w2_scale + ((size_t)s_act.expert[a] * (K >> 7) + blk) * n_ib + (ai - a * n_ib), s_w2s + i0);
         }
     }
     int left = mine * n_ib;   // units not yet issued
@@ -634,11 +641,18 @@ __global__ __launch_bounds__(kThreads) void moe_small_down_kernel(const SmallPar
         const int ns = slices_of(g);
         // row r's slice sl of the group at (r * gi + sl) * 128, its 16-byte chunk c at c ^ (r & 7)
         for (int s0 = 0; s0 < ns; s0 += 2) {
+            if (g > 0 || s0 > 0) {
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    if (s0 + h < ns) load_slice(g * s.gi + s0 + h, raw[h]);
+                // (waited for here: the first two slices' quantisation does not wait for the ring)
+#pragma unroll
+                for (int u = 0; u < kPasses; u++) asm volatile("" ::"v"(raw[0][u]), "v"(raw[1][u]));
+            }
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 const int sl = s0 + h, ib = g * s.gi + sl;
                 if (sl >= ns) break;
-                if (g > 0 || s0 > 0) load_slice(ib, raw[h]);
 #pragma unroll
                 for (int u = 0; u < kPasses; u++) {
                     if (u * kPassRows >= s.rows) break;
@@ -646,16 +660,18 @@ __global__ __launch_bounds__(kThreads) void moe_small_down_kernel(const SmallPar
                     float sa;
                     const uint2 o = quantise_row(raw[h][u], &sa);
                     if (row < s.rows) {
-                        *reinterpret_cast<uint2 *>(area + (row * s.gi + sl) * 128 + 16 * ((sub >> 1) ^ (row & 7)) + 8 * (sub & 1)) = o;
-                        if (sub == 0) s_sa[row * n_ib + ib] = sa;
+                        lds_store(area + (row * s.gi + sl) * 128 + 16 * ((sub >> 1) ^ (row & 7)) + 8 * (sub & 1), o);
+                        if (sub == 0) lds_store(&s_sa[row * n_ib + ib], sa);
                     }
                 }
             }
         }
         if (g == 0) {
-#pragma unroll
-            for (int u = 0; u < kW2sLoads; u++)
-                if (tid + u * kThreads < n_act * n_ib * 2) s_w2s[tid + u * kThreads] = w2s_reg[u];
+            // the w2 scales have arrived, the ring's loads may be outstanding
+            if (mine * n_ib >= SD)
+                wait_vmcnt<H * SD>();
+            else
+                drain_vmem();
             // a row that stands for others of its token takes their weights over, in ascending order (a fixed one: the result
             // does not depend on which wavefront comes first)
             if (repeats && tid < s.rows && s_act.same[tid] == 255) {
