@@ -113,17 +113,21 @@ __device__ __forceinline__ float divide(float a, float s, float r)
     return __builtin_fmaf(__builtin_fmaf(-t, s, a), r, t);
 }
 
-// the largest of the values of the 16 lanes of a row (lanes 16 k .. 16 k + 15), in all of them: rotations within the row
-__device__ __forceinline__ float max_of_16_lanes(float m)
+// the largest of the values (not negative, not NaN) of the 16 lanes of a row (lanes 16 k .. 16 k + 15), in all of them: rotations
+// within the row.  As integers, which such values compare as: a step is one instruction, where a float maximum is four.
+__device__ __forceinline__ float max_of_16_lanes(float v)
 {
-    auto turned = [](float v, auto by) {
-        const int b = __builtin_bit_cast(int, v);
-        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(b, b, 0x120 + decltype(by)::value, 0xf, 0xf, false));
+    unsigned m = __builtin_bit_cast(unsigned, v);
+    auto turned = [&](auto by) { return (unsigned)__builtin_amdgcn_mov_dpp((int)m, 0x120 + decltype(by)::value, 0xf, 0xf, true); };
+    auto step = [&](auto by) {
+        const unsigned o = turned(by);
+        m = m > o ? m : o;
     };
-    m = fmaxf(m, turned(m, std::integral_constant<int, 8>()));
-    m = fmaxf(m, turned(m, std::integral_constant<int, 4>()));
-    m = fmaxf(m, turned(m, std::integral_constant<int, 2>()));
-    return fmaxf(m, turned(m, std::integral_constant<int, 1>()));
+    step(std::integral_constant<int, 8>());
+    step(std::integral_constant<int, 4>());
+    step(std::integral_constant<int, 2>());
+    step(std::integral_constant<int, 1>());
+    return __builtin_bit_cast(float, m);
 }
 
 // 128 columns of a row on 16 lanes, 8 each: FP8 codes and the row's scale (in all 16 lanes)

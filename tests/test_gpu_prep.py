@@ -89,6 +89,20 @@ def test_align_where_the_wavefronts_of_a_segment_change(E):
         assert torch.equal(a.cpu(), b)
 
 
+@pytest.mark.parametrize("numel", [4096, 4500, 70000])
+@pytest.mark.parametrize("E", [256, 817, 818, 2045, 2046, 3580, 3581])
+def test_align_where_tables_and_cursors_fill_the_memory(E, numel):
+    """16, 8, 4 and 2 wavefronts place a segment, the last with more slots each than they keep in registers"""
+    from alpha_moe_python import prep_hip
+    g = torch.Generator().manual_seed(E)
+    ids = torch.randint(-1, E, (numel, 1), generator=g, dtype=torch.int32)
+    ids[100:1500] = E - 1
+    print(f"case align E={E} numel={numel}", flush=True)
+    got = prep_hip.moe_align_block_size(ids.to(DEV), 8, E)
+    for a, b in zip(got, O.align_reference(ids, 8, E)):
+        assert torch.equal(a.cpu(), b)
+
+
 @pytest.mark.parametrize("M,K,top_k,E,block,dtype", [
     (1, 128, 1, 3, 16, torch.bfloat16),        # one group, one slot
     (7, 7168, 9, 257, 8, torch.bfloat16),
