@@ -9,6 +9,8 @@
 //     equal to numel, one expert id per block (-1 past the padded total), and the padded total.
 //
 // Both are HBM-bound integer/byte passes: 16-byte loads, no matrix instructions.
+#include <type_traits>
+
 #include "moe_common.hpp"
 
 namespace alpha_moe {
@@ -19,7 +21,7 @@ constexpr int kAlignMaxSeg = 512;      // most segments before they get longer: 
                                        // (4 Mi slots, 4096 experts: 10.2 ms in 4096 segments, 272 us in 512;
                                        // 600 000 slots, 257 experts: 42 us in 586, 26 in 293)
 // Most routing slots one workgroup aligns by itself.  MI355X, one workgroup / two launches, 128 - 512 experts: 3072 slots
-// 8.5 - 10.2 / 9.4 - 10.9 us, 4096 9.8 - 11.7 / 9.4 - 11.2, 5120 11.0 - 13.2 / 9.7 - 11.1.
+// 5.8 - 6.9 / 7.1 - 7.9 us, 4096 6.8 - 7.8 / 7.0 - 8.0, 5120 8.4 - 9.8 / 7.1 - 8.0.
 constexpr int kAlignSmall = 4096;
 constexpr int kAlignMaxExperts = 4096;
 
@@ -84,25 +86,41 @@ __global__ __launch_bounds__(256) void quant_group128_kernel(const T *__restrict
 }
 
 // ---- alignment ---------------------------------------------------------------------------------------------
-// A stable counting sort of the routing slots by expert.  What bounds it is latency: a few hundred KiB of integers, so
-// everything serial counts.  A wavefront ranks 64 consecutive slots among the equal experts of its chunk with one ballot
-// per bit of the expert id (same_expert) - a loop over the chunk's distinct experts, ~60 LDS round trips for 64 slots
-// of 257 experts, is what took most of 398 us for 2997 slots and of 193 us for 73 728 - and every wavefront counts and
-// places a run of slots of its own behind cursors of its own.  MI355X, 257 experts: 9 us for 2997 slots, 12 us (two
-// launches) for 73 728; nine slots take 5.3 us (8.1 with a serial scan over the experts).
+// A stable counting sort of the routing slots by expert.  What bounds it is a chain of dependent steps on one workgroup of
+// sixteen wavefronts, where every instruction of all of them takes 16 cycles of the chain: round trips and instructions are
+// what is saved.  A wavefront ranks 64 consecutive slots among the equal experts of its chunk with a table of lane masks in LDS
+// (same_expert; a ballot per bit of the expert id was 72 instructions a chunk), keeps its slots in registers between counting and
+// placing, and counts and places a run of slots of its own behind cursors of its own.  MI355X, us in a graph of such calls,
+// before (ballots, slots read twice, prefix sums by LDS shuffles, divisions by the block size) / now: 9 slots of 257 experts
+// 5.2 / 3.9, 2997 slots 9.2 / 6.3, 4000 slots of 512 experts 11.3 / 7.9; in two launches 18 432 slots 10.6 / 7.9, 73 728 slots
+// 10.9 / 9.0, 8192 slots of 128 experts 9.1 / 6.9.
 typedef unsigned long long lanes_t;
+constexpr int kMasks = 256;   // entries of a wavefront's table of lane masks: the experts' low eight bits
+
+// LDS accesses of one wavefront complete in order; this keeps the compiler to the written order
+__device__ __forceinline__ void lds_order()
+{
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+}
 
 // The lanes of this wavefront whose slot has the same expert as this lane's (e < 0: no slot, no lanes); all 64 lanes
-// call it.
-__device__ __forceinline__ lanes_t same_expert(int e, int id_bits)
+// call it.  masks: the wavefront's table, zero before and after (its LDS accesses complete in order).
+__device__ __forceinline__ lanes_t same_expert(int e, int id_bits, lanes_t *masks)
 {
-    lanes_t same = __ballot(e >= 0);
-    for (int b = 0; b < id_bits; b++) {
+    lanes_t same = 0;
+    if (e >= 0) atomicOr(&masks[e & (kMasks - 1)], 1ull << (threadIdx.x & 63));
+    lds_order();
+    if (e >= 0) same = masks[e & (kMasks - 1)];
+    lds_order();
+    if (e >= 0) masks[e & (kMasks - 1)] = 0;
+    lds_order();
+    for (int b = 8; b < id_bits; b++) {   // the upper bits, one ballot each
         const bool set = (e >> b) & 1;
         const lanes_t with = __ballot(set);
         same &= set ? with : ~with;
     }
-    return e >= 0 ? same : 0;
+    return same;
 }
 
 __device__ __forceinline__ int expert_of_slot(const int32_t *ids, int i, int end, int E)
@@ -113,95 +131,158 @@ __device__ __forceinline__ int expert_of_slot(const int32_t *ids, int i, int end
 
 __device__ __forceinline__ lanes_t lanes_below() { return (1ull << (threadIdx.x & 63)) - 1ull; }
 
-// LDS accesses of one wavefront complete in order; this keeps the compiler to the written order
-__device__ __forceinline__ void lds_order()
+// The 64-slot chunks of ids[lo, hi) that a wavefront keeps in registers between counting and placing.
+constexpr int kKept = 4;
+struct Chunks {
+    int e[kKept];
+    lanes_t same[kKept];
+};
+
+__device__ __forceinline__ void load_chunks(const int32_t *ids, int lo, int hi, int E, Chunks &c)
 {
-    __builtin_amdgcn_wave_barrier();
-    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int k = 0; k < kKept; k++) c.e[k] = expert_of_slot(ids, lo + k * 64 + (threadIdx.x & 63), hi, E);
 }
 
-// counts[e] += slots of expert e in ids[lo, hi).  One wavefront, its own counters.
-__device__ __forceinline__ void count_run(const int32_t *ids, int lo, int hi, int E, int id_bits, uint16_t *counts)
+// counts[at] += n, 16-bit counts, without a round trip.  (Neighbouring wavefronts' counters may share a word.)
+__device__ __forceinline__ void add_count(uint16_t *counts, int at, int n)
 {
-    for (int base = lo; base < hi; base += 64) {
+    atomicAdd(reinterpret_cast<unsigned *>(counts) + (at >> 1), (unsigned)n << (16 * (at & 1)));
+}
+
+// cursors[e][column] += slots of expert e in ids[lo, hi).  One wavefront, its own column; c holds the first chunks' experts.
+__device__ __forceinline__ void count_run(const int32_t *ids, int lo, int hi, int E, int id_bits, lanes_t *masks,
+                                          uint16_t *cursors, int column, int n_waves, Chunks &c)
+{
+    auto count = [&](int e, lanes_t same) {
+        if (e >= 0 && (same & lanes_below()) == 0) add_count(cursors, e * n_waves + column, __builtin_popcountll(same));
+    };
+#pragma unroll
+    for (int k = 0; k < kKept; k++)
+        if (lo + k * 64 < hi) c.same[k] = same_expert(c.e[k], id_bits, masks);
+#pragma unroll
+    for (int k = 0; k < kKept; k++)
+        if (lo + k * 64 < hi) count(c.e[k], c.same[k]);
+    for (int base = lo + kKept * 64; base < hi; base += 64) {
         const int e = expert_of_slot(ids, base + (threadIdx.x & 63), hi, E);
-        const lanes_t same = same_expert(e, id_bits);
-        if (e >= 0 && (same & lanes_below()) == 0) counts[e] += (uint16_t)__builtin_popcountll(same);
-        lds_order();
+        count(e, same_expert(e, id_bits, masks));
     }
 }
 
-// sorted_ids[start[e] + cursor[e] ...] = the slots of expert e in ids[lo, hi), in order.  One wavefront, its own cursors.
-__device__ __forceinline__ void place_run(const int32_t *ids, int lo, int hi, int E, int id_bits, const int *start,
-                                          uint16_t *cursor, int32_t *sorted_ids)
+// sorted_ids[start(e) + cursor[e] ...] = the slots of expert e in ids[lo, hi), in order.  One wavefront, its own cursors
+// (a chunk's are read before they move on: LDS accesses of a wavefront complete in order).
+template <typename Start>
+__device__ __forceinline__ void place_run(const int32_t *ids, int lo, int hi, int E, int id_bits, lanes_t *masks, Start start,
+                                          uint16_t *cursors, int column, int n_waves, const Chunks &c,
+                                          int32_t *sorted_ids)
 {
-    for (int base = lo; base < hi; base += 64) {
+    auto place = [&](int e, lanes_t same) {   // the slot's place
+        int at = 0;
+        if (e >= 0) at = start(e) + cursors[e * n_waves + column];
+        lds_order();
+        if (e >= 0 && (same & lanes_below()) == 0) add_count(cursors, e * n_waves + column, __builtin_popcountll(same));
+        lds_order();
+        return at + __builtin_popcountll(same & lanes_below());
+    };
+    int at[kKept];
+#pragma unroll
+    for (int k = 0; k < kKept; k++)
+        if (lo + k * 64 < hi) at[k] = place(c.e[k], c.same[k]);
+#pragma unroll
+    for (int k = 0; k < kKept; k++)
+        if (lo + k * 64 < hi && c.e[k] >= 0) sorted_ids[at[k]] = lo + k * 64 + (threadIdx.x & 63);
+    for (int base = lo + kKept * 64; base < hi; base += 64) {
         const int i = base + (threadIdx.x & 63);
         const int e = expert_of_slot(ids, i, hi, E);
-        const lanes_t same = same_expert(e, id_bits);
-        const int rank = __builtin_popcountll(same & lanes_below());
-        const int at = e >= 0 ? cursor[e] : 0;
-        lds_order();
-        if (e >= 0) {
-            sorted_ids[start[e] + at + rank] = i;
-            if (rank == 0) cursor[e] = (uint16_t)(at + __builtin_popcountll(same));
-        }
-        lds_order();
+        const int to = place(e, same_expert(e, id_bits, masks));
+        if (e >= 0) sorted_ids[to] = i;
     }
 }
 
-// cursors[w][e] of the n_waves wavefronts: counts -> exclusive prefix over the wavefronts; returns the sum
-__device__ __forceinline__ int prefix_over_waves(uint16_t *cursors, int E, int e, int n_waves)
+// cursors[e][w] of the n_waves (2, 4, 8 or 16) wavefronts: counts -> exclusive prefix over the wavefronts; returns the sum
+__device__ __forceinline__ int prefix_over_waves(uint16_t *cursors, int e, int n_waves)
 {
     int run = 0;
-    for (int w = 0; w < n_waves; w++) {
-        const int t = cursors[w * E + e];
-        cursors[w * E + e] = (uint16_t)run;
-        run += t;
+    auto step = [&](unsigned two) {
+        const unsigned c0 = two & 0xffffu, c1 = two >> 16, first = run;
+        run += (int)(c0 + c1);
+        return first | (first + c0) << 16;
+    };
+    if (n_waves >= 8) {
+        v4i *c = reinterpret_cast<v4i *>(cursors + (size_t)e * n_waves);
+        v4i a = c[0], b = c[n_waves > 8 ? 1 : 0];
+#pragma unroll
+        for (int k = 0; k < 4; k++) a[k] = (int)step((unsigned)a[k]);
+        c[0] = a;
+        if (n_waves > 8) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) b[k] = (int)step((unsigned)b[k]);
+            c[1] = b;
+        }
+    } else {
+        unsigned *c = reinterpret_cast<unsigned *>(cursors + (size_t)e * n_waves);
+        const unsigned a = c[0], b = c[n_waves > 2 ? 1 : 0];
+        c[0] = step(a);
+        if (n_waves > 2) c[1] = step(b);
     }
     return run;
 }
 
-// Exclusive prefix sum over the n values of LDS array `vals`, in place; returns their sum.  All threads call it.
-__device__ int block_exclusive_scan(int *vals, int n, int *wave_sums /* [blockDim.x / 64] */)
+// Inclusive prefix sum over the wavefront, in registers (a step is a shift within rows of 16 lanes, or the last lane of the rows
+// before; through LDS, as __shfl_up goes, a step is a round trip).
+__device__ __forceinline__ int row_inclusive_scan(int v)
 {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
-    const int per = (n + blockDim.x - 1) / blockDim.x;
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // from 1, 2, 4, 8 lanes below in the row
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    return v;
+}
+__device__ __forceinline__ int wave_inclusive_scan(int v)
+{
+    v = row_inclusive_scan(v);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // lane 15 of rows 0 and 2 to rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // lane 31 to rows 2 and 3
+    return v;
+}
+
+// Exclusive prefix sum over the n values of LDS array `vals`, in place; returns their sum.  All 1024 threads call it.
+__device__ int block_exclusive_scan(int *vals, int n, int *wave_sums /* [16] */)
+{
+    const int per = (n + 1023) / 1024;
     const int lo = min((int)threadIdx.x * per, n), hi = min(lo + per, n);
-    int sum = 0;
-    for (int i = lo; i < hi; i++) sum += vals[i];
-    int incl = sum;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const int t = __shfl_up(incl, d);
-        if (lane >= d) incl += t;
+    int sum = 0, incl = 0;
+    if (__builtin_amdgcn_readfirstlane(lo < n)) {   // (a wavefront without values leaves the others its cycles)
+        for (int i = lo; i < hi; i++) sum += vals[i];
+        incl = wave_inclusive_scan(sum);
     }
-    if (lane == 63) wave_sums[wave] = incl;
-    __syncthreads();
-    int run = incl - sum, total = 0;
-    for (int w = 0; w < n_waves; w++) {
-        const int t = wave_sums[w];
-        if (w < wave) run += t;
-        total += t;
-    }
+    if ((threadIdx.x & 63) == 63) wave_sums[threadIdx.x >> 6] = incl;
+    lds_barrier();
+    const int sums = row_inclusive_scan(wave_sums[threadIdx.x & 15]);   // (of all sixteen wavefronts, in every row)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), total = __builtin_amdgcn_readlane(sums, 15);
+    int run = incl - sum + (wave > 0 ? __builtin_amdgcn_readlane(sums, wave - 1) : 0);
     for (int i = lo; i < hi; i++) {
-        const int t = vals[i];
+        const int v = vals[i];
         vals[i] = run;
-        run += t;
+        run += v;
     }
-    __syncthreads();
+    lds_barrier();
     return total;
 }
 
-__device__ __forceinline__ int pad_to(int v, int block_size) { return (v + block_size - 1) / block_size * block_size; }
-
-// expert_ids and the padded total from the starts of the experts' padded segments (total behind the last one): workgroup
-// `part` of `parts` writes its share.
-__device__ void write_blocks(const int *start, int E, int block_size, int total, int32_t *expert_ids, int n_blocks,
-                             int32_t *ntpp, int part, int parts)
+// v / block_size (a division is some forty instructions, of every wavefront)
+__device__ __forceinline__ int blocks_in(int v, int block_size)
 {
-    const int tid = part * blockDim.x + threadIdx.x, stride = parts * blockDim.x;
-    const int used = total / block_size;
+    return (block_size & (block_size - 1)) == 0 ? v >> __builtin_ctz(block_size) : v / block_size;
+}
+__device__ __forceinline__ int pad_to(int v, int block_size) { return blocks_in(v + block_size - 1, block_size) * block_size; }
+
+// expert_ids and the padded total from the starts of the experts' padded segments (total behind the last one): thread `tid` of
+// `stride` writes its share.
+__device__ void write_blocks(const int *start, int E, int block_size, int total, int32_t *expert_ids, int n_blocks,
+                             int32_t *ntpp, int tid, int stride)
+{
+    const int used = blocks_in(total, block_size);
     for (int b = tid; b < n_blocks; b += stride) {
         int e = -1;
         if (b < used) {   // the last expert whose segment starts at or before the block (empty segments start there too)
@@ -229,6 +310,9 @@ __device__ __forceinline__ void fill_sentinel(int32_t *sorted_ids, int sorted_nu
     for (int i = head + 4 * quads + tid; i < sorted_num; i += stride) sorted_ids[i] = numel;
 }
 
+// bytes of the cursors of n_waves wavefronts, whole 16 bytes
+__host__ __device__ constexpr size_t cursor_bytes(int n_waves, int E) { return ((size_t)n_waves * E * sizeof(uint16_t) + 15) & ~(size_t)15; }
+
 // One workgroup does everything (up to kAlignSmall slots).  n_waves of its wavefronts count and place `run` slots each.
 struct AlignSmall {
     const int32_t *ids;
@@ -246,29 +330,37 @@ __device__ __forceinline__ void align_small(const AlignSmall &a)
     const int numel = a.numel, E = a.E, id_bits = a.id_bits, block_size = a.block_size, sorted_num = a.sorted_num;
     const int n_waves = a.n_waves, run = a.run;
     int32_t *sorted_ids = a.sorted_ids;
-    extern __shared__ __attribute__((aligned(16))) int lds[];   // [E] starts | [16] | [n_waves][E] cursors (16 bit)
-    int *start = lds, *wave_sums = lds + E;
-    uint16_t *cursors = reinterpret_cast<uint16_t *>(lds + E + 16);
+    // [n_waves] tables of lane masks | [E][n_waves] cursors (16 bit, whole 16 bytes) | [16] the scan's sums | [E] starts
+    extern __shared__ __attribute__((aligned(16))) uint8_t mem[];
+    lanes_t *masks = reinterpret_cast<lanes_t *>(mem);
+    uint16_t *cursors = reinterpret_cast<uint16_t *>(masks + n_waves * kMasks);
+    const int zero_quads = (int)(cursor_bytes(n_waves, E) + n_waves * kMasks * sizeof(lanes_t)) / 16;
+    int *wave_sums = reinterpret_cast<int *>(mem) + 4 * zero_quads, *start = wave_sums + 16;
     const int wave = threadIdx.x >> 6;
-    for (int i = threadIdx.x; i < (n_waves * E + 1) / 2; i += blockDim.x) reinterpret_cast<int *>(cursors)[i] = 0;
+    const int lo = wave * run, hi = wave < n_waves ? min(lo + run, numel) : lo;
+    Chunks c;
+    load_chunks(ids, lo, hi, E, c);
+    for (int i = threadIdx.x; i < zero_quads; i += blockDim.x) reinterpret_cast<v4i *>(mem)[i] = (v4i){0, 0, 0, 0};
+    masks += wave * kMasks;
+    lds_barrier();
+    count_run(ids, lo, hi, E, id_bits, masks, cursors, wave, n_waves, c);
+    // (behind the use of the slots' experts: a load is waited for with everything issued behind it)
     fill_sentinel(sorted_ids, sorted_num, numel, threadIdx.x, blockDim.x);
-    __syncthreads();
-    const int lo = wave * run, hi = min(lo + run, numel);
-    if (wave < n_waves) count_run(ids, lo, hi, E, id_bits, cursors + wave * E);
-    __syncthreads();
-    for (int e = threadIdx.x; e < E; e += blockDim.x) start[e] = pad_to(prefix_over_waves(cursors, E, e, n_waves), block_size);
-    __syncthreads();
+    lds_barrier();
+    for (int e = threadIdx.x; e < E; e += blockDim.x) start[e] = pad_to(prefix_over_waves(cursors, e, n_waves), block_size);
+    lds_barrier();
     const int total = block_exclusive_scan(start, E, wave_sums);
-    // (the barriers above have also completed the sentinel fill before any slot is placed)
-    if (wave < n_waves) place_run(ids, lo, hi, E, id_bits, start, cursors + wave * E, sorted_ids);
-    write_blocks(start, E, block_size, total, a.expert_ids, a.n_blocks, a.ntpp, 0, 1);
+    drain_vmem();   // the sentinels are there before any slot is placed
+    lds_barrier();
+    place_run(ids, lo, hi, E, id_bits, masks, [&](int e) { return start[e]; }, cursors, wave, n_waves, c, sorted_ids);
+    // (wavefronts without slots take the first blocks)
+    write_blocks(start, E, block_size, total, a.expert_ids, a.n_blocks, a.ntpp, blockDim.x - 1 - threadIdx.x, blockDim.x);
 }
 
 __global__ __launch_bounds__(1024) void align_small_kernel(const AlignSmall a) { align_small(a); }
 
 // Both preparations of a layer call in one launch: workgroup 0 aligns, the others quantise.  Neither needs the other's
-// result, and at decode sizes each is ~5 us of latency: layer calls,
-// DeepSeek shard M=1 30.3 -> 26.3 us, M=7 63.8 -> 61.5, M=333 287 -> 283, Qwen3-30B M=61 104 -> 100.
+// result, and at decode sizes each is 2 - 6 us of latency.
 template <typename T>
 __global__ __launch_bounds__(1024) void prepare_small_kernel(const AlignSmall a, const T *__restrict__ x,
                                                              uint8_t *__restrict__ q, float *__restrict__ scale,
@@ -314,63 +406,75 @@ __global__ __launch_bounds__(256) void prepare_hist_kernel(const int32_t *__rest
 }
 
 // Pass 2, one workgroup per segment: every workgroup adds the histograms up itself (columns of two experts, the segments
-// split over the threads that share a column, sixteen in flight each; a third launch of one workgroup for the sums took
+// split over the threads that share a column, a thread's share in flight at once as far as twelve go; a third launch of one workgroup for the sums took
 // 17 - 42 us), scans the padded totals and places its segment, each of its n_waves wavefronts a part of it.
-// 1024 threads: every step is a dependent round trip of memory or LDS, and four times the threads take a quarter of the
-// rounds: 257 experts, 18 432 slots 13 -> 10 us, 73 728 slots 15 -> 11, 512 experts, 40 960 slots 12 -> 10 (before: 256).
+// 1024 threads: four times as many as 256 took a quarter of the rounds of dependent round trips (18 432 slots 13 -> 10 us, before
+// the rounds themselves were shortened).
 __global__ __launch_bounds__(1024) void align_place_kernel(const int32_t *__restrict__ ids, int numel, int E, int id_bits,
                                                            int block_size, const int *__restrict__ hist, int words,
                                                            int32_t *sorted_ids, int32_t *expert_ids, int n_blocks,
                                                            int32_t *ntpp, int n_waves, int seg_slots)
 {
-    // [2 words] starts | [2 words] slots of earlier segments | [n_waves][E] cursors (16 bit; first the scan's partial sums)
-    extern __shared__ __attribute__((aligned(16))) int lds[];
-    int *start = lds, *before = lds + 2 * words;
-    uint16_t *cursors = reinterpret_cast<uint16_t *>(lds + 4 * words);
+    // [n_waves] tables of lane masks | [E][n_waves] cursors (16 bit, whole 16 bytes) | [2 words] starts | [2 words] slots of
+    // earlier segments | [16] the scan's sums
+    extern __shared__ __attribute__((aligned(16))) uint8_t mem[];
+    lanes_t *masks = reinterpret_cast<lanes_t *>(mem);
+    uint16_t *cursors = reinterpret_cast<uint16_t *>(masks + n_waves * kMasks);
+    int *start = reinterpret_cast<int *>(mem + n_waves * kMasks * sizeof(lanes_t) + cursor_bytes(n_waves, E));
+    int *before = start + 2 * words, *wave_sums = before + 2 * words;
     const int wave = threadIdx.x >> 6, n_seg = gridDim.x, seg = blockIdx.x;
-    for (int i = threadIdx.x; i < 4 * words; i += blockDim.x) lds[i] = 0;
-    __syncthreads();
+    const int run = seg_slots / n_waves;
+    const int lo = seg * seg_slots + wave * run, hi = wave < n_waves ? min(lo + run, numel) : lo;
+    Chunks c;
+    load_chunks(ids, lo, hi, E, c);
+    const int zero_quads = (int)(reinterpret_cast<uint8_t *>(wave_sums) - mem) / 16;
+    for (int i = threadIdx.x; i < zero_quads; i += blockDim.x) reinterpret_cast<v4i *>(mem)[i] = (v4i){0, 0, 0, 0};
+    masks += wave * kMasks;
+    lds_barrier();
     const int share = words < (int)blockDim.x ? blockDim.x / words : 1;   // threads of a column
     const int part = words < (int)blockDim.x ? threadIdx.x / words : 0;
-    for (int c = (int)threadIdx.x - part * words; c < words && part < share; c += blockDim.x) {
-        int b0 = 0, b1 = 0, t0 = 0, t1 = 0;
-        for (int s0 = part; s0 < n_seg; s0 += 16 * share) {
-            unsigned v[16];
+    auto add_up = [&](auto in_flight) {
+        constexpr int U = decltype(in_flight)::value;
+        for (int col = (int)threadIdx.x - part * words; col < words && part < share; col += blockDim.x) {
+            int b0 = 0, b1 = 0, t0 = 0, t1 = 0;
+            for (int s0 = part; s0 < n_seg; s0 += U * share) {
+                unsigned v[U];
 #pragma unroll
-            for (int k = 0; k < 16; k++) v[k] = s0 + k * share < n_seg ? (unsigned)hist[(size_t)(s0 + k * share) * words + c] : 0u;
+                for (int k = 0; k < U; k++) v[k] = (unsigned)hist[(size_t)min(s0 + k * share, n_seg - 1) * words + col];
 #pragma unroll
-            for (int k = 0; k < 16; k++) {
-                const int c0 = v[k] & 0xffffu, c1 = v[k] >> 16;
-                t0 += c0;
-                t1 += c1;
-                if (s0 + k * share < seg) {
-                    b0 += c0;
-                    b1 += c1;
+                for (int k = 0; k < U; k++) {
+                    const unsigned w = s0 + k * share < n_seg ? v[k] : 0u;
+                    const int c0 = w & 0xffffu, c1 = w >> 16;
+                    t0 += c0;
+                    t1 += c1;
+                    if (s0 + k * share < seg) {
+                        b0 += c0;
+                        b1 += c1;
+                    }
                 }
             }
+            atomicAdd(&start[2 * col], t0);
+            atomicAdd(&start[2 * col + 1], t1);
+            atomicAdd(&before[2 * col], b0);
+            atomicAdd(&before[2 * col + 1], b1);
         }
-        atomicAdd(&start[2 * c], t0);
-        atomicAdd(&start[2 * c + 1], t1);
-        atomicAdd(&before[2 * c], b0);
-        atomicAdd(&before[2 * c + 1], b1);
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < 2 * words; i += blockDim.x) start[i] = pad_to(start[i], block_size);
-    __syncthreads();
-    const int total = block_exclusive_scan(start, E, lds + 4 * words);
-    for (int i = threadIdx.x; i < (n_waves * E + 1) / 2; i += blockDim.x) reinterpret_cast<int *>(cursors)[i] = 0;
-    write_blocks(start, E, block_size, total, expert_ids, n_blocks, ntpp, seg, n_seg);
-    __syncthreads();
-    const int run = seg_slots / n_waves;
-    const int lo = seg * seg_slots + wave * run, hi = min(lo + run, numel);
-    if (wave < n_waves) count_run(ids, lo, hi, E, id_bits, cursors + wave * E);
-    __syncthreads();
+    };
+    if (n_seg <= 2 * share)
+        add_up(std::integral_constant<int, 2>());
+    else if (n_seg <= 4 * share)
+        add_up(std::integral_constant<int, 4>());
+    else
+        add_up(std::integral_constant<int, 12>());
+    count_run(ids, lo, hi, E, id_bits, masks, cursors, wave, n_waves, c);
+    lds_barrier();
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
-        prefix_over_waves(cursors, E, e, n_waves);
-        start[e] += before[e];
+        prefix_over_waves(cursors, e, n_waves);
+        start[e] = pad_to(start[e], block_size);
     }
-    __syncthreads();
-    if (wave < n_waves) place_run(ids, lo, hi, E, id_bits, start, cursors + wave * E, sorted_ids);
+    lds_barrier();
+    const int total = block_exclusive_scan(start, E, wave_sums);
+    place_run(ids, lo, hi, E, id_bits, masks, [&](int e) { return start[e] + before[e]; }, cursors, wave, n_waves, c, sorted_ids);
+    write_blocks(start, E, block_size, total, expert_ids, n_blocks, ntpp, seg * blockDim.x + threadIdx.x, n_seg * blockDim.x);
 }
 
 // What is quantised beside an alignment (x == nullptr: nothing).
@@ -410,13 +514,16 @@ int align(const int32_t *topk_ids, int numel, int num_experts, int block_size, i
     int id_bits = 0;
     while ((1 << id_bits) < E) id_bits++;
     if (numel <= kAlignSmall) {
-        // as many wavefronts as there are chunks of 64 slots, and no more than have room for their cursors
-        int n_waves = (numel + 63) / 64;
-        if (n_waves > 16) n_waves = 16;
-        const int room = (40 << 10) / (E * (int)sizeof(uint16_t));
-        if (n_waves > room) n_waves = room;
+        // a power of two of wavefronts, as many as there are chunks of 64 slots, and no more than have room for their tables
+        // and cursors in 64 KiB of LDS
+        int n_waves = 2;
+        while (n_waves < 16 && n_waves * 64 < numel) n_waves *= 2;
+        auto lds_of = [&](int waves) {
+            return waves * kMasks * sizeof(lanes_t) + cursor_bytes(waves, E) + (16 + E) * sizeof(int);
+        };
+        while (lds_of(n_waves) > (64 << 10)) n_waves /= 2;
         const int run = ((numel + n_waves - 1) / n_waves + 63) / 64 * 64;
-        const size_t lds = (E + 16) * sizeof(int) + ((size_t)n_waves * E + 1) / 2 * sizeof(int);
+        const size_t lds = lds_of(n_waves);
         const AlignSmall a = {topk_ids, numel, E, id_bits, block_size, sorted_token_ids, sorted_num, expert_ids, n_blocks,
                               num_tokens_post_padded, n_waves, run};
         if (!z.x)
@@ -445,10 +552,13 @@ int align(const int32_t *topk_ids, int numel, int num_experts, int block_size, i
         hipLaunchKernelGGL(prepare_hist_kernel<uint16_t>, dim3(n_seg + quant_grid(z, 256)), dim3(256), words * sizeof(int),
                            hs, topk_ids, numel, E, hist, words, sorted_token_ids, sorted_num, n_seg, seg,
                            static_cast<const uint16_t *>(z.x), z.q, z.scale, n_groups);
-    // sixteen wavefronts where their cursors fit 32 KiB, at least four (64 KiB of LDS in all at kAlignMaxExperts)
-    const int n_waves = E <= 1024 ? 16 : E <= 2048 ? 8 : 4;
-    const int cursor_words = (n_waves * E + 1) / 2;
-    const size_t lds = (4 * words + (cursor_words > 16 ? cursor_words : 16)) * sizeof(int);
+    // as many wavefronts, sixteen at most, as have room for their tables and cursors in 64 KiB of LDS (at kAlignMaxExperts two)
+    int n_waves = 16;
+    auto lds_of = [&](int waves) {
+        return waves * kMasks * sizeof(lanes_t) + cursor_bytes(waves, E) + (4 * words + 16) * sizeof(int);
+    };
+    while (lds_of(n_waves) > (64 << 10)) n_waves /= 2;
+    const size_t lds = lds_of(n_waves);
     hipLaunchKernelGGL(align_place_kernel, dim3(n_seg), dim3(1024), lds, hs, topk_ids, numel, E, id_bits, block_size, hist,
                        words, sorted_token_ids, expert_ids, n_blocks, num_tokens_post_padded, n_waves, seg);
     return hipGetLastError() == hipSuccess ? ALPHA_MOE_OK : ALPHA_MOE_ERR_LAUNCH;
