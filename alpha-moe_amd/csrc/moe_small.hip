@@ -24,10 +24,10 @@
 //
 // Measured on MI355X, us a call, weights cold, streaming kernel / this one: DeepSeek-V3 shard M = 1 28.5 / 18.9, 4 48.5 /
 // 35.8, 8 77.4 / 60.5, 16 116.8 / 98.1; Qwen3-Next shard M = 1 23.4 / 12.8, 3 27.7 / 18.9, 16 61.5 / 51.1; Qwen3-30B shard
-// M = 1 27.1 / 17.9, 8 45.0 / 39.9, 16 61.0 / 58.1.  What bounds it: from M = 4 on the DeepSeek-V3 shard HBM (5.9 TB/s over the
-// first launch and 5.5 over the second at M = 16, launch and prologue included); below, the chain - at M = 1 2.5 us to the
-// first weight load, 6.5 us until 33 MB have landed, 2 us between the launches, 2.5 us to the second one's first load, 4.5 us
-// for its 16.5 MB.
+// M = 1 27.1 / 17.9, 8 45.0 / 39.9, 16 61.0 / 58.1 (this one is 1.0 - 2.5 us faster since: see the DOWN kernel).  What bounds
+// it: from M = 4 on the DeepSeek-V3 shard HBM (5.9 TB/s over the first launch and 5.5 over the second at M = 16, launch and
+// prologue included); below, the chain - at M = 1 2.5 us to the first weight load, 6.5 us until 33 MB have landed, 2 us between
+// the launches, then the second one's prologue and 4.5 us for its 16.5 MB.
 #include <mutex>
 #include <type_traits>
 
