@@ -356,13 +356,15 @@ void fused_experts(at::Tensor &hidden, const at::Tensor &topk_ids, const at::Ten
 {
     TORCH_CHECK_INDEX(topk_ids.dim() >= 2 && w.dim() >= 1, "topk_ids must be [M, top_k], w [E, N, K]");
     const int64_t top_k = topk_ids.size(1), E = w.size(0);
-    // (what prepare_inputs and the operator would refuse is left to them)
+    // (what prepare_inputs and the operator would refuse is left to them: the sizes and knobs are in the range of an int, from both
+    // sides, before they are narrowed)
     const bool whole = hidden.is_cuda() && hidden.dim() == 2 && hidden.scalar_type() == at::kBFloat16 && hidden.is_contiguous() &&
                        group_size == 128 && topk_ids.device() == hidden.device() && topk_ids.scalar_type() == at::kInt &&
                        topk_ids.is_contiguous() && hidden.size(0) <= 64 && topk_ids.numel() == hidden.size(0) * top_k &&
                        (reinterpret_cast<uintptr_t>(hidden.const_data_ptr()) & 15) == 0 && w.dim() == 3 &&
                        w.size(1) <= INT32_MAX && hidden.size(1) <= INT32_MAX && E <= INT32_MAX && top_k <= INT32_MAX &&
-                       block_m > 0 && block_m <= 128 && block_n <= 128 && warp_n <= 128 && stages <= 128 &&
+                       block_m > 0 && block_m <= 128 && block_n > 0 && block_n <= 128 && warp_n > 0 && warp_n <= 128 &&
+                       stages > 0 && stages <= 128 &&
                        alpha_moe_layer_call_supported(static_cast<int>(top_k), static_cast<int>(hidden.size(0)),
                                                       static_cast<int>(hidden.size(1)), static_cast<int>(w.size(1)),
                                                       static_cast<int>(E), static_cast<int>(block_m), static_cast<int>(block_n),

@@ -132,3 +132,23 @@ def test_layer_call_equals_its_three_steps_bit_for_bit(M, top_k, K, I, E, block_
             graph.replay()
             same(h, want)
             assert not torch.zeros(4, device=DEV).any()
+
+
+@pytest.mark.parametrize("M", [3, 40])
+@pytest.mark.parametrize("knob", ["block_m", "block_n", "warp_n", "stages"])
+def test_layer_call_refuses_knobs_that_only_their_low_32_bits_make_legal(knob, M):
+    """With and without the two-launch form: a legal value plus or minus 2**32 is no legal value."""
+    import alpha_moe  # noqa: F401
+    E, top_k, K, I = 4, 2, 256, 128
+    w13 = torch.zeros((E, 2 * I, K), device=DEV).to(torch.float8_e4m3fn)
+    w2 = torch.zeros((E, K, I), device=DEV).to(torch.float8_e4m3fn)
+    w13_s, w2_s = torch.ones((E, 2 * I // 128, K // 128), device=DEV), torch.ones((E, K // 128, I // 128), device=DEV)
+    ids = torch.arange(M * top_k, dtype=torch.int32, device=DEV).view(M, top_k) % E
+    legal = {"block_m": 16, "block_n": 32, "warp_n": 8, "stages": 4}
+    for value in (legal[knob] - 2 ** 32, legal[knob] + 2 ** 32, 0, -legal[knob]):
+        h = torch.ones((M, K), dtype=torch.bfloat16, device=DEV)
+        print(f"case layer call M={M} {knob}={value}", flush=True)
+        with pytest.raises(RuntimeError):
+            torch.ops.alpha_moe.fused_experts(h, ids, w13, w13_s, w2, w2_s, torch.ones((M, top_k), device=DEV), 128,
+                                              *{**legal, knob: value}.values(), 1.0)
+        assert bool((h == 1).all())
