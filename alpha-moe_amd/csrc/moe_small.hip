@@ -161,10 +161,8 @@ __device__ __forceinline__ uint2 quantise_row(const v4i raw, float *scale)
 // NKW: 128-byte K blocks per wavefront.  LAYER: what a layer call starts from - bf16 activations and the router's output -
 // is prepared here, by every workgroup for itself: the active experts come from a bit map of the rows' experts (ascending, as
 // the aligner sorts them), and a wavefront quantises its K range of all tokens while its first weights are on their way.  That
-// saves the preparation's launch (5.1 us of a chain of a few dependent steps on one workgroup, and the gap behind it).  MI355X,
-// cold weights, us a layer call, three launches / two: DeepSeek shard 1 token 31.9 / 28.0, 8 tokens 71.4 / 67.4, 16 tokens 109.8 /
-// 109.9 (there the activations, read at twice the width by 256 workgroups, take what the launch did); Qwen3-Next shard 24.7 /
-// 19.6, 44.8 / 38.8, 61.4 / 56.2; Qwen3-MoE shard 30.4 / 25.6, 48.4 / 43.6, 68.8 / 63.8.
+// saves the preparation's launch (a chain of a few dependent steps on one workgroup, and the gap behind it: 3.3 - 4 us of a graph
+// of layer calls); layer_pays() has both sides.
 template <int NKW, bool LAYER>
 __global__ __launch_bounds__(kThreads) void moe_small_up_kernel(const SmallParams s)
 {
@@ -764,13 +762,19 @@ struct SmallPlan {
     int nkw, up_parts, h, dcols, n_down, gi, ring, off_sa, off_w2s, lds_bytes;
 };
 
+// K blocks of a wavefront of the first launch: the variants there are
+int blocks_per_wave(int K)
+{
+    const int per_wave = (K / 128 + kWaves - 1) / kWaves;
+    return per_wave <= 1 ? 1 : per_wave <= 2 ? 2 : per_wave <= 4 ? 4 : 7;
+}
+
 SmallPlan make_plan(int top_k, int M, int K, int N, int block_m)
 {
     SmallPlan h = {};
     const int n_ib = N / 256, rows = M * top_k;
     if (M > kMaxTokens || rows > kMaxRows || n_ib > kMaxSlices || K > 128 * kWaves * 7 || block_m > 32) return h;
-    const int per_wave = (K / 128 + kWaves - 1) / kWaves;
-    h.nkw = per_wave <= 1 ? 1 : per_wave <= 2 ? 2 : per_wave <= 4 ? 4 : 7;
+    h.nkw = blocks_per_wave(K);
     const int cus = compute_units();
     h.up_parts = cus;
     // DOWN: one part per compute unit, whole groups of four columns (a lane's), at most 32
@@ -864,6 +868,17 @@ size_t small_workspace_bytes(int top_k, int M, int N)
 }
 
 bool layer_supported(int E) { return E <= kLayerExperts; }
+
+// The preparation's launch saved against what every workgroup of the first launch does instead: its eight wavefronts read and
+// quantise four tokens at a time, `nkw` K blocks each, so it grows with their product, and more of it hides behind the weights
+// the more experts are active.  MI355X, graphs of cold calls, us a layer call, three launches / two:
+//   1 group x 7 blocks    DeepSeek shard, 4 tokens 43.4 / 41.1; K = 7168, I = 128, top 1 15.4 / 14.3
+//   2 x 7                 DeepSeek shard, 8 tokens 68.2 / 66.7; K = 7168, I = 1024, top 4 66.3 / 65.4; I = 128, top 1 17.1 / 18.0
+//   4 x 2                 Qwen3-Next shard, 16 tokens 55.3 / 51.3; K = 2048, I = 128, top 1 14.6 / 13.4
+//   4 x 4                 K = 4096, 16 tokens: I = 256, top 8 58.5 / 57.6; I = 128, top 1 17.5 / 18.5
+//   3 x 7                 DeepSeek shard, 12 tokens 88.7 / 89.3; K = 5120, I = 256, top 8 60.4 / 61.5; I = 128, top 1 21.1 / 23.4
+//   4 x 7                 DeepSeek shard, 16 tokens 107.2 / 107.8; K = 6144, I = 256, top 8 75.8 / 78.7; I = 128, top 1 22.8 / 27.5
+bool layer_pays(int M, int K) { return (M + 3) / 4 * blocks_per_wave(K) <= 16; }
 
 hipError_t launch_small(const MoeParams &p, const uint16_t *x16, const int32_t *topk_ids, void *workspace, hipStream_t stream)
 {

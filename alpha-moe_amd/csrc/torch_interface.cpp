@@ -348,8 +348,8 @@ prepare_inputs(const at::Tensor &x, const at::Tensor &topk_ids, int64_t group_si
 }
 
 // A whole layer call: hidden_states [M, K] bf16 is quantised, the routing aligned, and the operator's result takes its
-// place.  The smallest batches do without the preparation and its tensors (alpha_moe_layer_call); otherwise this is
-// prepare_inputs and fused_moe_w8a8_up_down_store.
+// place.  The smallest batches do without the preparation and its tensors where that is faster (alpha_moe_layer_call_pays);
+// otherwise this is prepare_inputs and fused_moe_w8a8_up_down_store.
 void fused_experts(at::Tensor &hidden, const at::Tensor &topk_ids, const at::Tensor &w, const at::Tensor &w_scale,
                    const at::Tensor &w2, const at::Tensor &w2_scale, const at::Tensor &topk_weights, int64_t group_size,
                    int64_t block_m, int64_t block_n, int64_t warp_n, int64_t stages, double scaling_factor)
@@ -368,7 +368,8 @@ void fused_experts(at::Tensor &hidden, const at::Tensor &topk_ids, const at::Ten
                        alpha_moe_layer_call_supported(static_cast<int>(top_k), static_cast<int>(hidden.size(0)),
                                                       static_cast<int>(hidden.size(1)), static_cast<int>(w.size(1)),
                                                       static_cast<int>(E), static_cast<int>(block_m), static_cast<int>(block_n),
-                                                      static_cast<int>(warp_n), static_cast<int>(stages));
+                                                      static_cast<int>(warp_n), static_cast<int>(stages)) &&
+                       alpha_moe_layer_call_pays(static_cast<int>(hidden.size(0)), static_cast<int>(hidden.size(1)));
     if (!whole) {
         const auto [q, scale, sorted_ids, expert_ids, total] = prepare_inputs(hidden, topk_ids, group_size, block_m, E);
         run_fused_moe(q, scale, w, w_scale, w2, w2_scale, sorted_ids, expert_ids, total, topk_weights, hidden, top_k, block_m,

@@ -137,6 +137,19 @@ def test_prep_entry_points_refuse_bad_arguments_without_touching_a_device(lib):
     assert lib.alpha_moe_moe_align_block_size(8, 5000, 8, 16, 8, 5120, 8, 320, 8, None, 0, None) == 7
 
 
+def test_layer_call_pays_up_to_sixteen_token_groups_times_blocks(lib):
+    """groups of four tokens times K blocks of a wavefront (1, 2, 4 or 7): both sides of every border, and what no layer call is"""
+    lib.alpha_moe_layer_call_supported.restype = lib.alpha_moe_layer_call_pays.restype = ctypes.c_int
+    lib.alpha_moe_layer_call_supported.argtypes = [ctypes.c_int] * 9
+    lib.alpha_moe_layer_call_pays.argtypes = [ctypes.c_int] * 2
+    for K, most in ((128, 16), (1024, 16), (1152, 16), (2048, 16), (2176, 16), (4096, 16), (4224, 8), (5120, 8), (7168, 8)):
+        for M in range(1, 17):
+            assert lib.alpha_moe_layer_call_pays(M, K) == (M <= most), (M, K)
+            assert lib.alpha_moe_layer_call_supported(1, M, K, 256, 8, 16, 32, 8, 4), (M, K)
+    for M, K in ((0, 128), (-4, 128), (17, 128), (4, 0), (4, -128), (4, 65664)):
+        assert lib.alpha_moe_layer_call_pays(M, K) == 0
+
+
 def test_static_scratch_holds_every_batch_up_to_the_documented_sizes(lib):
     """With the shipped tables the entry point without a workspace takes every batch up to these sizes, also where a table
     keeps the streaming kernel and its fp32 rows (Qwen3-Next shard, 752 .. 768 tokens: 65.4 MiB)."""

@@ -152,3 +152,26 @@ def test_layer_call_refuses_knobs_that_only_their_low_32_bits_make_legal(knob, M
             torch.ops.alpha_moe.fused_experts(h, ids, w13, w13_s, w2, w2_s, torch.ones((M, top_k), device=DEV), 128,
                                               *{**legal, knob: value}.values(), 1.0)
         assert bool((h == 1).all())
+
+
+@pytest.mark.parametrize("M,K,whole", [(1, 4224, True), (8, 4224, True), (9, 4224, False), (8, 7168, True), (9, 7168, False),
+                                       (16, 4096, True), (16, 7168, False)])
+def test_layer_call_takes_two_launches_only_where_they_are_faster(M, K, whole):
+    """The two-launch form allocates nothing; the preparation returns five tensors."""
+    import alpha_moe  # noqa: F401
+    E, top_k, I = 8, 2, 128
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    w13 = torch.randn((E, 2 * I, K), generator=g, device=DEV).to(torch.float8_e4m3fn)
+    w2 = torch.randn((E, K, I), generator=g, device=DEV).to(torch.float8_e4m3fn)
+    w13_s, w2_s = torch.ones((E, 2 * I // 128, K // 128), device=DEV), torch.ones((E, K // 128, I // 128), device=DEV)
+    ids = torch.arange(M * top_k, dtype=torch.int32, device=DEV).view(M, top_k) % E
+    h, weights = torch.randn((M, K), generator=g, device=DEV).to(torch.bfloat16), torch.ones((M, top_k), device=DEV)
+
+    def call():
+        torch.ops.alpha_moe.fused_experts(h, ids, w13, w13_s, w2, w2_s, weights, 128, 16, 32, 8, 4, 1.0)
+
+    print(f"case route of a layer call M={M} K={K}", flush=True)
+    call()   # takes the scratch memory
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    call()
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == (0 if whole else 5)
