@@ -41,7 +41,7 @@ c_abi.alpha_moe_fused_moe_w8a8_up_down_prepacked.argtypes = (
 c_abi.alpha_moe_layer_call_supported.restype = ctypes.c_int
 c_abi.alpha_moe_layer_call_supported.argtypes = [ctypes.c_int] * 9
 c_abi.alpha_moe_layer_call_pays.restype = ctypes.c_int
-c_abi.alpha_moe_layer_call_pays.argtypes = [ctypes.c_int] * 2
+c_abi.alpha_moe_layer_call_pays.argtypes = [ctypes.c_int] * 9
 c_abi.alpha_moe_layer_call.restype = ctypes.c_int
 c_abi.alpha_moe_layer_call.argtypes = (
     [ctypes.c_void_p] * 8 + [ctypes.c_int] * 9 + [ctypes.c_float, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p])

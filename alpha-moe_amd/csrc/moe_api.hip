@@ -230,9 +230,11 @@ extern "C" int alpha_moe_layer_call_supported(int top_k, int M, int K, int N, in
     return layer_supported(num_experts) && choose_path(top_k, M, K, N, num_experts, (int)sorted_num, block_m, warp_n) == kSmall;
 }
 
-extern "C" int alpha_moe_layer_call_pays(int M, int K)
+extern "C" int alpha_moe_layer_call_pays(int top_k, int M, int K, int N, int num_experts, int block_m, int block_n, int warp_n,
+                                         int stages)
 {
-    return M > 0 && M <= 16 && K > 0 && K <= 128 * kMaxKBlocks && layer_pays(M, K);
+    return alpha_moe_layer_call_supported(top_k, M, K, N, num_experts, block_m, block_n, warp_n, stages) &&
+           layer_pays(top_k, M, K, N, num_experts);
 }
 
 extern "C" int alpha_moe_layer_call(const uint16_t *x, const int32_t *topk_ids, const uint8_t *w, const float *w_scale,

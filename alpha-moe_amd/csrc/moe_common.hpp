@@ -279,7 +279,7 @@ size_t small_workspace_bytes(int top_k, int M, int N);
 // x16, topk_ids: a layer call's bf16 activations and routing, prepared inside the first launch (the operator's inputs of p
 // are not read then; layer_supported()), or null.
 bool layer_supported(int E);
-bool layer_pays(int M, int K);   // ahead of the preparation and the operator one by one
+bool layer_pays(int top_k, int M, int K, int N, int E);   // ahead of the preparation and the operator one by one
 hipError_t launch_small(const MoeParams &p, const uint16_t *x16, const int32_t *topk_ids, void *workspace, hipStream_t stream);
 
 // Persistent work-queue kernel for decode-sized batches (block_m <= 32 and bounded sizes): split-K up items ->

@@ -870,15 +870,25 @@ size_t small_workspace_bytes(int top_k, int M, int N)
 bool layer_supported(int E) { return E <= kLayerExperts; }
 
 // The preparation's launch saved against what every workgroup of the first launch does instead: its eight wavefronts read and
-// quantise four tokens at a time, `nkw` K blocks each, so it grows with their product, and more of it hides behind the weights
-// the more experts are active.  MI355X, graphs of cold calls, us a layer call, three launches / two:
+// quantise four tokens at a time, `nkw` K blocks each, so it grows with their product, and the more weights follow the more of
+// it they hide.  MI355X, graphs of cold calls, us a layer call, three launches / two:
 //   1 group x 7 blocks    DeepSeek shard, 4 tokens 43.4 / 41.1; K = 7168, I = 128, top 1 15.4 / 14.3
 //   2 x 7                 DeepSeek shard, 8 tokens 68.2 / 66.7; K = 7168, I = 1024, top 4 66.3 / 65.4; I = 128, top 1 17.1 / 18.0
 //   4 x 2                 Qwen3-Next shard, 16 tokens 55.3 / 51.3; K = 2048, I = 128, top 1 14.6 / 13.4
 //   4 x 4                 K = 4096, 16 tokens: I = 256, top 8 58.5 / 57.6; I = 128, top 1 17.5 / 18.5
-//   3 x 7                 DeepSeek shard, 12 tokens 88.7 / 89.3; K = 5120, I = 256, top 8 60.4 / 61.5; I = 128, top 1 21.1 / 23.4
+//   3 x 7                 DeepSeek shard, 12 tokens 88.7 / 89.3; K = 7168, I = 256, top 2, 9 tokens 29.3 / 30.1; K = 4224, I = 256,
+//                         top 2, 12 tokens 27.8 / 30.3, I = 128, top 1, 9 tokens 17.0 / 20.5
 //   4 x 7                 DeepSeek shard, 16 tokens 107.2 / 107.8; K = 6144, I = 256, top 8 75.8 / 78.7; I = 128, top 1 22.8 / 27.5
-bool layer_pays(int M, int K) { return (M + 3) / 4 * blocks_per_wave(K) <= 16; }
+// Outside a graph the third launch and the five tensors of the preparation cost a caller that waits for each call 1 - 2 us more:
+// at 3 x 7 DeepSeek shard, 12 tokens 108.2 / 106.3, K = 7168, I = 256, top 2, 9 tokens 46.0 / 44.3 (99 MB of weights), but K = 4224,
+// I = 256, top 2, 12 tokens 45.2 / 45.2 (78 MB), I = 128, top 1, 9 tokens 34.7 / 36.0; at 4 x 7 DeepSeek shard 128.3 / 127.7, K = 5120,
+// I = 256, top 8 87.5 / 88.4.
+bool layer_pays(int top_k, int M, int K, int N, int E)
+{
+    const int steps = (M + 3) / 4 * blocks_per_wave(K);
+    const long long experts = (long long)M * top_k < E ? (long long)M * top_k : E;
+    return steps <= 16 || (steps <= 21 && experts * (N / 2) * 3 * K >= (80ll << 20));
+}
 
 hipError_t launch_small(const MoeParams &p, const uint16_t *x16, const int32_t *topk_ids, void *workspace, hipStream_t stream)
 {

@@ -365,11 +365,10 @@ void fused_experts(at::Tensor &hidden, const at::Tensor &topk_ids, const at::Ten
                        w.size(1) <= INT32_MAX && hidden.size(1) <= INT32_MAX && E <= INT32_MAX && top_k <= INT32_MAX &&
                        block_m > 0 && block_m <= 128 && block_n > 0 && block_n <= 128 && warp_n > 0 && warp_n <= 128 &&
                        stages > 0 && stages <= 128 &&
-                       alpha_moe_layer_call_supported(static_cast<int>(top_k), static_cast<int>(hidden.size(0)),
-                                                      static_cast<int>(hidden.size(1)), static_cast<int>(w.size(1)),
-                                                      static_cast<int>(E), static_cast<int>(block_m), static_cast<int>(block_n),
-                                                      static_cast<int>(warp_n), static_cast<int>(stages)) &&
-                       alpha_moe_layer_call_pays(static_cast<int>(hidden.size(0)), static_cast<int>(hidden.size(1)));
+                       alpha_moe_layer_call_pays(static_cast<int>(top_k), static_cast<int>(hidden.size(0)),
+                                                 static_cast<int>(hidden.size(1)), static_cast<int>(w.size(1)),
+                                                 static_cast<int>(E), static_cast<int>(block_m), static_cast<int>(block_n),
+                                                 static_cast<int>(warp_n), static_cast<int>(stages));
     if (!whole) {
         const auto [q, scale, sorted_ids, expert_ids, total] = prepare_inputs(hidden, topk_ids, group_size, block_m, E);
         run_fused_moe(q, scale, w, w_scale, w2, w2_scale, sorted_ids, expert_ids, total, topk_weights, hidden, top_k, block_m,

@@ -223,9 +223,9 @@ int alpha_moe_prepare_inputs(const void *x, int x_is_f32, uint8_t *q, float *sca
  */
 int alpha_moe_layer_call_supported(int top_k, int M, int K, int N, int num_experts, int block_m, int block_n, int warp_n,
                                    int stages);
-/* Of the calls that are taken: 1 where the call below is the faster way, 0 (above 8 tokens of more than 4096 columns) where
- * alpha_moe_prepare_inputs and the storing operator are. */
-int alpha_moe_layer_call_pays(int M, int K);
+/* 1 where the call below is taken and the faster way; 0 where it is not taken, or alpha_moe_prepare_inputs and the storing operator
+ * are faster (from 9 tokens of more than 4096 columns on, unless there are many weights to load). */
+int alpha_moe_layer_call_pays(int top_k, int M, int K, int N, int num_experts, int block_m, int block_n, int warp_n, int stages);
 int alpha_moe_layer_call(const uint16_t *x, const int32_t *topk_ids, const uint8_t *w, const float *w_scale,
                          const uint8_t *w2, const float *w2_scale, const float *topk_weights, uint16_t *out, int top_k, int M,
                          int K, int N, int num_experts, int block_m, int block_n, int warp_n, int stages,

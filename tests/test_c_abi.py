@@ -137,17 +137,26 @@ def test_prep_entry_points_refuse_bad_arguments_without_touching_a_device(lib):
     assert lib.alpha_moe_moe_align_block_size(8, 5000, 8, 16, 8, 5120, 8, 320, 8, None, 0, None) == 7
 
 
-def test_layer_call_pays_up_to_sixteen_token_groups_times_blocks(lib):
-    """groups of four tokens times K blocks of a wavefront (1, 2, 4 or 7): both sides of every border, and what no layer call is"""
-    lib.alpha_moe_layer_call_supported.restype = lib.alpha_moe_layer_call_pays.restype = ctypes.c_int
-    lib.alpha_moe_layer_call_supported.argtypes = [ctypes.c_int] * 9
-    lib.alpha_moe_layer_call_pays.argtypes = [ctypes.c_int] * 2
-    for K, most in ((128, 16), (1024, 16), (1152, 16), (2048, 16), (2176, 16), (4096, 16), (4224, 8), (5120, 8), (7168, 8)):
+def test_layer_call_pays_by_token_groups_times_blocks_and_by_weights(lib):
+    """groups of four tokens times K blocks of a wavefront (1, 2, 4 or 7): both sides of every border; at 3 x 7 the weights of the
+    experts there can be decide; a call that is not taken does not pay"""
+    pays, supported = lib.alpha_moe_layer_call_pays, lib.alpha_moe_layer_call_supported
+    pays.restype = supported.restype = ctypes.c_int
+    pays.argtypes = supported.argtypes = [ctypes.c_int] * 9
+    knobs = (16, 32, 8, 4)
+    for K, few, many in ((128, 16, 16), (1024, 16, 16), (1152, 16, 16), (2048, 16, 16), (2176, 16, 16), (4096, 16, 16),
+                         (4224, 8, 12), (5120, 8, 12), (7168, 8, 12)):
         for M in range(1, 17):
-            assert lib.alpha_moe_layer_call_pays(M, K) == (M <= most), (M, K)
-            assert lib.alpha_moe_layer_call_supported(1, M, K, 256, 8, 16, 32, 8, 4), (M, K)
-    for M, K in ((0, 128), (-4, 128), (17, 128), (4, 0), (4, -128), (4, 65664)):
-        assert lib.alpha_moe_layer_call_pays(M, K) == 0
+            assert supported(1, M, K, 256, 8, *knobs) == 1
+            assert pays(1, M, K, 256, 8, *knobs) == (M <= few), (M, K)
+            if K >= 2496:
+                assert pays(9, M, K, 512, 257, *knobs) == (M <= many), (M, K)
+    # at most rows, at most experts; 80 MiB of both weights: 15.2 experts of K = 7168, I = 256
+    assert [pays(1, 10, 7168, 2 * I, 64, *knobs) for I in (256, 384, 512)] == [0, 0, 1]
+    assert [pays(8, 10, 7168, 512, E, *knobs) for E in (15, 16)] == [0, 1]
+    assert pays(4, 17, 4096, 512, 8, *knobs) == 0 and pays(4, 8, 4096, 512, 8, 64, 32, 8, 4) == 0
+    for M, K in ((0, 128), (-4, 128), (4, 0), (4, -128), (4, 7296), (4, 130)):
+        assert pays(1, M, K, 256, 8, *knobs) == 0
 
 
 def test_static_scratch_holds_every_batch_up_to_the_documented_sizes(lib):

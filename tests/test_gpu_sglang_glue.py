@@ -154,12 +154,13 @@ def test_layer_call_refuses_knobs_that_only_their_low_32_bits_make_legal(knob, M
         assert bool((h == 1).all())
 
 
-@pytest.mark.parametrize("M,K,whole", [(1, 4224, True), (8, 4224, True), (9, 4224, False), (8, 7168, True), (9, 7168, False),
-                                       (16, 4096, True), (16, 7168, False)])
-def test_layer_call_takes_two_launches_only_where_they_are_faster(M, K, whole):
+@pytest.mark.parametrize("M,K,E,whole", [(1, 4224, 8, True), (8, 4224, 8, True), (9, 4224, 8, False), (8, 7168, 8, True),
+                                         (9, 7168, 8, False), (9, 7168, 64, True), (9, 4224, 64, False), (16, 4096, 8, True),
+                                         (16, 7168, 64, False)])
+def test_layer_call_takes_two_launches_only_where_they_are_faster(M, K, E, whole):
     """The two-launch form allocates nothing; the preparation returns five tensors."""
     import alpha_moe  # noqa: F401
-    E, top_k, I = 8, 2, 128
+    top_k, I = 2, 256
     g = torch.Generator(device=DEV).manual_seed(M + K)
     w13 = torch.randn((E, 2 * I, K), generator=g, device=DEV).to(torch.float8_e4m3fn)
     w2 = torch.randn((E, K, I), generator=g, device=DEV).to(torch.float8_e4m3fn)
@@ -170,7 +171,7 @@ def test_layer_call_takes_two_launches_only_where_they_are_faster(M, K, whole):
     def call():
         torch.ops.alpha_moe.fused_experts(h, ids, w13, w13_s, w2, w2_s, weights, 128, 16, 32, 8, 4, 1.0)
 
-    print(f"case route of a layer call M={M} K={K}", flush=True)
+    print(f"case route of a layer call M={M} K={K} E={E}", flush=True)
     call()   # takes the scratch memory
     before = torch.cuda.memory_stats()["allocation.all.allocated"]
     call()
