@@ -106,21 +106,42 @@ __device__ __forceinline__ void lds_order()
 
 // The lanes of this wavefront whose slot has the same expert as this lane's (e < 0: no slot, no lanes); all 64 lanes
 // call it.  masks: the wavefront's table, zero before and after (its LDS accesses complete in order).
+// Lanes that add to one table entry take turns.  FEW (few experts, many slots: few_experts()) is for inputs on which that is the
+// rule and not the exception: up to eight experts a ballot per bit of the id instead, otherwise the first lane's expert - the hot
+// one, if there is one - by a ballot and the others by the table.
+template <bool FEW>
 __device__ __forceinline__ lanes_t same_expert(int e, int id_bits, lanes_t *masks)
 {
+    lanes_t first = 0;
+    bool other = e >= 0;
+    if constexpr (FEW) {
+        if (id_bits <= 3) {
+            lanes_t same = __ballot(e >= 0);
+            for (int b = 0; b < id_bits; b++) {
+                const bool set = (e >> b) & 1;
+                const lanes_t with = __ballot(set);
+                same &= set ? with : ~with;
+            }
+            return e >= 0 ? same : 0;
+        }
+        const int e0 = __builtin_amdgcn_readfirstlane(e);
+        first = __ballot(e == e0);
+        first = e == e0 && e >= 0 ? first : 0;
+        other = e >= 0 && e != e0;
+    }
     lanes_t same = 0;
-    if (e >= 0) atomicOr(&masks[e & (kMasks - 1)], 1ull << (threadIdx.x & 63));
+    if (other) atomicOr(&masks[e & (kMasks - 1)], 1ull << (threadIdx.x & 63));
     lds_order();
-    if (e >= 0) same = masks[e & (kMasks - 1)];
+    if (other) same = masks[e & (kMasks - 1)];
     lds_order();
-    if (e >= 0) masks[e & (kMasks - 1)] = 0;
+    if (other) masks[e & (kMasks - 1)] = 0;
     lds_order();
     for (int b = 8; b < id_bits; b++) {   // the upper bits, one ballot each
         const bool set = (e >> b) & 1;
         const lanes_t with = __ballot(set);
         same &= set ? with : ~with;
     }
-    return same;
+    return same | first;
 }
 
 __device__ __forceinline__ int expert_of_slot(const int32_t *ids, int i, int end, int E)
@@ -151,6 +172,7 @@ __device__ __forceinline__ void add_count(uint16_t *counts, int at, int n)
 }
 
 // cursors[e][column] += slots of expert e in ids[lo, hi).  One wavefront, its own column; c holds the first chunks' experts.
+template <bool FEW>
 __device__ __forceinline__ void count_run(const int32_t *ids, int lo, int hi, int E, int id_bits, lanes_t *masks,
                                           uint16_t *cursors, int column, int n_waves, Chunks &c)
 {
@@ -159,19 +181,19 @@ __device__ __forceinline__ void count_run(const int32_t *ids, int lo, int hi, in
     };
 #pragma unroll
     for (int k = 0; k < kKept; k++)
-        if (lo + k * 64 < hi) c.same[k] = same_expert(c.e[k], id_bits, masks);
+        if (lo + k * 64 < hi) c.same[k] = same_expert<FEW>(c.e[k], id_bits, masks);
 #pragma unroll
     for (int k = 0; k < kKept; k++)
         if (lo + k * 64 < hi) count(c.e[k], c.same[k]);
     for (int base = lo + kKept * 64; base < hi; base += 64) {
         const int e = expert_of_slot(ids, base + (threadIdx.x & 63), hi, E);
-        count(e, same_expert(e, id_bits, masks));
+        count(e, same_expert<FEW>(e, id_bits, masks));
     }
 }
 
 // sorted_ids[start(e) + cursor[e] ...] = the slots of expert e in ids[lo, hi), in order.  One wavefront, its own cursors
 // (a chunk's are read before they move on: LDS accesses of a wavefront complete in order).
-template <typename Start>
+template <bool FEW, typename Start>
 __device__ __forceinline__ void place_run(const int32_t *ids, int lo, int hi, int E, int id_bits, lanes_t *masks, Start start,
                                           uint16_t *cursors, int column, int n_waves, const Chunks &c,
                                           int32_t *sorted_ids)
@@ -194,7 +216,7 @@ __device__ __forceinline__ void place_run(const int32_t *ids, int lo, int hi, in
     for (int base = lo + kKept * 64; base < hi; base += 64) {
         const int i = base + (threadIdx.x & 63);
         const int e = expert_of_slot(ids, i, hi, E);
-        const int to = place(e, same_expert(e, id_bits, masks));
+        const int to = place(e, same_expert<FEW>(e, id_bits, masks));
         if (e >= 0) sorted_ids[to] = i;
     }
 }
@@ -324,6 +346,7 @@ struct AlignSmall {
     int32_t *ntpp;
     int n_waves, run;
 };
+template <bool FEW>
 __device__ __forceinline__ void align_small(const AlignSmall &a)
 {
     const int32_t *__restrict__ ids = a.ids;
@@ -343,7 +366,7 @@ __device__ __forceinline__ void align_small(const AlignSmall &a)
     for (int i = threadIdx.x; i < zero_quads; i += blockDim.x) reinterpret_cast<v4i *>(mem)[i] = (v4i){0, 0, 0, 0};
     masks += wave * kMasks;
     lds_barrier();
-    count_run(ids, lo, hi, E, id_bits, masks, cursors, wave, n_waves, c);
+    count_run<FEW>(ids, lo, hi, E, id_bits, masks, cursors, wave, n_waves, c);
     // (behind the use of the slots' experts: a load is waited for with everything issued behind it)
     fill_sentinel(sorted_ids, sorted_num, numel, threadIdx.x, blockDim.x);
     lds_barrier();
@@ -352,21 +375,22 @@ __device__ __forceinline__ void align_small(const AlignSmall &a)
     const int total = block_exclusive_scan(start, E, wave_sums);
     drain_vmem();   // the sentinels are there before any slot is placed
     lds_barrier();
-    place_run(ids, lo, hi, E, id_bits, masks, [&](int e) { return start[e]; }, cursors, wave, n_waves, c, sorted_ids);
+    place_run<FEW>(ids, lo, hi, E, id_bits, masks, [&](int e) { return start[e]; }, cursors, wave, n_waves, c, sorted_ids);
     // (wavefronts without slots take the first blocks)
     write_blocks(start, E, block_size, total, a.expert_ids, a.n_blocks, a.ntpp, blockDim.x - 1 - threadIdx.x, blockDim.x);
 }
 
-__global__ __launch_bounds__(1024) void align_small_kernel(const AlignSmall a) { align_small(a); }
+template <bool FEW>
+__global__ __launch_bounds__(1024) void align_small_kernel(const AlignSmall a) { align_small<FEW>(a); }
 
 // Both preparations of a layer call in one launch: workgroup 0 aligns, the others quantise.  Neither needs the other's
 // result, and at decode sizes each is 2 - 6 us of latency.
-template <typename T>
+template <typename T, bool FEW>
 __global__ __launch_bounds__(1024) void prepare_small_kernel(const AlignSmall a, const T *__restrict__ x,
                                                              uint8_t *__restrict__ q, float *__restrict__ scale,
                                                              long long n_groups)
 {
-    if (blockIdx.x == 0) align_small(a);
+    if (blockIdx.x == 0) align_small<FEW>(a);
     else quant_groups<T>(x, q, scale, n_groups, (int)blockIdx.x - 1, (int)gridDim.x - 1);
 }
 
@@ -410,6 +434,7 @@ __global__ __launch_bounds__(256) void prepare_hist_kernel(const int32_t *__rest
 // 17 - 42 us), scans the padded totals and places its segment, each of its n_waves wavefronts a part of it.
 // 1024 threads: four times as many as 256 took a quarter of the rounds of dependent round trips (18 432 slots 13 -> 10 us, before
 // the rounds themselves were shortened).
+template <bool FEW>
 __global__ __launch_bounds__(1024) void align_place_kernel(const int32_t *__restrict__ ids, int numel, int E, int id_bits,
                                                            int block_size, const int *__restrict__ hist, int words,
                                                            int32_t *sorted_ids, int32_t *expert_ids, int n_blocks,
@@ -465,7 +490,7 @@ __global__ __launch_bounds__(1024) void align_place_kernel(const int32_t *__rest
         add_up(std::integral_constant<int, 4>());
     else
         add_up(std::integral_constant<int, 12>());
-    count_run(ids, lo, hi, E, id_bits, masks, cursors, wave, n_waves, c);
+    count_run<FEW>(ids, lo, hi, E, id_bits, masks, cursors, wave, n_waves, c);
     lds_barrier();
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
         prefix_over_waves(cursors, e, n_waves);
@@ -473,7 +498,7 @@ __global__ __launch_bounds__(1024) void align_place_kernel(const int32_t *__rest
     }
     lds_barrier();
     const int total = block_exclusive_scan(start, E, wave_sums);
-    place_run(ids, lo, hi, E, id_bits, masks, [&](int e) { return start[e] + before[e]; }, cursors, wave, n_waves, c, sorted_ids);
+    place_run<FEW>(ids, lo, hi, E, id_bits, masks, [&](int e) { return start[e] + before[e]; }, cursors, wave, n_waves, c, sorted_ids);
     write_blocks(start, E, block_size, total, expert_ids, n_blocks, ntpp, seg * blockDim.x + threadIdx.x, n_seg * blockDim.x);
 }
 
@@ -499,6 +524,14 @@ unsigned quant_grid(const Quant &z, int threads)
     const long long per = threads / 16, want = ((long long)z.M * (z.K / 128) + per - 1) / per, most = 8192 * 256 / threads;
     return (unsigned)(want < most ? want : most);
 }
+
+// Where same_expert() has to expect one expert on many lanes of a chunk.  MI355X, us in a graph of such calls, without / with
+// FEW, and in brackets without the table of lane masks (a ballot per bit for any number of experts): 4096 slots of 1 expert
+// 7.9 / 4.8 (6.2), of 2 evenly 6.7 / 5.1 (6.5), of 8 5.9 / 5.9 (7.4), all of 16 on one 8.2 / 5.6 (7.6), of 64 8.3 / 5.6 (8.5);
+// 4 Mi slots of 1 expert 57 / 39 (41), all of 64 on one 53 / 40 (46), half 44 / 41 (44), evenly 43 / 43 (45), all of 128 on one
+// 53 / 43 (50); from there on the table alone is ahead of ballots on any input (257 experts, all on one 57 / 54 (61)), and
+// below 1024 slots as well (300 of 1 expert 3.6 / 3.5 (4.3), 30 of 16 3.6 / 3.8 (4.6)).
+bool few_experts(int numel, int id_bits) { return id_bits <= 7 && numel >= 1024; }
 
 int align(const int32_t *topk_ids, int numel, int num_experts, int block_size, int32_t *sorted_token_ids, int sorted_num,
           int32_t *expert_ids, int n_blocks, int32_t *num_tokens_post_padded, void *workspace, size_t workspace_bytes,
@@ -526,14 +559,21 @@ int align(const int32_t *topk_ids, int numel, int num_experts, int block_size, i
         const size_t lds = lds_of(n_waves);
         const AlignSmall a = {topk_ids, numel, E, id_bits, block_size, sorted_token_ids, sorted_num, expert_ids, n_blocks,
                               num_tokens_post_padded, n_waves, run};
-        if (!z.x)
-            hipLaunchKernelGGL(align_small_kernel, dim3(1), dim3(1024), lds, hs, a);
-        else if (z.is_f32)
-            hipLaunchKernelGGL(prepare_small_kernel<float>, dim3(1 + quant_grid(z, 1024)), dim3(1024), lds, hs, a,
-                               static_cast<const float *>(z.x), z.q, z.scale, n_groups);
+        auto launch = [&](auto few) {
+            constexpr bool FEW = decltype(few)::value;
+            if (!z.x)
+                hipLaunchKernelGGL(align_small_kernel<FEW>, dim3(1), dim3(1024), lds, hs, a);
+            else if (z.is_f32)
+                hipLaunchKernelGGL((prepare_small_kernel<float, FEW>), dim3(1 + quant_grid(z, 1024)), dim3(1024), lds, hs, a,
+                                   static_cast<const float *>(z.x), z.q, z.scale, n_groups);
+            else
+                hipLaunchKernelGGL((prepare_small_kernel<uint16_t, FEW>), dim3(1 + quant_grid(z, 1024)), dim3(1024), lds, hs, a,
+                                   static_cast<const uint16_t *>(z.x), z.q, z.scale, n_groups);
+        };
+        if (few_experts(numel, id_bits))
+            launch(std::true_type());
         else
-            hipLaunchKernelGGL(prepare_small_kernel<uint16_t>, dim3(1 + quant_grid(z, 1024)), dim3(1024), lds, hs, a,
-                               static_cast<const uint16_t *>(z.x), z.q, z.scale, n_groups);
+            launch(std::false_type());
         return hipGetLastError() == hipSuccess ? ALPHA_MOE_OK : ALPHA_MOE_ERR_LAUNCH;
     }
     if (!workspace || workspace_bytes < alpha_moe_align_workspace_bytes(numel, E)) return ALPHA_MOE_ERR_WORKSPACE;
@@ -559,7 +599,8 @@ int align(const int32_t *topk_ids, int numel, int num_experts, int block_size, i
     };
     while (lds_of(n_waves) > (64 << 10)) n_waves /= 2;
     const size_t lds = lds_of(n_waves);
-    hipLaunchKernelGGL(align_place_kernel, dim3(n_seg), dim3(1024), lds, hs, topk_ids, numel, E, id_bits, block_size, hist,
+    const auto place = few_experts(numel, id_bits) ? align_place_kernel<true> : align_place_kernel<false>;
+    hipLaunchKernelGGL(place, dim3(n_seg), dim3(1024), lds, hs, topk_ids, numel, E, id_bits, block_size, hist,
                        words, sorted_token_ids, expert_ids, n_blocks, num_tokens_post_padded, n_waves, seg);
     return hipGetLastError() == hipSuccess ? ALPHA_MOE_OK : ALPHA_MOE_ERR_LAUNCH;
 }

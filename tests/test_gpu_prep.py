@@ -103,6 +103,35 @@ def test_align_where_tables_and_cursors_fill_the_memory(E, numel):
         assert torch.equal(a.cpu(), b)
 
 
+@pytest.mark.parametrize("kind", ["even", "one", "half", "none"])
+@pytest.mark.parametrize("numel", [1023, 1024, 4159])
+@pytest.mark.parametrize("E", [1, 8, 9, 128, 129])
+def test_align_of_few_experts(E, numel, kind):
+    """1024 slots and more of up to 128 experts are ranked without the lane masks (up to 8 experts), or with them behind the
+    first lane's expert; all slots on one expert, half of them, none valid, first lanes without an expert among them"""
+    from alpha_moe_python import prep_hip
+    g = torch.Generator().manual_seed(E * 7 + numel)
+    ids = torch.randint(-1, E + 1, (numel, 1), generator=g, dtype=torch.int32)
+    if kind == "one":
+        ids[:] = E - 1
+    elif kind == "half":
+        ids[torch.rand(numel, generator=g) < 0.5] = E // 2
+    elif kind == "none":
+        ids[:] = torch.where(torch.rand((numel, 1), generator=g) < 0.5, -1, E).to(torch.int32)
+    print(f"case align numel={numel} E={E} {kind}", flush=True)
+    got = prep_hip.moe_align_block_size(ids.to(DEV), 16, E)
+    flat = ids.flatten()
+    want, experts = [], []
+    for e in range(E):
+        slots = torch.nonzero(flat == e).flatten().tolist()
+        slots += [numel] * (-len(slots) % 16)
+        want += slots
+        experts += [e] * (len(slots) // 16)
+    assert got[2].item() == len(want)
+    assert got[0].tolist() == want + [numel] * (got[0].numel() - len(want))
+    assert got[1].tolist() == experts + [-1] * (got[1].numel() - len(experts))
+
+
 @pytest.mark.parametrize("M,K,top_k,E,block,dtype", [
     (1, 128, 1, 3, 16, torch.bfloat16),        # one group, one slot
     (7, 7168, 9, 257, 8, torch.bfloat16),
