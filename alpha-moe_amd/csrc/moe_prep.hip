@@ -430,8 +430,8 @@ __global__ __launch_bounds__(256) void prepare_hist_kernel(const int32_t *__rest
 }
 
 // Pass 2, one workgroup per segment: every workgroup adds the histograms up itself (columns of two experts, the segments
-// split over the threads that share a column, a thread's share in flight at once as far as twelve go; a third launch of one workgroup for the sums took
-// 17 - 42 us), scans the padded totals and places its segment, each of its n_waves wavefronts a part of it.
+// split over the threads that share a column, up to eight of a thread's in flight; a third launch of one workgroup for the sums
+// took 17 - 42 us), scans the padded totals and places its segment, each of its n_waves wavefronts a part of it.
 // 1024 threads: four times as many as 256 took a quarter of the rounds of dependent round trips (18 432 slots 13 -> 10 us, before
 // the rounds themselves were shortened).
 template <bool FEW>
@@ -458,17 +458,21 @@ __global__ __launch_bounds__(1024) void align_place_kernel(const int32_t *__rest
     lds_barrier();
     const int share = words < (int)blockDim.x ? blockDim.x / words : 1;   // threads of a column
     const int part = words < (int)blockDim.x ? threadIdx.x / words : 0;
-    auto add_up = [&](auto in_flight) {
-        constexpr int U = decltype(in_flight)::value;
+    // U segments in flight as long as there are as many, then R, of which those past the end are loaded twice and count nothing
+    auto add_up = [&](auto in_flight, auto rest) {
+        constexpr int U = decltype(in_flight)::value, R = decltype(rest)::value;
         for (int col = (int)threadIdx.x - part * words; col < words && part < share; col += blockDim.x) {
-            int b0 = 0, b1 = 0, t0 = 0, t1 = 0;
-            for (int s0 = part; s0 < n_seg; s0 += U * share) {
-                unsigned v[U];
+            int b0 = 0, b1 = 0, t0 = 0, t1 = 0, s0 = part;
+            auto take = [&](auto in_flight, auto all_there) {
+                constexpr int N = decltype(in_flight)::value;
+                constexpr bool ALL = decltype(all_there)::value;
+                unsigned v[N];
 #pragma unroll
-                for (int k = 0; k < U; k++) v[k] = (unsigned)hist[(size_t)min(s0 + k * share, n_seg - 1) * words + col];
+                for (int k = 0; k < N; k++)
+                    v[k] = (unsigned)hist[(size_t)(ALL ? s0 + k * share : min(s0 + k * share, n_seg - 1)) * words + col];
 #pragma unroll
-                for (int k = 0; k < U; k++) {
-                    const unsigned w = s0 + k * share < n_seg ? v[k] : 0u;
+                for (int k = 0; k < N; k++) {
+                    const unsigned w = ALL || s0 + k * share < n_seg ? v[k] : 0u;
                     const int c0 = w & 0xffffu, c1 = w >> 16;
                     t0 += c0;
                     t1 += c1;
@@ -477,19 +481,34 @@ __global__ __launch_bounds__(1024) void align_place_kernel(const int32_t *__rest
                         b1 += c1;
                     }
                 }
-            }
+                s0 += N * share;
+            };
+            if constexpr (U > R)
+                while (s0 + (U - 1) * share < n_seg) take(in_flight, std::true_type());
+            while (s0 < n_seg) take(rest, std::false_type());
             atomicAdd(&start[2 * col], t0);
             atomicAdd(&start[2 * col + 1], t1);
             atomicAdd(&before[2 * col], b0);
             atomicAdd(&before[2 * col + 1], b1);
         }
     };
+    // One round where eight segments a thread will do, with no more loads than there are segments to the next power of two; more
+    // rounds are bound by their loads, so none is made in vain before the last four.  More than eight in flight take the registers
+    // of a second workgroup per compute unit, which is what inputs of more than 256 segments run.  MI355X, us in a graph of such
+    // calls, twelve at a time with those past the end loaded twice / as it is: 40 960 slots, 512 experts (10 segments a thread)
+    // 9.6 / 9.4; 300 000 slots, 257 experts (42) 21.9 / 19.5, 1024 (147) 43.5 / 36.1, 4096 (293) 132 / 106; 2 Mi slots, 4096 experts
+    // (512) 248 / 208.  Sixteen and four took as long, twelve and four 0 - 10 % longer.
+    const std::integral_constant<int, 2> two;
+    const std::integral_constant<int, 4> four;
+    const std::integral_constant<int, 8> eight;
     if (n_seg <= 2 * share)
-        add_up(std::integral_constant<int, 2>());
+        add_up(two, two);
     else if (n_seg <= 4 * share)
-        add_up(std::integral_constant<int, 4>());
+        add_up(four, four);
+    else if (n_seg <= 8 * share)
+        add_up(eight, eight);
     else
-        add_up(std::integral_constant<int, 12>());
+        add_up(eight, four);
     count_run<FEW>(ids, lo, hi, E, id_bits, masks, cursors, wave, n_waves, c);
     lds_barrier();
     for (int e = threadIdx.x; e < E; e += blockDim.x) {

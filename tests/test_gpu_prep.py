@@ -103,6 +103,24 @@ def test_align_where_tables_and_cursors_fill_the_memory(E, numel):
         assert torch.equal(a.cpu(), b)
 
 
+@pytest.mark.parametrize("E", [1100, 2100])
+@pytest.mark.parametrize("segments", [5, 8, 9, 11, 12, 13, 16, 17, 20])
+def test_align_adds_up_the_segments_of_a_thread(segments, E):
+    """one thread per column (two columns a thread from 2049 experts on): up to eight segments in one round, then rounds of eight
+    and of four, the last one part-filled"""
+    from alpha_moe_python import prep_hip
+    g = torch.Generator().manual_seed(E + segments)
+    ids = torch.randint(-1, E + 1, (1024 * segments - 7, 1), generator=g, dtype=torch.int32)
+    print(f"case align segments={segments} E={E}", flush=True)
+    got = prep_hip.moe_align_block_size(ids.to(DEV), 8, E)
+    ids[(ids < 0) | (ids >= E)] = E   # (an expert of its own behind the last, cut off below)
+    s_ids, e_ids, total = O.align_reference(ids, 8, E + 1)
+    n = total.item() - -(-int((ids == E).sum()) // 8) * 8
+    assert got[2].item() == n
+    assert got[0][:n].tolist() == s_ids[:n].tolist() and bool((got[0][n:] == ids.numel()).all())
+    assert got[1][:n // 8].tolist() == e_ids[:n // 8].tolist() and bool((got[1][n // 8:] == -1).all())
+
+
 @pytest.mark.parametrize("kind", ["even", "one", "half", "none"])
 @pytest.mark.parametrize("numel", [1023, 1024, 4159])
 @pytest.mark.parametrize("E", [1, 8, 9, 128, 129])
