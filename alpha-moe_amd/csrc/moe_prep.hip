@@ -9,6 +9,7 @@
 //     equal to numel, one expert id per block (-1 past the padded total), and the padded total.
 //
 // Both are HBM-bound integer/byte passes: 16-byte loads, no matrix instructions.
+#include <mutex>
 #include <type_traits>
 
 #include "moe_common.hpp"
@@ -521,6 +522,24 @@ __global__ __launch_bounds__(1024) void align_place_kernel(const int32_t *__rest
     write_blocks(start, E, block_size, total, expert_ids, n_blocks, ntpp, seg * blockDim.x + threadIdx.x, n_seg * blockDim.x);
 }
 
+constexpr size_t kDefaultLds = 64 << 10;   // dynamic LDS a kernel may have without a word
+
+// The placement kernel's limit is raised once per device, not on every launch.
+hipError_t allow_place_lds()
+{
+    static std::mutex mu;
+    static bool done[64];
+    int dev = 0;
+    hipError_t err = hipGetDevice(&dev);
+    if (err != hipSuccess) return err;
+    std::lock_guard<std::mutex> lock(mu);
+    if (dev >= 0 && dev < 64 && done[dev]) return hipSuccess;
+    err = hipFuncSetAttribute(reinterpret_cast<const void *>(align_place_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              80 << 10);
+    if (err == hipSuccess && dev >= 0 && dev < 64) done[dev] = true;
+    return err;
+}
+
 // What is quantised beside an alignment (x == nullptr: nothing).
 struct Quant {
     const void *x;
@@ -573,7 +592,7 @@ int align(const int32_t *topk_ids, int numel, int num_experts, int block_size, i
         auto lds_of = [&](int waves) {
             return waves * kMasks * sizeof(lanes_t) + cursor_bytes(waves, E) + (16 + E) * sizeof(int);
         };
-        while (lds_of(n_waves) > (64 << 10)) n_waves /= 2;
+        while (lds_of(n_waves) > kDefaultLds) n_waves /= 2;
         const int run = ((numel + n_waves - 1) / n_waves + 63) / 64 * 64;
         const size_t lds = lds_of(n_waves);
         const AlignSmall a = {topk_ids, numel, E, id_bits, block_size, sorted_token_ids, sorted_num, expert_ids, n_blocks,
@@ -611,13 +630,17 @@ int align(const int32_t *topk_ids, int numel, int num_experts, int block_size, i
         hipLaunchKernelGGL(prepare_hist_kernel<uint16_t>, dim3(n_seg + quant_grid(z, 256)), dim3(256), words * sizeof(int),
                            hs, topk_ids, numel, E, hist, words, sorted_token_ids, sorted_num, n_seg, seg,
                            static_cast<const uint16_t *>(z.x), z.q, z.scale, n_groups);
-    // as many wavefronts, sixteen at most, as have room for their tables and cursors in 64 KiB of LDS (at kAlignMaxExperts two)
+    // as many wavefronts, sixteen at most, as have room for their tables and cursors in 64 KiB of LDS, but at least four (up to
+    // 72.1 KiB, from 3581 experts on; two workgroups per compute unit all the same): a segment is placed chunk by chunk, and two
+    // wavefronts take twice the chunks each.  MI355X, us in a graph of such calls, two / four wavefronts, 4096 experts: 8192 slots
+    // 15.1 / 11.8, 73 728 25.6 / 23.6, 600 000 119.5 / 115.4, 2 Mi 208 / 197.
     int n_waves = 16;
     auto lds_of = [&](int waves) {
         return waves * kMasks * sizeof(lanes_t) + cursor_bytes(waves, E) + (4 * words + 16) * sizeof(int);
     };
-    while (lds_of(n_waves) > (64 << 10)) n_waves /= 2;
+    while (n_waves > 4 && lds_of(n_waves) > kDefaultLds) n_waves /= 2;
     const size_t lds = lds_of(n_waves);
+    if (lds > kDefaultLds && allow_place_lds() != hipSuccess) return ALPHA_MOE_ERR_LAUNCH;
     const auto place = few_experts(numel, id_bits) ? align_place_kernel<true> : align_place_kernel<false>;
     hipLaunchKernelGGL(place, dim3(n_seg), dim3(1024), lds, hs, topk_ids, numel, E, id_bits, block_size, hist,
                        words, sorted_token_ids, expert_ids, n_blocks, num_tokens_post_padded, n_waves, seg);

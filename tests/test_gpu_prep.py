@@ -92,7 +92,8 @@ def test_align_where_the_wavefronts_of_a_segment_change(E):
 @pytest.mark.parametrize("numel", [4096, 4500, 70000])
 @pytest.mark.parametrize("E", [256, 817, 818, 2045, 2046, 3580, 3581])
 def test_align_where_tables_and_cursors_fill_the_memory(E, numel):
-    """16, 8, 4 and 2 wavefronts place a segment, the last with more slots each than they keep in registers"""
+    """16, 8 and 4 wavefronts place a segment, the last with more slots each than they keep in registers; 3581 experts and more of
+    them have more than 64 KiB of tables and cursors"""
     from alpha_moe_python import prep_hip
     g = torch.Generator().manual_seed(E)
     ids = torch.randint(-1, E, (numel, 1), generator=g, dtype=torch.int32)
