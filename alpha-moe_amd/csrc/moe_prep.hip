@@ -23,7 +23,7 @@ constexpr int kAlignMaxSeg = 512;      // most segments before they get longer: 
                                        // 600 000 slots, 257 experts: 42 us in 586, 26 in 293)
 // Most routing slots one workgroup aligns by itself.  MI355X, one workgroup / two launches, 128 - 512 experts: 3072 slots
 // 5.8 - 6.9 / 7.1 - 7.9 us, 4096 6.8 - 7.8 / 7.0 - 8.0, 5120 8.4 - 9.8 / 7.1 - 8.0.
-constexpr int kAlignSmall = 4096;
+constexpr int kAlignSmall = ALPHA_MOE_ALIGN_SLOTS_WITHOUT_WORKSPACE;
 constexpr int kAlignMaxExperts = 4096;
 
 // ---- quantisation ------------------------------------------------------------------------------------------

@@ -293,9 +293,9 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> moe_align_block_size(const at::Te
     const at::Device dev = topk_ids.device();
     at::Tensor sorted_ids = empty_on(dev, {sorted_num}, at::kInt), expert_ids = empty_on(dev, {n_blocks}, at::kInt),
                total = empty_on(dev, {1}, at::kInt);
-    size_t ws_bytes = 0;   // (up to 4096 slots need none)
+    size_t ws_bytes = 0;
     at::Tensor ws;
-    if (numel > 4096) {
+    if (numel > ALPHA_MOE_ALIGN_SLOTS_WITHOUT_WORKSPACE) {
         ws_bytes = alpha_moe_align_workspace_bytes(static_cast<int>(numel), static_cast<int>(num_experts));
         ws = empty_on(dev, {static_cast<int64_t>(ws_bytes)}, at::kByte);
     }
@@ -331,9 +331,9 @@ prepare_inputs(const at::Tensor &x, const at::Tensor &topk_ids, int64_t group_si
     const at::Device dev = topk_ids.device();
     at::Tensor sorted_ids = empty_on(dev, {sorted_num}, at::kInt), expert_ids = empty_on(dev, {n_blocks}, at::kInt),
                total = empty_on(dev, {1}, at::kInt);
-    size_t ws_bytes = 0;   // (up to 4096 slots need none)
+    size_t ws_bytes = 0;
     at::Tensor ws;
-    if (numel > 4096) {
+    if (numel > ALPHA_MOE_ALIGN_SLOTS_WITHOUT_WORKSPACE) {
         ws_bytes = alpha_moe_align_workspace_bytes(static_cast<int>(numel), static_cast<int>(num_experts));
         ws = empty_on(dev, {static_cast<int64_t>(ws_bytes)}, at::kByte);
     }

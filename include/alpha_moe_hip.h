@@ -196,9 +196,11 @@ int alpha_moe_per_token_group_quant_fp8(const void *x, int x_is_f32, uint8_t *q,
  *   expert_ids [n_blocks = ceil(sorted_num / block_size)]: the expert of each block, -1 past the padded total;
  *   num_tokens_post_padded [1]: the padded total
  * as the fused kernel reads them (fused_moe_w8a8_up_down_acc.cu:676-679,756-758).  Slots whose expert is outside
- * [0, num_experts) are dropped.  num_experts <= 4096.  Inputs of more than 4096 slots need a scratch buffer of
- * alpha_moe_align_workspace_bytes(numel, num_experts) bytes (any contents); smaller ones accept workspace == NULL.
+ * [0, num_experts) are dropped.  num_experts <= 4096.  Inputs of more than ALPHA_MOE_ALIGN_SLOTS_WITHOUT_WORKSPACE slots
+ * need a scratch buffer of alpha_moe_align_workspace_bytes(numel, num_experts) bytes (any contents); smaller ones accept
+ * workspace == NULL.
  */
+#define ALPHA_MOE_ALIGN_SLOTS_WITHOUT_WORKSPACE 4096
 size_t alpha_moe_align_workspace_bytes(int numel, int num_experts);
 int alpha_moe_moe_align_block_size(const int32_t *topk_ids, int numel, int num_experts, int block_size,
                                    int32_t *sorted_token_ids, int sorted_num, int32_t *expert_ids, int n_blocks,
