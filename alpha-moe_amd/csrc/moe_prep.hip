@@ -19,10 +19,10 @@ namespace {
 
 constexpr int kAlignSeg = 1024;        // routing slots per workgroup (segment) of the histogram and placement kernels, and
 constexpr int kAlignMaxSeg = 512;      // most segments before they get longer: every workgroup reads all segments' histograms
-                                       // (4 Mi slots, 4096 experts: 10.2 ms in 4096 segments, 272 us in 512;
-                                       // 600 000 slots, 257 experts: 42 us in 586, 26 in 293)
+                                       // (4 Mi slots, 4096 experts: 9.2 ms in 4096 segments, 225 us in 512;
+                                       // 600 000 slots, 257 experts: 35 us in 586, 23 in 293)
 // Most routing slots one workgroup aligns by itself.  MI355X, one workgroup / two launches, 128 - 512 experts: 3072 slots
-// 5.8 - 6.9 / 7.1 - 7.9 us, 4096 6.8 - 7.8 / 7.0 - 8.0, 5120 8.4 - 9.8 / 7.1 - 8.0.
+// 6.2 - 6.7 / 7.2 - 7.8 us, 4096 7.1 - 7.8 / 7.4 - 7.8, 5120 8.7 - 9.7 / 7.5 - 8.1.
 constexpr int kAlignSmall = ALPHA_MOE_ALIGN_SLOTS_WITHOUT_WORKSPACE;
 constexpr int kAlignMaxExperts = 4096;
 
@@ -93,8 +93,8 @@ __global__ __launch_bounds__(256) void quant_group128_kernel(const T *__restrict
 // (same_expert; a ballot per bit of the expert id was 72 instructions a chunk), keeps its slots in registers between counting and
 // placing, and counts and places a run of slots of its own behind cursors of its own.  MI355X, us in a graph of such calls,
 // before (ballots, slots read twice, prefix sums by LDS shuffles, divisions by the block size) / now: 9 slots of 257 experts
-// 5.2 / 3.9, 2997 slots 9.2 / 6.3, 4000 slots of 512 experts 11.3 / 7.9; in two launches 18 432 slots 10.6 / 7.9, 73 728 slots
-// 10.9 / 9.0, 8192 slots of 128 experts 9.1 / 6.9.
+// 5.4 / 4.1, 2997 slots 9.1 / 6.4, 4000 slots of 512 experts 11.1 / 7.8; in two launches 18 432 slots 11.1 / 8.4, 73 728 slots
+// 11.5 / 9.3, 600 000 slots 27.3 / 22.9, 8192 slots of 128 experts 9.7 / 7.5, 4 Mi slots of 4096 experts 273 / 225.
 typedef unsigned long long lanes_t;
 constexpr int kMasks = 256;   // entries of a wavefront's table of lane masks: the experts' low eight bits
 
