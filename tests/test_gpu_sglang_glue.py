@@ -76,11 +76,13 @@ def test_fused_experts_matches_the_oracle_on_the_checkpoint_tensors(M, tmp_path)
     (4, 5, 2176, 128, 40, 24), (5, 8, 4096, 384, 64, 32), (7, 9, 4224, 256, 257, 16),
     (8, 20, 2560, 128, 64, 8), (8, 8, 640, 256, 31, 64),
     (9, 4, 1152, 256, 33, 16), (16, 10, 3072, 128, 512, 8),         # the second eight tokens; the most tokens and rows
+    (12, 9, 7168, 256, 257, 16), (13, 8, 4224, 256, 64, 16), (16, 9, 7168, 256, 257, 16),   # ... with the widest K of a wavefront
     (17, 4, 1152, 256, 33, 16)])                                    # one token too many; blocks of 64: the three steps as well
 def test_layer_call_equals_its_three_steps_bit_for_bit(M, top_k, K, I, E, block_m):
     """The smallest batches are quantised and aligned inside the operator's first launch; quantiser, aligner and storing
     operator called one by one are the general path.  Rows with an expert twice, slots without an expert, an infinity, a
-    NaN and an all-zero group among them; int64 routing, a base that is not 16-byte aligned, replays of a graph."""
+    NaN and an all-zero group among them; a base that is not 16-byte aligned, replays of a graph; the C entry, which takes
+    every supported size, also where the binding calls the three steps because they are faster."""
     import alpha_moe
     from alpha_moe_python import prep_hip
     g = torch.Generator().manual_seed(M * 131 + K)
@@ -101,6 +103,7 @@ def test_layer_call_equals_its_three_steps_bit_for_bit(M, top_k, K, I, E, block_
             x[M - 1, K - 1], x[M // 2, K // 2] = float("inf"), float("nan")
             x[0, 0] = torch.finfo(torch.bfloat16).max
         x, ids, weights = x.to(DEV), ids.to(DEV), torch.rand((M, top_k), generator=g).to(DEV)
+        ids_were, weights_were = ids.clone(), weights.clone()
         print(f"case layer call M={M} top_k={top_k} K={K} I={I} E={E} block_m={block_m} {kind}", flush=True)
         q, q_s, *routing = prep_hip.prepare_inputs(x, ids, 128, block_m, E)
         want = torch.empty_like(x)
@@ -121,6 +124,16 @@ def test_layer_call_equals_its_three_steps_bit_for_bit(M, top_k, K, I, E, block_
         odd.copy_(x)
         call(odd)
         same(odd, want)
+        if taken:
+            sizes = (top_k, M, K, 2 * I, E)
+            ws = torch.zeros(alpha_moe.c_abi.alpha_moe_workspace_bytes(*sizes, M * top_k + E * (block_m - 1), block_m),
+                             dtype=torch.uint8, device=DEV)
+            out = torch.empty_like(x)
+            assert alpha_moe.c_abi.alpha_moe_layer_call(
+                x.data_ptr(), ids.data_ptr(), w13.data_ptr(), w13_s.data_ptr(), w2.data_ptr(), w2_s.data_ptr(),
+                weights.data_ptr(), out.data_ptr(), *sizes, block_m, 32, 8, 4, 2.5, ws.data_ptr(), ws.numel(),
+                torch.cuda.current_stream().cuda_stream) == 0
+            same(out, want)
         graph, stream = torch.cuda.CUDAGraph(), torch.cuda.Stream()
         with torch.cuda.stream(stream):
             call(h)   # scratch memory is per stream and is not allocated under capture
@@ -131,7 +144,7 @@ def test_layer_call_equals_its_three_steps_bit_for_bit(M, top_k, K, I, E, block_
             h.copy_(x)
             graph.replay()
             same(h, want)
-            assert not torch.zeros(4, device=DEV).any()
+        assert torch.equal(ids, ids_were) and torch.equal(weights, weights_were)   # nothing but hidden_states is written
 
 
 @pytest.mark.parametrize("M", [3, 40])
