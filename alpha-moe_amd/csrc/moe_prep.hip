@@ -494,11 +494,11 @@ __global__ __launch_bounds__(1024) void align_place_kernel(const int32_t *__rest
         }
     };
     // One round where eight segments a thread will do, with no more loads than there are segments to the next power of two; more
-    // rounds are bound by their loads, so none is made in vain before the last four.  More than eight in flight take the registers
-    // of a second workgroup per compute unit, which is what inputs of more than 256 segments run.  MI355X, us in a graph of such
-    // calls, twelve at a time with those past the end loaded twice / as it is: 40 960 slots, 512 experts (10 segments a thread)
-    // 9.6 / 9.4; 300 000 slots, 257 experts (42) 21.9 / 19.5, 1024 (147) 43.5 / 36.1, 4096 (293) 132 / 106; 2 Mi slots, 4096 experts
-    // (512) 248 / 208.  Sixteen and four took as long, twelve and four 0 - 10 % longer.
+    // rounds are bound by their loads, so none is made in vain before the last four.  Twelve at a time, those past the end loaded
+    // twice, also took 70 registers, which leave no room for a second workgroup per compute unit; inputs of more than 256 segments
+    // run two.  MI355X, us in a graph of such calls, so / as it is: 40 960 slots, 512 experts (10 segments a thread) 9.6 / 9.4;
+    // 300 000 slots, 257 experts (42) 21.9 / 19.5, 1024 (147) 43.5 / 36.1, 4096 (293) 132 / 106; 2 Mi slots, 4096 experts (512)
+    // 248 / 208.  Sixteen and then four took as long, twelve and then four 0 - 15 % longer.
     const std::integral_constant<int, 2> two;
     const std::integral_constant<int, 4> four;
     const std::integral_constant<int, 8> eight;
@@ -518,7 +518,8 @@ __global__ __launch_bounds__(1024) void align_place_kernel(const int32_t *__rest
     }
     lds_barrier();
     const int total = block_exclusive_scan(start, E, wave_sums);
-    place_run<FEW>(ids, lo, hi, E, id_bits, masks, [&](int e) { return start[e] + before[e]; }, cursors, wave, n_waves, c, sorted_ids);
+    place_run<FEW>(ids, lo, hi, E, id_bits, masks, [&](int e) { return start[e] + before[e]; }, cursors, wave, n_waves, c,
+                   sorted_ids);
     write_blocks(start, E, block_size, total, expert_ids, n_blocks, ntpp, seg * blockDim.x + threadIdx.x, n_seg * blockDim.x);
 }
 

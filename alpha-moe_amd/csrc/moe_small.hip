@@ -878,11 +878,12 @@ bool layer_supported(int E) { return E <= kLayerExperts; }
 //   4 x 4                 K = 4096, 16 tokens: I = 256, top 8 58.5 / 57.6; I = 128, top 1 17.5 / 18.5
 //   3 x 7                 DeepSeek shard, 12 tokens 88.7 / 89.3; K = 7168, I = 256, top 2, 9 tokens 29.3 / 30.1; K = 4224, I = 256,
 //                         top 2, 12 tokens 27.8 / 30.3, I = 128, top 1, 9 tokens 17.0 / 20.5
-//   4 x 7                 DeepSeek shard, 16 tokens 107.2 / 107.8; K = 6144, I = 256, top 8 75.8 / 78.7; I = 128, top 1 22.8 / 27.5
+//   4 x 7                 DeepSeek shard, 16 tokens 107.2 / 107.8; K = 6144, I = 256, top 8 75.8 / 78.7; K = 7168, I = 128, top 1
+//                         22.8 / 27.5
 // Outside a graph the third launch and the five tensors of the preparation cost a caller that waits for each call 1 - 2 us more:
-// at 3 x 7 DeepSeek shard, 12 tokens 108.2 / 106.3, K = 7168, I = 256, top 2, 9 tokens 46.0 / 44.3 (99 MB of weights), but K = 4224,
-// I = 256, top 2, 12 tokens 45.2 / 45.2 (78 MB), I = 128, top 1, 9 tokens 34.7 / 36.0; at 4 x 7 DeepSeek shard 128.3 / 127.7, K = 5120,
-// I = 256, top 8 87.5 / 88.4.
+// at 3 x 7 DeepSeek shard, 12 tokens 108.2 / 106.3, K = 7168, I = 256, top 2, 9 tokens 46.0 / 44.3 (99 MB of weights), but
+// K = 4224, I = 256, top 2, 12 tokens 45.2 / 45.2 (78 MB), I = 128, top 1, 9 tokens 34.7 / 36.0; at 4 x 7 DeepSeek shard
+// 128.3 / 127.7, K = 5120, I = 256, top 8 87.5 / 88.4.
 bool layer_pays(int top_k, int M, int K, int N, int E)
 {
     const int steps = (M + 3) / 4 * blocks_per_wave(K);
