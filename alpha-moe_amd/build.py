@@ -26,15 +26,15 @@ HIPCC = os.path.join(ROCM, "bin", "hipcc")
 # packed-fp32 VALU forms are switched off for every kernel in this library
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
              "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument"]
-# Per-source extras.  The tile kernel scales every matrix-instruction result into vector-register accumulators, so
+# Per-source extras.  The group kernel scales every matrix-instruction result into vector-register accumulators, so
 # the results must land in vector registers, not in accumulation registers that only a copy can read.
 HIP_SOURCES = {
     "moe_api.hip": [],
     "moe_direct.hip": [],
     "moe_small.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
     "moe_stream.hip": [],
-    "moe_tile.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
-    "moe_wide.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "moe_group.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "moe_reduce.hip": [],
     "moe_prep.hip": [],
 }
 

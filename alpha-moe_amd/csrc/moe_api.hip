@@ -21,7 +21,7 @@ TunableSlot g_tunables[kTunCount] = {
     {"ALPHA_MOE_LAG", kTunableUnset},         {"ALPHA_MOE_GRID", kTunableUnset},
     {"ALPHA_MOE_TILE_GPS", kTunableUnset},    {"ALPHA_MOE_TILE_LAG", kTunableUnset},
     {"ALPHA_MOE_TILE_GRID", kTunableUnset},   {"ALPHA_MOE_TILE_NT", kTunableUnset},
-    {"ALPHA_MOE_WIDE_PP", kTunableUnset},
+    {"ALPHA_MOE_WIDE_PP", kTunableUnset},     {"ALPHA_MOE_GROUP_PIECES", kTunableUnset},
 };
 
 void load_tunables_once()
@@ -31,7 +31,7 @@ void load_tunables_once()
             const char *e = getenv(t.name);
             if (!e) continue;
             if (!strcmp(t.name, "ALPHA_MOE_PATH"))
-                t.value = !strcmp(e, "direct") ? 1 : !strcmp(e, "stream") ? 2 : !strcmp(e, "tile") ? 3 : !strcmp(e, "wide") ? 4 : !strcmp(e, "small") ? 5 : kTunableUnset;
+                t.value = !strcmp(e, "direct") ? 1 : !strcmp(e, "stream") ? 2 : !strcmp(e, "group") ? 3 : !strcmp(e, "small") ? 5 : kTunableUnset;
             else
                 t.value = atoi(e);
         }
@@ -40,26 +40,20 @@ void load_tunables_once()
     (void)done;
 }
 
-enum Path { kDirect, kStream, kTile, kWide, kSmall };
+enum Path { kDirect, kStream, kGroup, kSmall };
 
 // At most 16 tokens: small kernels where they are ahead (small_pays).  Streaming kernel for row blocks of at most 32 rows
-// (decode); above that (prefill) warp_n picks the token tiles a wavefront multiplies per step: 8 -> wide kernel (macro blocks
-// of 256 rows), 4 -> tile kernel (one row block).  The direct kernel is the fallback for shapes none of them takes.
-Path choose_path(int top_k, int M, int K, int N, int E, int sorted_num, int block_m, int warp_n)
+// (decode), group kernel above that (prefill).  The direct kernel is the fallback for shapes none of them takes.
+Path choose_path(int top_k, int M, int K, int N, int E, int sorted_num, int block_m)
 {
     const bool s_ok = stream_supported(top_k, M, K, N, E, sorted_num, block_m);
-    const bool t_ok = tile_supported(top_k, M, K, N, E, sorted_num, block_m);
-    const bool w_ok = wide_supported(top_k, M, K, N, E, sorted_num, block_m);
     const int f = tunable(kTunPath, 0);
     if (f == 1) return kDirect;
     if (f == 2 && s_ok) return kStream;
-    if (f == 3 && t_ok) return kTile;
-    if (f == 4 && w_ok) return kWide;
     const bool small_ok = small_supported(top_k, M, K, N, block_m);
     if (small_ok && (f == 5 || (f == 0 && (!s_ok || small_pays(top_k, M, K, N, E))))) return kSmall;
     if (s_ok) return kStream;
-    if (w_ok && (warp_n == 8 || !t_ok)) return kWide;
-    if (t_ok) return kTile;
+    if (group_supported(top_k, M, K, N, E, sorted_num, block_m)) return kGroup;
     return kDirect;
 }
 
@@ -108,17 +102,13 @@ extern "C" size_t alpha_moe_workspace_bytes(int top_k, int M, int K, int N, int 
     const size_t stream = stream_supported(top_k, M, K, N, num_experts, sorted_num, block_m)
                               ? stream_workspace_bytes(top_k, M, K, N, num_experts, sorted_num, block_m)
                               : 0;
-    const size_t tile = tile_supported(top_k, M, K, N, num_experts, sorted_num, block_m)
-                            ? tile_workspace_bytes(top_k, M, K, N, num_experts, sorted_num, block_m)
-                            : 0;
-    const size_t wide = wide_supported(top_k, M, K, N, num_experts, sorted_num, block_m)
-                            ? wide_workspace_bytes(top_k, M, K, N, num_experts, sorted_num, block_m)
-                            : 0;
+    const size_t group = group_supported(top_k, M, K, N, num_experts, sorted_num, block_m)
+                             ? group_workspace_bytes(top_k, M, K, N, num_experts, sorted_num, block_m)
+                             : 0;
     const size_t small = small_supported(top_k, M, K, N, block_m) ? small_workspace_bytes(top_k, M, N) : 0;
     size_t m = direct > stream ? direct : stream;
     m = m > small ? m : small;
-    m = m > tile ? m : tile;
-    return m > wide ? m : wide;
+    return m > group ? m : group;
 }
 
 namespace {
@@ -156,15 +146,13 @@ int run_fused_moe(const uint8_t *x, const float *x_scale, const uint8_t *w, cons
 
     hipStream_t hs = static_cast<hipStream_t>(stream);
     hipError_t err;
-    const Path path = choose_path(top_k, M, K, N, num_experts, sorted_num, block_m, warp_n);
+    const Path path = choose_path(top_k, M, K, N, num_experts, sorted_num, block_m);
     if (path == kSmall) {
         err = launch_small(p, nullptr, nullptr, workspace, hs);
     } else if (path == kStream) {
         err = launch_stream(p, warp_n, stages, workspace, hs);
-    } else if (path == kWide) {
-        err = launch_wide(p, stages, workspace, hs);
-    } else if (path == kTile) {
-        err = launch_tile(p, stages, workspace, hs);
+    } else if (path == kGroup) {
+        err = launch_group(p, stages, workspace, hs);
     } else {
         // the fallback kernel reads the operator's own layout only
         if (prepacked) return ALPHA_MOE_ERR_SHAPE;
@@ -227,7 +215,7 @@ extern "C" int alpha_moe_layer_call_supported(int top_k, int M, int K, int N, in
     const int64_t sorted_num = (int64_t)M * top_k + (int64_t)num_experts * (block_m - 1);
     if (M <= 0 || top_k <= 0 || num_experts <= 0 || block_m <= 0 || sorted_num > INT32_MAX) return 0;
     if (alpha_moe_validate(top_k, M, K, N, num_experts, (int)sorted_num, block_m, block_n, warp_n, stages) != ALPHA_MOE_OK) return 0;
-    return layer_supported(num_experts) && choose_path(top_k, M, K, N, num_experts, (int)sorted_num, block_m, warp_n) == kSmall;
+    return layer_supported(num_experts) && choose_path(top_k, M, K, N, num_experts, (int)sorted_num, block_m) == kSmall;
 }
 
 extern "C" int alpha_moe_layer_call_pays(int top_k, int M, int K, int N, int num_experts, int block_m, int block_n, int warp_n,

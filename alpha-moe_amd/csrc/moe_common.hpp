@@ -86,13 +86,44 @@ __device__ __forceinline__ uint32_t pack_fp8x4(float a, float b, float c, float 
 }
 
 // SwiGLU on bf16-rounded gate/up, result rounded to bf16 (the reference keeps all three in bf16,
-// fused_moe_w8a8_up_down_acc.cu:76-79,919-946)
+// fused_moe_w8a8_up_down_acc.cu:76-79,919-946).  g / (1 + exp(-g)) as (g / 4) / ((1 + exp(-g)) / 4), whose divisor has a
+// reciprocal that is a normal number wherever the quotient is not 0; one residual correction of the product with it, and the
+// division's own fix-up of limits, infinities and NaN: half of the division's instructions.
 __device__ __forceinline__ float swiglu_bf16(float gate, float up)
 {
     const float g = round_bf16(gate);
     const float u = round_bf16(up);
-    return round_bf16(g / (1.0f + __expf(-g)) * u);
+    const float num = 0.25f * g, den = __builtin_fmaf(__expf(-g), 0.25f, 0.25f);
+    const float r = __builtin_amdgcn_rcpf(den);
+    const float t = num * r;
+    const float silu = __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-t, den, num), r, t), den, num);
+    return round_bf16(silu * u);
 }
+
+// a / s from r ~ 1 / s (one rounding off at most) by one residual correction: three instructions where the division takes
+// ten.  For s = 448 it is the quotient, for every bf16 row maximum; the FP8 codes are those of the exact division (the CPU tests
+// compare both, the codes for all mantissas of row maximum and value at eleven exponents).
+__device__ __forceinline__ float divide(float a, float s, float r)
+{
+    const float t = a * r;
+    return __builtin_fmaf(__builtin_fmaf(-t, s, a), r, t);
+}
+
+// FP8 codes of a 128-column row from its largest magnitude m (at least kAmaxFloor): scale = m / 448, codes of a / scale.
+// A row with an infinity: its scale is infinite, a finite value over it is 0 and an infinity over it NaN; NaN is clamped to -448
+// (as by the division itself).
+struct RowScale {
+    float scale, s, r;
+    __device__ __forceinline__ explicit RowScale(float m)
+    {
+        const bool inf = m == __builtin_inff();
+        scale = inf ? m : divide(m, kFp8Max, 1.0f / kFp8Max);
+        r = __builtin_amdgcn_rcpf(scale);
+        r = inf ? 0.f : __builtin_fmaf(__builtin_fmaf(-scale, r, 1.0f), r, r);
+        s = inf ? 0.f : scale;
+    }
+    __device__ __forceinline__ float code(float a) const { return clamp_fp8(divide(a, s, r)); }
+};
 
 __device__ __forceinline__ void atomic_add_f32(float *addr, float v)
 {
@@ -197,11 +228,8 @@ struct StreamCtl {
     int done;        // streaming kernel: workgroups that have left
     int epoch;       // stamp of the last completed launch on this workspace (any kernel family)
     int pad_e[2];
-    int tile_done;   // tile kernels: workgroups that have left
-    int pad0[2];
-    int tile_head[8];   // tile kernel: next work item of each of the eight queues
-    int pad1a[16];
-    int pad1;
+    int stamp;       // group kernel: the stamp of the launch that is running, until its reduce kernel makes it `epoch`
+    int pad0[27];
     int error;       // sticky: a bounded wait ran out (word kErrorWord of the workspace)
     int pad2[30];
 };
@@ -220,13 +248,11 @@ constexpr size_t kPrefixBytes = kOffLive + sizeof(int) * kMaxSlots;
 // (measured).
 // The stamp of a launch from that of the launch before it on this workspace: the odd numbers in turn, so never 0, which is
 // what a flag or a slot holds that no launch has stamped yet.  Flags and slots are compared for equality: nothing else is
-// up either, however many launches ago it was stamped.  (Without a branch: a comparison and a select here cost the wide
-// kernel's calls 7 - 10 %, again through its registers.)
+// up either, however many launches ago it was stamped.
 __device__ __forceinline__ int next_epoch(int epoch) { return (int)((unsigned)epoch + 2u) | 1; }
 
 // A whole wavefront, consecutive flags, one per lane: every poll is ONE load for up to 64 flags, so the wait costs one round
-// trip however many of them there are.  (The wide kernel's registers depend on those this function uses: handing the flags
-// out 64 at a time around the loop instead cost its calls 3 %.)
+// trip however many of them there are.
 __device__ __noinline__ inline void spin_all_eq(const int *addr, int count, int target, StreamCtl *ctl)
 {
     const int lane = threadIdx.x & 63;
@@ -248,17 +274,18 @@ __device__ __noinline__ inline void spin_all_eq(const int *addr, int count, int 
 // alpha_moe_set_tunable(): no launch ever calls getenv.  A value of kTunableUnset means "the library decides".
 constexpr int kTunableUnset = INT32_MIN;
 enum Tunable {
-    kTunPath,          // ALPHA_MOE_PATH: 1 direct, 2 stream, 3 tile, 4 wide, 5 small (where the family applies)
+    kTunPath,          // ALPHA_MOE_PATH: 1 direct, 2 stream, 3 or 4 group, 5 small (where the family applies)
     kTunStrictQueue,   // ALPHA_MOE_STRICT_QUEUE: 0 hands the first gridDim.x items of the streaming kernel out by index
     kTunKbpi,          // ALPHA_MOE_KBPI: K blocks per UP item of the streaming kernel
     kTunTpi,           // ALPHA_MOE_TPI: 16-column tiles per DOWN item of the streaming kernel
     kTunLag,           // ALPHA_MOE_LAG: row blocks between a block's UP and DOWN items in the streaming queue
     kTunGrid,          // ALPHA_MOE_GRID: workgroups of the streaming kernel
-    kTunTileGps,       // ALPHA_MOE_TILE_GPS: 64-column groups per DOWN item of the tile kernel
-    kTunTileLag,       // ALPHA_MOE_TILE_LAG
-    kTunTileGrid,      // ALPHA_MOE_TILE_GRID
-    kTunTileNt,        // ALPHA_MOE_TILE_NT: non-temporal weight loads 1 always, 0 never
-    kTunWidePp,        // ALPHA_MOE_WIDE_PP: up/gate items of the wide kernel with the wavefronts of a SIMD half a step apart
+    kTunTileGps,       // ALPHA_MOE_TILE_GPS: 64-column groups per DOWN item of the group kernel
+    kTunTileLag,       // ALPHA_MOE_TILE_LAG, ALPHA_MOE_TILE_GRID, ALPHA_MOE_WIDE_PP: of kernels that are gone; accepted, without effect
+    kTunTileGrid,
+    kTunTileNt,        // ALPHA_MOE_TILE_NT: non-temporal weight loads 1 always, 0 never (group kernel)
+    kTunWidePp,
+    kTunGroupPieces,   // ALPHA_MOE_GROUP_PIECES: most parts an UP item's contraction is taken in (group kernel)
     kTunCount
 };
 int tunable(Tunable which, int dflt);   // the override if one is set, else dflt
@@ -291,27 +318,22 @@ size_t stream_workspace_bytes(int top_k, int M, int K, int N, int E, int sorted_
 hipError_t launch_stream(const MoeParams &p, int warp_n, int stages, void *workspace, hipStream_t stream);
 
 
-// Tiled kernel for large batches: one workgroup per row block, token tiles shared through LDS, all I/128 slices in
-// one workgroup, per-slot bf16 result rows reduced by a second kernel.
-bool tile_supported(int top_k, int M, int K, int N, int E, int sorted_num, int block_m);
-size_t tile_workspace_bytes(int top_k, int M, int K, int N, int E, int sorted_num, int block_m);
-hipError_t launch_tile(const MoeParams &p, int stages, void *workspace, hipStream_t stream);
-
-// Wide kernel for large batches: macro blocks of up to 256 consecutive sorted rows of one expert (several row blocks),
-// twice the tokens per weight byte of the tile kernel; same per-slot result rows and reduce kernel.  block_m > 32.
-bool wide_supported(int top_k, int M, int K, int N, int E, int sorted_num, int block_m);
-size_t wide_workspace_bytes(int top_k, int M, int K, int N, int E, int sorted_num, int block_m);
-hipError_t launch_wide(const MoeParams &p, int stages, void *workspace, hipStream_t stream);
+// Row blocks above 32 rows (prefill): one item to a workgroup of four wavefronts - a row block x one slice of the intermediate, or x
+// a slab of output columns -, per-slot bf16 result rows added up by the reduce kernel.
+bool group_supported(int top_k, int M, int K, int N, int E, int sorted_num, int block_m);
+size_t group_workspace_bytes(int top_k, int M, int K, int N, int E, int sorted_num, int block_m);
+hipError_t launch_group(const MoeParams &p, int stages, void *workspace, hipStream_t stream);
 
 // out[t] = bf16(out[t] + sum over the token's live slots of y[slot]) (or bf16(sum) when p.overwrite).  Runs behind the
-// kernel that wrote the rows and closed the launch epoch.  Shared by the streaming, tile and wide kernels, which write each (token,
-// slot) row once into y.
+// kernel that wrote the rows, each (token, slot) row once.  Shared by the streaming and group kernels.
 struct RowsReduce {
     MoeParams p;
     StreamCtl *ctl;
-    const int *live;      // [slots] == epoch of the control block for rows written in this call
+    const int *live;      // [slots] == this launch's stamp for rows written in this call
     const void *y;        // [slots][K] bf16 or fp32
     int y_is_f32;
+    int *heads;           // group kernel: its eight queue counters, `head_stride` words apart; they go back to zero here, and the
+    int head_stride;      // launch epoch is closed.  Null: the kernel before has done both.
 };
 hipError_t launch_rows_reduce(const RowsReduce &r, hipStream_t stream);
 

@@ -1,0 +1,719 @@
+// Fused W8A8 MoE for row blocks above 32 rows (prefill and large decode batches): one launch of short-lived workgroups of four
+// wavefronts, two to a compute unit (three for blocks of at most 64 rows), each with one work item, then the row sums
+// (moe_rows_reduce_kernel).
+//
+// What bounds it: the weights and result rows at sizes where an expert has few rows (HBM), the path into a compute unit and the
+// matrix cores above.  Why independent workgroups: an item has phases that use nothing of what the others wait for - a chain of
+// round trips before its first load, the K loop, SwiGLU and requantisation, the acknowledgement of its stores - and a
+// workgroup that shares its compute unit with another one in a different phase hides them without any scheduling of ours.  The
+// persistent kernels of eight wavefronts that were here before (one row block, or 256 rows, to a workgroup that had the compute
+// unit to itself) spent a third of their time in those phases.  MI355X, layer
+// calls back to back, before and with this kernel (every launch of the call): Qwen3-30B M = 1024 200 -> 154 us, M = 8192 589 -> 486;
+// Qwen3-Next M = 4096 284 -> 236; DeepSeek shard M = 2048 421 -> 387, M = 8192 1040 -> 976.
+//
+// UP item: a row block x one 128-column slice of the intermediate (256 rows of w1).  Wavefront w multiplies slab rows
+// 64 w .. 64 w + 63 with all token tiles.  Nobody else reads its weights, so they go through a slot of 8 KiB of its own: the slot
+// is read into registers at the start of a step and refilled for the next one at once, which makes the registers the second
+// stage and leaves LDS for two stages of token tiles and for the second workgroup.  One barrier a step.  All loads are direct to LDS
+// and cover whole 128-byte lines (the register layout of the matrix operands - 16 rows x 64 bytes an instruction - is loaded at a
+// quarter of the rate).  A step's loads go out in a burst in front of its matrix work; handed out between the token tiles they
+// cost 2 %: the matrix instructions then wait for the memory path, which the other workgroup's matrix work would fill.
+// Then SwiGLU, the row maxima of the slice and the FP8 requantisation in registers; the operand tiles are put together in LDS
+// (4-byte stores to memory: 3 us an item more), stored, and the unit's flag is raised
+// (fused_moe_w8a8_up_down_acc.cu:863-994 of the reference).
+//
+// DOWN item: a row block x a slab of output columns, all slices; 64 columns to a wavefront and step, w2 through the same slots.
+// Up to two slices' tiles stay in LDS for the whole item (then no barrier either), more are streamed like tokens.  Each valid (token, slot)
+// row is written once, bf16, to y[slot] (fused_moe_w8a8_up_down_acc.cu:1007-1096 adds top_k * I/128 partial rows per token into the
+// output instead).
+//
+// Which item: eight queues, one per XCD (workgroups are dealt to the XCDs in turn), so that row blocks of one expert meet in one
+// L2; a workgroup draws a ticket from its queue's counter.  A queue holds the UP items of all its blocks, then the DOWN items, which
+// wait for flags of UP items EARLIER in the same queue: whoever drew those is running and waits for nothing, so every queue drains
+// with any number of resident workgroups.  (By workgroup index instead of a ticket: 1 - 2 % faster, but it needs workgroups to
+// start in order.  Workgroups that stay and take item after item: 5 - 15 % slower.)
+#include <mutex>
+#include <type_traits>
+
+#include "moe_common.hpp"
+
+namespace alpha_moe {
+namespace {
+
+constexpr int kGStages = 2;                // K steps whose token tiles are in the ring
+constexpr int kGSlot = 4 * 2048;           // a wavefront's four weight tiles of a K step
+constexpr int kGMaxKb = 128;               // most 128-byte K blocks (K <= 16384)
+constexpr int kGMaxW2s = 512;              // most w2 block scales of a DOWN item: launch_group cuts its slab to that
+constexpr int kGChunk = 8;                 // consecutive row blocks of a queue
+constexpr int kGHeadStride = 128;          // words between the queues' counters (lines of their own); behind one: the queue's arrivals
+constexpr int kGMaxRound = 96;             // most workgroups of a queue counted as running at a time
+constexpr int kGLongKb = 32;               // K blocks from which on UP items may be taken in parts
+constexpr int kGResidentIb = 2;            // slices whose requantised tiles fit the token ring for a whole DOWN item
+
+struct GroupParams {
+    MoeParams p;
+    StreamCtl *ctl;
+    int *head;        // next item of queue q at [q * kGHeadStride]
+    int *flag;        // [row block][n_ib] == epoch once the slice's tiles are in scratch
+    int *live;        // [slots] == epoch once y[slot] is written this launch
+    uint16_t *y;      // [slots][K] bf16
+    uint8_t *aqs;     // [row block][n_ib][tpb] requantised operand tiles of 2 KiB
+    float *sas;       // [row block][n_ib][tpb * 16] their per-token scales
+    int n_ib, nkb, n_mb_max;
+    int tpb;          // 16-row tile slots per row block in scratch
+    int gps, n_cs;    // 64-column groups per DOWN item (a multiple of 4), column slabs
+    int round;        // workgroups of a queue that run at a time
+    int max_pieces;   // most parts of an UP item's contraction
+    int xs_chunk;     // 1: a token's activation scales are fetched four K steps at a time (K / 128 a multiple of 4, x_scale
+                      // 16-byte aligned), 0: one step at a time
+    int w_nt;         // weights with non-temporal loads: 1 always, 0 never, -1 for experts with one row block
+};
+
+__device__ __forceinline__ int rfl(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// Direct-to-LDS loads of 16 and 4 bytes per lane from (wavefront-uniform base) + (per-lane offset) + (uniform offset): one scalar
+// addition a load, where the flat forms take a 64-bit address each.
+template <int AUX>
+__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t base, unsigned voff, unsigned soff, void *lds)
+{
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(base, (lptr_t)(uint32_t)(uintptr_t)lds, 16, (int)voff, (int)soff, 0, AUX);
+}
+template <int AUX>
+__device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t base, unsigned voff, unsigned soff, void *lds)
+{
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(base, (lptr_t)(uint32_t)(uintptr_t)lds, 4, (int)voff, (int)soff, 0, AUX);
+}
+
+// The 4 weight tiles of a wavefront's slot, as matrix operands in registers; the slot may be refilled afterwards.
+__device__ __forceinline__ void read_slot(v8i (&a)[4], const uint8_t *slot, int frag_lo, int frag_hi)
+{
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        a[k] = cat(*reinterpret_cast<const v4i *>(slot + k * 2048 + frag_lo), *reinterpret_cast<const v4i *>(slot + k * 2048 + frag_hi));
+    asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
+    wait_lds_reads();
+}
+
+// Operand reads of the multiply loop, written as instructions the compiler knows nothing about and waited for by count: it
+// would wait for ALL outstanding LDS reads before a tile's first matrix instruction, the next tile's (just issued) included.
+// LDS reads complete in order, so "at most the three reads just issued are outstanding" is what a tile needs.
+template <int OFF>
+__device__ __forceinline__ v4i lds_read16_raw(unsigned addr)
+{
+    v4i v;
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
+    return v;
+}
+__device__ __forceinline__ float lds_read4_raw(unsigned addr)
+{
+    float v;
+    asm volatile("ds_read_b32 %0, %1" : "=v"(v) : "v"(addr));
+    return v;
+}
+template <int N>
+__device__ __forceinline__ void lds_landed_but(v4i &lo, v4i &hi, float &f)
+{
+    asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(lo), "+v"(hi), "+v"(f) : "n"(N));
+}
+
+// 4 weight tiles in registers x T token tiles in LDS: acc[k][t] += (a_k x b_t) * f_t * (k odd ? sc1 : sc0).  A product is scaled
+// into its accumulator two matrix instructions after its own, so no wait states stand between the two.
+template <int T, int NT>
+__device__ __forceinline__ void multiply(const v8i (&a)[4], const uint8_t *b_tiles, const float *row, int row_stride, float sc0,
+                                         float sc1, v4f (&acc)[4][NT], int frag_lo, int frag_hi)
+{
+    const unsigned a_lo = (uint32_t)(uintptr_t)b_tiles + (unsigned)frag_lo, a_hi = (uint32_t)(uintptr_t)b_tiles + (unsigned)frag_hi;
+    const unsigned a_f = (uint32_t)(uintptr_t)row, f_stride = 4u * (unsigned)row_stride;
+    v4i b_lo = lds_read16_raw<0>(a_lo), b_hi = lds_read16_raw<0>(a_hi);
+    float f = lds_read4_raw(a_f);
+    v4f prod[2];
+    float fac[2];
+    auto tile = [&](auto tc) {
+        constexpr int t = decltype(tc)::value;
+        v4i n_lo = b_lo, n_hi = b_hi;
+        float n_f = f;
+        if constexpr (t + 1 < T) {
+            n_lo = lds_read16_raw<(t + 1) * 2048>(a_lo);
+            n_hi = lds_read16_raw<(t + 1) * 2048>(a_hi);
+            n_f = lds_read4_raw(a_f + (unsigned)(t + 1) * f_stride);
+            lds_landed_but<3>(b_lo, b_hi, f);
+        } else {
+            lds_landed_but<0>(b_lo, b_hi, f);
+        }
+        const v8i b = cat(b_lo, b_hi);
+        const float p0 = f * sc0, p1 = f * sc1;
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const v4f cur = mfma_fp8(a[k], b);
+            __builtin_amdgcn_sched_barrier(0);
+            if (t > 0 || k >= 2) {
+                v4f &dst = k >= 2 ? acc[k - 2][t] : acc[2 + k][t > 0 ? t - 1 : 0];
+                dst += prod[0] * fac[0];
+                asm volatile("" : "+v"(dst));
+            }
+            prod[0] = prod[1];
+            fac[0] = fac[1];
+            prod[1] = cur;
+            fac[1] = (k & 1) ? p1 : p0;
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        b_lo = n_lo;
+        b_hi = n_hi;
+        f = n_f;
+    };
+    tile(std::integral_constant<int, 0>{});
+    if constexpr (T > 1) tile(std::integral_constant<int, 1>{});
+    if constexpr (T > 2) tile(std::integral_constant<int, 2>{});
+    if constexpr (T > 3) tile(std::integral_constant<int, 3>{});
+    if constexpr (T > 4) tile(std::integral_constant<int, 4>{});
+    if constexpr (T > 5) tile(std::integral_constant<int, 5>{});
+    if constexpr (T > 6) tile(std::integral_constant<int, 6>{});
+    if constexpr (T > 7) tile(std::integral_constant<int, 7>{});
+    acc[2][T - 1] += prod[0] * fac[0];
+    acc[3][T - 1] += prod[1] * fac[1];
+}
+
+template <int NT>
+__global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const GroupParams s)
+{
+    using std::integral_constant;
+    extern __shared__ __attribute__((aligned(128))) uint8_t lds[];   // [4 wavefronts] weight slots, [kGStages][NT][2048] token tiles
+    union Tables {
+        struct {
+            union {
+                float xc[2 * NT * 64];   // chunked: [chunk & 1][token][step & 3]; else [step & 3][token]
+                float amax[4][NT * 16];  // behind the last step
+            };
+            float ws[2][kGMaxKb];
+        } up;
+        struct {
+            float sa[2][NT * 16];    // [slice or step & 1][token]
+            float w2s[kGMaxW2s];
+            float tw[NT * 16];
+        } down;
+    };
+    __shared__ __attribute__((aligned(16))) Tables tab;
+    __shared__ int s_row[NT * 16];   // UP: token of each row (0 for none); DOWN: slot of each row (-1: none)
+    __shared__ int s_slot[NT * 16];  // UP in pieces: slot of each row (-1: none)
+    __shared__ int s_last[2];
+    __shared__ int s_item;
+
+    const MoeParams &p = s.p;
+    const int tid = threadIdx.x, lane = tid & 63, w = rfl(tid >> 6);
+    const int n = lane & 15, q = lane >> 4;
+    const int K = p.K, I = p.N >> 1, nkb = s.nkb, n_ib = s.n_ib;
+    const int epoch = next_epoch(rfl(s.ctl->epoch));
+    int n_live = (rfl(p.ntpp[0]) + p.block_m - 1) / p.block_m;
+    n_live = n_live < s.n_mb_max ? n_live : s.n_mb_max;
+
+    const int f_n = (n >> 1) & 7;
+    const int frag_lo = n * 128 + 16 * (q ^ f_n);
+    const int frag_hi = n * 128 + 16 * ((q ^ f_n) ^ 4);
+    // direct-to-LDS load h of a tile: lane l fills position l & 7 of row 8h + l / 8
+    const int ld_row = lane >> 3;
+    unsigned ld_chunk[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) ld_chunk[h] = 16u * ((lane & 7) ^ (((8 * h + ld_row) >> 1) & 7));
+    uint8_t *slot = lds + w * kGSlot, *ring = lds + 4 * kGSlot;
+
+    // the only row block of its expert: nobody else will ask for the weights it streams
+    auto alone = [&](int mb, int e) {
+        if (s.w_nt >= 0) return s.w_nt != 0;
+        bool a = true;
+        if (mb > 0) a = rfl(p.expert_ids[mb - 1]) != e;
+        if (mb + 1 < n_live) a &= rfl(p.expert_ids[mb + 1]) != e;
+        return a;
+    };
+    auto tiles_of = [&]() {
+        int last = s_last[0];
+        if (NT > 4) last = s_last[1] > last ? s_last[1] : last;
+        return rfl((last >> 4) + 1);   // 0 when no row is valid
+    };
+    // run(T, non-temporal) with the smallest even T that holds the live tiles
+    auto pick = [&](int n_tiles, bool nt, auto run) {
+        auto sized = [&](auto ntc) {
+            if (NT >= 8 && n_tiles > 6) run(integral_constant<int, NT >= 8 ? 8 : NT>{}, ntc);
+            else if (NT >= 6 && n_tiles > 4) run(integral_constant<int, NT >= 6 ? 6 : NT>{}, ntc);
+            else if (n_tiles > 2) run(integral_constant<int, 4>{}, ntc);
+            else run(integral_constant<int, 2>{}, ntc);
+        };
+        if (nt) sized(std::true_type{});
+        else sized(std::false_type{});
+    };
+
+    // K steps [k0, k1); pieces > 1: the piece-th of that many parts of the contraction, `arrived` counts the finished ones
+    auto up_item = [&](int mb, int ib, int k0, int k1, int piece, int pieces, int *arrived) {
+        const int e = rfl(p.expert_ids[mb]);
+        if (e < 0 || e >= p.E) return;
+        const int row0 = mb * p.block_m;
+        const int n_rows = p.block_m < p.sorted_num - row0 ? p.block_m : p.sorted_num - row0;
+        if (tid < NT * 16) {
+            int id = -1;
+            if (tid < n_rows) id = p.sorted_ids[row0 + tid];
+            const int tk = id / p.top_k;
+            const bool ok = id >= 0 && tk < p.M;
+            s_row[tid] = ok ? tk : 0;
+            if (pieces > 1) s_slot[tid] = ok ? id : -1;
+            const unsigned long long okm = __ballot(ok);
+            if (lane == 0) s_last[w] = okm ? w * 64 + 63 - __builtin_clzll(okm) : -1;
+        }
+        const bool nt = alone(mb, e);
+        // Weights: matrix row r of tile a = (32-row group a / 2, gate | up a % 2) is slab row group * 32 + (r / 8) * 16 + r % 8 (+ 8
+        // for up), so the slab's j-th 8 rows are half (j >> 1) & 1 of tile 2 (j >> 2) + (j & 1).
+        const __amdgpu_buffer_rsrc_t wbuf = agent_buffer(p.w + (size_t)e * p.N * K + (size_t)(ib * 256 + w * 64) * p.w_rs);
+        unsigned w_voff[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) w_voff[h] = (unsigned)(ld_row * p.w_rs) + ld_chunk[h];
+        unsigned w_soff = (unsigned)(k0 * p.w_ks);
+        auto issue_w = [&](int j, auto aux) {   // j = 0 .. 7 in turn
+            dma16<decltype(aux)::value>(wbuf, w_voff[(j >> 1) & 1], w_soff, slot + (2 * (j >> 2) + (j & 1)) * 2048 + ((j >> 1) & 1) * 1024);
+            w_soff += (unsigned)(8 * p.w_rs);
+        };
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            if (nt) issue_w(j, integral_constant<int, 2>{});
+            else issue_w(j, integral_constant<int, 0>{});
+        }
+        if (w < 2) {   // this slice's gate (row 2*ib) and up (row 2*ib+1) scales
+            const __amdgpu_buffer_rsrc_t wsbuf = agent_buffer(p.w_scale + ((size_t)e * (p.N >> 7) + 2 * ib + w) * nkb);
+            for (int c = 0; c < nkb; c += 64)
+                if (lane < nkb - c) dma4<0>(wsbuf, 4u * lane, 4u * c, &tab.up.ws[w][c]);
+        }
+        lds_barrier();
+        const int n_tiles = tiles_of();
+        if (n_tiles > 0) {
+            const __amdgpu_buffer_rsrc_t xbuf = agent_buffer(p.x), xsbuf = agent_buffer(p.x_scale);
+            const bool xs_chunk = s.xs_chunk != 0;
+            v4f acc[4][NT];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int t = 0; t < NT; t++) acc[k][t] = (v4f){0.f, 0.f, 0.f, 0.f};
+            pick(n_tiles, nt, [&](auto tc, auto ntc) {
+                constexpr int T = decltype(tc)::value;   // token tiles multiplied, even
+                constexpr int AUX = decltype(ntc)::value ? 2 : 0;
+                constexpr int DM = T / 2;                // direct-to-LDS loads of a wavefront and step: 1 KiB halves of tiles
+                constexpr int XL = T * 4;                // tokens whose scales a wavefront fetches
+                unsigned x_off[DM];
+#pragma unroll
+                for (int j = 0; j < DM; j++) {
+                    const int hh = w * DM + j;
+                    x_off[j] = (unsigned)s_row[hh * 8 + ld_row] * (unsigned)K + ld_chunk[0];
+                    if (hh & 1) x_off[j] = x_off[j] - ld_chunk[0] + ld_chunk[1];
+                }
+                const unsigned xs_off = 4u * (unsigned)s_row[w * XL + (lane < XL ? lane : 0)] * (unsigned)nkb;
+                auto issue_xs = [&](int k) {
+                    if (!xs_chunk || (k & 3) == 0) {
+                        if (lane < XL) {
+                            if (xs_chunk) dma16<0>(xsbuf, xs_off, 4u * k, &tab.up.xc[(((k >> 2) & 1) * NT * 16 + w * XL) * 4]);
+                            else dma4<0>(xsbuf, xs_off, 4u * k, &tab.up.xc[(k & 3) * NT * 16 + w * XL]);
+                        }
+                    }
+                };
+                auto issue_x = [&](int k, int j) {
+                    dma16<0>(xbuf, x_off[j], 128u * k, ring + (k & (kGStages - 1)) * (NT * 2048) + w * (DM * 1024) + j * 1024);
+                };
+                const int row_stride = xs_chunk ? 64 : 16;
+                issue_xs(k0);
+#pragma unroll
+                for (int j = 0; j < DM; j++) issue_x(k0, j);
+                for (int k = k0; k < k1; k++) {
+                    wait_vmcnt<0>();   // this wavefront's loads of step k have landed
+                    lds_barrier();     // everybody's have, and step k - 1 is done with
+                    v8i a[4];
+                    float sc0 = tab.up.ws[0][k], sc1 = tab.up.ws[1][k];
+                    asm volatile("" : "+v"(sc0), "+v"(sc1));
+                    read_slot(a, slot, frag_lo, frag_hi);
+                    if (k + 1 < k1) {   // the next step's loads
+                        issue_xs(k + 1);
+                        w_soff = (unsigned)((k + 1) * p.w_ks);
+#pragma unroll
+                        for (int o = 0; o < 8; o++) issue_w(o, integral_constant<int, AUX>{});
+#pragma unroll
+                        for (int o = 0; o < DM; o++) issue_x(k + 1, o);
+                    }
+                    const float *row = xs_chunk ? &tab.up.xc[(((k >> 2) & 1) * NT * 16 + n) * 4 + (k & 3)]
+                                                : &tab.up.xc[(k & 3) * NT * 16 + n];
+                    multiply<T>(a, ring + (k & (kGStages - 1)) * (NT * 2048), row, row_stride, sc0, sc1, acc, frag_lo, frag_hi);
+                }
+            });
+
+            if (pieces > 1) {
+                // Partial sums go where the rows' results will be (nobody writes those before this unit's flag is up): 1 KiB
+                // of row y[slot] for each (slice, piece).  The last piece to arrive adds them up, in order.
+                const unsigned at = (unsigned)((ib * pieces) * 1024 + w * 256 + q * 16);
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    const int id = s_slot[t * 16 + n];
+                    if (id >= 0) {
+#pragma unroll
+                        for (int k = 0; k < 4; k++) stg128_agent(s.y, (unsigned)id * 2u * K + at + piece * 1024 + k * 64, acc[k][t]);
+                    }
+                }
+                wait_vmcnt<0>();
+                __syncthreads();
+                if (tid == 0) {
+                    const int before = __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (before == pieces - 1) store_agent(arrived, 0);
+                    s_item = before;
+                }
+                __syncthreads();
+                if (rfl(s_item) != pieces - 1) return;
+                acquire_fence();
+#pragma unroll
+                for (int t = 0; t < NT; t++) {
+                    const int id = s_slot[t * 16 + n];
+                    v4f sum[4] = {};
+                    if (id >= 0) {
+                        for (int o = 0; o < pieces; o++) {
+                            v4f v[4];
+#pragma unroll
+                            for (int k = 0; k < 4; k++) v[k] = __builtin_bit_cast(v4f, ldg128_agent(s.y, (unsigned)id * 2u * K + at + o * 1024 + k * 64));
+#pragma unroll
+                            for (int k = 0; k < 4; k++) sum[k] += v[k];
+                        }
+                    }
+#pragma unroll
+                    for (int k = 0; k < 4; k++) acc[k][t] = sum[k];
+                }
+            }
+            __syncthreads();   // the scales' place is the row maxima's from here on
+            // SwiGLU, per-token amax over the slice's 128 columns, FP8 requant into operand tiles
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                if (t < n_tiles) {
+                    float mx = 0.f;
+#pragma unroll
+                    for (int pr = 0; pr < 2; pr++)
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            const float v = swiglu_bf16(acc[2 * pr][t][j], acc[2 * pr + 1][t][j]);
+                            acc[2 * pr][t][j] = v;
+                            mx = fmaxf(mx, fabsf(v));
+                        }
+                    mx = fmaxf(mx, __shfl_xor(mx, 16));
+                    mx = fmaxf(mx, __shfl_xor(mx, 32));
+                    if (q == 0) tab.up.amax[w][t * 16 + n] = mx;
+                }
+            }
+            __syncthreads();
+            // the tiles are put together where the token ring was, then stored 16 bytes a lane
+            const size_t tile0 = ((size_t)mb * n_ib + ib) * s.tpb;
+#pragma unroll
+            for (int t = 0; t < NT; t++) {
+                if (t < n_tiles) {
+                    float mx = kAmaxFloor;
+#pragma unroll
+                    for (int wv = 0; wv < 4; wv++) mx = fmaxf(mx, tab.up.amax[wv][t * 16 + n]);
+                    const RowScale rs(mx);
+#pragma unroll
+                    for (int pr = 0; pr < 2; pr++) {
+                        const uint32_t packed =
+                            pack_fp8x4(rs.code(acc[2 * pr][t][0]), rs.code(acc[2 * pr][t][1]), rs.code(acc[2 * pr][t][2]),
+                                       rs.code(acc[2 * pr][t][3]));
+                        // columns w*32 + pr*16 + 4q .. +3 of token n: chunk w*2 + pr of the row, bytes 4q .. 4q+3 in it
+                        *reinterpret_cast<uint32_t *>(ring + t * 2048 + n * 128 + 16 * ((w * 2 + pr) ^ f_n) + 4 * q) = packed;
+                    }
+                    if (w == 0 && q == 0) stg32_agent(s.sas + (tile0 + t) * 16, 4u * n, __builtin_bit_cast(uint32_t, rs.scale));
+                }
+            }
+            lds_barrier();
+            for (int i = tid; i < n_tiles * 128; i += 256)
+                stg128_agent(s.aqs + tile0 * 2048, 16u * i, *reinterpret_cast<const v4f *>(ring + 16 * i));
+            wait_vmcnt<0>();
+        }
+        __syncthreads();
+        if (tid == 0) store_agent(&s.flag[mb * n_ib + ib], epoch);
+    };
+
+    auto down_item = [&](int mb, int cs, auto resident_c) {
+        constexpr bool RESIDENT = decltype(resident_c)::value;
+        const int e = rfl(p.expert_ids[mb]);
+        if (e < 0 || e >= p.E) return;
+        const int row0 = mb * p.block_m;
+        const int n_rows = p.block_m < p.sorted_num - row0 ? p.block_m : p.sorted_num - row0;
+        float tw = 0.f;
+        if (tid < NT * 16) {
+            int id = -1;
+            if (tid < n_rows) id = p.sorted_ids[row0 + tid];
+            const bool ok = id >= 0 && id / p.top_k < p.M;
+            s_row[tid] = ok ? id : -1;
+            if (ok) {
+                tw = p.topk_w[id];
+                if (cs == 0) s.live[id] = epoch;
+            }
+            const unsigned long long okm = __ballot(ok);
+            if (lane == 0) s_last[w] = okm ? w * 64 + 63 - __builtin_clzll(okm) : -1;
+        }
+        const int n_groups = K >> 6;
+        const int g0 = cs * s.gps;
+        const int g1 = g0 + s.gps < n_groups ? g0 + s.gps : n_groups;
+        const bool nt = alone(mb, e);
+        lds_barrier();
+        const int n_tiles = tiles_of();
+        if (n_tiles == 0) return;
+        const int rounds = (g1 - g0 + 3) >> 2;   // the slab's groups w, w + 4, ... of wavefront w; past the end: computed, not stored
+        const int n_steps = rounds * n_ib;
+        const __amdgpu_buffer_rsrc_t wbuf = agent_buffer(p.w2 + (size_t)e * K * I);
+        const __amdgpu_buffer_rsrc_t abuf = agent_buffer(s.aqs + (size_t)mb * n_ib * s.tpb * 2048);
+        const __amdgpu_buffer_rsrc_t sbuf = agent_buffer(s.sas + (size_t)mb * n_ib * s.tpb * 16);
+        // matrix row r of tile k is output column c0 + 16 (r / 4) + 4 k + r % 4: lane (n, q) collects 16 adjacent columns
+        unsigned w_voff[2];
+#pragma unroll
+        for (int h = 0; h < 2; h++) w_voff[h] = (unsigned)((16 * (lane >> 5) + (ld_row & 3)) * p.w2_rs) + ld_chunk[h];
+        pick(n_tiles, nt, [&](auto tc, auto ntc) {
+            constexpr int T = decltype(tc)::value;
+            constexpr int AUX = decltype(ntc)::value ? 2 : 0;
+            constexpr int DM = T / 2;
+            constexpr int XL = T * 4;
+            v4f acc[4][T];
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int t = 0; t < T; t++) acc[k][t] = (v4f){0.f, 0.f, 0.f, 0.f};
+            int li = 0, lib = 0, lg = g0 + w;   // next step to load: its number, slice and column group
+            unsigned w_soff = 0;
+            auto aim_w = [&]() {
+                const int grp = lg < g1 ? lg : g1 - 1;
+                w_soff = (unsigned)((grp << 6) * p.w2_rs + lib * p.w2_ks);
+            };
+            auto issue_w = [&](int o) {   // o = 0 .. 7 in turn
+                dma16<AUX>(wbuf, w_voff[o >> 2], w_soff, slot + (o & 3) * 2048 + (o >> 2) * 1024);
+                w_soff += (unsigned)((o == 3 ? 20 : 4) * p.w2_rs);
+            };
+            // slice ib's tiles (past the last one: that one again) and their scales
+            auto issue_x = [&](int ib, int stage, int j) {
+                {
+                    const int hh = w * DM + j, tt = hh >> 1;
+                    dma16<kAuxAgent>(abuf, (unsigned)(lane * 16),
+                                     (unsigned)((ib * s.tpb + (tt < n_tiles ? tt : n_tiles - 1)) * 2048 + (hh & 1) * 1024),
+                                     ring + stage * (NT * 2048) + hh * 1024);
+                }
+            };
+            auto issue_xs = [&](int ib, int stage) {
+                if (lane < XL) {
+                    const int r = w * XL + lane;
+                    dma4<kAuxAgent>(sbuf, 4u * (r < n_tiles * 16 ? r : 0), (unsigned)(ib * s.tpb * 64), &tab.down.sa[stage][w * XL]);
+                }
+            };
+            auto advance = [&]() {
+                li++;
+                if (++lib == n_ib) {
+                    lib = 0;
+                    lg += 4;
+                }
+            };
+            // the weights do not depend on the UP items
+            aim_w();
+#pragma unroll
+            for (int o = 0; o < 8; o++) issue_w(o);
+            if (w == 1) {
+                const __amdgpu_buffer_rsrc_t w2sbuf = agent_buffer(p.w2_scale + ((size_t)e * (K >> 7) + (g0 >> 1)) * n_ib);
+                const int count = ((g1 - g0 + 1) >> 1) * n_ib;
+                for (int c = 0; c < count; c += 64)
+                    if (lane < count - c) dma4<0>(w2sbuf, 4u * lane, 4u * c, &tab.down.w2s[c]);
+            }
+            if (tid < NT * 16) tab.down.tw[tid] = tw * p.scaling;
+            if (w == 0) spin_all_eq(&s.flag[mb * n_ib], n_ib, epoch, s.ctl);
+            lds_barrier();
+            if constexpr (RESIDENT) {
+                for (int ib = 0; ib < n_ib; ib++) {
+                    issue_xs(ib, ib);
+#pragma unroll
+                    for (int j = 0; j < DM; j++) issue_x(ib, ib, j);
+                }
+            } else {
+                issue_xs(0, 0);
+#pragma unroll
+                for (int j = 0; j < DM; j++) issue_x(0, 0, j);
+            }
+            advance();
+            wait_vmcnt<0>();
+            __syncthreads();
+            int cg = g0 + w, cib = 0;
+            for (int i = 0; i < n_steps; i++) {
+                if (!RESIDENT && i > 0) lds_barrier();   // everybody's loads of the step have landed, the step before is done with
+                v8i a[4];
+                read_slot(a, slot, frag_lo, frag_hi);
+                if (i + 1 < n_steps) {   // the next step's loads
+                    aim_w();
+#pragma unroll
+                    for (int o = 0; o < 8; o++) issue_w(o);
+                    if (!RESIDENT) {
+                        issue_xs(lib, li & 1);
+#pragma unroll
+                        for (int j = 0; j < DM; j++) issue_x(lib, li & 1, j);
+                    }
+                    advance();
+                }
+                const int st = RESIDENT ? cib : (i & 1);
+                const float ws2 = tab.down.w2s[(((cg < g1 ? cg : g1 - 1) - g0) >> 1) * n_ib + cib];
+                multiply<T>(a, ring + st * (NT * 2048), &tab.down.sa[st][n], 16, ws2, ws2, acc, frag_lo, frag_hi);
+                wait_vmcnt<0>();   // the next step's loads, before any result store is queued behind them
+                if (++cib == n_ib) {
+#pragma unroll
+                    for (int t = 0; t < T; t++) {
+                        const int slot_id = s_row[t * 16 + n];
+                        if (slot_id >= 0 && cg < g1) {
+                            const float tw = tab.down.tw[t * 16 + n];
+                            uint16_t *yp = s.y + (size_t)slot_id * K + (cg << 6) + 16 * q;
+#pragma unroll
+                            for (int half = 0; half < 2; half++) {
+                                const v4f lo = acc[2 * half][t] * tw, hi = acc[2 * half + 1][t] * tw;
+                                v4i o;
+                                o.x = (int)pack_bf16x2(lo[0], lo[1]);
+                                o.y = (int)pack_bf16x2(lo[2], lo[3]);
+                                o.z = (int)pack_bf16x2(hi[0], hi[1]);
+                                o.w = (int)pack_bf16x2(hi[2], hi[3]);
+                                *reinterpret_cast<v4i *>(yp + 8 * half) = o;
+                            }
+                        }
+#pragma unroll
+                        for (int k = 0; k < 4; k++) acc[k][t] = (v4f){0.f, 0.f, 0.f, 0.f};
+                    }
+                    cib = 0;
+                    cg += 4;
+                }
+            }
+        });
+    };
+
+    // ---- which item ---------------------------------------------------------------------------------------------------
+    const int q_id = blockIdx.x & 7;
+    if (blockIdx.x == 0 && tid == 0) s.ctl->stamp = epoch;   // for the reduce kernel, which closes the launch
+    if (tid == 0) s_item = __hip_atomic_fetch_add(s.head + q_id * kGHeadStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int item = rfl(s_item);
+    // This queue's live row blocks: whole rounds of chunks of kGChunk, what is left in chunks of an eighth of it
+    const int whole_chunks = n_live / (8 * kGChunk), left = n_live % (8 * kGChunk), chunk = (left + 7) >> 3;
+    const int rest = left - chunk * q_id;
+    const int nb = whole_chunks * kGChunk + (rest < 0 ? 0 : rest < chunk ? rest : chunk);
+    const int ups = nb * n_ib;
+    // Where one round of workgroups holds all UP items and K is long, each is taken in two parts: with a long item to two of a
+    // compute unit's three workgroups the loads in flight do not cover the memory's latency, and it is over when the slowest compute
+    // unit is (DeepSeek shard, 64-row blocks, whole -> two parts: M = 513 319 -> 308 us, 700 331 -> 316, 1024 353 -> 340, 1400 382 ->
+    // 369; three parts 317, 329, 349, 377).  Beyond one round the last one is left whole: parts of it cost more than they level
+    // (M = 2048 401 -> 411 us, 2500 430 -> 444).
+    const int pieces = ups < s.round && nkb >= kGLongKb ? s.max_pieces : 1;
+    const int up_items = ups * pieces;
+    const bool is_up = item < up_items;
+    const int unit_id = item / pieces, piece = item - unit_id * pieces;
+    const int k0 = is_up ? (nkb >> 2) * piece / pieces * 4 : 0;   // parts start at multiples of four K steps (the scales' chunks)
+    const int k1 = is_up && piece + 1 < pieces ? (nkb >> 2) * (piece + 1) / pieces * 4 : nkb;
+    const int i = is_up ? unit_id : item - up_items, per = is_up ? n_ib : s.n_cs;
+    const int j = i / per, off = i - j * per;
+    if (j >= nb) return;
+    const int mb = rfl(j < whole_chunks * kGChunk ? ((j / kGChunk) * 8 + q_id) * kGChunk + j % kGChunk
+                                                  : whole_chunks * 8 * kGChunk + chunk * q_id + j - whole_chunks * kGChunk);
+    if (is_up)
+        up_item(mb, rfl(off), rfl(k0), rfl(k1), rfl(piece), rfl(pieces), s.head + q_id * kGHeadStride + 1 + rfl(unit_id));
+    else if (n_ib <= kGResidentIb) down_item(mb, rfl(off), std::true_type());
+    else down_item(mb, rfl(off), std::false_type());
+}
+
+size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
+
+constexpr int dyn_lds(int nt) { return 4 * kGSlot + kGStages * nt * 2048; }
+
+typedef void (*GroupFn)(const GroupParams);
+
+hipError_t allow_dynamic_lds()
+{
+    static std::mutex mu;
+    static bool done[64];
+    int dev = 0;
+    hipError_t err = hipGetDevice(&dev);
+    if (err != hipSuccess) return err;
+    std::lock_guard<std::mutex> lock(mu);
+    if (dev >= 0 && dev < 64 && done[dev]) return hipSuccess;
+    const GroupFn fn[] = {moe_group_kernel<4>, moe_group_kernel<6>, moe_group_kernel<8>};
+    for (int i = 0; i < 3 && err == hipSuccess; i++)
+        err = hipFuncSetAttribute(reinterpret_cast<const void *>(fn[i]), hipFuncAttributeMaxDynamicSharedMemorySize, dyn_lds(4 + 2 * i));
+    if (err == hipSuccess && dev >= 0 && dev < 64) done[dev] = true;
+    return err;
+}
+
+}  // namespace
+
+bool group_supported(int top_k, int M, int K, int N, int E, int sorted_num, int block_m)
+{
+    (void)E;
+    const int n_ib = N / 256;
+    const int64_t n_mb = ((int64_t)sorted_num + block_m - 1) / block_m;
+    return block_m > 32 && K <= 128 * kGMaxKb && (K / 128) * n_ib <= 1024 && (int64_t)M * top_k <= kMaxSlots &&
+           n_mb * n_ib <= kMaxUnits;
+}
+
+size_t group_workspace_bytes(int top_k, int M, int K, int N, int E, int sorted_num, int block_m)
+{
+    (void)E;
+    const size_t n_mb = ((size_t)sorted_num + block_m - 1) / block_m;
+    const size_t tiles = n_mb * (N / 256) * ((block_m + 15) / 16);
+    return align_up(kPrefixBytes) + align_up((size_t)M * top_k * K * sizeof(uint16_t)) + align_up(tiles * 2048) +
+           align_up(tiles * 16 * sizeof(float));
+}
+
+hipError_t launch_group(const MoeParams &p, int stages, void *workspace, hipStream_t stream)
+{
+    uint8_t *ws = static_cast<uint8_t *>(workspace);
+    GroupParams s;
+    s.p = p;
+    s.n_ib = p.N / 256;
+    s.nkb = p.K / 128;
+    s.n_mb_max = (p.sorted_num + p.block_m - 1) / p.block_m;
+    s.tpb = (p.block_m + 15) / 16;
+    size_t off = align_up(kPrefixBytes);
+    s.ctl = reinterpret_cast<StreamCtl *>(ws);
+    s.head = reinterpret_cast<int *>(ws + kOffArrive);
+    s.flag = reinterpret_cast<int *>(ws + kOffFlag);
+    s.live = reinterpret_cast<int *>(ws + kOffLive);
+    s.y = reinterpret_cast<uint16_t *>(ws + off);
+    off += align_up((size_t)p.M * p.top_k * p.K * sizeof(uint16_t));
+    s.aqs = ws + off;
+    off += align_up((size_t)s.n_mb_max * s.n_ib * s.tpb * 2048);
+    s.sas = reinterpret_cast<float *>(ws + off);
+    const int e_gps = tunable(kTunTileGps, 0);
+    s.gps = e_gps > 0 ? (e_gps + 3) / 4 * 4 : 4 * ((5 * stages + s.n_ib - 1) / s.n_ib);
+    while (s.gps > 4 && s.gps / 2 * s.n_ib > kGMaxW2s) s.gps -= 4;
+    s.n_cs = ((p.K >> 6) + s.gps - 1) / s.gps;
+    s.xs_chunk = (s.nkb % 4 == 0 && reinterpret_cast<uintptr_t>(p.x_scale) % 16 == 0) ? 1 : 0;
+    s.w_nt = tunable(kTunTileNt, -1);
+    hipError_t err = allow_dynamic_lds();
+    if (err != hipSuccess) return err;
+    const unsigned chunk_rounds = (unsigned)((s.n_mb_max + 8 * kGChunk - 1) / (8 * kGChunk));
+    static const int cus = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            return 256;
+        return n;
+    }();
+    const int per_cu = s.tpb <= 4 ? 3 : 2;
+    s.round = (cus >= 8 ? cus / 8 : 1) * (s.tpb <= 4 ? 3 : 2);
+    if (s.round > kGMaxRound) s.round = kGMaxRound;
+    // The partial sums (1 KiB a row, slice and part) take the rows' places in y.
+    s.max_pieces = tunable(kTunGroupPieces, 2);
+    const int room = p.K * 2 / (1024 * s.n_ib);
+    if (s.max_pieces > room) s.max_pieces = room;
+    if ((int64_t)p.M * p.top_k * p.K * 2 > 0xffffffffll) s.max_pieces = 1;   // (their offsets are 32-bit)
+    if (s.max_pieces < 1) s.max_pieces = 1;
+    if (s.max_pieces > 8) s.max_pieces = 8;
+    const unsigned grid = 8 * (chunk_rounds * kGChunk * (s.n_ib + s.n_cs) + s.round * (s.max_pieces - 1));
+    const int nt = s.tpb <= 4 ? 4 : s.tpb <= 6 ? 6 : 8;
+    const GroupFn fn = nt == 4 ? moe_group_kernel<4> : nt == 6 ? moe_group_kernel<6> : moe_group_kernel<8>;
+    hipLaunchKernelGGL(fn, dim3(grid), dim3(256), dyn_lds(nt), stream, s);
+    err = hipGetLastError();
+    if (err != hipSuccess) return err;
+    RowsReduce r;
+    r.p = p;
+    r.ctl = s.ctl;
+    r.live = s.live;
+    r.y = s.y;
+    r.y_is_f32 = 0;
+    r.heads = s.head;
+    r.head_stride = kGHeadStride;
+    return launch_rows_reduce(r, stream);
+}
+
+}  // namespace alpha_moe

@@ -104,15 +104,6 @@ __device__ __forceinline__ void lds_store(float *at, float v)
     asm volatile("ds_write_b32 %0, %1" ::"v"(addr), "v"(v) : "memory");
 }
 
-// a / s from r ~ 1 / s (one rounding off at most) by one residual correction: three instructions where the division takes
-// ten.  For s = 448 it is the quotient, for every bf16 row maximum; the FP8 codes are those of the exact division (the CPU tests
-// compare both, the codes for all mantissas of row maximum and value at eleven exponents).
-__device__ __forceinline__ float divide(float a, float s, float r)
-{
-    const float t = a * r;
-    return __builtin_fmaf(__builtin_fmaf(-t, s, a), r, t);
-}
-
 // the largest of the values (not negative, not NaN) of the 16 lanes of a row (lanes 16 k .. 16 k + 15), in all of them: rotations
 // within the row.  As integers, which such values compare as: a step is one instruction, where a float maximum is four.
 __device__ __forceinline__ float max_of_16_lanes(float v)
@@ -143,18 +134,11 @@ __device__ __forceinline__ uint2 quantise_row(const v4i raw, float *scale)
 #pragma unroll
     for (int i = 0; i < 8; i++) m = fmaxf(m, fabsf(v[i]));
     m = max_of_16_lanes(m);
-    // a row with an infinity: its scale is infinite, a finite value over it is 0 and an infinity over it NaN; NaN is clamped
-    // to -448 (as in the other kernels)
-    const bool inf = m == __builtin_inff();
-    const float sa = inf ? m : divide(m, kFp8Max, 1.0f / kFp8Max);
-    float r = __builtin_amdgcn_rcpf(sa);
-    r = inf ? 0.f : __builtin_fmaf(__builtin_fmaf(-sa, r, 1.0f), r, r);
-    const float s = inf ? 0.f : sa;
-    auto code = [&](float a) { return clamp_fp8(divide(a, s, r)); };
+    const RowScale rs(m);
     uint2 o;
-    o.x = pack_fp8x4(code(v[0]), code(v[1]), code(v[2]), code(v[3]));
-    o.y = pack_fp8x4(code(v[4]), code(v[5]), code(v[6]), code(v[7]));
-    *scale = sa;
+    o.x = pack_fp8x4(rs.code(v[0]), rs.code(v[1]), rs.code(v[2]), rs.code(v[3]));
+    o.y = pack_fp8x4(rs.code(v[4]), rs.code(v[5]), rs.code(v[6]), rs.code(v[7]));
+    *scale = rs.scale;
     return o;
 }
 

@@ -846,6 +846,8 @@ hipError_t launch_stream(const MoeParams &p, int warp_n, int stages, void *works
     r.live = s.live;
     r.y = s.y;
     r.y_is_f32 = 1;
+    r.heads = nullptr;
+    r.head_stride = 0;
     return launch_rows_reduce(r, stream);
 }
 

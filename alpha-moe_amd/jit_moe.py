@@ -15,9 +15,8 @@ Differences, all on purpose:
     merges the result into an existing table;
   * on MI355X the knobs select this: row blocks of at most 32 rows take the streaming kernel (`warp_n` = wavefronts per
     workgroup, `stages` = depth of each wavefront's LDS ring) or, up to 16 tokens where they are ahead, the small kernels, to
-    which `block_n`, `warp_n` and `stages` mean nothing (their candidates differ by noise only); above that `warp_n` 4 takes the tile kernel (one row
-    block per item, four token tiles per wavefront), `warp_n` 8 the wide kernel (macro blocks of 256 rows, eight token
-    tiles per wavefront), and `stages` sets the length of their down-projection items.
+    which `block_n`, `warp_n` and `stages` mean nothing (their candidates differ by noise only); above that the group
+    kernel, in which `stages` sets the length of a down-projection item and `warp_n` means nothing.
 """
 import argparse
 import json

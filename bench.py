@@ -254,7 +254,7 @@ def main():
     def kernel_of(knobs):
         if knobs["block_m"] <= 32:
             return "moe_stream_kernel"
-        return "moe_wide_kernel" if knobs["warp_n"] == 8 else "moe_tile_kernel"
+        return "moe_group_kernel"
     if args.M >= 4096:   # prefill: the contraction is the bound (the weights stream once; from M ~ 8k the matrix time exceeds the HBM time)
         tflops = head["flops"] / head["launch_us_mean"] / 1e6
         roofline = {"bound": "mfma", "achieved": round(tflops, 1), "peak": FP8_PEAK_TFLOPS, "unit": "TFLOP/s",

@@ -186,6 +186,41 @@ def test_wide_kernel_up_loop_variants_give_the_same_bits():
                 assert torch.equal(outs[0], b), (K, M, knobs, "unaligned scales")
 
 
+@pytest.mark.parametrize("block_m", [40, 64, 72, 96, 104, 128])
+@pytest.mark.parametrize("K,I", [(384, 256), (512, 128), (640, 384), (4096, 256), (4224, 128)])
+def test_group_kernel_at_the_edges_of_its_tiles(block_m, K, I):
+    """Row blocks with one live row, one to eight live token tiles, the last row of a tile, a full block and one row more, an
+    expert without rows; one, two and three slices of the intermediate (up to two stay in LDS for a whole DOWN item, more are streamed);
+    column groups that are no multiple of a workgroup's four; K blocks in fours and singly (K / 128 = 3, 5, 33); and K from which on the
+    UP items of so few blocks are taken in two parts, whose sums the last part adds up (K = 4096, 4224: also as a whole)."""
+    rows = [1, 16, 17, 0, block_m - 1, block_m, block_m + 1, 33]
+    shape = Shape("ge", E=len(rows), top_k=1, K=K, I=I, shared_expert=False, routing="softmax_renorm", scaling_factor=1.2)
+    P = make_problem(make_weights(shape, device=DEV, seed=K + I), sum(rows), seed=block_m)
+    ids = torch.repeat_interleave(torch.arange(len(rows)), torch.tensor(rows))
+    perm = torch.randperm(P.M, generator=torch.Generator().manual_seed(block_m))
+    P.topk_ids = ids[perm].to(torch.int32).view(-1, 1).to(DEV)
+    refs = oracle_variants(P)
+
+    def check(out, what):
+        """With one expert to a token nothing averages out what a row's scale does: where the slice's largest activation is within
+        rounding noise of a bf16 boundary (of gate, up or their product), the scale moves by 2^-8 and about one code in sixteen - 8 or
+        so of 128 - by its spacing, 2^-3.5 of its value: sqrt(8) * 0.09 / sqrt(128) = 2.2 % of the row's root mean square, four times
+        that in the largest of K columns, where the output's largest value is five times it: 1.8e-2.  Such rows are few."""
+        o = out.float().cpu()
+        scale = refs[0].float().abs().max()
+        per_row = torch.stack([(o - r.float()).abs().amax(dim=1) for r in refs]).amin(dim=0) / scale
+        assert float(per_row.max()) <= 1.8e-2 and int((per_row > 1e-2).sum()) <= P.M // 64, (what, per_row.topk(4))
+
+    print(f"case group kernel block_m {block_m} K={K} I={I}", flush=True)
+    got = run_op(P, block_m, 64, 4, 1, via="c_abi")
+    check(got, f"block_m {block_m} K={K} I={I}")
+    assert torch.equal(got, run_op(P, block_m, 64, 4, 5, via="c_abi"))   # other column slabs
+    with tunables(ALPHA_MOE_GROUP_PIECES=1):
+        whole = run_op(P, block_m, 64, 4, 1, via="c_abi")
+    check(whole, f"block_m {block_m} K={K} I={I}, contraction not in parts")
+    assert K >= 4096 or torch.equal(got, whole)
+
+
 def test_store_variant_fallback_kernel():
     """129 K blocks are more than the tile and wide kernels take: the fallback kernel serves the call, and its store
     variant overwrites too."""
