@@ -12,9 +12,9 @@
 // Qwen3-Next M = 4096 284 -> 236; DeepSeek shard M = 2048 421 -> 387, M = 8192 1040 -> 976.
 //
 // UP item: a row block x one 128-column slice of the intermediate (256 rows of w1).  Wavefront w multiplies slab rows
-// 64 w .. 64 w + 63 with all token tiles.  Nobody else reads its weights, so they go through a slot of 8 KiB of its own: the slot
-// is read into registers at the start of a step and refilled for the next one at once, which makes the registers the second
-// stage and leaves LDS for two stages of token tiles and for the second workgroup.  One barrier a step.  All loads are direct to LDS
+// 64 w .. 64 w + 63 with all token tiles.  Nobody else reads its weights, so they go through a small ring of its own: a step's four
+// tiles are read into registers at its start and their places refilled at once, which makes the registers one more stage
+// and leaves LDS for two stages of token tiles and for the second workgroup.  One barrier a step.  All loads are direct to LDS
 // and cover whole 128-byte lines (the register layout of the matrix operands - 16 rows x 64 bytes an instruction - is loaded at a
 // quarter of the rate).  A step's loads go out in a burst in front of its matrix work; handed out between the token tiles they
 // cost 2 %: the matrix instructions then wait for the memory path, which the other workgroup's matrix work would fill.
@@ -22,7 +22,7 @@
 // (4-byte stores to memory: 3 us an item more), stored, and the unit's flag is raised
 // (fused_moe_w8a8_up_down_acc.cu:863-994 of the reference).
 //
-// DOWN item: a row block x a slab of output columns, all slices; 64 columns to a wavefront and step, w2 through the same slots.
+// DOWN item: a row block x a slab of output columns, all slices; 64 columns to a wavefront and step, w2 through the same ring.
 // Up to two slices' tiles stay in LDS for the whole item (then no barrier either), more are streamed like tokens.  Each valid (token, slot)
 // row is written once, bf16, to y[slot] (fused_moe_w8a8_up_down_acc.cu:1007-1096 adds top_k * I/128 partial rows per token into the
 // output instead).
@@ -40,14 +40,26 @@
 namespace alpha_moe {
 namespace {
 
-constexpr int kGStages = 2;                // K steps whose token tiles are in the ring
-constexpr int kGSlot = 4 * 2048;           // a wavefront's four weight tiles of a K step
+// Dynamic LDS: a ring of weight tiles for each wavefront and, behind them, a ring of the steps' token tiles.  Where K is short, what
+// token tiles a row block does not have is room for more of both in flight (Qwen3-30B shard, 128-row blocks of which most have
+// one to four tiles: M = 512 147 -> 144 us, 1024 165 -> 159.5; Qwen3-Next M = 1500 186 -> 184).  Where K is long, a few-row block that
+// runs ahead takes its neighbours' lines out of L2: DeepSeek shard M = 2048 408 -> 412 us, 8192 939 -> 955.
+constexpr int dyn_lds(int nt) { return nt <= 4 ? 48 * 1024 : 72 * 1024; }   // three workgroups to a compute unit, or two
+constexpr int x_stages(int nt, int t, bool deep)   // K steps of token tiles
+{
+    return deep && (dyn_lds(nt) - 3 * t * 2048) / 8192 >= 5 ? 3 : 2;
+}
+constexpr int w_tiles(int nt, int t, int stages, bool deep)   // weight tiles of a wavefront (four to a step)
+{
+    const int r = (dyn_lds(nt) - stages * t * 2048) / 8192;
+    return !deep ? 4 : r < 7 ? r : 7;
+}
 constexpr int kGMaxKb = 128;               // most 128-byte K blocks (K <= 16384)
 constexpr int kGMaxW2s = 512;              // most w2 block scales of a DOWN item: launch_group cuts its slab to that
 constexpr int kGChunk = 8;                 // consecutive row blocks of a queue
 constexpr int kGHeadStride = 128;          // words between the queues' counters (lines of their own); behind one: the queue's arrivals
 constexpr int kGMaxRound = 96;             // most workgroups of a queue counted as running at a time
-constexpr int kGLongKb = 32;               // K blocks from which on UP items may be taken in parts
+constexpr int kGLongKb = 32;               // K blocks from which on K counts as long
 constexpr int kGResidentIb = 2;            // slices whose requantised tiles fit the token ring for a whole DOWN item
 
 struct GroupParams {
@@ -84,12 +96,12 @@ __device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t base, unsigned voff,
     __builtin_amdgcn_raw_ptr_buffer_load_lds(base, (lptr_t)(uint32_t)(uintptr_t)lds, 4, (int)voff, (int)soff, 0, AUX);
 }
 
-// The 4 weight tiles of a wavefront's slot, as matrix operands in registers; the slot may be refilled afterwards.
-__device__ __forceinline__ void read_slot(v8i (&a)[4], const uint8_t *slot, int frag_lo, int frag_hi)
+// A step's four weight tiles as matrix operands in registers; their places in the ring may be refilled afterwards.
+__device__ __forceinline__ void read_weights(v8i (&a)[4], const uint8_t *const (&tile)[4], int frag_lo, int frag_hi)
 {
 #pragma unroll
     for (int k = 0; k < 4; k++)
-        a[k] = cat(*reinterpret_cast<const v4i *>(slot + k * 2048 + frag_lo), *reinterpret_cast<const v4i *>(slot + k * 2048 + frag_hi));
+        a[k] = cat(*reinterpret_cast<const v4i *>(tile[k] + frag_lo), *reinterpret_cast<const v4i *>(tile[k] + frag_hi));
     asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
     wait_lds_reads();
 }
@@ -178,7 +190,7 @@ template <int NT>
 __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const GroupParams s)
 {
     using std::integral_constant;
-    extern __shared__ __attribute__((aligned(128))) uint8_t lds[];   // [4 wavefronts] weight slots, [kGStages][NT][2048] token tiles
+    extern __shared__ __attribute__((aligned(128))) uint8_t lds[];   // [weight tile of the ring][wavefront][2048], [stage][token tile][2048]
     union Tables {
         struct {
             union {
@@ -215,7 +227,7 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
     unsigned ld_chunk[2];
 #pragma unroll
     for (int h = 0; h < 2; h++) ld_chunk[h] = 16u * ((lane & 7) ^ (((8 * h + ld_row) >> 1) & 7));
-    uint8_t *slot = lds + w * kGSlot, *ring = lds + 4 * kGSlot;
+    uint8_t *my_tiles = lds + w * 2048;   // place i of the wavefront's weight ring: + i * 8192
 
     // the only row block of its expert: nobody else will ask for the weights it streams
     auto alone = [&](int mb, int e) {
@@ -230,13 +242,18 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
         if (NT > 4) last = s_last[1] > last ? s_last[1] : last;
         return rfl((last >> 4) + 1);   // 0 when no row is valid
     };
-    // run(T, non-temporal) with the smallest even T that holds the live tiles
+    // run(T, non-temporal, deep rings) with the smallest even T that holds the live tiles
+    const bool short_k = nkb < kGLongKb;
     auto pick = [&](int n_tiles, bool nt, auto run) {
         auto sized = [&](auto ntc) {
-            if (NT >= 8 && n_tiles > 6) run(integral_constant<int, NT >= 8 ? 8 : NT>{}, ntc);
-            else if (NT >= 6 && n_tiles > 4) run(integral_constant<int, NT >= 6 ? 6 : NT>{}, ntc);
-            else if (n_tiles > 2) run(integral_constant<int, 4>{}, ntc);
-            else run(integral_constant<int, 2>{}, ntc);
+            auto few = [&](auto tc) {
+                if (short_k) run(tc, ntc, std::true_type{});
+                else run(tc, ntc, std::false_type{});
+            };
+            if (NT >= 8 && n_tiles > 6) run(integral_constant<int, NT >= 8 ? 8 : NT>{}, ntc, std::false_type{});
+            else if (NT >= 6 && n_tiles > 4) run(integral_constant<int, NT >= 6 ? 6 : NT>{}, ntc, std::false_type{});
+            else if (n_tiles > 2) few(integral_constant<int, 4>{});
+            else few(integral_constant<int, 2>{});
         };
         if (nt) sized(std::true_type{});
         else sized(std::false_type{});
@@ -259,21 +276,26 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
             if (lane == 0) s_last[w] = okm ? w * 64 + 63 - __builtin_clzll(okm) : -1;
         }
         const bool nt = alone(mb, e);
-        // Weights: matrix row r of tile a = (32-row group a / 2, gate | up a % 2) is slab row group * 32 + (r / 8) * 16 + r % 8 (+ 8
-        // for up), so the slab's j-th 8 rows are half (j >> 1) & 1 of tile 2 (j >> 2) + (j & 1).
+        // Weights: matrix row r of tile i = (32-row group i / 2, gate | up i % 2) is slab row group * 32 + (r / 8) * 16 + r % 8 (+ 8
+        // for up)
         const __amdgpu_buffer_rsrc_t wbuf = agent_buffer(p.w + (size_t)e * p.N * K + (size_t)(ib * 256 + w * 64) * p.w_rs);
         unsigned w_voff[2];
 #pragma unroll
         for (int h = 0; h < 2; h++) w_voff[h] = (unsigned)(ld_row * p.w_rs) + ld_chunk[h];
-        unsigned w_soff = (unsigned)(k0 * p.w_ks);
-        auto issue_w = [&](int j, auto aux) {   // j = 0 .. 7 in turn
-            dma16<decltype(aux)::value>(wbuf, w_voff[(j >> 1) & 1], w_soff, slot + (2 * (j >> 2) + (j & 1)) * 2048 + ((j >> 1) & 1) * 1024);
-            w_soff += (unsigned)(8 * p.w_rs);
+        auto issue_w = [&](int place, int k, int i, auto aux) {   // tile i of step k
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                dma16<decltype(aux)::value>(wbuf, w_voff[h], (unsigned)(k * p.w_ks + ((i >> 1) * 32 + (i & 1) * 8 + h * 16) * p.w_rs),
+                                            my_tiles + place * 8192 + h * 1024);
+        };
+        auto issue_rows = [&](int k, int j, auto aux) {   // the j-th eight rows of the slab, into a ring of four places
+            dma16<decltype(aux)::value>(wbuf, w_voff[(j >> 1) & 1], (unsigned)(k * p.w_ks + 8 * j * p.w_rs),
+                                        my_tiles + (2 * (j >> 2) + (j & 1)) * 8192 + ((j >> 1) & 1) * 1024);
         };
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            if (nt) issue_w(j, integral_constant<int, 2>{});
-            else issue_w(j, integral_constant<int, 0>{});
+        for (int i = 0; i < 4; i++) {
+            if (nt) issue_w(i, k0, i, integral_constant<int, 2>{});
+            else issue_w(i, k0, i, integral_constant<int, 0>{});
         }
         if (w < 2) {   // this slice's gate (row 2*ib) and up (row 2*ib+1) scales
             const __amdgpu_buffer_rsrc_t wsbuf = agent_buffer(p.w_scale + ((size_t)e * (p.N >> 7) + 2 * ib + w) * nkb);
@@ -290,11 +312,14 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
             for (int k = 0; k < 4; k++)
 #pragma unroll
                 for (int t = 0; t < NT; t++) acc[k][t] = (v4f){0.f, 0.f, 0.f, 0.f};
-            pick(n_tiles, nt, [&](auto tc, auto ntc) {
+            pick(n_tiles, nt, [&](auto tc, auto ntc, auto deepc) {
                 constexpr int T = decltype(tc)::value;   // token tiles multiplied, even
-                constexpr int AUX = decltype(ntc)::value ? 2 : 0;
+                constexpr integral_constant<int, decltype(ntc)::value ? 2 : 0> ntc_aux{};
                 constexpr int DM = T / 2;                // direct-to-LDS loads of a wavefront and step: 1 KiB halves of tiles
                 constexpr int XL = T * 4;                // tokens whose scales a wavefront fetches
+                constexpr bool DEEP = decltype(deepc)::value;
+                constexpr int S = x_stages(NT, T, DEEP), R = w_tiles(NT, T, S, DEEP);
+                uint8_t *ring = lds + R * 8192;
                 unsigned x_off[DM];
 #pragma unroll
                 for (int j = 0; j < DM; j++) {
@@ -311,31 +336,65 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
                         }
                     }
                 };
-                auto issue_x = [&](int k, int j) {
-                    dma16<0>(xbuf, x_off[j], 128u * k, ring + (k & (kGStages - 1)) * (NT * 2048) + w * (DM * 1024) + j * 1024);
+                auto issue_x = [&](int k, int stage) {
+#pragma unroll
+                    for (int j = 0; j < DM; j++) dma16<0>(xbuf, x_off[j], 128u * k, ring + stage * (T * 2048) + w * (DM * 1024) + j * 1024);
                 };
                 const int row_stride = xs_chunk ? 64 : 16;
+                // A step's loads are issued in this order: the scales and - with two stages - the token tiles of the step that is
+                // S - 1 ahead; weight tiles of the next step, into the places this step's have left; with three stages
+                // the token tiles here; weight tiles of the step after the next.  Loads complete in order, so at the start of a
+                // step what was issued behind its own last weight tile may still be on its way.
+                constexpr int BEHIND = 2 * (R - 4) + (S == 3 ? DM : 0);
                 issue_xs(k0);
+                issue_x(k0, 0);
+                if (k0 + 1 < k1) {
+                    if (S == 3) issue_xs(k0 + 1);
 #pragma unroll
-                for (int j = 0; j < DM; j++) issue_x(k0, j);
+                    for (int g = 4; g < R; g++) issue_w(g, k0 + 1, g & 3, ntc_aux);
+                    if (S == 3) issue_x(k0 + 1, 1);
+                }
+                int first = 0, stage = 0;   // the step's first weight tile, and its token tiles, in their rings
                 for (int k = k0; k < k1; k++) {
-                    wait_vmcnt<0>();   // this wavefront's loads of step k have landed
+                    if (k + 1 < k1) wait_vmcnt<BEHIND>();   // this wavefront's loads of step k have landed
+                    else wait_vmcnt<0>();
                     lds_barrier();     // everybody's have, and step k - 1 is done with
                     v8i a[4];
+                    int place[4];
+                    const uint8_t *tile[4];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        place[i] = first + i < R ? first + i : first + i - R;
+                        tile[i] = my_tiles + place[i] * 8192;
+                    }
+                    first = first + 4 < R ? first + 4 : first + 4 - R;
                     float sc0 = tab.up.ws[0][k], sc1 = tab.up.ws[1][k];
                     asm volatile("" : "+v"(sc0), "+v"(sc1));
-                    read_slot(a, slot, frag_lo, frag_hi);
-                    if (k + 1 < k1) {   // the next step's loads
-                        issue_xs(k + 1);
-                        w_soff = (unsigned)((k + 1) * p.w_ks);
+                    read_weights(a, tile, frag_lo, frag_hi);
+                    const int ahead = stage + S - 1 < S ? stage + S - 1 : stage - 1;
+                    if (k + S - 1 < k1) issue_xs(k + S - 1);
+                    if constexpr (R == 4) {
+                        // (all of a step's weights at once: in the order of their rows and in front of the tokens, which is 1 - 3 %
+                        // of a call of the DeepSeek shard at M = 8192, where row blocks of one expert share them in L2)
+                        if (k + 1 < k1) {
 #pragma unroll
-                        for (int o = 0; o < 8; o++) issue_w(o, integral_constant<int, AUX>{});
+                            for (int j = 0; j < 8; j++) issue_rows(k + 1, j, ntc_aux);
+                            issue_x(k + 1, ahead);
+                        }
+                    } else if (k + 1 < k1) {
+                        if (S == 2) issue_x(k + 1, ahead);
 #pragma unroll
-                        for (int o = 0; o < DM; o++) issue_x(k + 1, o);
+                        for (int i = 0; i < 8 - R; i++) issue_w(place[i], k + 1, (R + i) & 3, ntc_aux);
+                    }
+                    if (S == 3 && k + 2 < k1) issue_x(k + 2, ahead);
+                    if (R > 4 && k + 2 < k1) {
+#pragma unroll
+                        for (int i = 8 - R; i < 4; i++) issue_w(place[i], k + 2, (R + i) & 3, ntc_aux);
                     }
                     const float *row = xs_chunk ? &tab.up.xc[(((k >> 2) & 1) * NT * 16 + n) * 4 + (k & 3)]
                                                 : &tab.up.xc[(k & 3) * NT * 16 + n];
-                    multiply<T>(a, ring + (k & (kGStages - 1)) * (NT * 2048), row, row_stride, sc0, sc1, acc, frag_lo, frag_hi);
+                    multiply<T>(a, ring + stage * (T * 2048), row, row_stride, sc0, sc1, acc, frag_lo, frag_hi);
+                    stage = stage + 1 < S ? stage + 1 : 0;
                 }
             });
 
@@ -398,7 +457,7 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
                 }
             }
             __syncthreads();
-            // the tiles are put together where the token ring was, then stored 16 bytes a lane
+            // the tiles are put together where the weights were, then stored 16 bytes a lane
             const size_t tile0 = ((size_t)mb * n_ib + ib) * s.tpb;
 #pragma unroll
             for (int t = 0; t < NT; t++) {
@@ -413,14 +472,14 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
                             pack_fp8x4(rs.code(acc[2 * pr][t][0]), rs.code(acc[2 * pr][t][1]), rs.code(acc[2 * pr][t][2]),
                                        rs.code(acc[2 * pr][t][3]));
                         // columns w*32 + pr*16 + 4q .. +3 of token n: chunk w*2 + pr of the row, bytes 4q .. 4q+3 in it
-                        *reinterpret_cast<uint32_t *>(ring + t * 2048 + n * 128 + 16 * ((w * 2 + pr) ^ f_n) + 4 * q) = packed;
+                        *reinterpret_cast<uint32_t *>(lds + t * 2048 + n * 128 + 16 * ((w * 2 + pr) ^ f_n) + 4 * q) = packed;
                     }
                     if (w == 0 && q == 0) stg32_agent(s.sas + (tile0 + t) * 16, 4u * n, __builtin_bit_cast(uint32_t, rs.scale));
                 }
             }
             lds_barrier();
             for (int i = tid; i < n_tiles * 128; i += 256)
-                stg128_agent(s.aqs + tile0 * 2048, 16u * i, *reinterpret_cast<const v4f *>(ring + 16 * i));
+                stg128_agent(s.aqs + tile0 * 2048, 16u * i, *reinterpret_cast<const v4f *>(lds + 16 * i));
             wait_vmcnt<0>();
         }
         __syncthreads();
@@ -462,25 +521,34 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
         unsigned w_voff[2];
 #pragma unroll
         for (int h = 0; h < 2; h++) w_voff[h] = (unsigned)((16 * (lane >> 5) + (ld_row & 3)) * p.w2_rs) + ld_chunk[h];
-        pick(n_tiles, nt, [&](auto tc, auto ntc) {
+        pick(n_tiles, nt, [&](auto tc, auto ntc, auto deepc) {
             constexpr int T = decltype(tc)::value;
             constexpr int AUX = decltype(ntc)::value ? 2 : 0;
             constexpr int DM = T / 2;
             constexpr int XL = T * 4;
+            constexpr int R = w_tiles(NT, T, 2, decltype(deepc)::value);
+            uint8_t *ring = lds + R * 8192;
             v4f acc[4][T];
 #pragma unroll
             for (int k = 0; k < 4; k++)
 #pragma unroll
                 for (int t = 0; t < T; t++) acc[k][t] = (v4f){0.f, 0.f, 0.f, 0.f};
-            int li = 0, lib = 0, lg = g0 + w;   // next step to load: its number, slice and column group
-            unsigned w_soff = 0;
-            auto aim_w = [&]() {
+            // the step that is two ahead of the one multiplied: its slice and column group, and where its weights are
+            int lib = 0, lg = g0 + w;
+            auto aim = [&]() {
                 const int grp = lg < g1 ? lg : g1 - 1;
-                w_soff = (unsigned)((grp << 6) * p.w2_rs + lib * p.w2_ks);
+                return (unsigned)((grp << 6) * p.w2_rs + lib * p.w2_ks);
             };
-            auto issue_w = [&](int o) {   // o = 0 .. 7 in turn
-                dma16<AUX>(wbuf, w_voff[o >> 2], w_soff, slot + (o & 3) * 2048 + (o >> 2) * 1024);
-                w_soff += (unsigned)((o == 3 ? 20 : 4) * p.w2_rs);
+            auto advance = [&]() {
+                if (++lib == n_ib) {
+                    lib = 0;
+                    lg += 4;
+                }
+            };
+            auto issue_w = [&](int place, unsigned at, int i) {
+#pragma unroll
+                for (int h = 0; h < 2; h++)
+                    dma16<AUX>(wbuf, w_voff[h], at + (unsigned)((4 * i + 32 * h) * p.w2_rs), my_tiles + place * 8192 + h * 1024);
             };
             // slice ib's tiles (past the last one: that one again) and their scales
             auto issue_x = [&](int ib, int stage, int j) {
@@ -488,7 +556,7 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
                     const int hh = w * DM + j, tt = hh >> 1;
                     dma16<kAuxAgent>(abuf, (unsigned)(lane * 16),
                                      (unsigned)((ib * s.tpb + (tt < n_tiles ? tt : n_tiles - 1)) * 2048 + (hh & 1) * 1024),
-                                     ring + stage * (NT * 2048) + hh * 1024);
+                                     ring + stage * (T * 2048) + hh * 1024);
                 }
             };
             auto issue_xs = [&](int ib, int stage) {
@@ -497,17 +565,21 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
                     dma4<kAuxAgent>(sbuf, 4u * (r < n_tiles * 16 ? r : 0), (unsigned)(ib * s.tpb * 64), &tab.down.sa[stage][w * XL]);
                 }
             };
-            auto advance = [&]() {
-                li++;
-                if (++lib == n_ib) {
-                    lib = 0;
-                    lg += 4;
-                }
-            };
             // the weights do not depend on the UP items
-            aim_w();
+            unsigned at1, at2;   // weights of the next step and of the one after it
+            {
+                const unsigned at0 = aim();
 #pragma unroll
-            for (int o = 0; o < 8; o++) issue_w(o);
+                for (int i = 0; i < 4; i++) issue_w(i, at0, i);
+                advance();
+                at1 = aim();
+                if (n_steps > 1) {
+#pragma unroll
+                    for (int g = 4; g < R; g++) issue_w(g, at1, g & 3);
+                }
+                advance();
+                at2 = aim();
+            }
             if (w == 1) {
                 const __amdgpu_buffer_rsrc_t w2sbuf = agent_buffer(p.w2_scale + ((size_t)e * (K >> 7) + (g0 >> 1)) * n_ib);
                 const int count = ((g1 - g0 + 1) >> 1) * n_ib;
@@ -528,29 +600,51 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
 #pragma unroll
                 for (int j = 0; j < DM; j++) issue_x(0, 0, j);
             }
-            advance();
             wait_vmcnt<0>();
             __syncthreads();
-            int cg = g0 + w, cib = 0;
+            int cg = g0 + w, cib = 0, first = 0;
             for (int i = 0; i < n_steps; i++) {
                 if (!RESIDENT && i > 0) lds_barrier();   // everybody's loads of the step have landed, the step before is done with
                 v8i a[4];
-                read_slot(a, slot, frag_lo, frag_hi);
-                if (i + 1 < n_steps) {   // the next step's loads
-                    aim_w();
+                int place[4];
+                const uint8_t *tile[4];
 #pragma unroll
-                    for (int o = 0; o < 8; o++) issue_w(o);
-                    if (!RESIDENT) {
-                        issue_xs(lib, li & 1);
-#pragma unroll
-                        for (int j = 0; j < DM; j++) issue_x(lib, li & 1, j);
-                    }
-                    advance();
+                for (int t = 0; t < 4; t++) {
+                    place[t] = first + t < R ? first + t : first + t - R;
+                    tile[t] = my_tiles + place[t] * 8192;
                 }
+                first = first + 4 < R ? first + 4 : first + 4 - R;
+                read_weights(a, tile, frag_lo, frag_hi);
+                if (i + 1 < n_steps) {   // the next step's loads, as in the UP items
+                    if constexpr (!RESIDENT) {
+                        const int ib = cib + 1 < n_ib ? cib + 1 : 0;
+                        issue_xs(ib, (i + 1) & 1);
+#pragma unroll
+                        for (int j = 0; j < DM; j++) issue_x(ib, (i + 1) & 1, j);
+                    }
+                    if constexpr (R == 4) {
+#pragma unroll
+                        for (int o = 0; o < 8; o++)
+                            dma16<AUX>(wbuf, w_voff[o >> 2], at1 + (unsigned)((4 * (o & 3) + 32 * (o >> 2)) * p.w2_rs),
+                                       my_tiles + (o & 3) * 8192 + (o >> 2) * 1024);
+                    } else {
+#pragma unroll
+                        for (int t = 0; t < 8 - R; t++) issue_w(place[t], at1, (R + t) & 3);
+                    }
+                }
+                if (R > 4 && i + 2 < n_steps) {
+#pragma unroll
+                    for (int t = 8 - R; t < 4; t++) issue_w(place[t], at2, (R + t) & 3);
+                }
+                at1 = at2;
+                advance();
+                at2 = aim();
                 const int st = RESIDENT ? cib : (i & 1);
                 const float ws2 = tab.down.w2s[(((cg < g1 ? cg : g1 - 1) - g0) >> 1) * n_ib + cib];
-                multiply<T>(a, ring + st * (NT * 2048), &tab.down.sa[st][n], 16, ws2, ws2, acc, frag_lo, frag_hi);
-                wait_vmcnt<0>();   // the next step's loads, before any result store is queued behind them
+                multiply<T>(a, ring + st * (T * 2048), &tab.down.sa[st][n], 16, ws2, ws2, acc, frag_lo, frag_hi);
+                // the next step's loads have landed before any result store is queued behind them
+                if (i + 2 < n_steps) wait_vmcnt<2 * (R - 4)>();
+                else wait_vmcnt<0>();
                 if (++cib == n_ib) {
 #pragma unroll
                     for (int t = 0; t < T; t++) {
@@ -613,8 +707,6 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
 }
 
 size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
-
-constexpr int dyn_lds(int nt) { return 4 * kGSlot + kGStages * nt * 2048; }
 
 typedef void (*GroupFn)(const GroupParams);
 
