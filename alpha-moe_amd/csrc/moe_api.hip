@@ -364,4 +364,4 @@ extern "C" const char *alpha_moe_status_string(int status)
     }
 }
 
-extern "C" const char *alpha_moe_version(void) { return "0.7"; }
+extern "C" const char *alpha_moe_version(void) { return "0.8"; }

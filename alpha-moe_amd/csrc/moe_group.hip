@@ -30,7 +30,7 @@
 // Which item: eight queues, one per XCD (workgroups are dealt to the XCDs in turn), so that row blocks of one expert meet in one
 // L2; a workgroup draws a ticket from its queue's counter.  A queue holds the UP items of all its blocks, then the DOWN items, which
 // wait for flags of UP items EARLIER in the same queue: whoever drew those is running and waits for nothing, so every queue drains
-// with any number of resident workgroups.  (By workgroup index instead of a ticket: 1 - 2 % faster, but it needs workgroups to
+// with any number of resident workgroups.  (By workgroup index instead of a ticket: at most 1 % faster, but it needs workgroups to
 // start in order.  Workgroups that stay and take item after item: 5 - 15 % slower.)
 #include <mutex>
 #include <type_traits>
