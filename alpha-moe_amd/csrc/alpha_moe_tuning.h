@@ -9,6 +9,10 @@
  * The environment variables of the same names are read once, when the library is first used; no launch reads the
  * environment.  Not thread-safe against concurrent launches.  Results stay within the parity bar whatever is set.
  * Returns ALPHA_MOE_ERR_SHAPE for an unknown name.
+ *
+ * alpha_moe_group_plan tells how the group kernel would serve a call: plan = {tiles of 16 rows its variant takes in a row block,
+ * 64-column groups of a down-projection item, items' column slabs, w2 block scales an item's table holds}.  Returns
+ * ALPHA_MOE_ERR_SHAPE for a call that another kernel serves.  Host only.
  */
 #ifndef ALPHA_MOE_TUNING_H
 #define ALPHA_MOE_TUNING_H
@@ -16,6 +20,7 @@
 extern "C" {
 #endif
 int alpha_moe_set_tunable(const char *name, int value, int set);
+int alpha_moe_group_plan(int top_k, int M, int K, int N, int num_experts, int sorted_num, int block_m, int stages, int plan[4]);
 #ifdef __cplusplus
 }
 #endif

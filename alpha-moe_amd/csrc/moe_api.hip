@@ -78,6 +78,17 @@ extern "C" int alpha_moe_set_tunable(const char *name, int value, int set)
     return ALPHA_MOE_ERR_SHAPE;
 }
 
+extern "C" int alpha_moe_group_plan(int top_k, int M, int K, int N, int num_experts, int sorted_num, int block_m, int stages,
+                                    int plan[4])
+{
+    if (!plan) return ALPHA_MOE_ERR_NULL_POINTER;
+    const int rc = alpha_moe_validate(top_k, M, K, N, num_experts, sorted_num, block_m, 64, 4, stages);
+    if (rc != ALPHA_MOE_OK) return rc;
+    if (choose_path(top_k, M, K, N, num_experts, sorted_num, block_m) != kGroup) return ALPHA_MOE_ERR_SHAPE;
+    group_plan_numbers(K, N, block_m, stages, plan);
+    return ALPHA_MOE_OK;
+}
+
 extern "C" int alpha_moe_validate(int top_k, int M, int K, int N, int num_experts, int sorted_num, int block_m,
                                   int block_n, int warp_n, int stages)
 {

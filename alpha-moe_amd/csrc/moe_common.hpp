@@ -323,6 +323,8 @@ hipError_t launch_stream(const MoeParams &p, int warp_n, int stages, void *works
 bool group_supported(int top_k, int M, int K, int N, int E, int sorted_num, int block_m);
 size_t group_workspace_bytes(int top_k, int M, int K, int N, int E, int sorted_num, int block_m);
 hipError_t launch_group(const MoeParams &p, int stages, void *workspace, hipStream_t stream);
+// its variant, 64-column groups per DOWN item, column slabs, and the scales a DOWN item's table holds
+void group_plan_numbers(int K, int N, int block_m, int stages, int plan[4]);
 
 // out[t] = bf16(out[t] + sum over the token's live slots of y[slot]) (or bf16(sum) when p.overwrite).  Runs behind the
 // kernel that wrote the rows, each (token, slot) row once.  Shared by the streaming and group kernels.

@@ -54,8 +54,11 @@ constexpr int w_tiles(int nt, int t, int stages, bool deep)   // weight tiles of
     const int r = (dyn_lds(nt) - stages * t * 2048) / 8192;
     return !deep ? 4 : r < 7 ? r : 7;
 }
+constexpr int kGMaxExpertW2s = 1024;       // most w2 block scales of an expert, (K / 128) * (I / 128)
+// Most w2 block scales of a DOWN item; group_plan picks variant and slab so that they fit.  The variant with three workgroups to a compute
+// unit has no LDS for more than 512, the others' table holds all that an expert can have.
+constexpr int max_w2s(int nt) { return nt <= 4 ? 512 : kGMaxExpertW2s; }
 constexpr int kGMaxKb = 128;               // most 128-byte K blocks (K <= 16384)
-constexpr int kGMaxW2s = 512;              // most w2 block scales of a DOWN item: launch_group cuts its slab to that
 constexpr int kGChunk = 8;                 // consecutive row blocks of a queue
 constexpr int kGHeadStride = 128;          // words between the queues' counters (lines of their own); behind one: the queue's arrivals
 constexpr int kGMaxRound = 96;             // most workgroups of a queue counted as running at a time
@@ -201,7 +204,7 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
         } up;
         struct {
             float sa[2][NT * 16];    // [slice or step & 1][token]
-            float w2s[kGMaxW2s];
+            float w2s[max_w2s(NT)];
             float tw[NT * 16];
         } down;
     };
@@ -210,6 +213,8 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
     __shared__ int s_slot[NT * 16];  // UP in pieces: slot of each row (-1: none)
     __shared__ int s_last[2];
     __shared__ int s_item;
+    static_assert((NT <= 4 ? 3 : 2) * ((dyn_lds(NT) + (int)sizeof(Tables) + 2 * NT * 64 + 12 + 1279) / 1280 * 1280) <= 160 * 1024,
+                  "the workgroups of a compute unit share 160 KiB of LDS, handed out 1280 bytes at a time");
 
     const MoeParams &p = s.p;
     const int tid = threadIdx.x, lane = tid & 63, w = rfl(tid >> 6);
@@ -728,12 +733,33 @@ hipError_t allow_dynamic_lds()
 
 }  // namespace
 
+// The variant that serves a call and the output columns of its DOWN items.  A row block has up to nt 16-row tiles.  A slab has at least
+// four column groups, or all there are; where the scales of so few of them exceed the smallest variant's table (K >= 256: above 256
+// slices, K = 128: above 512), the next variant takes the call.
+struct GroupPlan {
+    int nt;          // template argument of the kernel
+    int gps, n_cs;   // 64-column groups per DOWN item (a multiple of 4), column slabs
+};
+
+static GroupPlan group_plan(int K, int N, int block_m, int stages)
+{
+    GroupPlan g;
+    const int n_ib = N / 256, tiles = (block_m + 15) / 16, groups = K >> 6;
+    const int fewest = (groups < 4 ? groups : 4) / 2 * n_ib;   // scales of the smallest slab
+    g.nt = tiles <= 4 && fewest <= max_w2s(4) ? 4 : tiles <= 6 ? 6 : 8;
+    const int e_gps = tunable(kTunTileGps, 0);
+    g.gps = e_gps > 0 ? ((e_gps < groups ? e_gps : groups) + 3) / 4 * 4 : 4 * ((5 * stages + n_ib - 1) / n_ib);
+    while (g.gps > 4 && g.gps / 2 * n_ib > max_w2s(g.nt)) g.gps -= 4;
+    g.n_cs = (groups + g.gps - 1) / g.gps;
+    return g;
+}
+
 bool group_supported(int top_k, int M, int K, int N, int E, int sorted_num, int block_m)
 {
     (void)E;
     const int n_ib = N / 256;
     const int64_t n_mb = ((int64_t)sorted_num + block_m - 1) / block_m;
-    return block_m > 32 && K <= 128 * kGMaxKb && (K / 128) * n_ib <= 1024 && (int64_t)M * top_k <= kMaxSlots &&
+    return block_m > 32 && K <= 128 * kGMaxKb && (K / 128) * n_ib <= kGMaxExpertW2s && (int64_t)M * top_k <= kMaxSlots &&
            n_mb * n_ib <= kMaxUnits;
 }
 
@@ -744,6 +770,15 @@ size_t group_workspace_bytes(int top_k, int M, int K, int N, int E, int sorted_n
     const size_t tiles = n_mb * (N / 256) * ((block_m + 15) / 16);
     return align_up(kPrefixBytes) + align_up((size_t)M * top_k * K * sizeof(uint16_t)) + align_up(tiles * 2048) +
            align_up(tiles * 16 * sizeof(float));
+}
+
+void group_plan_numbers(int K, int N, int block_m, int stages, int plan[4])
+{
+    const GroupPlan g = group_plan(K, N, block_m, stages);
+    plan[0] = g.nt;
+    plan[1] = g.gps;
+    plan[2] = g.n_cs;
+    plan[3] = max_w2s(g.nt);
 }
 
 hipError_t launch_group(const MoeParams &p, int stages, void *workspace, hipStream_t stream)
@@ -765,10 +800,10 @@ hipError_t launch_group(const MoeParams &p, int stages, void *workspace, hipStre
     s.aqs = ws + off;
     off += align_up((size_t)s.n_mb_max * s.n_ib * s.tpb * 2048);
     s.sas = reinterpret_cast<float *>(ws + off);
-    const int e_gps = tunable(kTunTileGps, 0);
-    s.gps = e_gps > 0 ? (e_gps + 3) / 4 * 4 : 4 * ((5 * stages + s.n_ib - 1) / s.n_ib);
-    while (s.gps > 4 && s.gps / 2 * s.n_ib > kGMaxW2s) s.gps -= 4;
-    s.n_cs = ((p.K >> 6) + s.gps - 1) / s.gps;
+    const GroupPlan plan = group_plan(p.K, p.N, p.block_m, stages);
+    const int nt = plan.nt;
+    s.gps = plan.gps;
+    s.n_cs = plan.n_cs;
     s.xs_chunk = (s.nkb % 4 == 0 && reinterpret_cast<uintptr_t>(p.x_scale) % 16 == 0) ? 1 : 0;
     s.w_nt = tunable(kTunTileNt, -1);
     hipError_t err = allow_dynamic_lds();
@@ -781,8 +816,7 @@ hipError_t launch_group(const MoeParams &p, int stages, void *workspace, hipStre
             return 256;
         return n;
     }();
-    const int per_cu = s.tpb <= 4 ? 3 : 2;
-    s.round = (cus >= 8 ? cus / 8 : 1) * (s.tpb <= 4 ? 3 : 2);
+    s.round = (cus >= 8 ? cus / 8 : 1) * (nt <= 4 ? 3 : 2);
     if (s.round > kGMaxRound) s.round = kGMaxRound;
     // The partial sums (1 KiB a row, slice and part) take the rows' places in y.
     s.max_pieces = tunable(kTunGroupPieces, 2);
@@ -792,7 +826,6 @@ hipError_t launch_group(const MoeParams &p, int stages, void *workspace, hipStre
     if (s.max_pieces < 1) s.max_pieces = 1;
     if (s.max_pieces > 8) s.max_pieces = 8;
     const unsigned grid = 8 * (chunk_rounds * kGChunk * (s.n_ib + s.n_cs) + s.round * (s.max_pieces - 1));
-    const int nt = s.tpb <= 4 ? 4 : s.tpb <= 6 ? 6 : 8;
     const GroupFn fn = nt == 4 ? moe_group_kernel<4> : nt == 6 ? moe_group_kernel<6> : moe_group_kernel<8>;
     hipLaunchKernelGGL(fn, dim3(grid), dim3(256), dyn_lds(nt), stream, s);
     err = hipGetLastError();

@@ -170,3 +170,35 @@ def test_static_scratch_holds_every_batch_up_to_the_documented_sizes(lib):
             bm = get_best_config(table, M)["block_m"]
             need = lib.alpha_moe_workspace_bytes(top_k, M, K, N, E, M * top_k + E * (bm - 1), bm)
             assert (need <= limit) == (M <= upto), (E, M, need)
+
+
+def test_group_kernel_slab_fits_its_scale_table(lib):
+    """Every (K, slices, row block, stages, slab override) the group kernel takes: the scales of the widest slab of output columns are
+    at most what the variant's LDS table holds.  (A slab has at least four column groups, so beyond 256 slices - 512 at
+    K = 128 - the smallest variant's table would be overrun.)"""
+    lib.alpha_moe_group_plan.restype = ctypes.c_int
+    lib.alpha_moe_group_plan.argtypes = [ctypes.c_int] * 8 + [ctypes.POINTER(ctypes.c_int)]
+    lib.alpha_moe_set_tunable.argtypes = [ctypes.c_char_p, ctypes.c_int, ctypes.c_int]
+    plan = (ctypes.c_int * 4)()
+    seen = set()
+    try:
+        for gps in (None, 1, 8, 13, 64, 1 << 30):
+            assert lib.alpha_moe_set_tunable(b"ALPHA_MOE_TILE_GPS", gps or 0, gps is not None) == 0
+            for kb in [*range(1, 18), 31, 33, 56, 63, 64, 100, 128]:
+                most = 1024 // kb
+                for n_ib in sorted({*range(1, min(most, 12) + 1), *range(13, most + 1, 37), 255, 256, 257, 300, 341, 342, 511, 512, 513, most}):
+                    for block_m in (40, 64, 72, 96, 104, 128):
+                        for stages in range(1, 6):
+                            rc = lib.alpha_moe_group_plan(1, 50, 128 * kb, 256 * n_ib, 1, 50 + block_m - 1, block_m, stages, plan)
+                            assert rc == (0 if n_ib <= most else 2), (kb, n_ib, rc)
+                            if rc:
+                                continue
+                            nt, per, slabs, table = plan
+                            groups = 2 * kb
+                            assert 16 * nt >= block_m and per % 4 == 0 and per > 0 and slabs == -(-groups // per)
+                            scales = max((min((c + 1) * per, groups) - c * per + 1) // 2 * n_ib for c in range(slabs))
+                            assert scales <= table, (kb, n_ib, block_m, stages, gps, tuple(plan), scales)
+                            seen.add((nt, block_m <= 64))
+    finally:
+        lib.alpha_moe_set_tunable(b"ALPHA_MOE_TILE_GPS", 0, 0)
+    assert seen == {(4, True), (6, True), (6, False), (8, False)}

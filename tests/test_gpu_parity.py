@@ -129,6 +129,18 @@ def test_more_than_64_slices_row_blocks_above_32():
         assert torch.equal(got, run_op(P, *knobs, via="c_abi"))
 
 
+@pytest.mark.parametrize("K,slices", [(128, 1024), (256, 300), (384, 341)])
+def test_most_slices_an_expert_can_have(K, slices):
+    """So many slices that two rows of w2 scales (one at K = 128) are more than the smallest variant's table holds: the next
+    variant serves row blocks of at most 64 rows too."""
+    shape = Shape("sx", E=2, top_k=1, K=K, I=slices * 128, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
+    P = make_problem(make_weights(shape, device=DEV, seed=7), 75, seed=7)
+    ref = oracle_out(P)
+    for knobs in ((64, 32, 8, 2), (96, 32, 8, 5), (128, 64, 4, 1)):
+        print(f"case {slices} slices K={K} knobs {knobs}", flush=True)
+        assert_parity(run_op(P, *knobs, via="c_abi"), ref, f"{slices} slices {knobs}")
+
+
 def test_prefill_kernels_fetch_activation_scales_both_ways():
     """The tile and wide kernels take a token's activation scales four K blocks at a time where the row of scales allows
     16-byte loads (K / 128 a multiple of 4, x_scale 16-byte aligned) and one at a time otherwise: both ways against the
