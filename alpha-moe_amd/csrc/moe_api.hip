@@ -43,7 +43,7 @@ void load_tunables_once()
 enum Path { kDirect, kStream, kGroup, kSmall };
 
 // At most 16 tokens: small kernels where they are ahead (small_pays).  Streaming kernel for row blocks of at most 32 rows
-// (decode), group kernel above that (prefill).  The direct kernel is the fallback for shapes none of them takes.
+// (decode), group kernel above that (prefill) and where the streaming kernel does not take so many rows.  The direct kernel is the fallback for shapes none of them takes.
 Path choose_path(int top_k, int M, int K, int N, int E, int sorted_num, int block_m)
 {
     const bool s_ok = stream_supported(top_k, M, K, N, E, sorted_num, block_m);

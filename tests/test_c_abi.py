@@ -202,3 +202,25 @@ def test_group_kernel_slab_fits_its_scale_table(lib):
     finally:
         lib.alpha_moe_set_tunable(b"ALPHA_MOE_TILE_GPS", 0, 0)
     assert seen == {(4, True), (6, True), (6, False), (8, False)}
+
+
+def test_small_row_blocks_beyond_the_streaming_kernel_take_the_group_kernel(lib):
+    """Row blocks of at most 32 rows whose fp32 result rows are more than 1 GiB, or with more than 64 experts to a token, are not the
+    streaming kernel's: the group kernel has them (and their scratch holds its bf16 rows) up to eight slices of the intermediate.
+    One row less, and the call and its scratch are the streaming kernel's."""
+    lib.alpha_moe_group_plan.restype = ctypes.c_int
+    lib.alpha_moe_group_plan.argtypes = [ctypes.c_int] * 8 + [ctypes.POINTER(ctypes.c_int)]
+    plan = (ctypes.c_int * 4)()
+
+    def grouped(top_k, M, K, N, E, bm):
+        return lib.alpha_moe_group_plan(top_k, M, K, N, E, M * top_k + E * (bm - 1), bm, 2, plan) == 0
+
+    def need(top_k, M, K, N, E, bm):
+        return lib.alpha_moe_workspace_bytes(top_k, M, K, N, E, M * top_k + E * (bm - 1), bm)
+    for bm in (8, 16, 24, 32):
+        assert not grouped(9, 4161, 7168, 512, 257, bm) and grouped(9, 4162, 7168, 512, 257, bm)
+        assert need(9, 4161, 7168, 512, 257, bm) > 4161 * 9 * 7168 * 4 > need(9, 4162, 7168, 512, 257, bm) > 4162 * 9 * 7168 * 2
+        assert not grouped(64, 40, 256, 256, 80, bm) and grouped(65, 40, 256, 256, 80, bm)
+        assert grouped(9, 5000, 7168, 256 * 8, 16, bm) and not grouped(9, 5000, 7168, 256 * 9, 16, bm)
+        assert not grouped(9, 5000, 128 * 128, 256 * 5, 16, bm) and grouped(9, 5000, 128 * 128, 256 * 4, 16, bm)
+    assert grouped(9, 64, 7168, 512, 257, 40)

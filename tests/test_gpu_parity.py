@@ -1108,6 +1108,28 @@ def _run_prepacked(P, packed, knobs, store=False, via="c_abi", out=None):
     return out
 
 
+@pytest.mark.parametrize("block_m", [8, 16, 32])
+def test_small_row_blocks_beyond_the_streaming_kernel(ds_weights, block_m):
+    """Too many fp32 rows for the streaming kernel (M * top_k * K * 4 bytes above 1 GiB), or more than 64 experts to a token: small row
+    blocks take the group kernel, on either weight layout, and give its bits."""
+    from alpha_moe_python.utils import prepack_weights
+    knobs = (block_m, 32, 8, 2)
+    P = make_problem(ds_weights, 4200, seed=block_m)
+    print(f"case ds M=4200 knobs {knobs}", flush=True)
+    got = run_op(P, *knobs, via="c_abi")
+    print("worst row", worst_row_error(P, got, n=48), flush=True)
+    assert torch.equal(got, run_op(P, 64, 64, 4, 3, via="c_abi"))
+    packed = prepack_weights(ds_weights.w1, ds_weights.w2)
+    assert torch.equal(got, _run_prepacked(P, packed, knobs))
+    for M in (20, 150):
+        shape = Shape("k65", E=70, top_k=65, K=384, I=256, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
+        Q = make_problem(make_weights(shape, device=DEV, seed=5), M, seed=5)
+        print(f"case top_k 65 M={M} knobs {knobs}", flush=True)
+        got = run_op(Q, *knobs, via="c_abi")
+        assert_parity_rows(got, oracle_variants(Q), f"top_k 65 M={M} {knobs}")
+        assert torch.equal(got, run_op(Q, 64, 64, 4, 3, via="c_abi"))
+
+
 def test_prepacked_weights_give_the_same_bits(c1, ds_weights, q3_weights, decode_path):
     """fused_moe_w8a8_up_down_prepacked on prepack_weights(w, w2) against the operator on w, w2: bit for bit, streaming
     and tile kernels, adding and storing, torch op and C ABI - on the CPU-sized case, the DeepSeek-V3 shard at M=256 and
