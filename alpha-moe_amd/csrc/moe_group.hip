@@ -311,7 +311,7 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
         lds_barrier();
         const int n_tiles = tiles_of();
         if (n_tiles > 0) {
-            const __amdgpu_buffer_rsrc_t xbuf = agent_buffer(p.x), xsbuf = agent_buffer(p.x_scale);
+            const __amdgpu_buffer_rsrc_t xsbuf = agent_buffer(p.x_scale);
             const bool xs_chunk = s.xs_chunk != 0;
             v4f acc[4][NT];
 #pragma unroll
@@ -342,9 +342,12 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
                         }
                     }
                 };
+                // (A step's columns are in the base and not in an offset: with 2^32 bytes of activations, the most there can be, the
+                // last row's last bytes would be past what a buffer's 32-bit size covers.)
                 auto issue_x = [&](int k, int stage) {
+                    const __amdgpu_buffer_rsrc_t xbuf = agent_buffer(p.x + 128u * (unsigned)k);
 #pragma unroll
-                    for (int j = 0; j < DM; j++) dma16<0>(xbuf, x_off[j], 128u * k, ring + stage * (T * 2048) + w * (DM * 1024) + j * 1024);
+                    for (int j = 0; j < DM; j++) dma16<0>(xbuf, x_off[j], 0u, ring + stage * (T * 2048) + w * (DM * 1024) + j * 1024);
                 };
                 const int row_stride = xs_chunk ? 64 : 16;
                 // A step's loads are issued in this order: the scales and - with two stages - the token tiles of the step that is

@@ -5,7 +5,7 @@ Bar (written out in gpu_util.py): max |err| / max |ref| <= 1e-2 and cosine >= 0.
 import pytest
 import torch
 
-from alpha_moe_python.workloads import SHAPES, Shape, make_problem, make_weights
+from alpha_moe_python.workloads import SHAPES, Problem, Shape, make_problem, make_weights
 from gpu_util import (assert_parity, assert_parity_rows, oracle_out, oracle_variants, run_op, sampled_tokens_match_oracle,
                       tunables, worst_row_error)
 
@@ -139,6 +139,26 @@ def test_most_slices_an_expert_can_have(K, slices):
     for knobs in ((64, 32, 8, 2), (96, 32, 8, 5), (128, 64, 4, 1)):
         print(f"case {slices} slices K={K} knobs {knobs}", flush=True)
         assert_parity(run_op(P, *knobs, via="c_abi"), ref, f"{slices} slices {knobs}")
+
+
+def test_activations_of_four_gibibytes():
+    """M = 262144 rows of K = 16384: as many slots, K blocks and activation bytes (2^32) as the group kernel takes.  The rows are 64 rows
+    over and over, with large values in the last columns, so that every output row has its own in a call on the 64 rows."""
+    M, n, K = 1 << 18, 64, 1 << 14
+    shape = Shape("x4g", E=1, top_k=1, K=K, I=128, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
+    P = make_problem(make_weights(shape, device=DEV, seed=3), n, seed=3)
+    P.x[:, -4:] = 448.0
+    with tunables(ALPHA_MOE_GROUP_PIECES=1):   # no parts of the contraction: none in the large call either
+        few = run_op(P, 128, 64, 4, 2, via="c_abi")
+    assert_parity(few, oracle_out(P), "64 rows")
+    again = M // n
+    Q = Problem(P.weights, M, P.x.view(torch.uint8).repeat(again, 1).view(P.x.dtype), P.x_scale.repeat(again, 1),
+                P.topk_ids.repeat(again, 1), P.topk_weights.repeat(again, 1))
+    Q.aligned[128] = (torch.arange(M, dtype=torch.int32, device=DEV), torch.zeros(M // 128, dtype=torch.int32, device=DEV),
+                      torch.tensor([M], dtype=torch.int32, device=DEV))
+    print("case x of 4 GiB", flush=True)
+    got = run_op(Q, 128, 64, 4, 2, via="c_abi", store=True).view(again, n, K)
+    assert all(torch.equal(got[i], few) for i in (*range(0, again, 97), again - 2, again - 1))
 
 
 def test_prefill_kernels_fetch_activation_scales_both_ways():
