@@ -110,38 +110,21 @@ __device__ __forceinline__ void read_weights(v8i (&a)[4], const uint8_t *const (
     wait_lds_reads();
 }
 
-// Operand reads of the multiply loop, written as instructions the compiler knows nothing about and waited for by count: it
-// would wait for ALL outstanding LDS reads before a tile's first matrix instruction, the next tile's (just issued) included.
-// LDS reads complete in order, so "at most the three reads just issued are outstanding" is what a tile needs.
-template <int OFF>
-__device__ __forceinline__ v4i lds_read16_raw(unsigned addr)
-{
-    v4i v;
-    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF));
-    return v;
-}
-__device__ __forceinline__ float lds_read4_raw(unsigned addr)
-{
-    float v;
-    asm volatile("ds_read_b32 %0, %1" : "=v"(v) : "v"(addr));
-    return v;
-}
-template <int N>
-__device__ __forceinline__ void lds_landed_but(v4i &lo, v4i &hi, float &f)
-{
-    asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(lo), "+v"(hi), "+v"(f) : "n"(N));
-}
+typedef const v4i __attribute__((address_space(3))) * lds_v4i;
+typedef const float __attribute__((address_space(3))) * lds_f32;
 
 // 4 weight tiles in registers x T token tiles in LDS: acc[k][t] += (a_k x b_t) * f_t * (k odd ? sc1 : sc0).  A product is scaled
-// into its accumulator two matrix instructions after its own, so no wait states stand between the two.
+// into its accumulator two matrix instructions after its own, so no wait states stand between the two.  A tile's operands are read while
+// the tile before it is multiplied; LDS reads complete in order and the compiler waits for them by count, so none waits for reads
+// behind its own - as long as they keep this order, which the scheduling barriers are for.
 template <int T, int NT>
 __device__ __forceinline__ void multiply(const v8i (&a)[4], const uint8_t *b_tiles, const float *row, int row_stride, float sc0,
                                          float sc1, v4f (&acc)[4][NT], int frag_lo, int frag_hi)
 {
-    const unsigned a_lo = (uint32_t)(uintptr_t)b_tiles + (unsigned)frag_lo, a_hi = (uint32_t)(uintptr_t)b_tiles + (unsigned)frag_hi;
-    const unsigned a_f = (uint32_t)(uintptr_t)row, f_stride = 4u * (unsigned)row_stride;
-    v4i b_lo = lds_read16_raw<0>(a_lo), b_hi = lds_read16_raw<0>(a_hi);
-    float f = lds_read4_raw(a_f);
+    const lds_v4i at_lo = (lds_v4i)(uint32_t)(uintptr_t)(b_tiles + frag_lo), at_hi = (lds_v4i)(uint32_t)(uintptr_t)(b_tiles + frag_hi);
+    const lds_f32 at_f = (lds_f32)(uint32_t)(uintptr_t)row;
+    v4i b_lo = *at_lo, b_hi = *at_hi;
+    float f = *at_f;
     v4f prod[2];
     float fac[2];
     auto tile = [&](auto tc) {
@@ -149,13 +132,11 @@ __device__ __forceinline__ void multiply(const v8i (&a)[4], const uint8_t *b_til
         v4i n_lo = b_lo, n_hi = b_hi;
         float n_f = f;
         if constexpr (t + 1 < T) {
-            n_lo = lds_read16_raw<(t + 1) * 2048>(a_lo);
-            n_hi = lds_read16_raw<(t + 1) * 2048>(a_hi);
-            n_f = lds_read4_raw(a_f + (unsigned)(t + 1) * f_stride);
-            lds_landed_but<3>(b_lo, b_hi, f);
-        } else {
-            lds_landed_but<0>(b_lo, b_hi, f);
+            n_lo = at_lo[(t + 1) * 128];
+            n_hi = at_hi[(t + 1) * 128];
+            n_f = at_f[(t + 1) * row_stride];
         }
+        __builtin_amdgcn_sched_barrier(0);
         const v8i b = cat(b_lo, b_hi);
         const float p0 = f * sc0, p1 = f * sc1;
         __builtin_amdgcn_sched_barrier(0);

@@ -224,3 +224,13 @@ def test_small_row_blocks_beyond_the_streaming_kernel_take_the_group_kernel(lib)
         assert grouped(9, 5000, 7168, 256 * 8, 16, bm) and not grouped(9, 5000, 7168, 256 * 9, 16, bm)
         assert not grouped(9, 5000, 128 * 128, 256 * 5, 16, bm) and grouped(9, 5000, 128 * 128, 256 * 4, 16, bm)
     assert grouped(9, 64, 7168, 512, 257, 40)
+
+
+def test_no_kernel_loads_in_inline_assembly():
+    """The compiler takes the output register of inline assembly as written when the instruction is issued: it may copy or reuse it
+    while a load is still on its way.  Loads are the compiler's own."""
+    csrc = os.path.join(ROOT, "alpha-moe_amd", "csrc")
+    load = re.compile(r'asm\b[^;]*?"[^"]*\b(ds_read|ds_load|global_load|buffer_load|flat_load|scratch_load|s_load|s_buffer_load)', re.S)
+    for name in sorted(os.listdir(csrc)):
+        text = open(os.path.join(csrc, name)).read()
+        assert not load.search(text), (name, load.search(text).group(0))
