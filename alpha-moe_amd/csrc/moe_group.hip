@@ -325,8 +325,9 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
                 };
                 // (A step's columns are in the base and not in an offset: with 2^32 bytes of activations, the most there can be, the
                 // last row's last bytes would be past what a buffer's 32-bit size covers.)
-                auto issue_x = [&](int k, int stage) {
-                    const __amdgpu_buffer_rsrc_t xbuf = agent_buffer(p.x + 128u * (unsigned)k);
+                const uint8_t *x_next = p.x + (size_t)(k0 * 128);   // columns of the next step to be asked for
+                auto issue_x = [&](int stage) {
+                    const __amdgpu_buffer_rsrc_t xbuf = agent_buffer(x_next);
 #pragma unroll
                     for (int j = 0; j < DM; j++) dma16<0>(xbuf, x_off[j], 0u, ring + stage * (T * 2048) + w * (DM * 1024) + j * 1024);
                 };
@@ -337,12 +338,16 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
                 // step what was issued behind its own last weight tile may still be on its way.
                 constexpr int BEHIND = 2 * (R - 4) + (S == 3 ? DM : 0);
                 issue_xs(k0);
-                issue_x(k0, 0);
+                issue_x(0);
+                x_next += 128;
                 if (k0 + 1 < k1) {
                     if (S == 3) issue_xs(k0 + 1);
 #pragma unroll
                     for (int g = 4; g < R; g++) issue_w(g, k0 + 1, g & 3, ntc_aux);
-                    if (S == 3) issue_x(k0 + 1, 1);
+                    if (S == 3) {
+                        issue_x(1);
+                        x_next += 128;
+                    }
                 }
                 int first = 0, stage = 0;   // the step's first weight tile, and its token tiles, in their rings
                 for (int k = k0; k < k1; k++) {
@@ -369,14 +374,14 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
                         if (k + 1 < k1) {
 #pragma unroll
                             for (int j = 0; j < 8; j++) issue_rows(k + 1, j, ntc_aux);
-                            issue_x(k + 1, ahead);
+                            issue_x(ahead);
                         }
                     } else if (k + 1 < k1) {
-                        if (S == 2) issue_x(k + 1, ahead);
+                        if (S == 2) issue_x(ahead);
 #pragma unroll
                         for (int i = 0; i < 8 - R; i++) issue_w(place[i], k + 1, (R + i) & 3, ntc_aux);
                     }
-                    if (S == 3 && k + 2 < k1) issue_x(k + 2, ahead);
+                    if (S == 3 && k + 2 < k1) issue_x(ahead);
                     if (R > 4 && k + 2 < k1) {
 #pragma unroll
                         for (int i = 8 - R; i < 4; i++) issue_w(place[i], k + 2, (R + i) & 3, ntc_aux);
@@ -384,6 +389,7 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
                     const float *row = xs_chunk ? &tab.up.xc[(((k >> 2) & 1) * NT * 16 + n) * 4 + (k & 3)]
                                                 : &tab.up.xc[(k & 3) * NT * 16 + n];
                     multiply<T>(a, ring + stage * (T * 2048), row, row_stride, sc0, sc1, acc, frag_lo, frag_hi);
+                    x_next += 128;
                     stage = stage + 1 < S ? stage + 1 : 0;
                 }
             });
