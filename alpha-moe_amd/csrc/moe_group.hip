@@ -44,7 +44,9 @@ namespace {
 // Dynamic LDS: a ring of weight tiles for each wavefront and, behind them, a ring of the steps' token tiles.  Where K is short, what
 // token tiles a row block does not have is room for more of both in flight (Qwen3-30B shard, 128-row blocks of which most have
 // one to four tiles: M = 512 147 -> 144 us, 1024 165 -> 159.5; Qwen3-Next M = 1500 186 -> 184).  Where K is long, a few-row block that
-// runs ahead takes its neighbours' lines out of L2: DeepSeek shard M = 2048 408 -> 412 us, 8192 939 -> 955.
+// runs ahead takes its neighbours' lines out of L2: DeepSeek shard M = 2048 408 -> 412 us, 8192 939 -> 955.  Between the two (128 experts,
+// six to a token, I = 512, 128-row blocks, us without -> with, M = 250 / 1000 / 6000): K = 3072 108 -> 106, 125 -> 126, 331 -> 327;
+// K = 4096 176 -> 166, 196 -> 191, 420 -> 423; K = 5120 174 -> 170, 201 -> 198, 526 -> 534; K = 6144 205 -> 203, 232 -> 231, 610 -> 616.
 constexpr int dyn_lds(int nt) { return nt <= 4 ? 48 * 1024 : 72 * 1024; }   // three workgroups to a compute unit, or two
 constexpr int x_stages(int nt, int t, bool deep)   // K steps of token tiles
 {
@@ -63,7 +65,8 @@ constexpr int kGMaxKb = 128;               // most 128-byte K blocks (K <= 16384
 constexpr int kGChunk = 8;                 // consecutive row blocks of a queue
 constexpr int kGHeadStride = 128;          // words between the queues' counters (lines of their own); behind one: the queue's arrivals
 constexpr int kGMaxRound = 96;             // most workgroups of a queue counted as running at a time
-constexpr int kGLongKb = 32;               // K blocks from which on K counts as long
+constexpr int kGDeepKb = 32;               // most K blocks with deep rings
+constexpr int kGPiecesKb = 32;             // fewest K blocks whose contraction may be taken in parts
 constexpr int kGResidentIb = 2;            // slices whose requantised tiles fit the token ring for a whole DOWN item
 
 struct GroupParams {
@@ -230,7 +233,7 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
         return rfl((last >> 4) + 1);   // 0 when no row is valid
     };
     // run(T, non-temporal, deep rings) with the smallest even T that holds the live tiles
-    const bool short_k = nkb < kGLongKb;
+    const bool short_k = nkb <= kGDeepKb;
     auto pick = [&](int n_tiles, bool nt, auto run) {
         auto sized = [&](auto ntc) {
             auto few = [&](auto tc) {
@@ -680,12 +683,12 @@ __global__ __launch_bounds__(256, NT <= 4 ? 3 : 2) void moe_group_kernel(const G
     const int rest = left - chunk * q_id;
     const int nb = whole_chunks * kGChunk + (rest < 0 ? 0 : rest < chunk ? rest : chunk);
     const int ups = nb * n_ib;
-    // Where one round of workgroups holds all UP items and K is long, each is taken in two parts: with a long item to two of a
-    // compute unit's three workgroups the loads in flight do not cover the memory's latency, and it is over when the slowest compute
-    // unit is (DeepSeek shard, 64-row blocks, whole -> two parts: M = 513 319 -> 308 us, 700 331 -> 316, 1024 353 -> 340, 1400 382 ->
-    // 369; three parts 317, 329, 349, 377).  Beyond one round the last one is left whole: parts of it cost more than they level
-    // (M = 2048 401 -> 411 us, 2500 430 -> 444).
-    const int pieces = ups < s.round && nkb >= kGLongKb ? s.max_pieces : 1;
+    // Where half a round of workgroups holds all UP items and K is long, each is taken in two parts, so that more loads are in flight.
+    // MI355X, 64-row blocks, by UP items of a queue's 96 workgroups, us whole -> two parts: K = 7168 47 items 196 -> 175, 66 271 -> 278,
+    // 68 304 -> 314; K = 6144 10 items 99 -> 73, 23 92 -> 85; K = 4096 24 items 87 -> 77, 33 110 -> 113.  More parts change nothing (three
+    // to eight at K = 6144, 10 items: 72 - 73).  Shorter K loses as often as it gains: K = 3072 74 -> 67 and, with 128-row blocks,
+    // 83 -> 92; K = 2560 65 -> 64 and 60 -> 70.
+    const int pieces = nkb >= kGPiecesKb && ups * s.max_pieces <= s.round ? s.max_pieces : 1;
     const int up_items = ups * pieces;
     const bool is_up = item < up_items;
     const int unit_id = item / pieces, piece = item - unit_id * pieces;
