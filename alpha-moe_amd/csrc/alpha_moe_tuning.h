@@ -3,7 +3,7 @@
  * (include/alpha_moe_hip.h) and free to change between versions.
  *
  * alpha_moe_set_tunable installs (set != 0) or clears (set == 0) a tuning override.  `name` is one of
- * ALPHA_MOE_PATH (1 direct, 2 stream, 3 or 4 group, 5 small), ALPHA_MOE_STRICT_QUEUE, ALPHA_MOE_KBPI, ALPHA_MOE_TPI,
+ * ALPHA_MOE_PATH (1 direct, 2 stream, 3 or 4 group, 5 small, each where it takes the call), ALPHA_MOE_STRICT_QUEUE, ALPHA_MOE_KBPI, ALPHA_MOE_TPI,
  * ALPHA_MOE_LAG, ALPHA_MOE_GRID, ALPHA_MOE_TILE_GPS, ALPHA_MOE_TILE_NT, ALPHA_MOE_GROUP_PIECES; ALPHA_MOE_TILE_LAG,
  * ALPHA_MOE_TILE_GRID and ALPHA_MOE_WIDE_PP belonged to kernels that are gone: accepted, without effect.
  * The environment variables of the same names are read once, when the library is first used; no launch reads the

@@ -19,10 +19,11 @@ TunableSlot g_tunables[kTunCount] = {
     {"ALPHA_MOE_PATH", kTunableUnset},        {"ALPHA_MOE_STRICT_QUEUE", kTunableUnset},
     {"ALPHA_MOE_KBPI", kTunableUnset},        {"ALPHA_MOE_TPI", kTunableUnset},
     {"ALPHA_MOE_LAG", kTunableUnset},         {"ALPHA_MOE_GRID", kTunableUnset},
-    {"ALPHA_MOE_TILE_GPS", kTunableUnset},    {"ALPHA_MOE_TILE_LAG", kTunableUnset},
-    {"ALPHA_MOE_TILE_GRID", kTunableUnset},   {"ALPHA_MOE_TILE_NT", kTunableUnset},
-    {"ALPHA_MOE_WIDE_PP", kTunableUnset},     {"ALPHA_MOE_GROUP_PIECES", kTunableUnset},
+    {"ALPHA_MOE_TILE_GPS", kTunableUnset},    {"ALPHA_MOE_TILE_NT", kTunableUnset},
+    {"ALPHA_MOE_GROUP_PIECES", kTunableUnset},
 };
+// of kernels that are gone: still taken, without effect
+const char *const kRetired[] = {"ALPHA_MOE_TILE_LAG", "ALPHA_MOE_TILE_GRID", "ALPHA_MOE_WIDE_PP"};
 
 void load_tunables_once()
 {
@@ -31,7 +32,7 @@ void load_tunables_once()
             const char *e = getenv(t.name);
             if (!e) continue;
             if (!strcmp(t.name, "ALPHA_MOE_PATH"))
-                t.value = !strcmp(e, "direct") ? 1 : !strcmp(e, "stream") ? 2 : !strcmp(e, "group") ? 3 : !strcmp(e, "small") ? 5 : kTunableUnset;
+                t.value = !strcmp(e, "direct") ? 1 : !strcmp(e, "stream") ? 2 : !strcmp(e, "group") || !strcmp(e, "tile") || !strcmp(e, "wide") ? 3 : !strcmp(e, "small") ? 5 : kTunableUnset;
             else
                 t.value = atoi(e);
         }
@@ -50,11 +51,12 @@ Path choose_path(int top_k, int M, int K, int N, int E, int sorted_num, int bloc
     const int f = tunable(kTunPath, 0);
     if (f == 1) return kDirect;
     if (f == 2 && s_ok) return kStream;
+    const bool g_ok = group_supported(top_k, M, K, N, E, sorted_num, block_m);
+    if ((f == 3 || f == 4) && g_ok) return kGroup;   // (two kernels once)
     const bool small_ok = small_supported(top_k, M, K, N, block_m);
     if (small_ok && (f == 5 || (f == 0 && (!s_ok || small_pays(top_k, M, K, N, E))))) return kSmall;
     if (s_ok) return kStream;
-    if (group_supported(top_k, M, K, N, E, sorted_num, block_m)) return kGroup;
-    return kDirect;
+    return g_ok ? kGroup : kDirect;
 }
 
 }  // namespace
@@ -75,6 +77,8 @@ extern "C" int alpha_moe_set_tunable(const char *name, int value, int set)
             t.value = set ? value : kTunableUnset;
             return ALPHA_MOE_OK;
         }
+    for (const char *n : kRetired)
+        if (!strcmp(name, n)) return ALPHA_MOE_OK;
     return ALPHA_MOE_ERR_SHAPE;
 }
 

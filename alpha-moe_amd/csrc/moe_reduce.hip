@@ -7,9 +7,11 @@ namespace {
 // out[t] = bf16(out[t] + sum over the token's live slots of y[slot]).
 // Row is the type of y: bf16 (prefill kernels) or fp32 (streaming kernel).  A thread loads 16 bytes of each row - 8 or 4
 // columns -, a workgroup covers 256 threads' columns of one token, and all rows of a token with up to 12 slots are in flight
-// at once.  Bound by HBM: the rows are read once.  Nothing else is waited for: the launch epoch was closed by the
-// kernel that wrote the rows.  (The last of this kernel's workgroups used to close it: arrivals at one counter are served
-// one by one, ~10 ns each, so 4096 workgroups took 41 us whatever they had to read.)
+// at once.  Bound by HBM: the rows are read once.  Nothing else is waited for.  Behind the streaming kernel, which closed the launch
+// epoch itself, that is all.  Behind the group kernel this launch ends the call: workgroup 0 sets the eight ticket counters back and
+// closes the epoch, so it has to follow every launch of that kernel on the workspace - the next one would find its queues
+// drawn empty.  (The last of this kernel's workgroups used to close it: arrivals at one counter are served one by one, ~10 ns each, so 4096
+// workgroups took 41 us whatever they had to read.)
 // MI355X, kernel trace, before and after: Qwen3-Next M=4096 60 -> 38 us, Qwen3-30B M=1024 18 -> 9.7 and M=8192 78 -> 46,
 // DeepSeek shard M=2048 76 -> 61 and M=8192 204 -> 198 (1.18 GB, 6.0 TB/s).  Workgroups that stride over tokens are slower
 // (M=8192 with 1024 of them: 220 us).

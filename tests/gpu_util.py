@@ -86,7 +86,7 @@ def assert_parity_rows(out, refs, what=""):
 
 @contextlib.contextmanager
 def tunables(**values):
-    """Tuning overrides of the library for the duration of a with-block: tunables(ALPHA_MOE_TILE_GRID=8)."""
+    """Tuning overrides of the library for the duration of a with-block: tunables(ALPHA_MOE_TILE_GPS=8)."""
     import alpha_moe
     for name, value in values.items():
         alpha_moe.set_tunable(name, value)

@@ -234,3 +234,16 @@ def test_no_kernel_loads_in_inline_assembly():
     for name in sorted(os.listdir(csrc)):
         text = open(os.path.join(csrc, name)).read()
         assert not load.search(text), (name, load.search(text).group(0))
+
+
+def test_kernel_choice_by_the_names_of_kernels_that_are_gone():
+    """ALPHA_MOE_PATH=tile and =wide chose kernels whose successor is the group kernel: like =group they keep the small kernels out of the
+    way, and their tunables are taken without effect."""
+    import subprocess
+    import sys
+    code = ("import ctypes, sys; L = ctypes.CDLL(sys.argv[1]); "
+            "print(L.alpha_moe_layer_call_supported(2, 4, 2048, 512, 8, 16, 32, 8, 4), "
+            "[L.alpha_moe_set_tunable(n, 1, 1) for n in (b'ALPHA_MOE_TILE_LAG', b'ALPHA_MOE_TILE_GRID', b'ALPHA_MOE_WIDE_PP', b'ALPHA_MOE_X')])")
+    for path, layer in (("", 1), ("group", 0), ("tile", 0), ("wide", 0), ("small", 1)):
+        out = subprocess.run([sys.executable, "-c", code, LIB], env=dict(os.environ, ALPHA_MOE_PATH=path), capture_output=True, text=True)
+        assert out.stdout.strip() == f"{layer} [0, 0, 0, 2]", (path, out.stdout, out.stderr)
