@@ -1,6 +1,7 @@
 """Shared helpers of the GPU parity tests: run the operator (through torch.ops or straight through the C ABI)
 and the CPU oracle on the same bits."""
 import contextlib
+import itertools
 
 import torch
 
@@ -82,6 +83,35 @@ def assert_parity_rows(out, refs, what=""):
     m = O.error_metrics(out, refs[0])
     assert float(per_row.max()) <= MAX_ABS_OVER_MAX_REF and m["cosine"] >= MIN_COSINE, (what, float(per_row.max()), m)
     return float(per_row.max())
+
+
+def rows_within_rounding_noise(P, token):
+    """What one token's row (top_k = 1) may be.  The up/gate sums in float64; those closer to a bf16 rounding boundary than the noise of
+    their fp32 accumulation (3e-7 of the sum of the terms' magnitudes: K / 128 additions, each 2^-25 of it off on average over
+    signs; the eight closest at most) rounded either way, and the scale of every slice as it is, or taken from the next bf16 value below or
+    above its largest activation, which may lie on a boundary itself."""
+    W, e = P.weights, int(P.topk_ids[token, 0])
+    I = P.shape.I
+    w1 = O.deinterleave_reference(W.w1[e:e + 1].cpu().view(torch.uint8), 8)[0].view(torch.float8_e4m3fn).double()
+    w1 *= O._expand_block_scale(O.deinterleave_reference(W.w1_scale[e:e + 1].cpu(), 1)[0], *w1.shape)
+    x = P.x[token].cpu().double() * P.x_scale[token].cpu().double().repeat_interleave(128)
+    sums, noise = w1 @ x, 3e-7 * (w1.abs() @ x.abs())
+    ulp = torch.exp2(torch.floor(torch.log2(sums.abs())) - 7)
+    below = torch.floor(sums / ulp) * ulp
+    margin = ((sums - below - 0.5 * ulp).abs() / noise).sort()
+    near = margin.indices[margin.values < 1.0][:8].tolist()
+    w2 = W.w2[e].cpu().float() * O._expand_block_scale(W.w2_scale[e].cpu(), P.shape.K, I)
+    rows = []
+    for up in itertools.product((False, True), repeat=len(near)):
+        h = sums.float().bfloat16().float()
+        for i, u in zip(near, up):
+            h[i] = below[i] + (ulp[i] if u else 0.0)
+        a = O._silu_mul(h[:I], h[I:]).bfloat16().float().reshape(I // 128, 128)
+        top = a.abs().amax(-1, keepdim=True).bfloat16().view(torch.int16)
+        for steps in itertools.product((0, -1, 1), repeat=I // 128):
+            s = (top + torch.tensor(steps, dtype=torch.int16).unsqueeze(1)).view(torch.bfloat16).float().clamp_min(O.AMAX_FLOOR) / O.FP8_MAX
+            rows.append(((a / s).clamp(-O.FP8_MAX, O.FP8_MAX).to(torch.float8_e4m3fn).float() * s).reshape(I))
+    return torch.stack(rows) @ w2.t() * (float(P.topk_weights[token, 0]) * P.shape.scaling_factor)
 
 
 @contextlib.contextmanager

@@ -6,8 +6,8 @@ import pytest
 import torch
 
 from alpha_moe_python.workloads import SHAPES, Problem, Shape, make_problem, make_weights
-from gpu_util import (assert_parity, assert_parity_rows, oracle_out, oracle_variants, run_op, sampled_tokens_match_oracle,
-                      tunables, worst_row_error)
+from gpu_util import (MAX_ABS_OVER_MAX_REF, assert_parity, assert_parity_rows, oracle_out, oracle_variants, rows_within_rounding_noise,
+                      run_op, sampled_tokens_match_oracle, tunables, worst_row_error)
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -47,7 +47,7 @@ def test_c_abi_workspace_is_reusable_without_clearing(c1, decode_path):
     for bm, bn, wn, st in [(16, 64, 4, 2), (16, 64, 4, 2), (8, 32, 8, 3), (64, 64, 4, 2), (32, 32, 8, 1), (16, 64, 4, 4)]:
         print(f"case c1 shared workspace knobs {(bm, bn, wn, st)}", flush=True)
         assert_parity(run_op(P, bm, bn, wn, st, via="c_abi", workspace=ws), ref, f"shared ws {(bm, bn, wn, st)}")
-    # a second problem of another size on the same buffer, streaming and tile kernels taking turns
+    # a second problem of another size on the same buffer, streaming and group kernels taking turns
     P2 = make_problem(P.weights, 150, seed=9)
     need = max(alpha_moe.c_abi.alpha_moe_workspace_bytes(P2.shape.top_k, P2.M, P2.shape.K, P2.shape.N, P2.shape.E,
                                                          P2.align(bm)[0].numel(), bm) for bm in (16, 64, 128))
@@ -89,7 +89,7 @@ def test_add_semantics_scaling_and_zero_weights(c1, decode_path):
 @pytest.mark.parametrize("knobs", [(16, 32, 8, 2), (16, 64, 4, 5), (64, 64, 4, 3), (128, 64, 4, 3)])
 def test_store_variant_overwrites_whatever_out_held(c1, knobs, decode_path):
     """fused_moe_w8a8_up_down_store: out = bf16(sum) on every element, NaN-filled or not, and bit for bit what the
-    adding call leaves in a zero-filled out - streaming and tile kernels, torch op and C ABI."""
+    adding call leaves in a zero-filled out - streaming and group kernels, torch op and C ABI."""
     P, ref = c1
     zero = run_op(P, *knobs, via="c_abi")
     assert_parity(zero, ref, f"knobs {knobs}")
@@ -106,8 +106,7 @@ def test_store_variant_overwrites_whatever_out_held(c1, knobs, decode_path):
 
 
 def test_nine_slices_row_blocks_above_32():
-    """Nine 128-column slices are more than the tile kernel takes: the wide kernel streams any number of them, whatever
-    (block_n, warp_n) asks for."""
+    """Nine 128-column slices: streamed by the DOWN items, whatever (block_n, warp_n) asks for."""
     shape = Shape("s9", E=6, top_k=2, K=256, I=1152, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
     W = make_weights(shape, device=DEV, seed=5)
     P = make_problem(W, 150, seed=5)
@@ -162,7 +161,7 @@ def test_activations_of_four_gibibytes():
 
 
 def test_prefill_kernels_fetch_activation_scales_both_ways():
-    """The tile and wide kernels take a token's activation scales four K blocks at a time where the row of scales allows
+    """The group kernel takes a token's activation scales four K blocks at a time where the row of scales allows
     16-byte loads (K / 128 a multiple of 4, x_scale 16-byte aligned) and one at a time otherwise: both ways against the
     oracle, and bit for bit against each other on the same problem."""
     for K in (384, 512, 640, 1024):
@@ -186,36 +185,29 @@ def test_prefill_kernels_fetch_activation_scales_both_ways():
             assert torch.equal(a, b), (K, knobs)
 
 
-def test_wide_kernel_up_loop_variants_give_the_same_bits():
-    """The wide kernel has two forms of its up/gate loop: both wavefronts of a SIMD in step, or half a step apart (one
-    multiplies a whole step alone, token tiles in blocks of four from the top down with a queue of pending products
-    that lives across steps, while the other loads).  ALPHA_MOE_WIDE_PP picks one (unset: by rows per expert).  Both
-    against the oracle and bit for bit against each other, over: one to sixteen live token tiles in a block and blocks
-    whose second wavefront of a pair has none; one, two, three, four and eight K steps (the loop's prologue issues
-    two steps of loads; activation scales are fetched four steps at a time from K = 512 on and singly otherwise, also
-    from a row of scales that is not 16-byte aligned); experts with one block of rows and with several."""
+def test_up_loop_of_a_few_steps():
+    """The up/gate loop over one, two, three, four, five and eight K steps (its prologue issues up to two steps of loads; activation scales
+    are fetched four steps at a time where K / 128 is a multiple of 4 and singly otherwise, also from a row of scales that is not
+    16-byte aligned), with experts of one block of rows and of several: against the oracle, and the same bits for two block sizes."""
     for K, M in ((128, 150), (256, 300), (384, 40), (512, 700), (1024, 300), (512, 9), (640, 150)):
         shape = Shape("pp", E=6, top_k=4, K=K, I=256, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
         W = make_weights(shape, device=DEV, seed=K + M)
         P = make_problem(W, M, seed=K + M)
         ref = oracle_out(P)
+        outs = []
         for knobs in ((128, 32, 8, 2), (48, 32, 8, 1)):
-            outs = []
-            for pp in (0, 1):
-                print(f"case up loop K={K} M={M} knobs {knobs} ALPHA_MOE_WIDE_PP={pp}", flush=True)
-                with tunables(ALPHA_MOE_WIDE_PP=pp):
-                    outs.append(run_op(P, *knobs, via="c_abi"))
-                assert_parity(outs[-1], ref, f"K={K} M={M} {knobs} pp={pp}")
-            assert torch.equal(outs[0], outs[1]), (K, M, knobs)
+            print(f"case up loop K={K} M={M} knobs {knobs}", flush=True)
+            outs.append(run_op(P, *knobs, via="c_abi"))
+            assert_parity(outs[-1], ref, f"K={K} M={M} {knobs}")
             if K == 512 and M == 700:
                 aligned = P.x_scale
                 raw = torch.empty(aligned.numel() + 1, dtype=torch.float32, device=DEV)
                 raw[1:].copy_(aligned.flatten())
                 P.x_scale = raw[1:].view_as(aligned)
-                with tunables(ALPHA_MOE_WIDE_PP=1):
-                    b = run_op(P, *knobs, via="c_abi")
+                b = run_op(P, *knobs, via="c_abi")
                 P.x_scale = aligned
-                assert torch.equal(outs[0], b), (K, M, knobs, "unaligned scales")
+                assert torch.equal(outs[-1], b), (K, M, knobs, "unaligned scales")
+        assert torch.equal(outs[0], outs[1]), (K, M)
 
 
 @pytest.mark.parametrize("block_m", [40, 64, 72, 96, 104, 128])
@@ -234,14 +226,19 @@ def test_group_kernel_at_the_edges_of_its_tiles(block_m, K, I):
     refs = oracle_variants(P)
 
     def check(out, what):
-        """With one expert to a token nothing averages out what a row's scale does: where the slice's largest activation is within
-        rounding noise of a bf16 boundary (of gate, up or their product), the scale moves by 2^-8 and about one code in sixteen - 8 or
-        so of 128 - by its spacing, 2^-3.5 of its value: sqrt(8) * 0.09 / sqrt(128) = 2.2 % of the row's root mean square, four times
-        that in the largest of K columns, where the output's largest value is five times it: 1.8e-2.  Such rows are few."""
+        """Every row within the bar of the oracle or one of its neighbours.  With one expert to a token nothing averages out what one
+        sum on a rounding boundary does - a large activation's FP8 code one further, or the scale of all 128 -, and several of a row
+        may fall each its own way, where no common nudge of the sums reaches them: such a row, one of a problem at most, has
+        to be within the bar of one of the rows that the rounding of its own sums allows."""
         o = out.float().cpu()
         scale = refs[0].float().abs().max()
         per_row = torch.stack([(o - r.float()).abs().amax(dim=1) for r in refs]).amin(dim=0) / scale
-        assert float(per_row.max()) <= 1.8e-2 and int((per_row > 1e-2).sum()) <= P.M // 64, (what, per_row.topk(4))
+        far = (per_row > MAX_ABS_OVER_MAX_REF).nonzero().flatten().tolist()
+        assert len(far) <= 1, (what, per_row.topk(4))
+        for t in far:
+            nearest = float((o[t] - rows_within_rounding_noise(P, t)).abs().amax(dim=1).min() / scale)
+            print(f"{what}: row {t} {float(per_row[t]):.2e} from the oracle, {nearest:.2e} from the nearest within rounding noise", flush=True)
+            assert nearest <= MAX_ABS_OVER_MAX_REF, (what, t, float(per_row[t]), nearest)
 
     print(f"case group kernel block_m {block_m} K={K} I={I}", flush=True)
     got = run_op(P, block_m, 64, 4, 1, via="c_abi")
@@ -254,7 +251,7 @@ def test_group_kernel_at_the_edges_of_its_tiles(block_m, K, I):
 
 
 def test_store_variant_fallback_kernel():
-    """129 K blocks are more than the tile and wide kernels take: the fallback kernel serves the call, and its store
+    """129 K blocks are more than the group kernel takes: the fallback kernel serves the call, and its store
     variant overwrites too."""
     from alpha_moe_python.workloads import Shape
     shape = Shape("fb", E=6, top_k=2, K=16512, I=128, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
@@ -289,7 +286,7 @@ def test_prefill_rows_are_summed_for_any_top_k(top_k):
     P = make_problem(W, 70, seed=top_k)
     ref = oracle_out(P)
     junk = torch.full((P.M, shape.K), float("nan"), dtype=torch.bfloat16, device=DEV)
-    for knobs in ((48, 64, 4, 3), (64, 32, 8, 2)):   # tile kernel, wide kernel
+    for knobs in ((48, 64, 4, 3), (64, 32, 8, 2)):
         print(f"case rows top_k={top_k} knobs {knobs}", flush=True)
         for store in (False, True, False):           # one workspace: every call has to see its own rows as live
             out = junk.clone() if store else None
@@ -345,8 +342,8 @@ def test_deepseek_shard_decode_full_size(ds_weights, M, knobs):
 
 
 @pytest.mark.parametrize("knobs", [(48, 64, 4, 3), (64, 32, 8, 2), (128, 64, 4, 3)])
-def test_deepseek_shard_prefill_tile_kernel(ds_weights, knobs):
-    """Row blocks above 32 rows go to the tile kernel: M=256 of the DeepSeek-V3 shard against the oracle."""
+def test_deepseek_shard_prefill_group_kernel(ds_weights, knobs):
+    """Row blocks above 32 rows go to the group kernel: M=256 of the DeepSeek-V3 shard against the oracle."""
     P = make_problem(ds_weights, 256, seed=1)
     print(f"case ds M=256 knobs {knobs}", flush=True)
     m = assert_parity(run_op(P, *knobs, via="c_abi"), oracle_out(P), f"ds M=256 knobs {knobs}")
@@ -428,8 +425,8 @@ def q3_weights():
 
 @pytest.mark.parametrize("M,knobs", [(64, (16, 32, 8, 5)), (64, (32, 64, 4, 3)), (200, (64, 64, 4, 3)), (200, (128, 64, 4, 2))])
 def test_qwen3_30b_zipf_shard_against_oracle(q3_weights, M, knobs):
-    """Load imbalance: E=128, top_k=8, K=2048, I=768 (six 128-column slices), Zipf(1.2) expert popularity.  With six
-    slices a 128-row block's requantised tiles do not fit LDS at once: its DOWN items serve the tokens in two parts."""
+    """Load imbalance: E=128, top_k=8, K=2048, I=768 (six 128-column slices), Zipf(1.2) expert popularity.  Six
+    slices are more than a DOWN item of the group kernel keeps in LDS: it streams them."""
     P = make_problem(q3_weights, M, seed=0)
     print(f"case q3 M={M} knobs {knobs}", flush=True)
     m = assert_parity(run_op(P, *knobs, via="c_abi"), oracle_out(P), f"q3 M={M} knobs {knobs}")
@@ -492,12 +489,9 @@ def test_grid_fits_the_device(ds_weights, knobs):
     assert_parity(out, oracle_out(P), f"ds M=64 knobs {knobs}")
 
 
-def test_tile_kernel_result_independent_of_item_schedule():
-    """The tile kernel's work items (up/gate slices, slabs of output columns) may run on any workgroup in any order
-    that respects their flags: few workgroups (every one serves all eight queues), down items right behind their
-    up/gate items, the smallest and the largest column slabs, cached or non-temporal weight loads - the output is
-    the same bit for bit, and agrees with the oracle.  K=640 gives 10 column groups: the last slab is ragged and
-    some wavefront pairs have no group in it."""
+def test_group_kernel_result_independent_of_item_schedule():
+    """The smallest and the largest column slabs, cached or non-temporal weight loads: the output is the same bit for bit, and agrees
+    with the oracle.  K=640 gives 10 column groups: the last slab is ragged and some wavefronts have no group in it."""
     from alpha_moe_python.workloads import Shape
     shape = Shape("sched", E=12, top_k=3, K=640, I=256, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
     W = make_weights(shape, device=DEV, seed=3)
@@ -507,13 +501,32 @@ def test_tile_kernel_result_independent_of_item_schedule():
         print(f"case sched M=300 block_m {block_m} default schedule", flush=True)
         base = run_op(P, block_m, 64, 4, 3, via="c_abi")
         assert_parity(base, ref, f"sched block_m {block_m}")
-        for env in ({"ALPHA_MOE_TILE_GRID": 8}, {"ALPHA_MOE_TILE_LAG": 1}, {"ALPHA_MOE_TILE_GPS": 4},
-                    {"ALPHA_MOE_TILE_GPS": 1000}, {"ALPHA_MOE_TILE_NT": 1}, {"ALPHA_MOE_TILE_NT": 0},
-                    {"ALPHA_MOE_TILE_GRID": 16, "ALPHA_MOE_TILE_LAG": 2, "ALPHA_MOE_TILE_GPS": 8}):
+        for env in ({"ALPHA_MOE_TILE_GPS": 4}, {"ALPHA_MOE_TILE_GPS": 1000}, {"ALPHA_MOE_TILE_NT": 1}, {"ALPHA_MOE_TILE_NT": 0},
+                    {"ALPHA_MOE_TILE_NT": 1, "ALPHA_MOE_TILE_GPS": 8}):
             print(f"case sched M=300 block_m {block_m} {env}", flush=True)
             with tunables(**env):
                 got = run_op(P, block_m, 64, 4, 3, via="c_abi")
             assert torch.equal(got, base), (block_m, env)
+
+
+@pytest.mark.parametrize("blocks,I", [(1, 128), (1, 512), (7, 512), (8, 128), (9, 512), (63, 128), (64, 128), (65, 512), (72, 128), (130, 128)])
+def test_group_kernel_deals_every_block_to_a_queue(blocks, I):
+    """Row blocks around the eight queues and their chunks (whole rounds of 64 blocks, what is left in eighths), each block an expert of
+    its own: whole, in two parts and in as many as y has room for (K = 4096: eight with one slice, two with four), any slab."""
+    shape = Shape("dq", E=blocks, top_k=1, K=4096, I=I, shared_expert=False, routing="softmax_renorm", scaling_factor=1.0)
+    P = make_problem(make_weights(shape, device=DEV, seed=blocks), 2 * blocks + 1, seed=blocks)
+    P.topk_ids = (torch.arange(P.M, device=DEV) % blocks).to(torch.int32).view(-1, 1)
+    refs = oracle_variants(P)
+    with tunables(ALPHA_MOE_GROUP_PIECES=1):
+        whole = run_op(P, 64, 64, 4, 2, via="c_abi")
+    assert_parity_rows(whole, refs, f"{blocks} blocks I={I} whole")
+    for parts in (2, 3, 5, 8):
+        print(f"case {blocks} blocks I={I} parts {parts}", flush=True)
+        with tunables(ALPHA_MOE_GROUP_PIECES=parts):
+            got = run_op(P, 64, 64, 4, 2, via="c_abi")
+            assert_parity_rows(got, refs, f"{blocks} blocks I={I} parts {parts}")
+            with tunables(ALPHA_MOE_TILE_GPS=16):
+                assert torch.equal(got, run_op(P, 64, 64, 4, 2, via="c_abi"))
 
 
 @pytest.mark.parametrize("knobs", [(16, 32, 8, 5), (64, 64, 4, 3)])
@@ -634,10 +647,10 @@ def test_workspace_check_reports_an_expired_wait(c1):
     import alpha_moe
     P, ref = c1
     need = max(alpha_moe.c_abi.alpha_moe_workspace_bytes(P.shape.top_k, P.M, P.shape.K, P.shape.N, P.shape.E,
-                                                         P.align(bm)[0].numel(), bm) for bm in (16, 64))
+                                                         P.align(bm)[0].numel(), bm) for bm in (16, 64, 128))
     ws = torch.zeros(need, dtype=torch.uint8, device=DEV)
     stream = torch.cuda.current_stream().cuda_stream
-    families = ((2, (16, 32, 8, 5)), (5, (16, 32, 8, 5)), (3, (64, 64, 4, 3)), (4, (64, 32, 8, 2)))   # streaming, small, tile, wide
+    families = ((2, (16, 32, 8, 5)), (5, (16, 32, 8, 5)), (3, (64, 64, 4, 3)), (3, (128, 32, 8, 2)))   # streaming, small, group
     for path, knobs in families:
         with tunables(ALPHA_MOE_PATH=path):
             assert_parity(run_op(P, *knobs, via="c_abi", workspace=ws), ref, f"path {path} knobs {knobs}")
@@ -660,7 +673,7 @@ def test_workspace_check_reports_an_expired_wait(c1):
     assert alpha_moe.c_abi.alpha_moe_workspace_check(ws.data_ptr(), stream) == 0
 
 
-@pytest.mark.parametrize("path,knobs", [(2, (16, 32, 8, 5)), (5, (16, 32, 8, 5)), (3, (64, 64, 4, 3)), (4, (64, 32, 8, 2))])
+@pytest.mark.parametrize("path,knobs", [(2, (16, 32, 8, 5)), (5, (16, 32, 8, 5)), (3, (64, 64, 4, 3)), (3, (128, 32, 8, 2))])
 @pytest.mark.parametrize("epoch,stamps", [(-5, -5), (-5, 0), (2 ** 31 - 5, 0), (2 ** 31 - 5, -(2 ** 31) + 5)])
 def test_epoch_of_a_workspace_may_wrap(c1, path, knobs, epoch, stamps):
     """Four calls over the wrap of the launch epoch and over its change of sign.  Flags and slots hold the stamp of an earlier
@@ -1152,7 +1165,7 @@ def test_small_row_blocks_beyond_the_streaming_kernel(ds_weights, block_m):
 
 def test_prepacked_weights_give_the_same_bits(c1, ds_weights, q3_weights, decode_path):
     """fused_moe_w8a8_up_down_prepacked on prepack_weights(w, w2) against the operator on w, w2: bit for bit, streaming
-    and tile kernels, adding and storing, torch op and C ABI - on the CPU-sized case, the DeepSeek-V3 shard at M=256 and
+    and group kernels, adding and storing, torch op and C ABI - on the CPU-sized case, the DeepSeek-V3 shard at M=256 and
     the Zipf shard at M=200 (six slices)."""
     from alpha_moe_python.utils import prepack_weights
     P, ref = c1

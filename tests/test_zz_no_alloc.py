@@ -42,7 +42,7 @@ def test_static_scratch_entry_point_matches_the_workspace_entry_point():
         assert_parity(got, oracle_out(P, knobs[0]), f"static ds M={P.M}")
     Wc = make_weights(SHAPES["c1"], device=DEV, seed=0)
     mid = make_problem(Wc, 200, seed=33)
-    print("case static c1 M=200 tile kernel", flush=True)
+    print("case static c1 M=200 group kernel", flush=True)
     rc, got = run_static(mid, 64, 64, 4, 3)
     assert rc == 0 and torch.equal(got, run_op(mid, 64, 64, 4, 3, via="c_abi"))
     pre = torch.full((small.M, small.shape.K), 0.5, dtype=torch.bfloat16, device=DEV)
