@@ -51,7 +51,7 @@ Path choose_path(int top_k, int M, int K, int N, int E, int sorted_num, int bloc
     const int f = tunable(kTunPath, 0);
     if (f == 1) return kDirect;
     if (f == 2 && s_ok) return kStream;
-    const bool g_ok = group_supported(top_k, M, K, N, E, sorted_num, block_m);
+    const bool g_ok = group_supported(top_k, M, K, N, sorted_num, block_m, s_ok);
     if ((f == 3 || f == 4) && g_ok) return kGroup;   // (two kernels once)
     const bool small_ok = small_supported(top_k, M, K, N, block_m);
     if (small_ok && (f == 5 || (f == 0 && (!s_ok || small_pays(top_k, M, K, N, E))))) return kSmall;
@@ -114,10 +114,9 @@ extern "C" size_t alpha_moe_workspace_bytes(int top_k, int M, int K, int N, int 
     // both kernel families keep their bookkeeping out of each other's way: the streaming kernel's self-maintaining
     // prefix comes first, the direct kernel's accumulator (cleared on every call) after it
     const size_t direct = stream_prefix_bytes() + (size_t)M * (size_t)K * sizeof(float);
-    const size_t stream = stream_supported(top_k, M, K, N, num_experts, sorted_num, block_m)
-                              ? stream_workspace_bytes(top_k, M, K, N, num_experts, sorted_num, block_m)
-                              : 0;
-    const size_t group = group_supported(top_k, M, K, N, num_experts, sorted_num, block_m)
+    const bool streams = stream_supported(top_k, M, K, N, num_experts, sorted_num, block_m);
+    const size_t stream = streams ? stream_workspace_bytes(top_k, M, K, N, num_experts, sorted_num, block_m) : 0;
+    const size_t group = group_supported(top_k, M, K, N, sorted_num, block_m, streams)
                              ? group_workspace_bytes(top_k, M, K, N, num_experts, sorted_num, block_m)
                              : 0;
     const size_t small = small_supported(top_k, M, K, N, block_m) ? small_workspace_bytes(top_k, M, N) : 0;

@@ -319,7 +319,7 @@ hipError_t launch_stream(const MoeParams &p, int warp_n, int stages, void *works
 
 // Row blocks above 32 rows (prefill), smaller ones where the streaming kernel does not take the call: one item to a workgroup of four wavefronts - a row block x one slice of the intermediate, or x
 // a slab of output columns -, per-slot bf16 result rows added up by the reduce kernel.
-bool group_supported(int top_k, int M, int K, int N, int E, int sorted_num, int block_m);
+bool group_supported(int top_k, int M, int K, int N, int sorted_num, int block_m, bool streams);   // streams: stream_supported()
 size_t group_workspace_bytes(int top_k, int M, int K, int N, int E, int sorted_num, int block_m);
 hipError_t launch_group(const MoeParams &p, int stages, void *workspace, hipStream_t stream);
 // its variant, 64-column groups per DOWN item, column slabs, and the scales a DOWN item's table holds

@@ -752,10 +752,10 @@ static GroupPlan group_plan(int K, int N, int block_m, int stages)
 // more than 64 experts to a token) come here up to eight slices and 512 scales, beyond which the fallback kernel has them: its sums
 // are fp32 throughout, those of the rows here are not.  MI355X, DeepSeek shard, 16- and 32-row blocks, here / in the fallback
 // kernel: M = 4200 1.12 and 0.77 ms / 7.3 and 7.3 ms, M = 8192 2.00 and 1.35 / 14.2 and 14.1.
-bool group_supported(int top_k, int M, int K, int N, int E, int sorted_num, int block_m)
+bool group_supported(int top_k, int M, int K, int N, int sorted_num, int block_m, bool streams)
 {
     const int n_ib = N / 256;
-    if (block_m <= 32 && (n_ib > 8 || (K / 128) * n_ib > 512 || stream_supported(top_k, M, K, N, E, sorted_num, block_m))) return false;
+    if (block_m <= 32 && (streams || n_ib > 8 || (K / 128) * n_ib > 512)) return false;
     const int64_t n_mb = ((int64_t)sorted_num + block_m - 1) / block_m;
     return K <= 128 * kGMaxKb && (K / 128) * n_ib <= kGMaxExpertW2s && (int64_t)M * top_k <= kMaxSlots &&
            n_mb * n_ib <= kMaxUnits;
