@@ -825,8 +825,10 @@ hipError_t launch_group(const MoeParams &p, int stages, void *workspace, hipStre
     if (s.max_pieces > 8) s.max_pieces = 8;
     const unsigned grid = 8 * (chunk_rounds * kGChunk * (s.n_ib + s.n_cs) + s.round * (s.max_pieces - 1));
     const GroupFn fn = nt == 4 ? moe_group_kernel<4> : nt == 6 ? moe_group_kernel<6> : moe_group_kernel<8>;
-    hipLaunchKernelGGL(fn, dim3(grid), dim3(256), dyn_lds(nt), stream, s);
-    err = hipGetLastError();
+    // (Each launch's own status: hipGetLastError() also reports what other calls of the thread left behind, and to stop here, with the
+    // tickets drawn, would leave the workspace's queues empty for the calls that follow.)
+    void *args[] = {&s};
+    err = hipLaunchKernel(reinterpret_cast<const void *>(fn), dim3(grid), dim3(256), args, dyn_lds(nt), stream);
     if (err != hipSuccess) return err;
     RowsReduce r;
     r.p = p;

@@ -83,9 +83,10 @@ hipError_t launch_rows_reduce(const RowsReduce &r, hipStream_t stream)
     const int cols = r.y_is_f32 ? 1024 : 2048;   // of a workgroup
     const int chunks = (r.p.K + cols - 1) / cols;
     const dim3 grid((unsigned)(r.p.M * chunks));
-    if (r.y_is_f32) hipLaunchKernelGGL(moe_rows_reduce_kernel<float>, grid, dim3(256), 0, stream, r, chunks);
-    else hipLaunchKernelGGL(moe_rows_reduce_kernel<uint16_t>, grid, dim3(256), 0, stream, r, chunks);
-    return hipGetLastError();
+    typedef void (*Fn)(const RowsReduce, int);
+    const Fn fn = r.y_is_f32 ? moe_rows_reduce_kernel<float> : moe_rows_reduce_kernel<uint16_t>;
+    void *args[] = {const_cast<RowsReduce *>(&r), const_cast<int *>(&chunks)};
+    return hipLaunchKernel(reinterpret_cast<const void *>(fn), grid, dim3(256), args, 0, stream);   // (this launch's own status)
 }
 
 }  // namespace alpha_moe
