@@ -72,6 +72,19 @@ at::Tensor workspace_for(const at::Device &dev, hipStream_t stream, size_t bytes
     return slot.current;
 }
 
+// After a refused launch: what the call's other launches left in the control prefix is undefined, so the next call on the
+// stream gets a buffer of its own.
+void forget_workspace(const at::Device &dev, hipStream_t stream)
+{
+    std::lock_guard<std::mutex> lock(g_scratch_mu);
+    auto it = g_scratch.find({dev.index(), static_cast<void *>(stream)});
+    if (it == g_scratch.end()) return;
+    StreamScratch &slot = it->second;
+    if (slot.current.defined() && slot.current_seen_by_capture) slot.retired.push_back(slot.current);
+    slot.current = at::Tensor();
+    slot.current_seen_by_capture = false;
+}
+
 // scratch_buffers(like): [buffers alive, bytes of the current one, bytes kept for earlier graph captures] of
 // (like's device, the current stream) - for tests and memory accounting.
 std::vector<int64_t> scratch_buffers(const at::Tensor &like)
@@ -215,6 +228,7 @@ void run_fused_moe(const at::Tensor &x, const at::Tensor &x_scale, const at::Ten
             static_cast<int>(block_n), static_cast<int>(warp_n), static_cast<int>(stages),
             static_cast<float>(scaling_factor), ws.data_ptr(), static_cast<size_t>(ws.numel()),
             static_cast<void *>(stream)));
+    if (rc == ALPHA_MOE_ERR_LAUNCH) forget_workspace(dev, stream);
     TORCH_CHECK(rc == ALPHA_MOE_OK, "alpha_moe_fused_moe_w8a8_up_down failed: ", alpha_moe_status_string(rc));
 }
 
@@ -394,6 +408,7 @@ void fused_experts(at::Tensor &hidden, const at::Tensor &topk_ids, const at::Ten
         x, static_cast<int>(top_k), static_cast<int>(M), static_cast<int>(K), static_cast<int>(N), static_cast<int>(E),
         static_cast<int>(block_m), static_cast<int>(block_n), static_cast<int>(warp_n), static_cast<int>(stages),
         static_cast<float>(scaling_factor), ws.data_ptr(), static_cast<size_t>(ws.numel()), static_cast<void *>(stream));
+    if (rc == ALPHA_MOE_ERR_LAUNCH) forget_workspace(dev, stream);
     TORCH_CHECK(rc == ALPHA_MOE_OK, "alpha_moe_layer_call failed: ", alpha_moe_status_string(rc));
 }
 

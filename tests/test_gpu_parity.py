@@ -700,6 +700,30 @@ def test_an_error_of_another_call_does_not_spoil_the_workspace(c1, knobs, decode
     assert torch.equal(run_op(P2, *knobs, via="c_abi", store=True, workspace=ws), want)
 
 
+def test_a_refused_launch_costs_the_binding_its_scratch(c1, decode_path):
+    """A launch that reports an error (another call's: nothing is wrong with it) raises; the scratch buffer, whose control prefix the call may
+    have left half-way, is not used again."""
+    import alpha_moe
+    P, ref = c1
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        assert_parity(run_op(P, 16, 32, 8, 5), ref, "before")
+        kept = torch.ops.alpha_moe.scratch_buffers(P.x)
+        s_ids, e_ids, total = P.align(16)
+        out, W = torch.zeros((P.M, P.shape.K), dtype=torch.bfloat16, device=DEV), P.weights
+        stream.synchronize()
+        assert kept[0] == 1 and alpha_moe.c_abi.hipSetDevice(4096) != 0
+        try:
+            with pytest.raises(RuntimeError, match="launch"):
+                torch.ops.alpha_moe.fused_moe_w8a8_up_down(P.x, P.x_scale, W.w1, W.w1_scale, W.w2, W.w2_scale, s_ids, e_ids, total,
+                                                           P.topk_weights, out, P.shape.top_k, 16, 32, 8, 5, P.shape.scaling_factor)
+        finally:
+            alpha_moe.c_abi.hipGetLastError()
+        assert torch.ops.alpha_moe.scratch_buffers(P.x)[0] == 0
+        assert_parity(run_op(P, 16, 32, 8, 5), ref, "after")
+        assert torch.ops.alpha_moe.scratch_buffers(P.x) == kept
+
+
 @pytest.mark.parametrize("path,knobs", [(2, (16, 32, 8, 5)), (5, (16, 32, 8, 5)), (3, (64, 64, 4, 3)), (3, (128, 32, 8, 2))])
 @pytest.mark.parametrize("epoch,stamps", [(-5, -5), (-5, 0), (2 ** 31 - 5, 0), (2 ** 31 - 5, -(2 ** 31) + 5)])
 def test_epoch_of_a_workspace_may_wrap(c1, path, knobs, epoch, stamps):
